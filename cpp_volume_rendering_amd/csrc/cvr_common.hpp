@@ -78,13 +78,18 @@ __device__ __forceinline__ f3 norm3(f3 v) {
 }
 __device__ __forceinline__ f3 ld3(const float* p) { return mk3(p[0], p[1], p[2]); }
 
-// Camera ray of pixel (px, py), ray_marching_1p.comp:164-170.
+// Camera ray of pixel (px, py), ray_marching_1p.comp:164-170.  The fused operations are
+// spelled out so that every kernel marches the same ray bit for bit (the compiler would
+// choose which product of a sum to fuse by the code around it).
 __device__ __forceinline__ f3 camera_ray(const RayFrame& rf, int px, int py) {
-  float vx = ((float(px) + 0.5f) / float(rf.W)) * 2.0f - 1.0f;
-  float vy = ((float(py) + 0.5f) / float(rf.H)) * 2.0f - 1.0f;
-  float a = vx * rf.tanfov * rf.aspect, b = vy * rf.tanfov;
-  f3 d = ld3(rf.s) * a + ld3(rf.u) * b + ld3(rf.f);
-  return norm3(d);
+  const float vx = __builtin_fmaf((float(px) + 0.5f) / float(rf.W), 2.0f, -1.0f);
+  const float vy = __builtin_fmaf((float(py) + 0.5f) / float(rf.H), 2.0f, -1.0f);
+  const float a = vx * rf.tanfov * rf.aspect, b = vy * rf.tanfov;
+  const float bu[3] = {b * rf.u[0], b * rf.u[1], b * rf.u[2]};
+  const f3 d = mk3(__builtin_fmaf(rf.s[0], a, bu[0]) + rf.f[0], __builtin_fmaf(rf.s[1], a, bu[1]) + rf.f[1],
+                   __builtin_fmaf(rf.s[2], a, bu[2]) + rf.f[2]);
+  const float l2 = __builtin_fmaf(d.z, d.z, __builtin_fmaf(d.x, d.x, d.y * d.y));
+  return d * (1.0f / sqrtf(l2));
 }
 
 // Slab test against [-G/2, G/2], ray_bbox_intersection.comp:18-52.

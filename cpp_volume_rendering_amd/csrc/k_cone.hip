@@ -10,9 +10,11 @@
 // level whose Gaussian sigma matches the cone radius there (LINEAR_MIPMAP_LINEAR +
 // the border falloff of GetGaussianExtinction, :92-112).
 //
-// Per step the level index is wave-uniform, so the level geometry stays in SGPRs;
+// The march is queue_march's (cvr_queue.hpp): 256^3 at 1024^2 177 -> 90 ms, at 512^2
+// 162 -> 34 ms, at 128^2 146 -> 7.7 ms.  Per step the level index is wave-uniform, so the level geometry stays in SGPRs;
 // the step schedule is read with scalar loads from a small device table.
 #include "cvr_cone.hpp"
+#include "cvr_queue.hpp"
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -22,56 +24,26 @@ namespace cvr {
 template <typename T, int F>
 __global__ __launch_bounds__(256) void k_cone_render(RayFrame rf, VolGeom g, PyrGeom pg, const void* __restrict__ pyr,
                                                      ConeK K, const float4* __restrict__ tf, int ntf, float step,
-                                                     float et, float4* __restrict__ out,
+                                                     float et, int rays, float4* __restrict__ out,
                                                      unsigned long long* __restrict__ counters) {
   extern __shared__ float4 s_tf[];
+  __shared__ WaveQueue queue[4];
   for (int i = threadIdx.x; i < ntf; i += blockDim.x) s_tf[i] = tf[i];
   __syncthreads();
-  const int bid = xcd_remap(blockIdx.x, gridDim.x);
-  const int tiles_x = (rf.W + 15) >> 4;
-  int tx, ty;
-  super_tile(bid, tiles_x, (rf.H + 15) >> 4, 16, 16, tx, ty);
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int px = tx * 16 + (w & 1) * 8 + (lane & 7);
-  const int py = ty * 16 + (w >> 1) * 8 + (lane >> 3);
-  if (px >= rf.W || py >= rf.H) return;
-  const f3 dir = camera_ray(rf, px, py);
-  const f3 eye = ld3(rf.eye);
-  float tn, tf_;
-  float4 dst = make_float4(0.f, 0.f, 0.f, 0.f);
+  const int gw = xcd_remap(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), nw = gridDim.x * 4;
   unsigned int nsamp = 0, nshade = 0;
   const float ka = K.apply_occ ? K.ka : 0.f, kd = K.apply_sdw ? K.kd : 0.f;
   const float inv_k = 1.0f / (ka + kd);
-  if (ray_box(eye, dir, g.G, tn, tf_)) {
-    f3 k, up, right;
-    occ_frame(dir, k, up, right);
-    const f3 L = ld3(K.L);
-    const float D = fabsf(tf_ - tn);
-    const f3 tp = eye + dir * tn + mk3(0.5f * g.G[0], 0.5f * g.G[1], 0.5f * g.G[2]);
-    for (int j = 0; j < kMaxSamples; ++j) {
-      const float s = float(j) * step;
-      if (!(s < D)) break;
-      const float h = fminf(step, D - s);
-      const f3 p = tp + dir * (s + 0.5f * h);
-      float4 src = sample_tf(s_tf, ntf, sample_volume_oct<T>(g, p));
-      ++nsamp;
-      if (src.w > 0.0f) {
-        ++nshade;
-        const float Io = K.apply_occ ? ct_occlusion<F>(pyr, pg, K, p, k, up, right) : 0.f;
-        const float Is = K.apply_sdw ? cone_T<F>(pyr, pg, K.ss, K.n_steps, p, L) : 0.f;
-        const float m = inv_k * (Io * ka + Is * kd);
-        src.x *= m; src.y *= m; src.z *= m;
-        const float a = 1.0f - __expf(-src.w * h);
-        const float wgt = (1.0f - dst.w) * a;
-        dst.x += wgt * src.x;
-        dst.y += wgt * src.y;
-        dst.z += wgt * src.z;
-        dst.w += wgt;
-        if (dst.w > et) break;
-      }
-    }
-  }
-  out[size_t(py) * rf.W + px] = dst;
+  const f3 L = ld3(K.L);
+  const float spec[3] = {0.f, 0.f, 0.f};
+  queue_march<T>(rf, g, s_tf, ntf, step, et, gw, nw, rays, spec, queue[threadIdx.x >> 6], out, nsamp, nshade,
+                 [&](f3 p, f3 dir) {
+                   f3 k, up, right;
+                   occ_frame(dir, k, up, right);
+                   const float Io = K.apply_occ ? ct_occlusion<F>(pyr, pg, K, p, k, up, right) : 0.f;
+                   const float Is = K.apply_sdw ? cone_T<F>(pyr, pg, K.ss, K.n_steps, p, L) : 0.f;
+                   return Lit{inv_k * (Io * ka + Is * kd), 0.f};
+                 });
   if (counters) {
     atomicAdd(&counters[0], (unsigned long long)nsamp);
     atomicAdd(&counters[1], (unsigned long long)nshade);
@@ -266,15 +238,18 @@ int launch_cone(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* o
   ConeK K = cone_constants(c, P, L);
   VolGeom g = geom_of(c);
   const float step = P.step_size > 0 ? P.step_size : default_step(c);
-  const int tiles = ((rf.W + 15) / 16) * ((rf.H + 15) / 16);
   const size_t shm = size_t(c->tf_size) * sizeof(float4);
   if (shm > 64 * 1024) { set_error("cone renderer: transfer function larger than 4096 entries"); return -4; }
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   float4* o4 = reinterpret_cast<float4*>(out);
+  // one ray per wavefront: a batch of 64 samples takes 9 x 64 cone steps, so an unfilled
+  // last one weighs less than the evenness (1024^2: 90.2 ms, 90.7 with two rays, 92.3 with
+  // four, 100 with sixteen; 128^2: 7.7, 8.2 and 9.2)
+  const QueueShape qs = queue_shape(rf, 1, 1);
   with_types(c->dtype, c->pyr.fmt, [&](auto t, auto f) {
     using T = typename decltype(t)::type;
-    hipLaunchKernelGGL((k_cone_render<T, decltype(f)::value>), dim3(tiles), dim3(256), shm, st, rf, g, c->pyr,
-                       c->d_pyr_oct, K, c->d_tf_rgbt, c->tf_size, step, P.et_threshold, o4, cnt);
+    hipLaunchKernelGGL((k_cone_render<T, decltype(f)::value>), dim3(qs.blocks), dim3(256), shm, st, rf, g, c->pyr,
+                       c->d_pyr_oct, K, c->d_tf_rgbt, c->tf_size, step, P.et_threshold, qs.rays, o4, cnt);
   });
   CVR_HIP_CHECK(hipGetLastError());
   return 0;

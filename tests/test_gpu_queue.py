@@ -1,0 +1,49 @@
+"""Frames of the renderers that shade samples through a wavefront queue, at the sizes where
+it can go wrong: one pixel, one ray past a tile, rays of fewer and of several times 64
+samples, samples from several rays in one batch, and one or more rays per wavefront."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from cpp_volume_rendering_amd import native as N
+from cpp_volume_rendering_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-3
+
+# (volume side, width, height, alpha limit): 24 voxels give rays of at most 83 samples, 96
+# at a low opacity several hundred
+SIZES = [(24, 1, 1, 0.95), (24, 17, 3, 0.95), (24, 33, 31, 0.3), (96, 16, 16, 0.02), (96, 5, 18, 0.95)]
+
+
+def scene(tech, n, w, h, alpha_max, **params):
+    wl = W.cone_blobs(n=n, width=w, height=h, seed=31)
+    rgb, a = W.seeded_tf(131, 4, alpha_max=alpha_max)
+    r = N.Renderer(tech)
+    r.set_volume(wl.volume, wl.scale)
+    r.set_transfer_function(rgb, a)
+    p = r.params()
+    for k, v in params.items():
+        if k == "base_res":
+            p.base_res[:] = list(v)
+        else:
+            setattr(p, k, v)
+    r.set_params(p)
+    r.collect_stats()
+    img = r.render(wl.camera(), w, h, light=wl.light())
+    return wl, O.OTF(rgb, a), r, r.params(), img
+
+
+def check(img, ref, m):
+    s = O.compare(img, ref, m, TOL, 1)
+    print(s)
+    assert s["max_abs"] <= TOL, s
+    assert s["n_over_tol"] <= 0.005 * s["n_pixels"] + 1, s
+
+
+@pytest.mark.parametrize("n,w,h,alpha_max", SIZES)
+def test_cone(n, w, h, alpha_max):
+    wl, tf, r, p, img = scene(N.CONE_TRACE, n, w, h, alpha_max, n_steps=8)
+    pyr = O.OPyr.build(wl.volume, tf, nlev=6)
+    ref, m = O.render_cone(wl.volume, tf, pyr, O.cone_params(wl.grid, wl.light(), n_steps=8), wl.camera(), w, h)
+    check(img, ref, m)
