@@ -16,6 +16,10 @@ TOL = 2e-3
 SIZES = [(24, 1, 1, 0.95), (24, 17, 3, 0.95), (24, 33, 31, 0.3), (96, 16, 16, 0.02), (96, 5, 18, 0.95)]
 
 
+# frames of more than one ray per wavefront, the last of them past the image
+MANY = [(24, 97, 71, 0.95), (24, 160, 131, 0.3)]
+
+
 def scene(tech, n, w, h, alpha_max, **params):
     wl = W.cone_blobs(n=n, width=w, height=h, seed=31)
     rgb, a = W.seeded_tf(131, 4, alpha_max=alpha_max)
@@ -46,4 +50,12 @@ def test_cone(n, w, h, alpha_max):
     wl, tf, r, p, img = scene(N.CONE_TRACE, n, w, h, alpha_max, n_steps=8)
     pyr = O.OPyr.build(wl.volume, tf, nlev=6)
     ref, m = O.render_cone(wl.volume, tf, pyr, O.cone_params(wl.grid, wl.light(), n_steps=8), wl.camera(), w, h)
+    check(img, ref, m)
+
+
+@pytest.mark.parametrize("n,w,h,alpha_max", SIZES + MANY)
+def test_dos(n, w, h, alpha_max):
+    wl, tf, r, p, img = scene(N.DOS, n, w, h, alpha_max, apply_shadow=1, shadow_type=2, base_res=(24, 24, 24))
+    pyr = O.OPyr.build(wl.volume, tf, base=(24, 24, 24))
+    ref, m = O.render_dos(wl.volume, tf, pyr, O.dos_params(p, wl.grid, wl.light()), wl.camera(), w, h)
     check(img, ref, m)
