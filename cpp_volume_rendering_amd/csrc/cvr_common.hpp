@@ -202,6 +202,28 @@ __device__ __forceinline__ float volume_oct_lerp(const VolGeom& g, typename VolO
   return quad_lerp(a, b, fx, fy, fz) * (sizeof(T) == 1 ? (1.0f / 255.0f) : (1.0f / 65535.0f));
 }
 
+// The same with the block's weights kept between the load and the lerp.
+template <typename T> struct VolTap {
+  typename VolOct<T>::type rec;
+  float fx, fy, fz;
+};
+template <typename T>
+__device__ __forceinline__ VolTap<T> volume_tap_load(const VolGeom& g, f3 p) {
+  VolTap<T> t;
+  int x0, y0, z0;
+  quad_axis_f(p.x * g.tex_mul[0] - 0.5f, g.vmax[0], x0, t.fx);
+  quad_axis_f(p.y * g.tex_mul[1] - 0.5f, g.vmax[1], y0, t.fy);
+  quad_axis_f(p.z * g.tex_mul[2] - 0.5f, g.vmax[2], z0, t.fz);
+  t.rec = static_cast<const typename VolOct<T>::type*>(g.oct)[brick_index(x0, y0, z0, g.nbx, g.nby)];
+  return t;
+}
+template <typename T>
+__device__ __forceinline__ float volume_tap_lerp(const VolTap<T>& t) {
+  float4 a, b;
+  VolOct<T>::f(t.rec, a, b);
+  return quad_lerp(a, b, t.fx, t.fy, t.fz) * (sizeof(T) == 1 ? (1.0f / 255.0f) : (1.0f / 65535.0f));
+}
+
 // Trilinear sample of the raw volume at world-in-box position p (texture space
 // [0, G]); returns the normalised density v/255 or v/65535
 // (structuredgridvolume.cpp:121-151 + GL_LINEAR, utils.cpp:8-9).

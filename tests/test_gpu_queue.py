@@ -59,3 +59,11 @@ def test_dos(n, w, h, alpha_max):
     pyr = O.OPyr.build(wl.volume, tf, base=(24, 24, 24))
     ref, m = O.render_dos(wl.volume, tf, pyr, O.dos_params(p, wl.grid, wl.light()), wl.camera(), w, h)
     check(img, ref, m)
+
+
+@pytest.mark.parametrize("n,w,h,alpha_max", SIZES)
+@pytest.mark.parametrize("shadow_type", [0, 2])
+def test_ground_truth(n, w, h, alpha_max, shadow_type):
+    wl, tf, r, p, img = scene(N.CONE_GT, n, w, h, alpha_max, occ_rays=3, sdw_rays=2, shadow_type=shadow_type)
+    ref, m = O.render_gt(wl.volume, tf, O.gt_params(p, wl.grid, wl.light()), wl.camera(), w, h)
+    check(img, ref, m)
