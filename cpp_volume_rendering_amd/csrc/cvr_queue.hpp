@@ -89,18 +89,18 @@ __device__ __forceinline__ bool tiled_pixel(const RayFrame& rf, int i, int& px, 
 }
 inline int tiled_pixels(const RayFrame& rf) { return ((rf.W + 15) / 16) * ((rf.H + 15) / 16) * 256; }
 
-// Rays per wavefront and workgroups of four wavefronts of a frame: at most `most` rays (a
+// Rays per wavefront and workgroups (of `waves` wavefronts) of a frame: at most `most` rays (a
 // power of two up to 64) while that leaves `min_waves` wavefronts.  More rays leave fewer
 // part-filled last batches, fewer rays more wavefronts to even out; where the two lines lie
 // is each renderer's, measured over frame sizes.
 struct QueueShape {
   int rays, blocks;
 };
-inline QueueShape queue_shape(const RayFrame& rf, int most, int min_waves) {
+inline QueueShape queue_shape(const RayFrame& rf, int most, int min_waves, int waves = 4) {
   const int n = tiled_pixels(rf);
   int rays = 1;
   while (rays < most && n / (rays * 2) >= min_waves) rays *= 2;
-  return QueueShape{rays, (n / rays + 3) / 4};
+  return QueueShape{rays, (n / rays + waves - 1) / waves};
 }
 
 // Marches rays gw, gw + nw, gw + 2 nw, ... (`rays` of them, at most 64) of the frame and

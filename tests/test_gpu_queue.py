@@ -67,3 +67,29 @@ def test_ground_truth(n, w, h, alpha_max, shadow_type):
     wl, tf, r, p, img = scene(N.CONE_GT, n, w, h, alpha_max, occ_rays=3, sdw_rays=2, shadow_type=shadow_type)
     ref, m = O.render_gt(wl.volume, tf, O.gt_params(p, wl.grid, wl.light()), wl.camera(), w, h)
     check(img, ref, m)
+
+
+@pytest.mark.parametrize("n,w,h,alpha_max", SIZES + MANY)
+@pytest.mark.parametrize("shadow_type", [0, 1])
+def test_ebs(n, w, h, alpha_max, shadow_type):
+    wl, tf, r, p, img = scene(N.EBS, n, w, h, alpha_max, shadow_type=shadow_type)
+    prm = O.ebs_params(p, wl.light())
+    prm.sdw_max_dist = np.float32(0.75) * np.float32(np.linalg.norm(wl.grid))
+    ref, m = O.render_ebs(wl.volume, tf, O.sat(wl.volume, tf), prm, wl.camera(), w, h)
+    check(img, ref, m)
+
+
+def test_ebs_tables_that_leave_room_for_one_queue():
+    """A 4096-entry transfer function and a shadow chain of 2700 boxes: 146 KiB of LDS beside
+    a single wavefront's queue."""
+    wl = W.cone_blobs(n=24, width=33, height=31, seed=31)
+    rgb, a = W.seeded_tf(131, 4, max_density=4095)
+    r = N.Renderer(N.EBS)
+    r.set_volume(wl.volume, wl.scale)
+    r.set_transfer_function(rgb, a, max_density=4095)
+    # a sample's chain stops at the volume's edge, far before its table does
+    p = r.set_params(shadow_type=1, sdw_max_dist=7300.0)
+    img = r.render(wl.camera(), 33, 31, light=wl.light())
+    tf = O.OTF(rgb, a, max_density=4095)
+    ref, m = O.render_ebs(wl.volume, tf, O.sat(wl.volume, tf), O.ebs_params(p, wl.light()), wl.camera(), 33, 31)
+    check(img, ref, m)
