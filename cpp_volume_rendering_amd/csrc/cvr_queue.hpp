@@ -45,28 +45,28 @@ struct Lit {
 };
 
 constexpr int kQueueCap = 128;  // a step adds at most 64 to fewer than 64 waiting
-struct WaveQueue {
+// kRays: the most rays a wavefront takes (LDS: 4 KiB and 48 bytes a ray).
+template <int kRays> struct WaveQueue {
   float4 a[kQueueCap];  // position, compositing weight
   float4 b[kQueueCap];  // weight * rgb, ray (bits)
-  float4 dir[64];       // camera-ray direction of each of the wavefront's rays
-  float acc[64][4];     // and its accumulated colour
+  float4 tp[kRays];     // each of the wavefront's rays: entry point (texture space), length
+  float4 dir[kRays];    // direction
+  float4 acc[kRays];    // accumulated colour, opacity
 };
 
-__device__ __forceinline__ float lane_value(float v, int lane) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
-}
-// Lane k - 1's value; `first` in lane 0.
-__device__ __forceinline__ float left_lane(float v, float first) {
+// Lane k - 1's value within each group of kSub lanes; `first` in the group's first lane.
+template <int kSub> __device__ __forceinline__ float left_lane(float v, float first) {
+  constexpr int ctrl = kSub == 64 ? 0x138 : 0x111;  // wave_shr:1, row_shr:1
   return __int_as_float(
-      __builtin_amdgcn_update_dpp(__float_as_int(first), __float_as_int(v), 0x138 /* wave_shr:1 */, 0xf, 0xf, false));
+      __builtin_amdgcn_update_dpp(__float_as_int(first), __float_as_int(v), ctrl, 0xf, 0xf, false));
 }
 // Opacity after each lane's sample: w_k = w_(k-1) + (1 - w_(k-1)) alpha_k, w_(-1) = w.
-// Every round makes one more lane final; three instructions each.
-__device__ __forceinline__ float opacity_scan(float alpha, float w) {
+// Every round makes one more lane of the group final; three instructions each.
+template <int kSub> __device__ __forceinline__ float opacity_scan(float alpha, float w) {
   float v = w;
 #pragma unroll
-  for (int k = 0; k < 64; ++k) {
-    const float b = left_lane(v, w);
+  for (int k = 0; k < kSub; ++k) {
+    const float b = left_lane<kSub>(v, w);
     v = __builtin_fmaf(1.0f - b, alpha, b);
   }
   return v;
@@ -103,110 +103,155 @@ inline QueueShape queue_shape(const RayFrame& rf, int most, int min_waves, int w
   return QueueShape{rays, (n / rays + waves - 1) / waves};
 }
 
-// Marches rays gw, gw + nw, gw + 2 nw, ... (`rays` of them, at most 64) of the frame and
-// writes their pixels; gw: this wavefront's number, nw: all wavefronts.  shade(p, dir) lights
-// one sample (in texture space) for each active lane; spec: specular colour of Lit::s.
-template <typename T, class Shade>
+__device__ __forceinline__ float lane_value(float v, int lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
+}
+// A value all 64 lanes share, in a scalar register; a group's value as it is.
+template <int kSub> __device__ __forceinline__ float group_uniform(float v) {
+  return kSub == 64 ? __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))) : v;
+}
+
+// The pixels of a frame's wavefronts: ray k of wavefront gw of nw, kGroups neighbouring rays
+// side by side and the groups far apart.
+template <int kSub> struct FramePixels {
+  const RayFrame& rf;
+  int gw, nw;
+  __device__ __forceinline__ bool operator()(int k, int& px, int& py) const {
+    constexpr int kGroups = 64 / kSub;
+    return tiled_pixel(rf, (gw + k / kGroups * nw) * kGroups + k % kGroups, px, py);
+  }
+};
+
+// Marches `rays` rays (at most kRays <= 64), ray k that of pixel pix(k, px, py) (false: no pixel), and
+// writes their pixels: 64 / kSub rays at a time, kSub samples of each per step.
+// shade(on, p, dir) lights one sample (in texture space) per lane; kWhole: all 64 lanes call
+// it together, `on` says which have a sample; otherwise only those with one.  spec:
+// specular colour of Lit::s.
+template <typename T, int kSub, bool kWhole, int kRays, class Pix, class Shade>
 __device__ __forceinline__ void queue_march(const RayFrame& rf, const VolGeom& g, const float4* s_tf, int ntf,
-                                            float step, float et, int gw, int nw, int rays, const float* spec,
-                                            WaveQueue& Q, float4* __restrict__ out, unsigned int& nsamp,
-                                            unsigned int& nshade, Shade&& shade) {
+                                            float step, float et, int rays, Pix&& pix, const float* spec,
+                                            WaveQueue<kRays>& Q, float4* __restrict__ out, unsigned int& nsamp, unsigned int& nshade,
+                                            Shade&& shade) {
   typedef typename VolOct<T>::type RT;
-  const int lane = threadIdx.x & 63;
-  // lane r sets up the wavefront's ray r
+  static_assert(kSub == 64 || kSub == 16, "groups are wavefronts or DPP rows");
+  constexpr uint64_t kGroupMask = kSub == 64 ? ~0ull : (1ull << (kSub & 63)) - 1ull;
+  const int lane = threadIdx.x & 63, sub = lane % kSub, base = lane - sub;
+  const uint64_t below = (1ull << lane) - 1ull, below_group = (1ull << base) - 1ull;
+  // lane k sets up ray k; the rays that hit the box are listed in order
   int px = 0, py = 0;
-  const bool inside = lane < rays && tiled_pixel(rf, gw + lane * nw, px, py);
-  float D_r = 0.f, w_r = 0.f;
-  f3 tp_r = mk3(0.f, 0.f, 0.f), dir_r = tp_r;
+  const bool inside = lane < rays && pix(lane, px, py);
   bool hit = false;
+  float4 tp_k = make_float4(0.f, 0.f, 0.f, 0.f), dir_k = tp_k;
   if (inside) {
-    const f3 eye = ld3(rf.eye);
-    dir_r = camera_ray(rf, px, py);
+    const f3 eye = ld3(rf.eye), d = camera_ray(rf, px, py);
     float tn, tf_;
-    hit = ray_box(eye, dir_r, g.G, tn, tf_);
-    D_r = fabsf(tf_ - tn);
-    tp_r = mk3(__builtin_fmaf(dir_r.x, tn, eye.x), __builtin_fmaf(dir_r.y, tn, eye.y),
-               __builtin_fmaf(dir_r.z, tn, eye.z));
-    tp_r = tp_r + mk3(0.5f * g.G[0], 0.5f * g.G[1], 0.5f * g.G[2]);
-    Q.dir[lane] = make_float4(dir_r.x, dir_r.y, dir_r.z, 0.f);
-    Q.acc[lane][0] = Q.acc[lane][1] = Q.acc[lane][2] = 0.f;
+    hit = ray_box(eye, d, g.G, tn, tf_);
+    f3 t = mk3(__builtin_fmaf(d.x, tn, eye.x), __builtin_fmaf(d.y, tn, eye.y), __builtin_fmaf(d.z, tn, eye.z));
+    t = t + mk3(0.5f * g.G[0], 0.5f * g.G[1], 0.5f * g.G[2]);
+    tp_k = make_float4(t.x, t.y, t.z, fabsf(tf_ - tn));
+    dir_k = make_float4(d.x, d.y, d.z, 0.f);
+  }
+  const uint64_t hits = __ballot(hit);
+  const int nhit = __popcll(hits), slot = __popcll(hits & below);
+  if (hit) {
+    Q.tp[slot] = tp_k;
+    Q.dir[slot] = dir_k;
+    Q.acc[slot] = make_float4(0.f, 0.f, 0.f, 0.f);
   }
   wave_lds_sync();
-  uint64_t left = __ballot(hit);  // rays not begun
-  int ray = -1, jb = 0, head = 0, count = 0;
-  float w = 0.f, D = 0.f;
-  f3 tp = tp_r, dir = dir_r;
+  f3 tp = mk3(0.f, 0.f, 0.f), dir = tp;
+  float D = 0.f;
+  int ray = -1, jb = 0;                  // the group's ray and next sample
+  int next = 0, head = 0, count = 0;     // next ray, queue: the same in every lane
+  float w = 0.f;
   RT rec = {};
-  for (;;) {
-    while (count < 64) {
-      if (ray < 0) {
-        if (!left) break;
-        ray = __builtin_ctzll(left);
-        left &= left - 1;
-        D = lane_value(D_r, ray);
-        tp = mk3(lane_value(tp_r.x, ray), lane_value(tp_r.y, ray), lane_value(tp_r.z, ray));
-        dir = mk3(lane_value(dir_r.x, ray), lane_value(dir_r.y, ray), lane_value(dir_r.z, ray));
+  // a new ray for the groups without one, and the blocks of every group's next samples: in
+  // flight under the queue and the shading (past a ray's end the position is finite and its
+  // clamped block in bounds)
+  auto advance = [&]() {
+    const uint64_t need = __ballot(ray < 0 && sub == 0);
+    if (need && next < nhit) {
+      const int mine = next + __popcll(need & below_group);
+      if (ray < 0 && mine < nhit) {
+        ray = mine;
+        const float4 t = Q.tp[mine], d = Q.dir[mine];
+        tp = mk3(group_uniform<kSub>(t.x), group_uniform<kSub>(t.y), group_uniform<kSub>(t.z));
+        dir = mk3(group_uniform<kSub>(d.x), group_uniform<kSub>(d.y), group_uniform<kSub>(d.z));
+        D = group_uniform<kSub>(t.w);
         jb = 0;
         w = 0.f;
-        rec = volume_oct_load<T>(g, ray_sample_pos(ray_sample(lane, step, D), tp, dir));
       }
-      const RaySample r = ray_sample(jb + lane, step, D);
-      const f3 p = ray_sample_pos(r, tp, dir);
-      const float4 src = sample_tf(s_tf, ntf, volume_oct_lerp<T>(g, rec, p));
-      // the next step's block, in flight under the compositing and the shading (past the
-      // ray's end the position is finite and its clamped block in bounds)
-      rec = volume_oct_load<T>(g, ray_sample_pos(ray_sample(jb + 64 + lane, step, D), tp, dir));
-      const uint64_t valid = __ballot(r.s < D && jb + lane < kMaxSamples);
-      const bool opaque = ((valid >> lane) & 1) && src.w > 0.0f;
-      uint64_t taken = valid;  // the samples the ray comes to
-      uint64_t m = __ballot(opaque);
-      if (m) {
-        const float alpha = opaque ? 1.0f - __expf(-src.w * r.h) : 0.f;
-        const float wa = opacity_scan(alpha, w);
-        const float mine = (1.0f - left_lane(wa, w)) * alpha;
-        const uint64_t over = __ballot(wa > et);
-        w = lane_value(wa, 63);
-        if (over) {
-          const int k = __builtin_ctzll(over);  // the ray ends with sample k
-          taken &= (2ull << k) - 1ull;
-          m &= (2ull << k) - 1ull;
-          w = lane_value(wa, k);
-          jb = kMaxSamples;
+      next = min(nhit, next + __popcll(need));
+    }
+    if (ray >= 0) rec = volume_oct_load<T>(g, ray_sample_pos(ray_sample(jb + sub, step, D), tp, dir));
+  };
+  advance();
+  for (;;) {
+    while (count < 64 && __any(ray >= 0)) {
+      f3 p = tp;
+      float4 src = make_float4(0.f, 0.f, 0.f, 0.f);
+      float mine = 0.f;
+      bool emit = false;
+      const int emit_ray = ray;
+      if (ray >= 0) {
+        const RaySample r = ray_sample(jb + sub, step, D);
+        p = ray_sample_pos(r, tp, dir);
+        src = sample_tf(s_tf, ntf, volume_oct_lerp<T>(g, rec, p));
+        const bool valid = r.s < D && jb + sub < kMaxSamples;
+        const bool opaque = valid && src.w > 0.0f;
+        bool taken = valid;  // the ray comes to this sample
+        bool ended = !((__ballot(valid) >> (base + kSub - 1)) & 1);
+        if (__any(opaque)) {
+          const float alpha = opaque ? 1.0f - __expf(-src.w * r.h) : 0.f;
+          const float wa = opacity_scan<kSub>(alpha, w);
+          mine = (1.0f - left_lane<kSub>(wa, w)) * alpha;
+          const uint64_t over = (__ballot(wa > et) >> base) & kGroupMask;
+          const int last = over ? __builtin_ctzll(over) : kSub - 1;  // over: the ray ends with that sample
+          w = kSub == 64 ? lane_value(wa, last) : __shfl(wa, base + last);
+          taken = valid && sub <= last;
+          ended = ended || over != 0;
         }
-        if ((m >> lane) & 1) {
-          const int i = (head + count + __popcll(m & ((1ull << lane) - 1ull))) & (kQueueCap - 1);
-          Q.a[i] = make_float4(p.x, p.y, p.z, mine);
-          Q.b[i] = make_float4(mine * src.x, mine * src.y, mine * src.z, __int_as_float(ray));
+        emit = opaque && taken;
+        nsamp += taken;
+        nshade += emit;
+        jb += kSub;
+        if (ended || jb >= kMaxSamples) {
+          if (sub == 0) Q.acc[ray].w = w;
+          ray = -1;
         }
-        count += __popcll(m);
       }
-      nsamp += (taken >> lane) & 1;
-      nshade += (m >> lane) & 1;
-      jb += 64;
-      if (valid != ~0ull || jb >= kMaxSamples) {
-        if (lane == ray) w_r = w;
-        ray = -1;
+      const uint64_t m = __ballot(emit);
+      if (emit) {
+        const int i = (head + count + __popcll(m & below)) & (kQueueCap - 1);
+        Q.a[i] = make_float4(p.x, p.y, p.z, mine);
+        Q.b[i] = make_float4(mine * src.x, mine * src.y, mine * src.z, __int_as_float(emit_ray));
       }
+      count += __popcll(m);
+      advance();
     }
     if (count == 0) break;
     wave_lds_sync();
     const int n = min(count, 64);
-    if (lane < n) {
-      const int i = (head + lane) & (kQueueCap - 1);
+    const bool on = lane < n;
+    if (kWhole || on) {
+      const int i = (head + (on ? lane : 0)) & (kQueueCap - 1);
       const float4 a = Q.a[i], b = Q.b[i];
       const int r = __float_as_int(b.w);
       const float4 d = Q.dir[r];
-      const Lit l = shade(mk3(a.x, a.y, a.z), mk3(d.x, d.y, d.z));
-      const float ws = a.w * l.s;
-      atomicAdd(&Q.acc[r][0], __builtin_fmaf(b.x, l.m, spec[0] * ws));
-      atomicAdd(&Q.acc[r][1], __builtin_fmaf(b.y, l.m, spec[1] * ws));
-      atomicAdd(&Q.acc[r][2], __builtin_fmaf(b.z, l.m, spec[2] * ws));
+      const Lit l = shade(on, mk3(a.x, a.y, a.z), mk3(d.x, d.y, d.z));
+      if (on) {
+        const float ws = a.w * l.s;
+        atomicAdd(&Q.acc[r].x, __builtin_fmaf(b.x, l.m, spec[0] * ws));
+        atomicAdd(&Q.acc[r].y, __builtin_fmaf(b.y, l.m, spec[1] * ws));
+        atomicAdd(&Q.acc[r].z, __builtin_fmaf(b.z, l.m, spec[2] * ws));
+      }
     }
     head = (head + n) & (kQueueCap - 1);
     count -= n;
     wave_lds_sync();
   }
-  if (inside) out[size_t(py) * rf.W + px] = make_float4(Q.acc[lane][0], Q.acc[lane][1], Q.acc[lane][2], w_r);
+  wave_lds_sync();
+  if (inside) out[size_t(py) * rf.W + px] = hit ? Q.acc[slot] : make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
 }  // namespace cvr

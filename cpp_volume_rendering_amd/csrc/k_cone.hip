@@ -10,8 +10,8 @@
 // level whose Gaussian sigma matches the cone radius there (LINEAR_MIPMAP_LINEAR +
 // the border falloff of GetGaussianExtinction, :92-112).
 //
-// The march is queue_march's (cvr_queue.hpp): 256^3 at 1024^2 177 -> 90 ms, at 512^2
-// 162 -> 34 ms, at 128^2 146 -> 7.7 ms.  Per step the level index is wave-uniform, so the level geometry stays in SGPRs;
+// The march is queue_march's (cvr_queue.hpp): 256^3 at 1024^2 177 -> 72 ms, at
+// 200 x 150 of a 100 x 90 x 80 volume 43 -> 1.4 ms.  Per step the level index is wave-uniform, so the level geometry stays in SGPRs;
 // the step schedule is read with scalar loads from a small device table.
 #include "cvr_cone.hpp"
 #include "cvr_queue.hpp"
@@ -21,13 +21,16 @@
 
 namespace cvr {
 
+// One ray per wavefront: a batch of 64 samples takes 9 x 64 cone steps, so an unfilled last
+// one weighs less than the evenness (128^2: 7.7 ms, 8.2 with two rays, 9.2 with four).
+constexpr int kRays = 1;
 template <typename T, int F>
 __global__ __launch_bounds__(256) void k_cone_render(RayFrame rf, VolGeom g, PyrGeom pg, const void* __restrict__ pyr,
                                                      ConeK K, const float4* __restrict__ tf, int ntf, float step,
                                                      float et, int rays, float4* __restrict__ out,
                                                      unsigned long long* __restrict__ counters) {
   extern __shared__ float4 s_tf[];
-  __shared__ WaveQueue queue[4];
+  __shared__ WaveQueue<kRays> queue[4];
   for (int i = threadIdx.x; i < ntf; i += blockDim.x) s_tf[i] = tf[i];
   __syncthreads();
   const int gw = xcd_remap(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), nw = gridDim.x * 4;
@@ -36,8 +39,8 @@ __global__ __launch_bounds__(256) void k_cone_render(RayFrame rf, VolGeom g, Pyr
   const float inv_k = 1.0f / (ka + kd);
   const f3 L = ld3(K.L);
   const float spec[3] = {0.f, 0.f, 0.f};
-  queue_march<T>(rf, g, s_tf, ntf, step, et, gw, nw, rays, spec, queue[threadIdx.x >> 6], out, nsamp, nshade,
-                 [&](f3 p, f3 dir) {
+  queue_march<T, 64, false>(rf, g, s_tf, ntf, step, et, rays, FramePixels<64>{rf, gw, nw}, spec, queue[threadIdx.x >> 6], out, nsamp, nshade,
+                 [&](bool, f3 p, f3 dir) {
                    f3 k, up, right;
                    occ_frame(dir, k, up, right);
                    const float Io = K.apply_occ ? ct_occlusion<F>(pyr, pg, K, p, k, up, right) : 0.f;
@@ -242,10 +245,7 @@ int launch_cone(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* o
   if (shm > 64 * 1024) { set_error("cone renderer: transfer function larger than 4096 entries"); return -4; }
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   float4* o4 = reinterpret_cast<float4*>(out);
-  // one ray per wavefront: a batch of 64 samples takes 9 x 64 cone steps, so an unfilled
-  // last one weighs less than the evenness (1024^2: 90.2 ms, 90.7 with two rays, 92.3 with
-  // four, 100 with sixteen; 128^2: 7.7, 8.2 and 9.2)
-  const QueueShape qs = queue_shape(rf, 1, 1);
+  const QueueShape qs = queue_shape(rf, kRays, 1);
   with_types(c->dtype, c->pyr.fmt, [&](auto t, auto f) {
     using T = typename decltype(t)::type;
     hipLaunchKernelGGL((k_cone_render<T, decltype(f)::value>), dim3(qs.blocks), dim3(256), shm, st, rf, g, c->pyr,

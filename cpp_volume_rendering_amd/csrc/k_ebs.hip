@@ -387,6 +387,9 @@ __device__ __forceinline__ void ebs_load_rows(const ShadowRow* __restrict__ rows
   __syncthreads();
 }
 
+// Up to 64 rays per wavefront while every SIMD has one (1024^2 47 ms with one ray, 32 with 16,
+// 30.8 with 64; 200 x 150 0.69, 0.52 with 16, 0.48 with 32 (1040 wavefronts), 0.61 with 64).
+constexpr int kRays = 64;
 // The march is queue_march's (cvr_queue.hpp).  One wavefront per SIMD: the box streams keep
 // four corner records in flight per lane, which with the FP64 interpolation takes more than
 // the 256 architectural VGPRs; at one wavefront per SIMD the excess lives in AGPRs instead of
@@ -401,7 +404,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
            float4* __restrict__ out, unsigned long long* __restrict__ counters) {
   extern __shared__ float4 smem[];
   const int waves = blockDim.x >> 6;
-  WaveQueue* queue = reinterpret_cast<WaveQueue*>(smem);
+  WaveQueue<kRays>* queue = reinterpret_cast<WaveQueue<kRays>*>(smem);
   float4* s_tf = reinterpret_cast<float4*>(queue + waves);
   ShadowRow* s_rows = reinterpret_cast<ShadowRow*>(s_tf + ntf);
   for (int i = threadIdx.x; i < ntf; i += blockDim.x) s_tf[i] = tf[i];
@@ -412,8 +415,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   unsigned int nsamp = 0, nshade = 0, nbox = 0;
   const float ka = k.apply_occ ? k.ka : 0.f, kd = k.apply_sdw ? k.kd : 0.f;
   const float inv_k = 1.0f / (ka + kd);
-  queue_march<T>(rf, k.g, s_tf, ntf, step, et, gw, nw, rays, ph.spec, queue[threadIdx.x >> 6], out, nsamp, nshade,
-                 [&](f3 p, f3) {
+  queue_march<T, 64, false>(rf, k.g, s_tf, ntf, step, et, rays, FramePixels<64>{rf, gw, nw}, ph.spec, queue[threadIdx.x >> 6], out, nsamp, nshade,
+                 [&](bool, f3 p, f3) {
                    float Io = 0.f, Is = 0.f;
                    if (k.apply_occ) {
                      Io = ebs_ao<L>(sat, k, p);
@@ -589,11 +592,9 @@ int launch_ebs(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* ou
   }
   // four wavefronts per workgroup, fewer where the tables leave no room for their queues
   int waves = 4;
-  while (waves > 1 && tables + size_t(waves) * sizeof(WaveQueue) > 160 * 1024) waves /= 2;
-  const size_t shm = tables + size_t(waves) * sizeof(WaveQueue);
-  // up to 64 rays per wavefront while every SIMD has one (1024^2 47 ms with one ray, 32 with 16,
-  // 30.8 with 64; 200 x 150 0.69, 0.52 with 16, 0.48 with 32 (1040 wavefronts), 0.61 with 64)
-  const QueueShape qs = queue_shape(rf, 64, 1024, waves);
+  while (waves > 1 && tables + size_t(waves) * sizeof(WaveQueue<kRays>) > 160 * 1024) waves /= 2;
+  const size_t shm = tables + size_t(waves) * sizeof(WaveQueue<kRays>);
+  const QueueShape qs = queue_shape(rf, kRays, 1024, waves);
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   const void* sat = P.sat_layout == 1 ? static_cast<const void*>(c->d_sat) : c->d_sat_oct;
   const ShadowRow* rows = static_cast<const ShadowRow*>(c->d_ebs_rows);

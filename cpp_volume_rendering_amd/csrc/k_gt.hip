@@ -90,6 +90,9 @@ __device__ __forceinline__ float gt_cone(const VolGeom& g, const float2* s_ext, 
   return S / W;
 }
 
+// One ray per wavefront: a batch is tens to thousands of light-ray steps (256^2 with 16 + 4
+// rays 8.9 ms, 9.3 with two).
+constexpr int kRays = 1;
 // The march is queue_march's (cvr_queue.hpp).  128^3 at 256^2 with 16 + 4 rays per sample:
 // 313 -> 8.9 ms (one dependent read per light-ray step at one wavefront per SIMD before).
 template <typename T>
@@ -97,7 +100,7 @@ __global__ __launch_bounds__(256) void k_gt_render(RayFrame rf, VolGeom g, GtK K
                                                    int ntf, float step, float et, int rays, float4* __restrict__ out,
                                                    unsigned long long* __restrict__ counters) {
   extern __shared__ float4 s_tf[];
-  __shared__ WaveQueue queue[4];
+  __shared__ WaveQueue<kRays> queue[4];
   float2* s_ext = reinterpret_cast<float2*>(s_tf + ntf);
   for (int i = threadIdx.x; i < ntf; i += blockDim.x) s_tf[i] = tf[i];
   for (int i = threadIdx.x; i <= ntf; i += blockDim.x) s_ext[i] = make_float2(tf[max(i - 1, 0)].w, tf[min(i, ntf - 1)].w);
@@ -108,8 +111,8 @@ __global__ __launch_bounds__(256) void k_gt_render(RayFrame rf, VolGeom g, GtK K
   const float inv_k = 1.0f / (ka + kd);
   const f3 half = mk3(0.5f * g.G[0], 0.5f * g.G[1], 0.5f * g.G[2]);
   const float spec[3] = {0.f, 0.f, 0.f};
-  queue_march<T>(rf, g, s_tf, ntf, step, et, gw, nw, rays, spec, queue[threadIdx.x >> 6], out, nsamp, nshade,
-                 [&](f3 p, f3 dir) {
+  queue_march<T, 64, false>(rf, g, s_tf, ntf, step, et, rays, FramePixels<64>{rf, gw, nw}, spec, queue[threadIdx.x >> 6], out, nsamp, nshade,
+                 [&](bool, f3 p, f3 dir) {
                    float Io = 0.f, Is = 0.f;
                    if (K.apply_occ) {
                      const f3 right = norm3(cross3(dir, mk3(0.f, 1.f, 0.f)));
@@ -231,9 +234,7 @@ int launch_gt(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out
     return CVR_ERR_UNSUPPORTED;
   }
   const size_t shm = size_t(c->tf_size) * sizeof(float4) + size_t(c->tf_size + 1) * sizeof(float2);
-  // one ray per wavefront: a batch is tens to thousands of light-ray steps (256^2 with 16 + 4
-  // rays 8.9 ms, 9.3 with two)
-  const QueueShape qs = queue_shape(rf, 1, 1);
+  const QueueShape qs = queue_shape(rf, kRays, 1);
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   float4* o4 = reinterpret_cast<float4*>(out);
   if (c->dtype == CVR_U8)
