@@ -264,12 +264,13 @@ __device__ __forceinline__ float4 sample_tf(const float4* __restrict__ tf, int T
 // and at any moment the 8 XCDs hold 8 consecutive supertiles, i.e. one compact region
 // of the image whose part of the volume the shared MALL then serves to all of them.
 // (Giving each XCD a contiguous eighth of the image instead was 22 % slower on the
-// 512^3 surrogate frame: 8 distant regions share nothing in the MALL.)  Workgroups past
+// 512^3 surrogate frame: 8 distant regions share nothing in the MALL.)  Groups of
+// 1 << kLog2 workgroups for launches of smaller workgroups.  Workgroups past
 // the last full run of 512 keep their index; a permutation for every grid size.
-__device__ __forceinline__ int xcd_remap(int bid, int nblocks) {
-  if (bid >= (nblocks >> 9) << 9) return bid;
+__device__ __forceinline__ int xcd_remap(int bid, int nblocks, int kLog2 = 6) {
+  if (bid >= (nblocks >> (kLog2 + 3)) << (kLog2 + 3)) return bid;
   const int x = bid & 7, k = bid >> 3;
-  return ((k >> 6) << 9) | (x << 6) | (k & 63);
+  return ((k >> kLog2) << (kLog2 + 3)) | (x << kLog2) | (k & ((1 << kLog2) - 1));
 }
 
 // Workgroup index -> tile of a tiles_x x tiles_y grid of tile_px-wide tiles, in

@@ -15,7 +15,7 @@
 //  - opaque samples go to a queue in LDS; whenever it holds 64, every lane shades one and
 //    adds it to its pixel's colour in LDS.  A wavefront's rays share the queue, so all of
 //    its lanes shade until its last batch.
-// A wavefront's rays lie far apart in the image: neighbours are alike, and a wavefront of
+// A wavefront's rays lie some way apart in the image: neighbours are alike, and a wavefront of
 // long rays would end last.
 #pragma once
 #include "cvr_common.hpp"
@@ -78,29 +78,48 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Pixel i of the image in 16 x 16 tiles, row-major, of 2 x 2 pixel groups; false past the
-// image's edges.  After xcd_remap, the 64 workgroups an XCD takes in turn are one tile (the
-// 256^3 cone-traced frame at 1024^2: 90 ms, 117 ms in rows of 8 x 8 tiles).
-__device__ __forceinline__ bool tiled_pixel(const RayFrame& rf, int i, int& px, int& py) {
-  const int tiles_x = (rf.W + 15) >> 4, t = i >> 8;
-  px = (t % tiles_x) * 16 + ((i >> 1) & 14) + (i & 1);
-  py = (t / tiles_x) * 16 + ((i >> 4) & 14) + ((i >> 1) & 1);
+// Pixel i of the image in square tiles of 1 << tile_log2 pixels (at most 64), row-major, each in
+// Z order; false past the image's edges.
+__device__ __forceinline__ bool tiled_pixel(const RayFrame& rf, int tile_log2, int i, int& px, int& py) {
+  const int tiles_x = (rf.W + (1 << tile_log2) - 1) >> tile_log2, t = i >> (2 * tile_log2), j = i & ((1 << (2 * tile_log2)) - 1);
+  auto even = [](int v) {  // bits 0, 2, 4, ... of v
+    v &= 0x555;
+    v = (v | (v >> 1)) & 0x333;
+    v = (v | (v >> 2)) & 0x70f;
+    return (v | (v >> 4)) & 0x3f;
+  };
+  px = ((t % tiles_x) << tile_log2) + even(j);
+  py = ((t / tiles_x) << tile_log2) + even(j >> 1);
   return px < rf.W && py < rf.H;
 }
-inline int tiled_pixels(const RayFrame& rf) { return ((rf.W + 15) / 16) * ((rf.H + 15) / 16) * 256; }
+inline int tiled_pixels(const RayFrame& rf, int tile_log2) {
+  const int m = 1 << tile_log2;
+  return ((rf.W + m - 1) / m) * ((rf.H + m - 1) / m) * m * m;
+}
 
-// Rays per wavefront and workgroups (of `waves` wavefronts) of a frame: at most `most` rays (a
-// power of two up to 64) while that leaves `min_waves` wavefronts.  More rays leave fewer
-// part-filled last batches, fewer rays more wavefronts to even out; where the two lines lie
-// is each renderer's, measured over frame sizes.
+// How a frame's rays are dealt out: `rays` per unit (a wavefront, or a workgroup whose four
+// wavefronts share them: parts 4), the tile whose pixels the units take in turn, workgroups,
+// and runs of 1 << xcd_log2 workgroups per XCD (xcd_remap).
 struct QueueShape {
-  int rays, blocks;
+  int rays, parts, tile_log2, blocks, xcd_log2;
 };
-inline QueueShape queue_shape(const RayFrame& rf, int most, int min_waves, int waves = 4) {
-  const int n = tiled_pixels(rf);
-  int rays = 1;
-  while (rays < most && n / (rays * 2) >= min_waves) rays *= 2;
-  return QueueShape{rays, (n / rays + waves - 1) / waves};
+// Tiles of 64 x 64 pixels: a unit's rays lie 32 (rays 4) or 16 (rays 16) pixels apart, so long
+// and short ones mix, while the units that run at once stay together (256^3 cone-traced frame
+// at 512^2: 18.7 ms, 23.7 ms in 16 x 16 tiles; EBS 5.0 and 6.6 ms; DOS 4.5 and 6.0 ms).
+// Narrower frames take smaller tiles.  xcd_px: pixels an XCD takes in a row.
+inline QueueShape queue_shape(const RayFrame& rf, int rays, int parts, int xcd_px, int waves = 4) {
+  const int side = rf.W < rf.H ? rf.W : rf.H;
+  QueueShape q{rays, parts, 2, 0, 0};
+  while (q.tile_log2 < 6 && 1 << q.tile_log2 < side) ++q.tile_log2;
+  const int per_wg = rays * waves / parts;  // pixels of a workgroup
+  q.blocks = (tiled_pixels(rf, q.tile_log2) + per_wg - 1) / per_wg;
+  while (per_wg << q.xcd_log2 < xcd_px) ++q.xcd_log2;
+  return q;
+}
+// The unit of this wavefront.
+template <int kParts> __device__ __forceinline__ int queue_unit(int xcd_log2) {
+  const int waves = int(blockDim.x) >> 6, bid = xcd_remap(blockIdx.x, gridDim.x, xcd_log2);
+  return kParts > 1 ? bid : bid * waves + int(threadIdx.x >> 6);
 }
 
 __device__ __forceinline__ float lane_value(float v, int lane) {
@@ -111,31 +130,40 @@ template <int kSub> __device__ __forceinline__ float group_uniform(float v) {
   return kSub == 64 ? __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))) : v;
 }
 
-// The pixels of a frame's wavefronts: ray k of wavefront gw of nw, kGroups neighbouring rays
-// side by side and the groups far apart.
-template <int kSub> struct FramePixels {
+// The pixels of unit u of a frame: the units of a tile take its pixels in turn, `group`
+// neighbours at a time.
+struct FramePixels {
   const RayFrame& rf;
-  int gw, nw;
+  int tile_log2, first, stride, group;
+  __device__ __forceinline__ FramePixels(const RayFrame& r, const QueueShape& q, int u, int g = 1)
+      : rf(r), tile_log2(q.tile_log2), group(g) {
+    stride = (1 << (2 * q.tile_log2)) / q.rays;  // units of a tile
+    first = u / stride * (1 << (2 * q.tile_log2)) + u % stride * g;
+  }
   __device__ __forceinline__ bool operator()(int k, int& px, int& py) const {
-    constexpr int kGroups = 64 / kSub;
-    return tiled_pixel(rf, (gw + k / kGroups * nw) * kGroups + k % kGroups, px, py);
+    return tiled_pixel(rf, tile_log2, first + k / group * stride * group + k % group, px, py);
   }
 };
 
 // Marches `rays` rays (at most kRays <= 64), ray k that of pixel pix(k, px, py) (false: no pixel), and
 // writes their pixels: 64 / kSub rays at a time, kSub samples of each per step.
+// kParts > 1: that many wavefronts of a workgroup march the same rays, each shading every
+// kParts-th batch, and the first adds up their colours (every wavefront of the workgroup
+// makes this call once; Q: the first one's queue, the others' follow).
 // shade(on, p, dir) lights one sample (in texture space) per lane; kWhole: all 64 lanes call
 // it together, `on` says which have a sample; otherwise only those with one.  spec:
 // specular colour of Lit::s.
-template <typename T, int kSub, bool kWhole, int kRays, class Pix, class Shade>
+template <typename T, int kSub, bool kWhole, int kParts, int kRays, class Pix, class Shade>
 __device__ __forceinline__ void queue_march(const RayFrame& rf, const VolGeom& g, const float4* s_tf, int ntf,
                                             float step, float et, int rays, Pix&& pix, const float* spec,
-                                            WaveQueue<kRays>& Q, float4* __restrict__ out, unsigned int& nsamp, unsigned int& nshade,
+                                            WaveQueue<kRays>* queues, float4* __restrict__ out, unsigned int& nsamp, unsigned int& nshade,
                                             Shade&& shade) {
   typedef typename VolOct<T>::type RT;
   static_assert(kSub == 64 || kSub == 16, "groups are wavefronts or DPP rows");
   constexpr uint64_t kGroupMask = kSub == 64 ? ~0ull : (1ull << (kSub & 63)) - 1ull;
   const int lane = threadIdx.x & 63, sub = lane % kSub, base = lane - sub;
+  const int part = kParts > 1 ? int(threadIdx.x >> 6) % kParts : 0;
+  WaveQueue<kRays>& Q = queues[part];
   const uint64_t below = (1ull << lane) - 1ull, below_group = (1ull << base) - 1ull;
   // lane k sets up ray k; the rays that hit the box are listed in order
   int px = 0, py = 0;
@@ -162,7 +190,7 @@ __device__ __forceinline__ void queue_march(const RayFrame& rf, const VolGeom& g
   f3 tp = mk3(0.f, 0.f, 0.f), dir = tp;
   float D = 0.f;
   int ray = -1, jb = 0;                  // the group's ray and next sample
-  int next = 0, head = 0, count = 0;     // next ray, queue: the same in every lane
+  int next = 0, head = 0, count = 0, batch = 0;  // next ray, queue: the same in every lane
   float w = 0.f;
   RT rec = {};
   // a new ray for the groups without one, and the blocks of every group's next samples: in
@@ -212,8 +240,8 @@ __device__ __forceinline__ void queue_march(const RayFrame& rf, const VolGeom& g
           ended = ended || over != 0;
         }
         emit = opaque && taken;
-        nsamp += taken;
-        nshade += emit;
+        nsamp += taken && part == 0;
+        nshade += emit && part == 0;
         jb += kSub;
         if (ended || jb >= kMaxSamples) {
           if (sub == 0) Q.acc[ray].w = w;
@@ -232,8 +260,9 @@ __device__ __forceinline__ void queue_march(const RayFrame& rf, const VolGeom& g
     if (count == 0) break;
     wave_lds_sync();
     const int n = min(count, 64);
-    const bool on = lane < n;
-    if (kWhole || on) {
+    const bool on = lane < n, mine = kParts == 1 || batch % kParts == part;
+    ++batch;
+    if (mine && (kWhole || on)) {
       const int i = (head + (on ? lane : 0)) & (kQueueCap - 1);
       const float4 a = Q.a[i], b = Q.b[i];
       const int r = __float_as_int(b.w);
@@ -251,7 +280,21 @@ __device__ __forceinline__ void queue_march(const RayFrame& rf, const VolGeom& g
     wave_lds_sync();
   }
   wave_lds_sync();
-  if (inside) out[size_t(py) * rf.W + px] = hit ? Q.acc[slot] : make_float4(0.f, 0.f, 0.f, 0.f);
+  if (kParts > 1) __syncthreads();
+  if (inside && part == 0) {
+    float4 c = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (hit) {
+      c = Q.acc[slot];
+      for (int i = 1; i < kParts; ++i) {
+        const float4 d = queues[i].acc[slot];
+        c.x += d.x;
+        c.y += d.y;
+        c.z += d.z;
+      }
+    }
+    out[size_t(py) * rf.W + px] = c;
+  }
+  if (kParts > 1) __syncthreads();  // before the queues are used again
 }
 
 }  // namespace cvr

@@ -10,8 +10,8 @@
 // level whose Gaussian sigma matches the cone radius there (LINEAR_MIPMAP_LINEAR +
 // the border falloff of GetGaussianExtinction, :92-112).
 //
-// The march is queue_march's (cvr_queue.hpp): 256^3 at 1024^2 177 -> 72 ms, at
-// 200 x 150 of a 100 x 90 x 80 volume 43 -> 1.4 ms.  Per step the level index is wave-uniform, so the level geometry stays in SGPRs;
+// The march is queue_march's (cvr_queue.hpp): 256^3 at 1024^2 177 -> 69 ms, at
+// 512^2 162 -> 18.7 ms, at 128^2 146 -> 1.9 ms.  Per step the level index is wave-uniform, so the level geometry stays in SGPRs;
 // the step schedule is read with scalar loads from a small device table.
 #include "cvr_cone.hpp"
 #include "cvr_queue.hpp"
@@ -21,25 +21,23 @@
 
 namespace cvr {
 
-// One ray per wavefront: a batch of 64 samples takes 9 x 64 cone steps, so an unfilled last
-// one weighs less than the evenness (128^2: 7.7 ms, 8.2 with two rays, 9.2 with four).
-constexpr int kRays = 1;
-template <typename T, int F>
+constexpr int kRays = 4;
+template <typename T, int F, int kParts>
 __global__ __launch_bounds__(256) void k_cone_render(RayFrame rf, VolGeom g, PyrGeom pg, const void* __restrict__ pyr,
                                                      ConeK K, const float4* __restrict__ tf, int ntf, float step,
-                                                     float et, int rays, float4* __restrict__ out,
+                                                     float et, QueueShape qs, float4* __restrict__ out,
                                                      unsigned long long* __restrict__ counters) {
   extern __shared__ float4 s_tf[];
   __shared__ WaveQueue<kRays> queue[4];
   for (int i = threadIdx.x; i < ntf; i += blockDim.x) s_tf[i] = tf[i];
   __syncthreads();
-  const int gw = xcd_remap(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), nw = gridDim.x * 4;
+  const int u = queue_unit<kParts>(qs.xcd_log2);
   unsigned int nsamp = 0, nshade = 0;
   const float ka = K.apply_occ ? K.ka : 0.f, kd = K.apply_sdw ? K.kd : 0.f;
   const float inv_k = 1.0f / (ka + kd);
   const f3 L = ld3(K.L);
   const float spec[3] = {0.f, 0.f, 0.f};
-  queue_march<T, 64, false>(rf, g, s_tf, ntf, step, et, rays, FramePixels<64>{rf, gw, nw}, spec, queue[threadIdx.x >> 6], out, nsamp, nshade,
+  queue_march<T, 64, false, kParts>(rf, g, s_tf, ntf, step, et, qs.rays, FramePixels(rf, qs, u), spec, kParts > 1 ? queue : queue + (threadIdx.x >> 6), out, nsamp, nshade,
                  [&](bool, f3 p, f3 dir) {
                    f3 k, up, right;
                    occ_frame(dir, k, up, right);
@@ -245,11 +243,18 @@ int launch_cone(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* o
   if (shm > 64 * 1024) { set_error("cone renderer: transfer function larger than 4096 entries"); return -4; }
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   float4* o4 = reinterpret_cast<float4*>(out);
-  const QueueShape qs = queue_shape(rf, kRays, 1);
+  // small frames: workgroups whose wavefronts share their rays (128^2 1.9 ms, 3.4 ms with rays
+  // of their own; 512^2 18.7 and 19.9; 1024^2 70.4 and 68.6)
+  const bool shared = size_t(rf.W) * rf.H < (1 << 19);
+  const QueueShape qs = queue_shape(rf, kRays, shared ? 4 : 1, shared ? 64 : 256);
   with_types(c->dtype, c->pyr.fmt, [&](auto t, auto f) {
     using T = typename decltype(t)::type;
-    hipLaunchKernelGGL((k_cone_render<T, decltype(f)::value>), dim3(qs.blocks), dim3(256), shm, st, rf, g, c->pyr,
-                       c->d_pyr_oct, K, c->d_tf_rgbt, c->tf_size, step, P.et_threshold, qs.rays, o4, cnt);
+    auto launch = [&](auto parts) {
+      hipLaunchKernelGGL((k_cone_render<T, decltype(f)::value, decltype(parts)::value>), dim3(qs.blocks), dim3(256), shm,
+                         st, rf, g, c->pyr, c->d_pyr_oct, K, c->d_tf_rgbt, c->tf_size, step, P.et_threshold, qs, o4, cnt);
+    };
+    if (shared) launch(std::integral_constant<int, 4>{});
+    else launch(std::integral_constant<int, 1>{});
   });
   CVR_HIP_CHECK(hipGetLastError());
   return 0;

@@ -16,8 +16,8 @@
 // section on the axis, then 3 then 7 sub-cones that inherit their parent's optical
 // depth, trapezoid sums of amplitude * extinction, I = exp(-depth) averaged over the
 // sub-cones (the 7-packing weights its ring by the adjacent weight).  The march is
-// queue_march's (cvr_queue.hpp; 256^3 at 1024^2 with shadows 41.5 -> 16.1 ms, at 200 x 150
-// 7.2 -> 0.27 ms).  The table row
+// queue_march's (cvr_queue.hpp; 256^3 at 1024^2 with shadows 41.5 -> 15.6 ms, at 200 x 150
+// 7.2 -> 0.26 ms).  The table row
 // index is wave-uniform, so rows arrive through scalar loads and the level geometry
 // stays in SGPRs.
 #include "cvr_cone.hpp"
@@ -133,27 +133,24 @@ __device__ __forceinline__ float dos_shadow(const void* __restrict__ pyr, const 
   return dos_cone<F>(pyr, pg, K.sdw, K.sdw_rows, p, k, v1, u1);
 }
 
-// Up to 8 rays per wavefront while 3072 wavefronts are left: 1024^2 26.7 ms with one ray, 24.2
-// with eight, 25.2 with 64; 200 x 150 0.34, 0.32 and 0.73; 100 x 100 1.16 with four (3136
-// wavefronts), 1.51 with eight.
-constexpr int kRays = 8;
-template <typename T, int F>
+constexpr int kRays = 4;
+template <typename T, int F, int kParts>
 __global__ __launch_bounds__(256) void k_dos_render(RayFrame rf, VolGeom g, PyrGeom pg, const void* __restrict__ pyr,
                                                     DosK K, const float4* __restrict__ tf, int ntf, float step, float et,
-                                                    PhongK ph, const float4* __restrict__ grad, int rays,
+                                                    PhongK ph, const float4* __restrict__ grad, QueueShape qs,
                                                     float4* __restrict__ out,
                                                     unsigned long long* __restrict__ counters) {
   extern __shared__ float4 s_tf[];
   __shared__ WaveQueue<kRays> queue[4];
   for (int i = threadIdx.x; i < ntf; i += blockDim.x) s_tf[i] = tf[i];
   __syncthreads();
-  const int gw = xcd_remap(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), nw = gridDim.x * 4;
+  const int u = queue_unit<kParts>(qs.xcd_log2);
   const f3 eye = ld3(rf.eye);
   const f3 half = mk3(0.5f * g.G[0], 0.5f * g.G[1], 0.5f * g.G[2]);
   unsigned int nsamp = 0, nshade = 0;
   const float ka = K.apply_occ ? K.ka : 0.f, kd = K.apply_sdw ? K.kd : 0.f;
   const float inv_k = 1.0f / (ka + kd);
-  queue_march<T, 64, false>(rf, g, s_tf, ntf, step, et, rays, FramePixels<64>{rf, gw, nw}, ph.spec, queue[threadIdx.x >> 6], out, nsamp, nshade,
+  queue_march<T, 64, false, kParts>(rf, g, s_tf, ntf, step, et, qs.rays, FramePixels(rf, qs, u), ph.spec, kParts > 1 ? queue : queue + (threadIdx.x >> 6), out, nsamp, nshade,
                  [&](bool, f3 p, f3 dir) {
                    const f3 wp = p - half;
                    float Io = 0.f, Is = 0.f;
@@ -454,11 +451,19 @@ int launch_dos(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* ou
   }
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   float4* o4 = reinterpret_cast<float4*>(out);
-  const QueueShape qs = queue_shape(rf, kRays, 3072);
+  // small frames: workgroups whose wavefronts share their rays (100 x 100 0.41 ms, 0.82 ms with
+  // rays of their own; 200 x 150 0.26 and 0.48; 400 x 300 2.2 and 1.7; 1024^2 19.4 and 15.6)
+  const bool shared = size_t(rf.W) * rf.H < (1 << 16);
+  const QueueShape qs = queue_shape(rf, kRays, shared ? 4 : 1, shared ? 64 : 256);
   with_types(c->dtype, c->pyr.fmt, [&](auto t, auto f) {
     using T = typename decltype(t)::type;
-    hipLaunchKernelGGL((k_dos_render<T, decltype(f)::value>), dim3(qs.blocks), dim3(256), shm, st, rf, g, c->pyr,
-                       c->d_pyr_oct, K, c->d_tf_rgbt, c->tf_size, step, P.et_threshold, ph, c->d_grad, qs.rays, o4, cnt);
+    auto launch = [&](auto parts) {
+      hipLaunchKernelGGL((k_dos_render<T, decltype(f)::value, decltype(parts)::value>), dim3(qs.blocks), dim3(256), shm, st,
+                         rf, g, c->pyr, c->d_pyr_oct, K, c->d_tf_rgbt, c->tf_size, step, P.et_threshold, ph, c->d_grad, qs,
+                         o4, cnt);
+    };
+    if (shared) launch(std::integral_constant<int, 4>{});
+    else launch(std::integral_constant<int, 1>{});
   });
   CVR_HIP_CHECK(hipGetLastError());
   return CVR_OK;

@@ -387,20 +387,18 @@ __device__ __forceinline__ void ebs_load_rows(const ShadowRow* __restrict__ rows
   __syncthreads();
 }
 
-// Up to 64 rays per wavefront while every SIMD has one (1024^2 47 ms with one ray, 32 with 16,
-// 30.8 with 64; 200 x 150 0.69, 0.52 with 16, 0.48 with 32 (1040 wavefronts), 0.61 with 64).
-constexpr int kRays = 64;
+constexpr int kRays = 16;
 // The march is queue_march's (cvr_queue.hpp).  One wavefront per SIMD: the box streams keep
 // four corner records in flight per lane, which with the FP64 interpolation takes more than
 // the 256 architectural VGPRs; at one wavefront per SIMD the excess lives in AGPRs instead of
 // scratch memory.  kPoint: the point light's shadows, a variant of its own (its per-sample
 // cone geometry takes registers the table's lookups do without).  256^3 u16 at 1024^2 with
-// shadows, light table: 66 ms one ray per lane, 30.8 ms queued, 23.1 ms with everything
-// inlined so that no kernel argument is copied to scratch memory; 28.9 ms at two wavefronts
-// per SIMD.
-template <typename T, int L, bool kPoint>
+// shadows, light table: 66 ms one ray per lane, 23.1 ms queued (30.8 ms with
+// kernel arguments copied to scratch memory for functions called, 28.9 ms at two wavefronts per
+// SIMD), 16.0 ms with the rays dealt out as in queue_shape.
+template <typename T, int L, bool kPoint, int kParts>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_ebs(RayFrame rf, EbsK k, const float4* __restrict__ tf, int ntf, const void* __restrict__ sat,
-           const ShadowRow* __restrict__ rows, float step, float et, PhongK ph, const float4* __restrict__ grad, int rays,
+           const ShadowRow* __restrict__ rows, float step, float et, PhongK ph, const float4* __restrict__ grad, QueueShape qs,
            float4* __restrict__ out, unsigned long long* __restrict__ counters) {
   extern __shared__ float4 smem[];
   const int waves = blockDim.x >> 6;
@@ -410,12 +408,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   for (int i = threadIdx.x; i < ntf; i += blockDim.x) s_tf[i] = tf[i];
   ebs_load_rows(rows, k.nrows, s_rows);
   const int nrows = k.nrows;
-  const int gw = xcd_remap(blockIdx.x, gridDim.x) * waves + (threadIdx.x >> 6), nw = gridDim.x * waves;
+  const int u = queue_unit<kParts>(qs.xcd_log2);
   const f3 eye = ld3(rf.eye);
   unsigned int nsamp = 0, nshade = 0, nbox = 0;
   const float ka = k.apply_occ ? k.ka : 0.f, kd = k.apply_sdw ? k.kd : 0.f;
   const float inv_k = 1.0f / (ka + kd);
-  queue_march<T, 64, false>(rf, k.g, s_tf, ntf, step, et, rays, FramePixels<64>{rf, gw, nw}, ph.spec, queue[threadIdx.x >> 6], out, nsamp, nshade,
+  queue_march<T, 64, false, kParts>(rf, k.g, s_tf, ntf, step, et, qs.rays, FramePixels(rf, qs, u), ph.spec, kParts > 1 ? queue : queue + (threadIdx.x >> 6), out, nsamp, nshade,
                  [&](bool, f3 p, f3) {
                    float Io = 0.f, Is = 0.f;
                    if (k.apply_occ) {
@@ -594,19 +592,26 @@ int launch_ebs(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* ou
   int waves = 4;
   while (waves > 1 && tables + size_t(waves) * sizeof(WaveQueue<kRays>) > 160 * 1024) waves /= 2;
   const size_t shm = tables + size_t(waves) * sizeof(WaveQueue<kRays>);
-  const QueueShape qs = queue_shape(rf, kRays, 1024, waves);
+  // small frames: workgroups whose wavefronts share their rays (100 x 100 0.51 ms, 1.0 ms with
+  // rays of their own; 400 x 300, point light 3.6 and 4.3; 512^2 5.3 and 5.0; 1024^2 19.4 and 16.0)
+  const bool shared = waves == 4 && size_t(rf.W) * rf.H < 200000;
+  const QueueShape qs = queue_shape(rf, kRays, shared ? 4 : 1, shared ? 64 : 256, waves);
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   const void* sat = P.sat_layout == 1 ? static_cast<const void*>(c->d_sat) : c->d_sat_oct;
   const ShadowRow* rows = static_cast<const ShadowRow*>(c->d_ebs_rows);
   float4* o4 = reinterpret_cast<float4*>(out);
-  auto launch = [&](auto t, auto l, auto pt) {
-    hipLaunchKernelGGL((k_ebs<typename decltype(t)::type, decltype(l)::value, decltype(pt)::value>), dim3(qs.blocks),
+  auto launch = [&](auto t, auto l, auto pt, auto parts) {
+    hipLaunchKernelGGL((k_ebs<typename decltype(t)::type, decltype(l)::value, decltype(pt)::value, decltype(parts)::value>), dim3(qs.blocks),
                        dim3(64 * waves), shm, st, rf, k, c->d_tf_rgbt, c->tf_size, sat, rows, step, P.et_threshold, ph,
-                       c->d_grad, qs.rays, o4, cnt);
+                       c->d_grad, qs, o4, cnt);
   };
   auto by_light = [&](auto t, auto l) {
-    if (P.apply_shadow && P.shadow_type != 1) launch(t, l, std::true_type{});
-    else launch(t, l, std::false_type{});
+    auto by_size = [&](auto pt) {
+      if (shared) launch(t, l, pt, std::integral_constant<int, 4>{});
+      else launch(t, l, pt, std::integral_constant<int, 1>{});
+    };
+    if (P.apply_shadow && P.shadow_type != 1) by_size(std::true_type{});
+    else by_size(std::false_type{});
   };
   auto by_layout = [&](auto t) {
     if (P.sat_layout == 1) by_light(t, std::integral_constant<int, 1>{});

@@ -90,14 +90,12 @@ __device__ __forceinline__ float gt_cone(const VolGeom& g, const float2* s_ext, 
   return S / W;
 }
 
-// One ray per wavefront: a batch is tens to thousands of light-ray steps (256^2 with 16 + 4
-// rays 8.9 ms, 9.3 with two).
-constexpr int kRays = 1;
+constexpr int kRays = 4;
 // The march is queue_march's (cvr_queue.hpp).  128^3 at 256^2 with 16 + 4 rays per sample:
-// 313 -> 8.9 ms (one dependent read per light-ray step at one wavefront per SIMD before).
+// 313 -> 5.7 ms (one dependent read per light-ray step at one wavefront per SIMD before).
 template <typename T>
 __global__ __launch_bounds__(256) void k_gt_render(RayFrame rf, VolGeom g, GtK K, const float4* __restrict__ tf,
-                                                   int ntf, float step, float et, int rays, float4* __restrict__ out,
+                                                   int ntf, float step, float et, QueueShape qs, float4* __restrict__ out,
                                                    unsigned long long* __restrict__ counters) {
   extern __shared__ float4 s_tf[];
   __shared__ WaveQueue<kRays> queue[4];
@@ -105,13 +103,13 @@ __global__ __launch_bounds__(256) void k_gt_render(RayFrame rf, VolGeom g, GtK K
   for (int i = threadIdx.x; i < ntf; i += blockDim.x) s_tf[i] = tf[i];
   for (int i = threadIdx.x; i <= ntf; i += blockDim.x) s_ext[i] = make_float2(tf[max(i - 1, 0)].w, tf[min(i, ntf - 1)].w);
   __syncthreads();
-  const int gw = xcd_remap(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6), nw = gridDim.x * 4;
+  const int u = queue_unit<4>(qs.xcd_log2);
   unsigned int nsamp = 0, nshade = 0;
   const float ka = K.apply_occ ? K.ka : 0.f, kd = K.apply_sdw ? K.kd : 0.f;
   const float inv_k = 1.0f / (ka + kd);
   const f3 half = mk3(0.5f * g.G[0], 0.5f * g.G[1], 0.5f * g.G[2]);
   const float spec[3] = {0.f, 0.f, 0.f};
-  queue_march<T, 64, false>(rf, g, s_tf, ntf, step, et, rays, FramePixels<64>{rf, gw, nw}, spec, queue[threadIdx.x >> 6], out, nsamp, nshade,
+  queue_march<T, 64, false, 4>(rf, g, s_tf, ntf, step, et, qs.rays, FramePixels(rf, qs, u), spec, queue, out, nsamp, nshade,
                  [&](bool, f3 p, f3 dir) {
                    float Io = 0.f, Is = 0.f;
                    if (K.apply_occ) {
@@ -234,15 +232,18 @@ int launch_gt(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out
     return CVR_ERR_UNSUPPORTED;
   }
   const size_t shm = size_t(c->tf_size) * sizeof(float4) + size_t(c->tf_size + 1) * sizeof(float2);
-  const QueueShape qs = queue_shape(rf, kRays, 1);
+  // workgroups whose wavefronts share their rays: a batch is tens to thousands of light-ray
+  // steps (128^3 at 256^2 with 16 + 4 rays 5.7 ms, 13.7 ms with rays of their own; 256^3 at 512^2
+  // with 4 + 1 11.5 and 12.2)
+  const QueueShape qs = queue_shape(rf, kRays, 4, 64);
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   float4* o4 = reinterpret_cast<float4*>(out);
   if (c->dtype == CVR_U8)
     hipLaunchKernelGGL(k_gt_render<uint8_t>, dim3(qs.blocks), dim3(256), shm, st, rf, g, K, c->d_tf_rgbt, c->tf_size,
-                       step, P.et_threshold, qs.rays, o4, cnt);
+                       step, P.et_threshold, qs, o4, cnt);
   else
     hipLaunchKernelGGL(k_gt_render<uint16_t>, dim3(qs.blocks), dim3(256), shm, st, rf, g, K, c->d_tf_rgbt, c->tf_size,
-                       step, P.et_threshold, qs.rays, o4, cnt);
+                       step, P.et_threshold, qs, o4, cnt);
   CVR_HIP_CHECK(hipGetLastError());
   return CVR_OK;
 }
