@@ -1,8 +1,9 @@
 // Surrogate network inference shared by the single-frame and batched renderers:
 // bf16 MFMA types and layout constants, the wavefront-cooperative forward pass,
-// and the per-tile surrogate march.
+// and the surrogate march.
 #pragma once
 #include "cvr_cone.hpp"
+#include "cvr_queue.hpp"
 
 namespace cvr {
 
@@ -148,142 +149,57 @@ struct NnK {
   int exact_all;                 // validation gate failed: every sample uses the exact tracer
 };
 
-// Shape of the work of one wavefront: an (1 << tw_log2) x (64 >> tw_log2) pixel tile
-// (four of them, 2 x 2, per workgroup), and how many of the wave's marching lanes
-// must be waiting on a shaded sample before the wave gathers their features and runs
-// the network together (`park`: a fraction of the active lanes; 0 = as soon as one
-// waits).  Neither changes any pixel: every ray takes the same samples in the same
-// order and the network maps each sample independently of the others.
-struct NnSched {
-  int tw_log2;
-  float park;
-  int span;  // wave tiles per wave (pixels handed out as lanes free up)
-};
-
 NnK nn_consts(cvr_ctx* c);
 ConeK cone_constants(const cvr_ctx* c, const cvr_cone_params& P, const float L[3]);
 void light_dir(const RayFrame& rf, const cvr_light* light, float L[3]);
 
-// Renders one workgroup tile of frame `rf`: 2 x 2 waves, each owning `span` wave tiles
-// of the NnSched shape stacked along y.  A lane whose ray ends writes its pixel and,
-// once enough lanes of the wave are idle, takes the wave's next unrendered pixel, so the
-// wave keeps its lanes busy until its pixels run out instead of idling behind its
-// longest ray.  sW/sB/s_tf: the network and transfer function staged in LDS; sXw: this
-// wave's LDS scratch.  Counters (samples, shaded, exact fallbacks) accumulate into cnt.
+// Rays of a wavefront's queue and samples per step of each: four rays at a time share a
+// step, so that the in-order opacity recurrence takes 16 rounds, not 64 (512^3 at 1024^2 4.74 ms,
+// 4.95 with 64 samples of one ray; from inside a 200 x 190 x 180 volume at 700 x 500 2.64 and 3.0).
+constexpr int kNnRays = 16, kNnSub = 16;
+
+// Marches a wavefront's rays (queue_march, pixels from pix) with the surrogate as the
+// lighting: the wave gathers its 64 samples' features and runs the network over them
+// together.  sW/sB/s_tf: the network and transfer function staged in LDS; sXw: this wave's
+// LDS scratch.  Counters (samples, shaded, exact fallbacks) accumulate into cnt.
 // kExact: a sample whose inputs leave the training range takes the exact cone tracer's
-// answers; without it the tile is only marked (the return value: some lane of this wave
-// met such a sample) for a second pass with kExact, and its pixels are provisional.
+// answers; without it the rays are only marked (the return value: some sample of this wave
+// left the range) for a second pass with kExact, and their pixels are provisional.
 // Which samples a ray takes and their opacities do not depend on the shading, so both
-// passes march a tile identically.
-template <typename T, int F, bool kExact = true>
-__device__ __forceinline__ bool nn_tile(const RayFrame& rf, const VolGeom& g, const PyrGeom& pg,
-                                        const void* __restrict__ pyr, const ConeK& K, const NnK& nk,
-                                        const NnSched& sc, const short* sW, const float* sB, float* sXw,
-                                        const float4* s_tf, int ntf, float step, float et, float4* __restrict__ out,
-                                        int tx, int ty, unsigned int* cnt) {
-  const int tl = sc.tw_log2, tw = 1 << tl, th = 64 >> tl, span = sc.span;
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int x0 = tx * 2 * tw + (w & 1) * tw;
-  const int y0 = (ty * 2 + (w >> 1)) * th * span;
-  const int total = 64 * span;
-  const f3 eye = ld3(rf.eye);
-  const f3 half = mk3(0.5f * g.G[0], 0.5f * g.G[1], 0.5f * g.G[2]);
+// passes march it identically.
+template <typename T, int F, bool kExact, class Pix>
+__device__ __forceinline__ bool nn_march(const RayFrame& rf, const VolGeom& g, const PyrGeom& pg,
+                                         const void* __restrict__ pyr, const ConeK& K, const NnK& nk, const short* sW,
+                                         const float* sB, float* sXw, const float4* s_tf, int ntf, float step, float et,
+                                         int rays, Pix&& pix, WaveQueue<kNnRays>& Q, float4* __restrict__ out,
+                                         unsigned int* cnt) {
   const float ka = K.apply_occ ? K.ka : 0.f, kd = K.apply_sdw ? K.kd : 0.f;
   const float inv_k = 1.0f / (ka + kd);
   const f3 L = ld3(K.L);
-  const uint64_t below = (1ull << lane) - 1ull;
-  // per-lane ray state (pix < 0: idle)
-  int pix = -1, px = 0, py = 0, j = 0;
-  float D = 0.f, h = 0.f;
-  f3 dir = mk3(0.f, 0.f, 1.f), tp = eye, p = eye;  // the occlusion axis is -dir
-  float4 dst = make_float4(0.f, 0.f, 0.f, 0.f), src = dst;
-  // The corner block of the lane's next sample, loaded as soon as the current sample is
-  // known, so that its read is in flight while the wave gathers and shades (sample j sits
-  // at the midpoint of [s, s + h], s = j step, h = min(step, D - s); past the end of the
-  // ray the position is still finite and its clamped block in bounds).
-  typedef typename VolOct<T>::type RT;
-  auto pos = [&](int jj) {
-    const float s = float(jj) * step;
-    return tp + dir * (s + 0.5f * fminf(step, D - s));
-  };
-  RT rec = {};
-  bool parked = false, ood_seen = false;
-  int next = 0;  // wave-uniform: next pixel of the span to hand out
-  for (;;) {
-    const uint64_t idle = __ballot(pix < 0);
-    const int n_idle = __popcll(idle);
-    if (next < total && (n_idle >= 16 || n_idle == 64)) {
-      // hand the next pixels to the idle lanes, in lane order
-      const int mine = next + __popcll(idle & below);
-      if (pix < 0 && mine < total) {
-        const int t = mine >> 6, l = mine & 63;
-        px = x0 + (l & (tw - 1));
-        py = y0 + t * th + (l >> tl);
-        float tn = 0.f, tf_ = 0.f;
-        if (px < rf.W && py < rf.H) {
-          dir = camera_ray(rf, px, py);
-          if (ray_box(eye, dir, g.G, tn, tf_)) {
-            pix = mine;
-            D = fabsf(tf_ - tn);
-            tp = eye + dir * tn + half;
-            j = 0;
-            dst = make_float4(0.f, 0.f, 0.f, 0.f);
-            rec = volume_oct_load<T>(g, pos(0));
-          } else {
-            out[size_t(py) * rf.W + px] = make_float4(0.f, 0.f, 0.f, 0.f);  // the ray misses the box
-          }
+  const float spec[3] = {0.f, 0.f, 0.f};
+  bool ood_seen = false;
+  queue_march<T, kNnSub, true, 1>(
+      rf, g, s_tf, ntf, step, et, rays, pix, spec, &Q, out, cnt[0], cnt[1], [&](bool on, f3 p, f3 dir) {
+        float f[kNFeat];
+        bool ood = false;
+        float bo = 0.f, bs = 0.f;
+        if (on) {
+          nn_feats<F>(pyr, pg, K.ft, p, mk3(-dir.x, -dir.y, -dir.z), L, f);
+#pragma unroll
+          for (int c = 0; c < kNFeat; ++c) ood |= (f[c] < nk.lo[c]) | (f[c] > nk.hi[c]);
+          // the network-free estimate now, so the features die inside the network's input staging
+          nn_base(f, float(K.n_occ - 1) * K.ring_cos, bo, bs);
+        } else {
+#pragma unroll
+          for (int c = 0; c < kNFeat; ++c) f[c] = 0.f;
         }
-      }
-      next += n_idle;
-    }
-    const bool busy = pix >= 0;
-    if (!__any(busy)) {
-      if (next >= total) break;
-      continue;
-    }
-    // one sample of every marching lane; a lane whose sample needs shading parks on it
-    // (keeps p, h, src) while the others march on
-    bool finished = false;
-    if (busy && !parked) {
-      const float s = float(j) * step;
-      if (!(s < D) || j >= kMaxSamples) {
-        finished = true;
-      } else {
-        h = fminf(step, D - s);
-        p = tp + dir * (s + 0.5f * h);
-        src = sample_tf(s_tf, ntf, volume_oct_lerp<T>(g, rec, p));
-        rec = volume_oct_load<T>(g, pos(j + 1));
-        ++cnt[0];
-        if (src.w > 0.f) parked = true;
-        else ++j;
-      }
-    }
-    // the wave shades all parked samples together once enough lanes wait, or when every
-    // marching lane waits
-    const int np = __popcll(__ballot(parked)), na = __popcll(__ballot(busy && !finished));
-    if (np > 0 && (np == na || float(np) >= sc.park * float(na))) {
-      float f[kNFeat];
-      bool ood = false;
-      float bo = 0.f, bs = 0.f;
-      if (parked) {
-        nn_feats<F>(pyr, pg, K.ft, p, mk3(-dir.x, -dir.y, -dir.z), L, f);
-#pragma unroll
-        for (int c = 0; c < kNFeat; ++c) ood |= (f[c] < nk.lo[c]) | (f[c] > nk.hi[c]);
-        // the network-free estimate now, so the features die inside the network's input staging
-        nn_base(f, float(K.n_occ - 1) * K.ring_cos, bo, bs);
-      } else {
-#pragma unroll
-        for (int c = 0; c < kNFeat; ++c) f[c] = 0.f;
-      }
-      float Io, Is;
-      mlp_wave(sW, sB, sXw, f, Io, Is);
-      if (parked) {
+        float Io, Is;
+        mlp_wave(sW, sB, sXw, f, Io, Is);
         Io += bo;
         Is += bs;
-        ++cnt[1];
         if (!kExact) {
           ood_seen |= ood;
-        } else if (ood || nk.exact_all) {
+        } else if (on && (ood || nk.exact_all)) {
           ++cnt[2];
           f3 k, up, right;
           occ_frame(dir, k, up, right);
@@ -292,23 +208,8 @@ __device__ __forceinline__ bool nn_tile(const RayFrame& rf, const VolGeom& g, co
         }
         Io = fminf(fmaxf(Io, 0.f), 1.f);
         Is = fminf(fmaxf(Is, 0.f), 1.f);
-        const float m = inv_k * (Io * ka + Is * kd);
-        const float a = 1.0f - __expf(-src.w * h);
-        const float wgt = (1.0f - dst.w) * a;
-        dst.x += wgt * src.x * m;
-        dst.y += wgt * src.y * m;
-        dst.z += wgt * src.z * m;
-        dst.w += wgt;
-        ++j;
-        parked = false;
-        if (dst.w > et) finished = true;
-      }
-    }
-    if (finished) {
-      out[size_t(py) * rf.W + px] = dst;
-      pix = -1;
-    }
-  }
+        return Lit{inv_k * (Io * ka + Is * kd), 0.f};
+      });
   return __any(ood_seen);
 }
 

@@ -1,14 +1,19 @@
 // Batched surrogate rendering (gfx950): many (volume, camera, light) jobs in one
 // persistent launch, captured in a HIP graph.
 //
-// Work items are (job, workgroup tile) pairs.  With 8 queues the tiles of every job are
-// cut into 8 bands of tile rows and band x goes to queue x; a workgroup starts on the
-// queue of the XCD it runs on (the hardware deals workgroups round-robin over the 8
-// XCDs, so blockIdx % 8), which keeps neighbouring tiles of one image in one XCD's L2,
-// and steals from the other queues once its own is empty.  Items are ordered volume by
-// volume (largest volume first), so a workgroup restages the network and transfer
-// function in LDS only when the volume changes.  Each tile is rendered by the same
-// device code as the single-frame surrogate renderer.
+// Work items are runs of 16 x span pixels of a wave tile, pulled by single wavefronts.  With 8
+// queues the supertiles of every job are dealt to them in turn; a wavefront starts on the
+// queue of the XCD it runs on (the hardware deals workgroups round-robin over the 8 XCDs, so
+// blockIdx % 8), which keeps neighbouring tiles of one image in one XCD's L2, and steals from
+// the other queues once its own is empty.  A workgroup goes through the volumes and holds one
+// volume's network and transfer function in LDS: its wavefronts wait for each other only
+// between volumes (with a barrier at each item, of 256 pixels, they waited for the slowest of
+// four).  Workgroups begin with different volumes, so that all of them are in work at once: when
+// every workgroup began with the largest, each volume had its own tail of waiting wavefronts.
+// 32 images of 256^2 over four volumes of 64^3 to 256^3: 6.6 ms with a barrier at each item, 4.7
+// from the largest on, 4.0 now; 8 of 138 x 147 over four of 43 x 43 x 62: 0.69, 1.10 and 0.41.
+// Which item a queue position is follows from its number, so there is no item list.  Each item
+// is rendered by the same device code as the single-frame surrogate renderer.
 #include "cvr_nn.hpp"
 #include <algorithm>
 #include <cmath>
@@ -38,65 +43,109 @@ struct JobDesc {
   int vol;
 };
 
-constexpr int kQueues = 8;
+constexpr int kQueues = 8, kMaxVolumes = 64;
+
+// The jobs of one volume (a range of the job order), largest volume first.
+struct VolJobs {
+  int vol, first, count;
+};
+// Tiles of an image in supertiles of 64, dealt to the queues in turn, each cut into kCuts items.
+constexpr int kCuts = 4;
+struct BatchShape {
+  int tiles_x, tiles_y, tw_log2, span, nq, nvols;
+};
+// Tiles of one image in queue q.
+__host__ __device__ inline int queue_tiles(const BatchShape& s, int q) {
+  const int t = s.tiles_x * s.tiles_y, st = (t + 63) >> 6;  // tiles, supertiles
+  if (q >= st) return 0;
+  const int mine = (st - 1 - q) / s.nq + 1;
+  return (st - 1) % s.nq == q ? (mine - 1) * 64 + t - (st - 1) * 64 : mine * 64;
+}
+
+// The pixels of an item: from pixel `first` of a stack of wave tiles, row by row.
+struct TilePixels {
+  const RayFrame& rf;
+  int x0, y0, tw_log2, first;
+  __device__ __forceinline__ bool operator()(int k, int& px, int& py) const {
+    k += first;
+    px = x0 + (k & ((1 << tw_log2) - 1));
+    py = y0 + (k >> tw_log2);
+    return px < rf.W && py < rf.H;
+  }
+};
 
 // Clears the queue heads and the counters (a kernel, so that it can sit in the graph).
-__global__ __launch_bounds__(64) void k_batch_reset(unsigned int* __restrict__ heads,
+__global__ __launch_bounds__(kQueues * kMaxVolumes) void k_batch_reset(unsigned int* __restrict__ heads,
                                                     unsigned long long* __restrict__ counters) {
-  if (threadIdx.x < kQueues) heads[threadIdx.x] = 0u;
+  heads[threadIdx.x] = 0u;
   if (threadIdx.x < 4) counters[threadIdx.x] = 0ull;
 }
 
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_batch_render(const VolDesc* __restrict__ vols, const JobDesc* __restrict__ jobs,
-                                                      const int2* __restrict__ items, const int* __restrict__ qoff,
-                                                      int nq, int tiles_x, NnSched sc, size_t img_px,
+                                                      const VolJobs* __restrict__ vjobs, const int* __restrict__ order,
+                                                      BatchShape bs, size_t img_px,
                                                       float4* __restrict__ out, unsigned int* __restrict__ heads,
                                                       unsigned long long* __restrict__ counters) {
   __shared__ __align__(16) short sW[kPackShorts];
   __shared__ __align__(16) float sB[kNBias];
   __shared__ __align__(16) float sX[4][kWaveScratch];
-  __shared__ int s_item;
+  __shared__ WaveQueue<kNnRays> queue[4];
+  __shared__ int s_left;
   extern __shared__ float4 s_tf[];
-  const int home = int(blockIdx.x) % nq;
-  int loaded = -1;
+  const int home = int(blockIdx.x) % bs.nq, w = threadIdx.x >> 6;
+  const int tw = 1 << bs.tw_log2, th = (64 >> bs.tw_log2) * bs.span, item_px = 64 * bs.span / kCuts;
   unsigned int cnt[3] = {0, 0, 0};
-  for (int qi = 0; qi < nq; ++qi) {
-    const int q = (home + qi) % nq;
-    const int base = qoff[q], n = qoff[q + 1] - base;
-    for (;;) {
-      if (threadIdx.x == 0) s_item = int(atomicAdd(&heads[q], 1u));
-      __syncthreads();
-      const int idx = __builtin_amdgcn_readfirstlane(s_item);
-      __syncthreads();  // every lane has read s_item before lane 0 may write it again
-      if (idx >= n) break;
-      const int2 it = items[base + idx];  // (job, tile)
-      const int job = __builtin_amdgcn_readfirstlane(it.x), tile = __builtin_amdgcn_readfirstlane(it.y);
-      const JobDesc& J = jobs[job];
-      const VolDesc& V = vols[J.vol];
-      if (J.vol != loaded) {
-        // the barrier above guarantees no wave still reads the previous volume's tables
-        nn_stage(V.wpack, V.bpack, V.tf, V.ntf, sW, sB, s_tf);
-        loaded = J.vol;
-        __syncthreads();
-      }
-      ConeK K = V.K;
-      K.L[0] = J.L[0];
-      K.L[1] = J.L[1];
-      K.L[2] = J.L[2];
-      float4* o = out + size_t(job) * img_px;
-#define CVR_BATCH_TILE(TT, FF)                                                                                    \
-  nn_tile<TT, FF>(J.rf, V.g, V.pg, V.pyr, K, V.nk, sc, sW, sB, sX[threadIdx.x >> 6], s_tf, V.ntf, V.step, V.et, o, \
-                  tile % tiles_x, tile / tiles_x, cnt)
-      switch (V.g.dtype * 3 + V.pg.fmt) {
-        case 0: CVR_BATCH_TILE(uint8_t, 0); break;
-        case 1: CVR_BATCH_TILE(uint8_t, 1); break;
-        case 2: CVR_BATCH_TILE(uint8_t, 2); break;
-        case 3: CVR_BATCH_TILE(uint16_t, 0); break;
-        case 4: CVR_BATCH_TILE(uint16_t, 1); break;
-        default: CVR_BATCH_TILE(uint16_t, 2); break;
-      }
-#undef CVR_BATCH_TILE
+  for (int vi = 0; vi < bs.nvols; ++vi) {
+    const int v = (int(blockIdx.x) / bs.nq + vi) % bs.nvols;
+    const VolJobs vj = vjobs[v];
+    unsigned int* vheads = heads + v * kQueues;
+    if (threadIdx.x == 0) {
+      int left = 0;
+      for (int q = 0; q < bs.nq; ++q)
+        left |= int(__hip_atomic_load(&vheads[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) <
+                vj.count * queue_tiles(bs, q) * kCuts;
+      s_left = left;
     }
+    __syncthreads();  // and no wavefront reads the volume before's tables any more
+    const int left = s_left;
+    __syncthreads();  // every lane has read s_left
+    if (!left) continue;
+    const VolDesc& V = vols[vj.vol];
+    nn_stage(V.wpack, V.bpack, V.tf, V.ntf, sW, sB, s_tf);
+    __syncthreads();
+    for (int qi = 0; qi < bs.nq; ++qi) {
+      const int q = (home + qi) % bs.nq, per_job = queue_tiles(bs, q) * kCuts, n = vj.count * per_job;
+      for (;;) {
+        int idx = 0;
+        if ((threadIdx.x & 63) == 0) idx = int(atomicAdd(&vheads[q], 1u));
+        idx = __builtin_amdgcn_readfirstlane(idx);
+        if (idx >= n) break;
+        const int job = order[vj.first + idx / per_job], r = idx % per_job, cut = r % kCuts, t = r / kCuts;
+        int tx, ty;
+        super_tile(((t >> 6) * bs.nq + q) * 64 + (t & 63), bs.tiles_x, bs.tiles_y, tw, 16, tx, ty);
+        const JobDesc& J = jobs[job];
+        ConeK K = V.K;
+        K.L[0] = J.L[0];
+        K.L[1] = J.L[1];
+        K.L[2] = J.L[2];
+        float4* o = out + size_t(job) * img_px;
+#define CVR_BATCH_ITEM(TT, FF)                                                                                      \
+  for (int p = 0; p < item_px; p += kNnRays)                                                                        \
+  nn_march<TT, FF, true>(J.rf, V.g, V.pg, V.pyr, K, V.nk, sW, sB, sX[w], s_tf, V.ntf, V.step, V.et,                 \
+                         kNnRays,          \
+                         TilePixels{J.rf, tx * tw, ty * th, bs.tw_log2, cut * item_px + p}, queue[w], o, cnt)
+        switch (V.g.dtype * 3 + V.pg.fmt) {
+          case 0: CVR_BATCH_ITEM(uint8_t, 0); break;
+          case 1: CVR_BATCH_ITEM(uint8_t, 1); break;
+          case 2: CVR_BATCH_ITEM(uint8_t, 2); break;
+          case 3: CVR_BATCH_ITEM(uint16_t, 0); break;
+          case 4: CVR_BATCH_ITEM(uint16_t, 1); break;
+          default: CVR_BATCH_ITEM(uint16_t, 2); break;
+        }
+#undef CVR_BATCH_ITEM
+      }
+    }
+    __syncthreads();
   }
   if (counters) {
     atomicAdd(&counters[0], (unsigned long long)cnt[0]);
@@ -158,11 +207,12 @@ struct cvr_batch {
   // device side
   VolDesc* d_vols = nullptr;
   JobDesc* d_jobs = nullptr;
-  int2* d_items = nullptr;
-  int* d_qoff = nullptr;
+  VolJobs* d_vjobs = nullptr;
+  int* d_order = nullptr;
   unsigned int* d_heads = nullptr;
   unsigned long long* d_counters = nullptr;
-  size_t cap_vols = 0, cap_jobs = 0, cap_items = 0;
+  size_t cap_vols = 0, cap_jobs = 0, cap_vjobs = 0, cap_order = 0;
+  int n_vjobs = 0;
   int max_ntf = 0;
   // graph of (reset, render) for the current jobs / tuning / output
   hipStream_t cap = nullptr;
@@ -295,35 +345,22 @@ int build_tables(cvr_batch* b) {
     if (cells[va] != cells[vc]) return cells[va] > cells[vc];
     return va < vc;
   });
-  const int tl = tw_log2_of(b->tune.tile_w), tw = 1 << tl, th = (64 >> tl) * b->tune.span;
-  const int tiles_x = (b->W + 2 * tw - 1) / (2 * tw), tiles_y = (b->H + 2 * th - 1) / (2 * th);
-  const int nq = b->tune.queues;
-  // Every image's tiles in supertile order (super_tile); with 8 queues (one per XCD:
-  // workgroup b starts at queue b % 8) queue q takes supertiles q, q + 8, ... of each
-  // image, so the 8 XCDs render 8 adjacent supertiles of one image at a time, as the
-  // single-frame renderers' block order does.
-  std::vector<std::vector<int2>> q(nq);
-  for (int j : order)
-    for (int b = 0; b < tiles_x * tiles_y; ++b) {
-      int tx, ty;
-      super_tile(b, tiles_x, tiles_y, 2 * tw, 16, tx, ty);
-      q[(b >> 6) % nq].push_back(make_int2(j, ty * tiles_x + tx));
-    }
-  std::vector<int2> items;
-  std::vector<int> qoff(kQueues + 1, 0);
-  for (int i = 0; i < nq; ++i) {
-    qoff[i] = int(items.size());
-    items.insert(items.end(), q[i].begin(), q[i].end());
+  std::vector<VolJobs> vj;
+  for (int i = 0; i < nj; ++i) {
+    const int v = b->jobs[order[i]].volume;
+    if (vj.empty() || vj.back().vol != v) vj.push_back(VolJobs{v, i, 0});
+    ++vj.back().count;
   }
-  for (int i = nq; i <= kQueues; ++i) qoff[i] = int(items.size());
+  b->n_vjobs = int(vj.size());
   int rc;
   if ((rc = grow(reinterpret_cast<void**>(&b->d_vols), b->cap_vols, vd.size() * sizeof(VolDesc)))) return rc;
   if ((rc = grow(reinterpret_cast<void**>(&b->d_jobs), b->cap_jobs, jd.size() * sizeof(JobDesc)))) return rc;
-  if ((rc = grow(reinterpret_cast<void**>(&b->d_items), b->cap_items, items.size() * sizeof(int2)))) return rc;
+  if ((rc = grow(reinterpret_cast<void**>(&b->d_vjobs), b->cap_vjobs, vj.size() * sizeof(VolJobs)))) return rc;
+  if ((rc = grow(reinterpret_cast<void**>(&b->d_order), b->cap_order, order.size() * sizeof(int)))) return rc;
   CVR_HIP_CHECK(hipMemcpy(b->d_vols, vd.data(), vd.size() * sizeof(VolDesc), hipMemcpyHostToDevice));
   CVR_HIP_CHECK(hipMemcpy(b->d_jobs, jd.data(), jd.size() * sizeof(JobDesc), hipMemcpyHostToDevice));
-  CVR_HIP_CHECK(hipMemcpy(b->d_items, items.data(), items.size() * sizeof(int2), hipMemcpyHostToDevice));
-  CVR_HIP_CHECK(hipMemcpy(b->d_qoff, qoff.data(), qoff.size() * sizeof(int), hipMemcpyHostToDevice));
+  CVR_HIP_CHECK(hipMemcpy(b->d_vjobs, vj.data(), vj.size() * sizeof(VolJobs), hipMemcpyHostToDevice));
+  CVR_HIP_CHECK(hipMemcpy(b->d_order, order.data(), order.size() * sizeof(int), hipMemcpyHostToDevice));
   b->tables_dirty = false;
   return CVR_OK;
 }
@@ -333,15 +370,13 @@ int build_graph(cvr_batch* b, float* out) {
   int ncu = 0;
   CVR_HIP_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, b->device));
   const int grid = std::max(1, ncu * b->tune.workgroups_per_cu);
-  const int tl = tw_log2_of(b->tune.tile_w), tw = 1 << tl;
-  const int tiles_x = (b->W + 2 * tw - 1) / (2 * tw);
-  NnSched sc{tl, b->tune.shade_batch, b->tune.span};
+  const int tl = tw_log2_of(b->tune.tile_w), tw = 1 << tl, th = (64 >> tl) * b->tune.span;
+  const BatchShape bs{(b->W + tw - 1) / tw, (b->H + th - 1) / th, tl, b->tune.span, b->tune.queues, b->n_vjobs};
   const size_t shm = size_t(b->max_ntf) * sizeof(float4);
   CVR_HIP_CHECK(hipStreamBeginCapture(b->cap, hipStreamCaptureModeThreadLocal));
-  hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(64), 0, b->cap, b->d_heads, b->d_counters);
-  hipLaunchKernelGGL(k_batch_render, dim3(grid), dim3(256), shm, b->cap, b->d_vols, b->d_jobs, b->d_items, b->d_qoff,
-                     b->tune.queues, tiles_x, sc, size_t(b->W) * b->H, reinterpret_cast<float4*>(out), b->d_heads,
-                     b->d_counters);
+  hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(kQueues * kMaxVolumes), 0, b->cap, b->d_heads, b->d_counters);
+  hipLaunchKernelGGL(k_batch_render, dim3(grid), dim3(256), shm, b->cap, b->d_vols, b->d_jobs, b->d_vjobs, b->d_order, bs,
+                     size_t(b->W) * b->H, reinterpret_cast<float4*>(out), b->d_heads, b->d_counters);
   const hipError_t le = hipGetLastError();
   hipGraph_t g = nullptr;
   const hipError_t ce = hipStreamEndCapture(b->cap, &g);
@@ -440,9 +475,8 @@ int cvr_batch_create(int device, int width, int height, cvr_batch_handle* out) {
   b->device = device;
   b->W = width;
   b->H = height;
-  if (hipMalloc(&b->d_heads, kQueues * sizeof(unsigned int)) != hipSuccess ||
+  if (hipMalloc(&b->d_heads, kQueues * kMaxVolumes * sizeof(unsigned int)) != hipSuccess ||
       hipMalloc(&b->d_counters, 4 * sizeof(unsigned long long)) != hipSuccess ||
-      hipMalloc(&b->d_qoff, (kQueues + 1) * sizeof(int)) != hipSuccess ||
       hipStreamCreateWithFlags(&b->cap, hipStreamNonBlocking) != hipSuccess) {
     cvr_batch_destroy(b);
     set_error("cvr_batch_create: HIP allocation failed");
@@ -457,8 +491,8 @@ void cvr_batch_destroy(cvr_batch_handle b) {
   Guard gd(b->device);
   (void)hipDeviceSynchronize();
   drop_graph(b);
-  for (void* p : {static_cast<void*>(b->d_vols), static_cast<void*>(b->d_jobs), static_cast<void*>(b->d_items),
-                  static_cast<void*>(b->d_qoff), static_cast<void*>(b->d_heads), static_cast<void*>(b->d_counters)})
+  for (void* p : {static_cast<void*>(b->d_vols), static_cast<void*>(b->d_jobs), static_cast<void*>(b->d_vjobs),
+                  static_cast<void*>(b->d_order), static_cast<void*>(b->d_heads), static_cast<void*>(b->d_counters)})
     if (p) (void)hipFree(p);
   if (b->cap) (void)hipStreamDestroy(b->cap);
   delete b;
@@ -469,7 +503,7 @@ int cvr_batch_add_volume(cvr_batch_handle b, cvr_handle h, int* index) {
   if (h->technique != CVR_CONE_NN) { set_error("cvr_batch_add_volume: the handle must be CVR_CONE_NN"); return CVR_ERR_UNSUPPORTED; }
   if (h->device != b->device) { set_error("cvr_batch_add_volume: handle on another device"); return CVR_ERR_INVALID; }
   if (!h->d_vol || !h->d_tf_rgbt) { set_error("cvr_batch_add_volume: volume and transfer function must be set"); return CVR_ERR_STATE; }
-  if (b->vols.size() >= 64) { set_error("cvr_batch_add_volume: at most 64 volumes"); return CVR_ERR_INVALID; }
+  if (b->vols.size() >= size_t(kMaxVolumes)) { set_error("cvr_batch_add_volume: at most 64 volumes"); return CVR_ERR_INVALID; }
   b->vols.push_back(h);
   if (index) *index = int(b->vols.size()) - 1;
   b->tables_dirty = b->dirty = true;
@@ -503,10 +537,9 @@ int cvr_batch_set_tuning(cvr_batch_handle b, const cvr_batch_tuning* t) {
   if (!b || !t) { set_error("cvr_batch_set_tuning: null argument"); return CVR_ERR_INVALID; }
   int rc = check_tuning(*t);
   if (rc) return rc;
-  const bool items_change = t->tile_w != b->tune.tile_w || t->queues != b->tune.queues || t->span != b->tune.span ||
-                            t->step_scale != b->tune.step_scale;
+  // the step is in the volume descriptors, the work shape in the captured launch
+  if (t->step_scale != b->tune.step_scale) b->tables_dirty = true;
   b->tune = *t;
-  if (items_change) b->tables_dirty = true;
   b->dirty = true;
   return CVR_OK;
 }
@@ -566,8 +599,8 @@ int cvr_batch_autotune(cvr_batch_handle b, float* out, int stride, void* hip_str
     return CVR_OK;
   };
   // the step schedule first (its images against the step_scale 1 images of the same
-  // jobs), then coordinate descent over tile width, shading batch, queues, workgroups
-  // per CU and span at the chosen step
+  // jobs), then coordinate descent over tile width, queues, workgroups per CU and span at the
+  // chosen step
   cvr_batch_tuning cur = b->tune;
   cur.step_rmse = 0.0;
   double cur_ms = 0;
@@ -575,21 +608,19 @@ int cvr_batch_autotune(cvr_batch_handle b, float* out, int stride, void* hip_str
   if (cur.max_step_rmse > 0.f) rc = tune_step(b, out, st, time_of, cur, cur_ms);
   else rc = time_of(cur, &cur_ms);
   const int tws[] = {4, 8, 16, 32};
-  const float sbs[] = {0.f, 0.25f, 0.5f, 0.75f, 1.f};
   const int qs[] = {1, kQueues};
   const int wgs[] = {1, 2, 3};
   const int spans[] = {1, 2, 4, 8};
-  for (int pass = 0; pass < 5 && rc == CVR_OK; ++pass) {
-    const int nopt = pass == 0 ? 4 : pass == 1 ? 5 : pass == 2 ? 2 : pass == 3 ? 3 : 4;
+  for (int pass = 0; pass < 4 && rc == CVR_OK; ++pass) {
+    const int nopt = pass == 0 ? 4 : pass == 1 ? 2 : pass == 2 ? 3 : 4;
     for (int o = 0; o < nopt && rc == CVR_OK; ++o) {
       cvr_batch_tuning t = cur;
       if (pass == 0) t.tile_w = tws[o];
-      if (pass == 1) t.shade_batch = sbs[o];
-      if (pass == 2) t.queues = qs[o];
-      if (pass == 3) t.workgroups_per_cu = wgs[o];
-      if (pass == 4) t.span = spans[o];
-      if (t.tile_w == cur.tile_w && t.shade_batch == cur.shade_batch && t.queues == cur.queues &&
-          t.workgroups_per_cu == cur.workgroups_per_cu && t.span == cur.span)
+      if (pass == 1) t.queues = qs[o];
+      if (pass == 2) t.workgroups_per_cu = wgs[o];
+      if (pass == 3) t.span = spans[o];
+      if (t.tile_w == cur.tile_w && t.queues == cur.queues && t.workgroups_per_cu == cur.workgroups_per_cu &&
+          t.span == cur.span)
         continue;
       double ms = 0;
       rc = time_of(t, &ms);

@@ -593,37 +593,38 @@ __global__ void k_feat_range(const float* __restrict__ X, int n, unsigned int* _
 }
 
 // ---------------------------------------------------------------- surrogate renderer
-// Two passes over the same tiles.  kExact = false renders every tile with the network
-// alone and marks (redo[tile] = 1) the tiles where some sample's inputs left the
-// training range; kExact = true then renders only the marked tiles again, exact cone
-// tracer for those samples, and clears their marks, so every mark is 0 between frames.
+// Two passes over the same rays.  kExact = false renders every ray with the network alone
+// and marks (redo[workgroup] = 1) the workgroups where some sample's inputs left the
+// training range; kExact = true then renders only the marked workgroups' rays again, exact
+// cone tracer for those samples, and clears their marks, so every mark is 0 between frames.
 // The first pass carries no exact-tracer code (its registers and scalar state serve the
 // march, the features and the network alone); the second costs one launch when nothing
 // is marked.  Counters: samples and shaded samples from the first pass, exact fallbacks
-// from the second (which marches a tile exactly as the first did).
+// from the second (which marches a ray exactly as the first did).  A wavefront takes
+// the rays of `sets` units.
 template <typename T, int F, bool kExact>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_nn_render(RayFrame rf, VolGeom g, PyrGeom pg, const void* __restrict__ pyr,
-                                                   ConeK K, NnK nk, NnSched sc, const short* __restrict__ wpack,
+                                                   ConeK K, NnK nk, const short* __restrict__ wpack,
                                                    const float* __restrict__ bpack, const float4* __restrict__ tf,
-                                                   int ntf, float step, float et, float4* __restrict__ out,
+                                                   int ntf, float step, float et, QueueShape qs, int sets,
+                                                   float4* __restrict__ out,
                                                    unsigned int* __restrict__ redo, unsigned long long* __restrict__ counters) {
   __shared__ __align__(16) short sW[kPackShorts];
   __shared__ __align__(16) float sB[kNBias];
   __shared__ __align__(16) float sX[4][kWaveScratch];
+  __shared__ WaveQueue<kNnRays> queue[4];
   extern __shared__ float4 s_tf[];
-  const int bid = xcd_remap(blockIdx.x, gridDim.x);
+  const int bid = xcd_remap(blockIdx.x, gridDim.x, qs.xcd_log2);
   if (kExact && redo[bid] == 0u) return;  // the same word for every thread of the block
   nn_stage(wpack, bpack, tf, ntf, sW, sB, s_tf);
   __syncthreads();
   if (kExact && threadIdx.x == 0) redo[bid] = 0u;  // every thread has read it (barrier above)
-  const int tw = 1 << sc.tw_log2;
-  const int tiles_x = (rf.W + 2 * tw - 1) / (2 * tw);
+  const int w = threadIdx.x >> 6, u = bid * 4 + w;
   unsigned int cnt[3] = {0, 0, 0};
-  const int th = (64 >> sc.tw_log2) * sc.span;
-  int tx, ty;
-  super_tile(bid, tiles_x, (rf.H + 2 * th - 1) / (2 * th), 2 * tw, 16, tx, ty);
-  const bool marked = nn_tile<T, F, kExact>(rf, g, pg, pyr, K, nk, sc, sW, sB, sX[threadIdx.x >> 6], s_tf, ntf, step,
-                                            et, out, tx, ty, cnt);
+  bool marked = false;
+  for (int s = 0; s < sets; ++s)
+    marked |= nn_march<T, F, kExact>(rf, g, pg, pyr, K, nk, sW, sB, sX[w], s_tf, ntf, step, et, qs.rays,
+                                     FramePixels(rf, qs, u * sets + s, 64 / kNnSub), queue[w], out, cnt);
   if (!kExact && marked && (threadIdx.x & 63) == 0) redo[bid] = 1u;
   if (counters) {
     if (!kExact) {
@@ -898,19 +899,26 @@ NnK nn_consts(cvr_ctx* c) {
   return nk;
 }
 
-// Work shape of a surrogate frame: the schedule and the number of workgroup tiles.
-static NnSched nn_sched(const cvr_nn_params& N) {
-  NnSched sc{0, N.shade_batch, N.span};
-  while ((1 << sc.tw_log2) < N.tile_w) ++sc.tw_log2;
-  return sc;
+// A surrogate frame's rays: 16 per wavefront, 4 in small frames (512^3 at 1024^2 4.74 ms and
+// 4.89 ms; 100 x 90 x 80 at 200 x 150 0.2 and 0.1 ms).  A wavefront takes its rays of `sets`
+// units: more than one for frames of more than kMaxBlocks workgroups, whose marks would not
+// fit cvr_render_noalloc's array.
+constexpr int kMaxBlocks = 1 << 16;
+static QueueShape nn_shape(const RayFrame& rf, int& sets) {
+  QueueShape q = queue_shape(rf, size_t(rf.W) * rf.H < (1 << 16) ? 4 : 16, 1, 64);
+  sets = (q.blocks + kMaxBlocks - 1) / kMaxBlocks;
+  q.blocks = (q.blocks + sets - 1) / sets;
+  return q;
 }
-static int nn_tiles(const NnSched& sc, const RayFrame& rf) {
-  const int tw = 1 << sc.tw_log2, th = (64 / tw) * sc.span;
-  return ((rf.W + 2 * tw - 1) / (2 * tw)) * ((rf.H + 2 * th - 1) / (2 * th));
+// The workgroup tiles of the frame as cvr_render_noalloc counts them against its limit:
+// 2 x 2 wave tiles of tile_w x 64 / tile_w pixels, `span` of them stacked.
+static long long noalloc_tiles(const cvr_nn_params& N, const RayFrame& rf) {
+  const int tw = N.tile_w, th = (64 / tw) * N.span;
+  return (long long)((rf.W + 2 * tw - 1) / (2 * tw)) * ((rf.H + 2 * th - 1) / (2 * th));
 }
 
 // The frame of a prepared, trained handle: the exact tracer when the validation gate is
-// closed, else the two passes of k_nn_render over `redo` (one word per workgroup tile,
+// closed, else the two passes of k_nn_render over `redo` (one word per workgroup,
 // zero on entry and left zero by the second pass).  Allocates nothing.
 static int nn_frame(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out, unsigned int* redo,
                     unsigned long long* cnt, hipStream_t st) {
@@ -929,8 +937,8 @@ static int nn_frame(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, floa
   }
   VolGeom g = geom_of(c);
   const float step = N.cone.step_size > 0 ? N.cone.step_size : default_step(c);
-  const NnSched sc = nn_sched(N);
-  const int tiles = nn_tiles(sc, rf);
+  int sets = 1;
+  const QueueShape sh = nn_shape(rf, sets);
   const size_t shm = size_t(c->tf_size) * sizeof(float4);
   if (shm > 32 * 1024) { set_error("surrogate renderer: transfer function larger than 2048 entries"); return -4; }
   short* wp = static_cast<short*>(c->d_nn_pack);
@@ -939,10 +947,10 @@ static int nn_frame(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, floa
   with_types(c->dtype, c->pyr.fmt, [&](auto t, auto f) {
     using T = typename decltype(t)::type;
     constexpr int FF = decltype(f)::value;
-    hipLaunchKernelGGL((k_nn_render<T, FF, false>), dim3(tiles), dim3(256), shm, st, rf, g, c->pyr, c->d_pyr_oct, K,
-                       nk, sc, wp, bp, c->d_tf_rgbt, c->tf_size, step, N.cone.et_threshold, o4, redo, cnt);
-    hipLaunchKernelGGL((k_nn_render<T, FF, true>), dim3(tiles), dim3(256), shm, st, rf, g, c->pyr, c->d_pyr_oct, K,
-                       nk, sc, wp, bp, c->d_tf_rgbt, c->tf_size, step, N.cone.et_threshold, o4, redo, cnt);
+    hipLaunchKernelGGL((k_nn_render<T, FF, false>), dim3(sh.blocks), dim3(256), shm, st, rf, g, c->pyr, c->d_pyr_oct,
+                       K, nk, wp, bp, c->d_tf_rgbt, c->tf_size, step, N.cone.et_threshold, sh, sets, o4, redo, cnt);
+    hipLaunchKernelGGL((k_nn_render<T, FF, true>), dim3(sh.blocks), dim3(256), shm, st, rf, g, c->pyr, c->d_pyr_oct,
+                       K, nk, wp, bp, c->d_tf_rgbt, c->tf_size, step, N.cone.et_threshold, sh, sets, o4, redo, cnt);
   });
   CVR_HIP_CHECK(hipGetLastError());
   return 0;
@@ -956,8 +964,9 @@ int launch_nn(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out
     rc = nn_train(c, st);
     if (rc) return rc;
   }
-  const int tiles = nn_tiles(nn_sched(N), rf);
-  // tile marks for the second pass: zero when allocated, and the second pass clears
+  int sets = 1;
+  const int tiles = nn_shape(rf, sets).blocks;
+  // workgroup marks for the second pass: zero when allocated, and the second pass clears
   // what the first sets
   if (size_t(tiles) > c->nn_redo_cap) {
     if (c->d_nn_redo) CVR_HIP_CHECK(hipFree(c->d_nn_redo));
@@ -980,6 +989,7 @@ int launch_nn(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out
 // own copy of `scratch` (256 KiB) until the process ends; host code uses only the
 // address hipGetSymbolAddress gives for the current device, never the array's name.
 constexpr int kNoAllocMaxTiles = 1 << 16;
+static_assert(kMaxBlocks <= kNoAllocMaxTiles, "a frame's marks fit the array");
 static __device__ __align__(256) unsigned int scratch[kNoAllocMaxTiles];
 constexpr int kMaxDevices = 64;
 static unsigned int* g_scratch[kMaxDevices];
@@ -1029,7 +1039,7 @@ extern "C" int cvr_render_noalloc(cvr_handle h, const cvr_camera* cam, const cvr
     return CVR_ERR_STATE;
   }
   const RayFrame rf = frame_of(cam, width, height);
-  const int tiles = nn_tiles(nn_sched(h->nn), rf);
+  const long long tiles = noalloc_tiles(h->nn, rf);
   if (tiles > kNoAllocMaxTiles) {
     set_error("cvr_render_noalloc: the frame needs " + std::to_string(tiles) + " workgroup tiles, above the limit of " +
               std::to_string(kNoAllocMaxTiles) + " (4096 x 4096 pixels at 4 x 16-pixel wave tiles)");
@@ -1053,7 +1063,9 @@ extern "C" int cvr_render_noalloc(cvr_handle h, const cvr_camera* cam, const cvr
   if (rc) return rc;
   hipStream_t st = static_cast<hipStream_t>(hip_stream);
   // the marks must start at zero: a fill kernel (not a memset node) keeps the call capturable
-  hipLaunchKernelGGL(k_clear_marks, dim3((tiles + 255) / 256), dim3(256), 0, st, marks, tiles);
+  int sets = 1;
+  const int blocks = nn_shape(rf, sets).blocks;
+  hipLaunchKernelGGL(k_clear_marks, dim3((blocks + 255) / 256), dim3(256), 0, st, marks, blocks);
   CVR_HIP_CHECK(hipGetLastError());
   return nn_frame(h, rf, light, out_device, marks, nullptr, st);
 }

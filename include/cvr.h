@@ -233,13 +233,13 @@ typedef struct cvr_nn_params {
   float ood_margin;     /* inputs this far outside the training range use the exact tracer (0.02) */
   int force_exact;      /* nonzero: every sample uses the exact tracer */
   uint64_t seed;        /* training-set and initialisation seed */
-  /* Work shape of the renderer (pixels do not depend on it): wavefront tile width in
-   * pixels (4, 8, 16 or 32; the height is 64 / width) and the fraction of a wave's
-   * marching lanes that must wait on a shaded sample before the wave shades them
-   * together (0: as soon as one waits). */
+  /* Work shape (pixels do not depend on it; a single frame takes its shape from its size
+   * and reads these only for the limit of cvr_render_noalloc, 65536 tiles of 2 x 2 stacks
+   * of `span` wave tiles): wavefront tile width in pixels (4, 8, 16 or 32; the height is
+   * 64 / width), a fraction in [0, 1] without effect, and the stack's height. */
   int tile_w;           /* 4 */
   float shade_batch;    /* 0.75 */
-  int span;             /* wave tiles per wavefront, handed to lanes as their rays end: 1, 2, 4 or 8 (1) */
+  int span;             /* wave tiles of a stack: 1, 2, 4 or 8 (1) */
 } cvr_nn_params;
 
 typedef struct cvr_nn_report {
@@ -464,10 +464,10 @@ typedef struct cvr_job {
  * pixels, within the image error the autotuner accepts for it. */
 typedef struct cvr_batch_tuning {
   int tile_w;            /* wavefront tile width: 4, 8, 16 or 32 pixels (height 64 / width) */
-  float shade_batch;     /* fraction of marching lanes that wait before a shading pass, [0, 1] */
+  float shade_batch;     /* [0, 1], without effect: samples are always shaded 64 at a time */
   int queues;            /* 1: one global queue; 8: one queue per XCD with stealing */
   int workgroups_per_cu; /* persistent workgroups per compute unit, 1..4 */
-  int span;              /* wave tiles per wavefront, handed to lanes as their rays end: 1, 2, 4 or 8 */
+  int span;              /* wave tiles of a stack, which makes four work items: 1, 2, 4 or 8 */
   double ms;             /* autotune: the measured time of the chosen shape */
   float step_scale;      /* multiplier of every member's march step (its cone.step_size, or the
                             default half-voxel step), [0.25, 4]; 1 = each member's own step.  The

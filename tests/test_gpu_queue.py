@@ -93,3 +93,24 @@ def test_ebs_tables_that_leave_room_for_one_queue():
     tf = O.OTF(rgb, a, max_density=4095)
     ref, m = O.render_ebs(wl.volume, tf, O.sat(wl.volume, tf), O.ebs_params(p, wl.light()), wl.camera(), 33, 31)
     check(img, ref, m)
+
+
+@pytest.mark.parametrize("n,w,h,alpha_max", SIZES + MANY + [(24, 257, 259, 0.95)])
+def test_surrogate(n, w, h, alpha_max):
+    """4 and 16 rays per wavefront, four of them marching side by side."""
+    wl = W.cone_blobs(n=n, width=w, height=h, seed=31)
+    rgb, a = W.seeded_tf(131, 4, alpha_max=alpha_max)
+    r = N.Renderer(N.CONE_NN)
+    r.set_volume(wl.volume, wl.scale)
+    r.set_transfer_function(rgb, a)
+    rng = np.random.default_rng(3)
+    wts = rng.normal(0, 0.1, N.lib().cvr_nn_param_count()).astype(np.float32)
+    r.nn_set_weights(wts)
+    r.collect_stats()
+    img = r.render(wl.camera(), w, h, light=wl.light())
+    tf = O.OTF(rgb, a)
+    pyr = O.OPyr.build(wl.volume, tf, nlev=7)
+    ref, m, counts = O.render_nn(wl.volume, tf, pyr, O.cone_params(wl.grid, wl.light()), wts, wl.camera(), w, h)
+    check(img, ref, m)
+    # near-tied exits may take a sample more or less
+    assert abs(int(r.stats().shaded_samples) - int(counts[0])) <= 0.001 * counts[0] + 4
