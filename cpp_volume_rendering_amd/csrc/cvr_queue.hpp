@@ -54,22 +54,40 @@ template <int kRays> struct WaveQueue {
   float4 acc[kRays];    // accumulated colour, opacity
 };
 
-// Lane k - 1's value within each group of kSub lanes; `first` in the group's first lane.
-template <int kSub> __device__ __forceinline__ float left_lane(float v, float first) {
-  constexpr int ctrl = kSub == 64 ? 0x138 : 0x111;  // wave_shr:1, row_shr:1
-  return __int_as_float(
-      __builtin_amdgcn_update_dpp(__float_as_int(first), __float_as_int(v), ctrl, 0xf, 0xf, false));
+// Opacity before each lane's sample: w_0 = w, w_(k+1) = w_k + (1 - w_k) alpha_k, in order.
+// Lane k takes alpha_0 with the row shift by k, alpha_1 with that by k - 1, and so on; shifts
+// that reach past its row's first lane read 0, which leaves w as it is, bit for bit.
+// (In assembly: the compiler keeps the shift apart from the fused multiply-add, 3 instructions a
+// round for 2.  The wait is for the shift's source, if it was written just before.)
+__device__ __forceinline__ float opacity_rounds(float alpha, float w) {
+#define CVR_ROUND(d)                                                                  \
+  "v_sub_f32_e32 %1, 1.0, %0\n"                                                       \
+  "v_fmac_f32_dpp %0, %2, %1 row_shr:" #d " row_mask:0xf bank_mask:0xf bound_ctrl:1\n"
+  float t;
+  asm("s_nop 1\n" CVR_ROUND(15) CVR_ROUND(14) CVR_ROUND(13) CVR_ROUND(12) CVR_ROUND(11) CVR_ROUND(10) CVR_ROUND(9)
+          CVR_ROUND(8) CVR_ROUND(7) CVR_ROUND(6) CVR_ROUND(5) CVR_ROUND(4) CVR_ROUND(3) CVR_ROUND(2) CVR_ROUND(1)
+      : "+v"(w), "=&v"(t)
+      : "v"(alpha));
+#undef CVR_ROUND
+  return w;
 }
-// Opacity after each lane's sample: w_k = w_(k-1) + (1 - w_(k-1)) alpha_k, w_(-1) = w.
-// Every round makes one more lane of the group final; three instructions each.
-template <int kSub> __device__ __forceinline__ float opacity_scan(float alpha, float w) {
-  float v = w;
+__device__ __forceinline__ float opacity_after(float alpha, float w) { return __builtin_fmaf(alpha, 1.0f - w, w); }
+// A whole wavefront's 64 samples: each round shifts every lane's value by one lane, and makes
+// one more lane final.
+__device__ __forceinline__ float left_lane(float v, float first) {  // wave_shr:1; `first` in lane 0
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(__float_as_int(first), __float_as_int(v), 0x138, 0xf, 0xf, false));
+}
+template <int kSub> __device__ __forceinline__ float opacity_before(float alpha, float w) {
+  if (kSub == 16) return opacity_rounds(alpha, w);
+  float b = w;
 #pragma unroll
-  for (int k = 0; k < kSub; ++k) {
-    const float b = left_lane<kSub>(v, w);
-    v = __builtin_fmaf(1.0f - b, alpha, b);
-  }
-  return v;
+  for (int k = 0; k < 63; ++k) b = left_lane(opacity_after(alpha, b), w);
+  return b;
+}
+// The last lane's value of each row of 16.
+__device__ __forceinline__ float row_last(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x15f, 0xf, 0xf, true));
 }
 
 __device__ __forceinline__ void wave_lds_sync() {
@@ -231,8 +249,8 @@ __device__ __forceinline__ void queue_march(const RayFrame& rf, const VolGeom& g
         bool ended = !((__ballot(valid) >> (base + kSub - 1)) & 1);
         if (__any(opaque)) {
           const float alpha = opaque ? 1.0f - __expf(-src.w * r.h) : 0.f;
-          const float wa = opacity_scan<kSub>(alpha, w);
-          mine = (1.0f - left_lane<kSub>(wa, w)) * alpha;
+          const float wb = opacity_before<kSub>(alpha, w), wa = opacity_after(alpha, wb);
+          mine = (1.0f - wb) * alpha;
           const uint64_t over = (__ballot(wa > et) >> base) & kGroupMask;
           const int last = over ? __builtin_ctzll(over) : kSub - 1;  // over: the ray ends with that sample
           w = kSub == 64 ? lane_value(wa, last) : __shfl(wa, base + last);
@@ -295,6 +313,147 @@ __device__ __forceinline__ void queue_march(const RayFrame& rf, const VolGeom& g
     out[size_t(py) * rf.W + px] = c;
   }
   if (kParts > 1) __syncthreads();  // before the queues are used again
+}
+
+// sample_tf of a table with its first and last entry twice, for d in [0, 1] (a density is, to
+// a rounding): the two entries lie side by side, and no index needs a clamp.
+__device__ __forceinline__ float4 sample_tf_padded(const float4* tf, int ntf, float d) {
+  const float x = d * float(ntf) - 0.5f, fl = floorf(x), f = x - fl;
+  const float4* e = tf + int(fl);
+  const float4 a = e[1], b = e[2];
+  return make_float4(a.x + f * (b.x - a.x), a.y + f * (b.y - a.y), a.z + f * (b.z - a.z), a.w + f * (b.w - a.w));
+}
+__device__ __forceinline__ void stage_tf_padded(float4* s_tf, const float4* __restrict__ tf, int ntf) {
+  for (int i = threadIdx.x; i < ntf + 2; i += blockDim.x) s_tf[i] = tf[min(max(i - 1, 0), ntf - 1)];
+}
+
+// The march whose lighting costs less than the queue: lit(p) gives the factor of the colour of
+// the sample at p where it is met.  A lane adds up its own samples' colours and a group of 16 lanes
+// adds up its lanes' when its ray ends.  Takes rays as queue_march does.
+template <int kRays> struct RayList {
+  float4 tp[kRays];   // entry point (texture space), length
+  float4 dir[kRays];  // direction, pixel (bits)
+};
+template <typename T, bool kPadded, int kRays, class Pix, class Lit1>
+__device__ __forceinline__ void plain_march(const RayFrame& rf, const VolGeom& g, const float4* tfp, int ntf,
+                                            float step, float et, int rays, Pix&& pix, const float* spec, RayList<kRays>& Q,
+                                            float4* __restrict__ out, unsigned int& nsamp, unsigned int& nshade,
+                                            Lit1&& lit) {
+  constexpr int kSub = 16;
+  const int lane = threadIdx.x & 63, sub = lane % kSub, base = lane - sub;
+  const uint64_t below = (1ull << lane) - 1ull, below_group = (1ull << base) - 1ull;
+  int px = 0, py = 0;
+  const bool inside = lane < rays && pix(lane, px, py);
+  bool hit = false;
+  f3 t = mk3(0.f, 0.f, 0.f), d = t;
+  float len = 0.f;
+  if (inside) {
+    const f3 eye = ld3(rf.eye);
+    d = camera_ray(rf, px, py);
+    float tn, tf_;
+    hit = ray_box(eye, d, g.G, tn, tf_);
+    t = mk3(__builtin_fmaf(d.x, tn, eye.x), __builtin_fmaf(d.y, tn, eye.y), __builtin_fmaf(d.z, tn, eye.z));
+    t = t + mk3(0.5f * g.G[0], 0.5f * g.G[1], 0.5f * g.G[2]);
+    len = fabsf(tf_ - tn);
+    if (!hit) out[size_t(py) * rf.W + px] = make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  const uint64_t hits = __ballot(hit);
+  const int nhit = __popcll(hits), slot = __popcll(hits & below);
+  if (nhit == 0) return;
+  if (hit) {
+    Q.tp[slot] = make_float4(t.x, t.y, t.z, len);
+    Q.dir[slot] = make_float4(d.x, d.y, d.z, __int_as_float(py * rf.W + px));
+  }
+  wave_lds_sync();
+  f3 tp, dir;
+  float4 acc;  // this lane's share of the colour; opacity of the ray
+  float D;
+  int ray, jb, next = 0, pixel;
+  // the next rays for the groups without one (ray -1: none left, and D below every s)
+  auto take = [&]() {
+    const uint64_t need = __ballot(ray < 0 && sub == 0);
+    if (ray < 0) {
+      const int mine = next + __popcll(need & below_group), i = min(mine, nhit - 1);
+      const float4 a = Q.tp[i], b = Q.dir[i];
+      ray = mine < nhit ? mine : -1;
+      tp = mk3(a.x, a.y, a.z);
+      dir = mk3(b.x, b.y, b.z);
+      D = ray < 0 ? -1.f : a.w;
+      pixel = __float_as_int(b.w);
+      jb = sub;
+      acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    next += __popcll(need);
+  };
+  auto load = [&](RaySample& s, VolTap<T>& v) {
+    s = ray_sample(jb, step, D);
+    v = volume_tap_load<T>(g, ray_sample_pos(s, tp, dir));
+  };
+  ray = -1;
+  take();
+  // One step; the next step's blocks are in flight under it.  False: no rays left.
+  auto go = [&](const RaySample& r, const VolTap<T>& tap, RaySample& r1, VolTap<T>& tap1) {
+    const bool in_range = jb < kMaxSamples;
+    jb += kSub;
+    load(r1, tap1);
+    const float d = volume_tap_lerp<T>(tap);
+    const float4 src = kPadded ? sample_tf_padded(tfp, ntf, d) : sample_tf(tfp, ntf, d);
+    const bool valid = r.s < D && in_range;
+    const bool opaque = valid && src.w > 0.0f;
+    const float alpha = opaque ? 1.0f - __expf(-src.w * r.h) : 0.f;
+    const uint64_t valids = __ballot(valid);
+    float wa = acc.w;
+    uint64_t over = 0;
+    bool taken = valid;
+    if (__any(opaque)) {
+      const float wb = opacity_before<kSub>(alpha, acc.w);
+      wa = opacity_after(alpha, wb);
+      over = __ballot(wa > et);
+      // the ray ends with the first sample over: those after it are not taken
+      taken = valid && !(wb > et);
+      float mine = taken ? (1.0f - wb) * alpha : 0.f;
+      if (opaque && taken) {
+        const Lit l = lit(ray_sample_pos(r, tp, dir));
+        const float ws = mine * l.s;
+        mine *= l.m;
+        acc.x = __builtin_fmaf(spec[0], ws, acc.x);
+        acc.y = __builtin_fmaf(spec[1], ws, acc.y);
+        acc.z = __builtin_fmaf(spec[2], ws, acc.z);
+      }
+      acc.x = __builtin_fmaf(mine, src.x, acc.x);
+      acc.y = __builtin_fmaf(mine, src.y, acc.y);
+      acc.z = __builtin_fmaf(mine, src.z, acc.z);
+      acc.w = row_last(wa);
+      nshade += opaque && taken;
+    }
+    nsamp += taken;
+    if (over | ~valids) {
+      // some group's ray has ended (or some group has none)
+      const unsigned int mine = (unsigned int)(over >> base) & 0xffffu;
+      const bool ended = mine != 0 || !((valids >> (base + kSub - 1)) & 1);
+      if (__any(ended && ray >= 0)) {
+        float4 c = acc;
+        if (mine) c.w = __shfl(wa, base + __builtin_ctz(mine));
+#pragma unroll
+        for (int o = kSub / 2; o > 0; o /= 2) {
+          c.x += __shfl_xor(c.x, o);
+          c.y += __shfl_xor(c.y, o);
+          c.z += __shfl_xor(c.z, o);
+        }
+        if (ended && ray >= 0 && sub == 0) out[pixel] = c;
+        if (ended) ray = -1;
+        take();
+        if (!__any(ray >= 0)) return false;
+        if (ended) load(r1, tap1);
+      }
+    }
+    return true;
+  };
+  RaySample ra, rb;
+  VolTap<T> ta, tb;
+  load(ra, ta);
+  while (go(ra, ta, rb, tb) && go(rb, tb, ra, ta)) {
+  }
 }
 
 }  // namespace cvr

@@ -114,3 +114,44 @@ def test_surrogate(n, w, h, alpha_max):
     check(img, ref, m)
     # near-tied exits may take a sample more or less
     assert abs(int(r.stats().shaded_samples) - int(counts[0])) <= 0.001 * counts[0] + 4
+
+
+# (density entries, 8 or 16 bits): the smallest tables, the largest staged one, one read from memory
+@pytest.mark.parametrize("entries,bits", [(2, 8), (256, 8), (4096, 16), (5000, 16)])
+@pytest.mark.parametrize("n,w,h,alpha_max", SIZES + MANY)
+@pytest.mark.parametrize("phong", [0, 1])
+def test_plain(n, w, h, alpha_max, entries, bits, phong):
+    wl = W.cone_blobs(n=n, width=w, height=h, seed=31)
+    vol = wl.volume if bits == 8 else (wl.volume.astype(np.uint16) * 257)
+    rgb, a = W.seeded_tf(131, 4, alpha_max=alpha_max)
+    if entries == 2:
+        rgb, a = rgb[[0, -1]], a[[0, -1]]
+    rgb[:, 3] = np.round(rgb[:, 3] * (entries - 1) / 255)
+    a[:, 1] = rgb[:, 3]
+    r = N.Renderer(N.RC1P)
+    r.set_volume(vol, wl.scale)
+    r.set_transfer_function(rgb, a, max_density=entries - 1)
+    p = r.params()
+    p.apply_gradient_shading, p.shininess = phong, 20.0
+    r.set_params(p)
+    img = r.render(wl.camera(), w, h, light=wl.light())
+    tf = O.OTF(rgb, a, max_density=entries - 1)
+    if phong:
+        ph = O.phong(p.gradient_type, wl.light(), ka=p.ka, kd=p.kd, ks=p.ks, shininess=p.shininess)
+        ref, m = O.render_rc1p_phong(vol, tf, ph, wl.camera(), w, h)
+    else:
+        ref, m = O.render_rc1p(vol, tf, wl.camera(), w, h)
+    check(img, ref, m)
+
+
+@pytest.mark.parametrize("n,w,h,alpha_max", SIZES + MANY)
+@pytest.mark.parametrize("phong", [0, 1])
+def test_light_cache(n, w, h, alpha_max, phong):
+    wl, tf, r, p, img = scene(N.EBS, n, w, h, alpha_max, light_cache=1, apply_phong=phong)
+    g = r.light_cache()
+    if phong:
+        ph = O.phong(p.gradient_type, wl.light(), ka=p.ka, kd=p.kd, ks=p.ks, shininess=p.shininess)
+        ref, m = O.render_lc_phong(wl.volume, tf, g, 1, 1, p.ka, p.kd, ph, wl.camera(), w, h, scale=wl.scale)
+    else:
+        ref, m = O.render_lc(wl.volume, tf, g, 1, 1, p.ka, p.kd, wl.camera(), w, h, scale=wl.scale)
+    check(img, ref, m)
