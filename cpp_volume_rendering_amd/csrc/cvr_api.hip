@@ -210,7 +210,6 @@ static void defaults(int technique, void* p) {
 static void free_all(cvr_ctx* c) {
   if (c->d_vol) (void)hipFree(c->d_vol);
   if (c->d_tf_rgbt) (void)hipFree(c->d_tf_rgbt);
-  if (c->d_tf_rgba) (void)hipFree(c->d_tf_rgba);
   if (c->d_sat) (void)hipFree(c->d_sat);
   if (c->d_sat_oct) (void)hipFree(c->d_sat_oct);
   if (c->d_ext_lut) (void)hipFree(c->d_ext_lut);
@@ -219,6 +218,8 @@ static void free_all(cvr_ctx* c) {
   if (c->d_ms_frame) (void)hipFree(c->d_ms_frame);
   if (c->d_pyr) (void)hipFree(c->d_pyr);
   if (c->d_pyr_oct) (void)hipFree(c->d_pyr_oct);
+  if (c->d_pyr_work) (void)hipFree(c->d_pyr_work);
+  if (c->h_nn_io) (void)hipHostFree(c->h_nn_io);
   if (c->d_nn_redo) (void)hipFree(c->d_nn_redo);
   if (c->d_vol_oct) (void)hipFree(c->d_vol_oct);
   if (c->d_cone_tab) (void)hipFree(c->d_cone_tab);
@@ -228,7 +229,7 @@ static void free_all(cvr_ctx* c) {
   if (c->d_grad) (void)hipFree(c->d_grad);
   if (c->d_ebs_rows) (void)hipFree(c->d_ebs_rows);
   for (void* p : {static_cast<void*>(c->d_nn_w), static_cast<void*>(c->d_nn_g), static_cast<void*>(c->d_nn_m),
-                  static_cast<void*>(c->d_nn_v), static_cast<void*>(c->d_nn_scalar), c->d_nn_pack, c->d_nn_tpack,
+                  static_cast<void*>(c->d_nn_v), c->d_nn_pack, c->d_nn_tpack,
                   static_cast<void*>(c->d_nn_slabs)})
     if (p) (void)hipFree(p);
   for (hipEvent_t e : c->ev_sat)
@@ -335,6 +336,8 @@ int cvr_set_volume(cvr_handle h, int nx, int ny, int nz, int dtype, float sx, fl
       return CVR_ERR_NOMEM;
     }
   }
+  // frames in flight on any stream may still read the volume and its corner blocks
+  CVR_HIP_CHECK(hipDeviceSynchronize());
   CVR_HIP_CHECK(hipMemcpy(h->d_vol, voxels, bytes, is_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice));
   h->nx = nx; h->ny = ny; h->nz = nz; h->dtype = dtype;
   if (const int rc = build_volume_oct(h, nullptr)) return rc;
@@ -387,7 +390,8 @@ int cvr_set_transfer_function(cvr_handle h, int max_density, int extinction_inpu
       tab[size_t(x) * 4 + 3] = double(a0) + diff * k;
     }
   }
-  std::vector<float4> rgbt(T), rgba(T);
+  std::vector<float4> both(size_t(T) * 2);  // RGBt, then RGBA
+  float4 *rgbt = both.data(), *rgba = rgbt + T;
   for (int i = 0; i < T; ++i) {
     const float r = float(tab[i * 4]), g = float(tab[i * 4 + 1]), b = float(tab[i * 4 + 2]);
     const float v4 = float(tab[i * 4 + 3]);
@@ -399,16 +403,15 @@ int cvr_set_transfer_function(cvr_handle h, int max_density, int extinction_inpu
   DeviceGuard dg(h->device);
   if (h->tf_size != T) {
     if (h->d_tf_rgbt) CVR_HIP_CHECK(hipFree(h->d_tf_rgbt));
-    if (h->d_tf_rgba) CVR_HIP_CHECK(hipFree(h->d_tf_rgba));
     h->d_tf_rgbt = h->d_tf_rgba = nullptr;
-    if (hipMalloc(&h->d_tf_rgbt, T * sizeof(float4)) != hipSuccess ||
-        hipMalloc(&h->d_tf_rgba, T * sizeof(float4)) != hipSuccess) {
+    if (hipMalloc(&h->d_tf_rgbt, both.size() * sizeof(float4)) != hipSuccess) {
+      h->d_tf_rgbt = nullptr;
       set_error("cvr_set_transfer_function: out of device memory");
       return CVR_ERR_NOMEM;
     }
+    h->d_tf_rgba = h->d_tf_rgbt + T;
   }
-  CVR_HIP_CHECK(hipMemcpy(h->d_tf_rgbt, rgbt.data(), T * sizeof(float4), hipMemcpyHostToDevice));
-  CVR_HIP_CHECK(hipMemcpy(h->d_tf_rgba, rgba.data(), T * sizeof(float4), hipMemcpyHostToDevice));
+  CVR_HIP_CHECK(hipMemcpy(h->d_tf_rgbt, both.data(), both.size() * sizeof(float4), hipMemcpyHostToDevice));
   h->tf_size = T;
   h->tf_max_density = max_density;
   h->tf_ext_input = extinction_input != 0;
@@ -893,22 +896,53 @@ int cvr_nn_eval(cvr_handle h, int n, const float* X, float* Y, int path) {
   return CVR_OK;
 }
 
+// One step of an optimiser outside the library.  The kernels read the samples from a pinned buffer
+// and write the gradient behind them, so the call waits once; the buffer is kept up to this size
+// (16384 samples: 126 us with device buffers made in the call and a wait for each of four copies, 101
+// with kept buffers and queued copies, 81 now, of which 14 copy the samples and 37 are the kernels').
+constexpr size_t kNnIoKept = size_t(64) << 20;
+
 int cvr_nn_gradient(cvr_handle h, int n, const float* X, const float* T, float* grad, float* loss) {
   int rc = nn_check(h);
   if (rc) return rc;
   if (!X || !T || !grad || n < 1) { set_error("cvr_nn_gradient: null argument"); return CVR_ERR_INVALID; }
   if (!h->d_nn_w) { set_error("cvr_nn_gradient: no network yet"); return CVR_ERR_STATE; }
   DeviceGuard dg(h->device);
-  DevBuf dx, dt;
-  CVR_HIP_CHECK(hipMalloc(&dx.p, size_t(n) * 16 * 4));
-  CVR_HIP_CHECK(hipMalloc(&dt.p, size_t(n) * 2 * 4));
-  CVR_HIP_CHECK(hipMemcpy(dx.p, X, size_t(n) * 16 * 4, hipMemcpyHostToDevice));
-  CVR_HIP_CHECK(hipMemcpy(dt.p, T, size_t(n) * 2 * 4, hipMemcpyHostToDevice));
-  rc = nn_gradient(h, static_cast<float*>(dx.p), static_cast<float*>(dt.p), n, nullptr);
+  const size_t xn = size_t(n) * 16, tn = size_t(n) * 2, gn = size_t(nn_param_count()) + 1;
+  const size_t bytes = (xn + tn + gn) * sizeof(float);
+  if (bytes > kNnIoKept) {
+    DevBuf dx, dt;
+    CVR_HIP_CHECK(hipMalloc(&dx.p, xn * sizeof(float)));
+    CVR_HIP_CHECK(hipMalloc(&dt.p, tn * sizeof(float)));
+    CVR_HIP_CHECK(hipMemcpy(dx.p, X, xn * sizeof(float), hipMemcpyHostToDevice));
+    CVR_HIP_CHECK(hipMemcpy(dt.p, T, tn * sizeof(float), hipMemcpyHostToDevice));
+    rc = nn_gradient(h, static_cast<float*>(dx.p), static_cast<float*>(dt.p), n, h->d_nn_g, nullptr);
+    if (rc) return rc;
+    CVR_HIP_CHECK(hipDeviceSynchronize());
+    CVR_HIP_CHECK(hipMemcpy(grad, h->d_nn_g, (gn - 1) * sizeof(float), hipMemcpyDeviceToHost));
+    if (loss) CVR_HIP_CHECK(hipMemcpy(loss, h->d_nn_scalar, sizeof(float), hipMemcpyDeviceToHost));
+    return CVR_OK;
+  }
+  if (h->nn_io_bytes != bytes) {
+    if (h->h_nn_io) CVR_HIP_CHECK(hipHostFree(h->h_nn_io));
+    h->h_nn_io = nullptr;
+    h->nn_io_bytes = 0;
+    if (hipHostMalloc(reinterpret_cast<void**>(&h->h_nn_io), bytes, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      h->h_nn_io = nullptr;
+      set_error("cvr_nn_gradient: out of pinned host memory");
+      return CVR_ERR_NOMEM;
+    }
+    h->nn_io_bytes = bytes;
+  }
+  float *hx = h->h_nn_io, *ht = hx + xn, *hg = ht + tn;
+  std::memcpy(hx, X, xn * sizeof(float));
+  std::memcpy(ht, T, tn * sizeof(float));
+  rc = nn_gradient(h, hx, ht, n, hg, nullptr);
+  CVR_HIP_CHECK(hipStreamSynchronize(nullptr));  // also on errors: the kernels read the kept buffer
   if (rc) return rc;
-  CVR_HIP_CHECK(hipDeviceSynchronize());
-  CVR_HIP_CHECK(hipMemcpy(grad, h->d_nn_g, size_t(nn_param_count()) * 4, hipMemcpyDeviceToHost));
-  if (loss) CVR_HIP_CHECK(hipMemcpy(loss, h->d_nn_scalar, 4, hipMemcpyDeviceToHost));
+  std::memcpy(grad, hg, (gn - 1) * sizeof(float));
+  if (loss) *loss = hg[gn - 1];
   return CVR_OK;
 }
 

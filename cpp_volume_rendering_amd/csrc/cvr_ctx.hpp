@@ -59,6 +59,7 @@ struct cvr_ctx {
   float sx = 1, sy = 1, sz = 1;
   void* d_vol = nullptr;
   void* d_vol_oct = nullptr;  // corner blocks of the voxels, 8 x u8 / 8 x u16 (k_quad.hip)
+  size_t vol_oct_bytes = 0;
 
   // transfer function (host FP64 table as TransferFunction1D::BuildLinear builds it)
   int tf_max_density = 255;
@@ -86,6 +87,9 @@ struct cvr_ctx {
 
   // Gaussian extinction pyramid (cone tracers, surrogate)
   float* d_pyr = nullptr;
+  size_t pyr_bytes = 0, pyr_oct_bytes = 0;
+  void* d_pyr_work = nullptr;  // opacities and separable passes of a build, kept up to kPyrWorkKept bytes
+  size_t pyr_work_bytes = 0;
   void* d_pyr_oct = nullptr;   // corner blocks of every level (PyrGeom::fmt, k_quad.hip)
   cvr::PyrGeom pyr{};
   cvr::PyrKey pyr_key{};
@@ -97,6 +101,8 @@ struct cvr_ctx {
 
   // directional occlusion shading: section tables (occlusion rows, then shadow rows)
   cvr::DosTable dos_occ, dos_sdw;
+  cvr_dos_cone dos_cones_for[2] = {};  // the cones and sigma of the tables in d_dos_rows
+  double dos_sigma_for = 0.0;          // 0: none
   float4* d_dos_rows = nullptr;
   size_t dos_rows_cap = 0;
 
@@ -112,6 +118,8 @@ struct cvr_ctx {
   void* d_nn_tpack = nullptr;      // bf16 training packs (forward, biases, W^T tiles)
   float* d_nn_slabs = nullptr;     // per-64-sample gradient slabs of a training step
   size_t nn_slabs_cap = 0;
+  float* h_nn_io = nullptr;        // cvr_nn_gradient: samples, gradient and loss (pinned, at most kNnIoKept bytes)
+  size_t nn_io_bytes = 0;
   float nn_lo[16] = {0}, nn_hi[16] = {0};
   bool nn_trained = false;
   uint64_t nn_version = 0;  // bumped whenever the weights or the input range change
@@ -168,6 +176,8 @@ int lc_prepare(cvr_ctx* c, const int res[3]);
 int launch_lc_render(cvr_ctx* c, const RayFrame& rf, int apply_occ, int apply_sdw, float ka, float kd, float step,
                      float et, const PhongK& ph, float* out, hipStream_t st);
 int launch_ebs(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out, hipStream_t st);
+// a device buffer of exactly `bytes`: *p if it has that size, else a new one in its place
+int sized_buffer(void** p, size_t* have, size_t bytes);
 int build_volume_oct(cvr_ctx* c, hipStream_t st);
 int build_pyramid_oct(cvr_ctx* c, size_t total, int fmt, hipStream_t st);
 int build_pyramid(cvr_ctx* c, int base_x, int base_y, int base_z, float sigma0, int nlev, int fmt, hipStream_t st);
@@ -188,7 +198,7 @@ int launch_dos(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* ou
 int nn_alloc(cvr_ctx* c);
 int nn_pack(cvr_ctx* c, hipStream_t st);
 int nn_train(cvr_ctx* c, hipStream_t st);
-int nn_gradient(cvr_ctx* c, const float* d_X, const float* d_T, int n, hipStream_t st);
+int nn_gradient(cvr_ctx* c, const float* d_X, const float* d_T, int n, float* grad, hipStream_t st);
 int nn_eval(cvr_ctx* c, const float* d_X, int n, float* d_Y, int packed, hipStream_t st);
 int launch_nn(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out, hipStream_t st);
 int nn_param_count();

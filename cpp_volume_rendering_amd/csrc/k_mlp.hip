@@ -657,11 +657,11 @@ static int ensure(void** p, size_t bytes) {
 int nn_alloc(cvr_ctx* c) {
   int rc = 0;
   rc |= ensure(reinterpret_cast<void**>(&c->d_nn_w), kNParams * sizeof(float));
-  rc |= ensure(reinterpret_cast<void**>(&c->d_nn_g), kNParams * sizeof(float));
+  rc |= ensure(reinterpret_cast<void**>(&c->d_nn_g), (kNParams + 64) * sizeof(float));
   rc |= ensure(reinterpret_cast<void**>(&c->d_nn_m), kNParams * sizeof(float));
   rc |= ensure(reinterpret_cast<void**>(&c->d_nn_v), kNParams * sizeof(float));
   rc |= ensure(reinterpret_cast<void**>(&c->d_nn_pack), kPackShorts * sizeof(short) + kNBias * sizeof(float));
-  rc |= ensure(reinterpret_cast<void**>(&c->d_nn_scalar), 64 * sizeof(float));
+  c->d_nn_scalar = c->d_nn_g ? c->d_nn_g + kNParams : nullptr;  // the loss, behind the gradient
   return rc ? -5 : 0;
 }
 
@@ -715,22 +715,24 @@ static int train_buffers(cvr_ctx* c, int n) {
 }
 
 // The update kernel in one of its modes (0: gradient sum, 1: Adam step, 2: packs only).
-static void launch_update(cvr_ctx* c, int nslabs, int mode, float lr, float bc1, float bc2, hipStream_t st) {
+static void launch_update(cvr_ctx* c, int nslabs, int mode, float lr, float bc1, float bc2, hipStream_t st,
+                          float* grad = nullptr) {
   hipLaunchKernelGGL(k_mlp_update, dim3((kNParams + 1 + kUpdParams - 1) / kUpdParams), dim3(kUpdParams * kUpdParts), 0, st,
                      c->d_nn_slabs, nslabs, mode,
-                     c->d_nn_w, c->d_nn_g, c->d_nn_m, c->d_nn_v, lr, 0.9f, 0.999f, 1e-8f, bc1, bc2,
-                     static_cast<unsigned char*>(c->d_nn_tpack), static_cast<short*>(c->d_nn_pack), c->d_nn_scalar);
+                     c->d_nn_w, grad ? grad : c->d_nn_g, c->d_nn_m, c->d_nn_v, lr, 0.9f, 0.999f, 1e-8f, bc1, bc2,
+                     static_cast<unsigned char*>(c->d_nn_tpack), static_cast<short*>(c->d_nn_pack),
+                     grad ? grad + kNParams : c->d_nn_scalar);
 }
 
-// Gradient of L = sum (y - t)^2 / (2 n) over n samples at the current weights.
-int nn_gradient(cvr_ctx* c, const float* d_X, const float* d_T, int n, hipStream_t st) {
+// Gradient of L = sum (y - t)^2 / (2 n) over n samples at the current weights, and the loss behind it.
+int nn_gradient(cvr_ctx* c, const float* d_X, const float* d_T, int n, float* grad, hipStream_t st) {
   int rc = train_buffers(c, n);
   if (rc) return rc;
   const int chunks = (n + kTrainChunk - 1) / kTrainChunk;
   launch_update(c, 0, 2, 0.f, 1.f, 1.f, st);  // the packs of the current weights
   hipLaunchKernelGGL(k_mlp_train, dim3(chunks), dim3(64 * kTrainWaves), 0, st,
                      static_cast<const unsigned char*>(c->d_nn_tpack), d_X, d_T, n, float(n), c->d_nn_slabs);
-  launch_update(c, chunks, 0, 0.f, 1.f, 1.f, st);
+  launch_update(c, chunks, 0, 0.f, 1.f, 1.f, st, grad);
   CVR_HIP_CHECK(hipGetLastError());
   return 0;
 }

@@ -227,6 +227,11 @@ PyrKey pyr_key_for(const cvr_ctx* c, int base_x, int base_y, int base_z, float s
   return key;
 }
 
+// A volume that changes every frame rebuilds its pyramid every frame: allocating and freeing
+// its four buffers and the volume's corner blocks took longer than the build (the next 256^3 step and
+// its DOS frame 1.6 to 9 ms with them, 0.54 without).
+constexpr size_t kPyrWorkKept = size_t(1) << 30;
+
 int build_pyramid(cvr_ctx* c, int base_x, int base_y, int base_z, float sigma0, int nlev, int fmt, hipStream_t st) {
   if (base_x < 1 || base_y < 1 || base_z < 1) { set_error("pyramid: base resolution must be >= 1"); return -1; }
   if (!(sigma0 > 0)) { set_error("pyramid: sigma0 must be > 0"); return -1; }
@@ -260,15 +265,8 @@ int build_pyramid(cvr_ctx* c, int base_x, int base_y, int base_z, float sigma0, 
   VolGeom g = geom_of(c);
   for (int k = 0; k < 3; ++k) pg.G[k] = g.G[k];
   pg.one = 1.0f;
-  if (c->d_pyr) CVR_HIP_CHECK(hipFree(c->d_pyr));
-  c->d_pyr = nullptr;
-  float* d_op = nullptr;
-  if (hipMalloc(&c->d_pyr, total * sizeof(float)) != hipSuccess || hipMalloc(&d_op, total * sizeof(float)) != hipSuccess) {
-    if (c->d_pyr) (void)hipFree(c->d_pyr);
-    c->d_pyr = nullptr;
-    set_error("pyramid: out of device memory");
-    return -5;
-  }
+  // frames in flight on any stream may still read the pyramid that is built over
+  CVR_HIP_CHECK(hipDeviceSynchronize());
   // separable path per level: voxel spacing and sigma commensurate on every axis (true at
   // every level of the default configurations; a level whose size was rounded down from
   // an odd one may not be, and takes the direct build)
@@ -284,12 +282,19 @@ int build_pyramid(cvr_ctx* c, int base_x, int base_y, int base_z, float sigma0, 
       tmp_floats = std::max(tmp_floats, size_t(sax[i][0].len) * sax[i][1].len * sax[i][2].len +
                                             size_t(pg.dims[i][0]) * sax[i][1].len * sax[i][2].len);
   }
-  float* d_tmp = nullptr;
-  if (tmp_floats && hipMalloc(&d_tmp, tmp_floats * sizeof(float)) != hipSuccess) {
-    (void)hipGetLastError();
-    d_tmp = nullptr;
+  // opacities of every level, then the temporaries of the largest level's passes
+  int rc = sized_buffer(reinterpret_cast<void**>(&c->d_pyr), &c->pyr_bytes, total * sizeof(float));
+  if (!rc) rc = sized_buffer(&c->d_pyr_work, &c->pyr_work_bytes, (total + tmp_floats) * sizeof(float));
+  if (rc == CVR_ERR_NOMEM && c->d_pyr) {
     std::fill(sep.begin(), sep.end(), 0);  // no room for the temporaries: the direct build needs none
+    rc = sized_buffer(&c->d_pyr_work, &c->pyr_work_bytes, total * sizeof(float));
   }
+  if (rc) {
+    if (rc == CVR_ERR_NOMEM) set_error("pyramid: out of device memory");
+    return -5;
+  }
+  float* d_op = static_cast<float*>(c->d_pyr_work);
+  float* d_tmp = d_op + total;
   SepW gw;
   double gsum = 0;
   for (int t = 0; t < 7; ++t) {
@@ -349,16 +354,15 @@ int build_pyramid(cvr_ctx* c, int base_x, int base_y, int base_z, float sigma0, 
                        a[2].len, 2, a[2].m, a[2].q, bz, gw, norm);
     CVR_HIP_CHECK(hipGetLastError());
   }
-  if (d_tmp) {
-    CVR_HIP_CHECK(hipStreamSynchronize(st));
-    CVR_HIP_CHECK(hipFree(d_tmp));
-  }
   hipLaunchKernelGGL(k_pyr_tau, dim3(unsigned((total + 255) / 256)), dim3(256), 0, st, d_op, c->d_pyr, total);
   CVR_HIP_CHECK(hipGetLastError());
-  CVR_HIP_CHECK(hipStreamSynchronize(st));
-  CVR_HIP_CHECK(hipFree(d_op));
   c->pyr = pg;
-  if (build_pyramid_oct(c, btotal, fmt, st) != CVR_OK) return -5;
+  if (build_pyramid_oct(c, btotal, fmt, st) != CVR_OK) return -5;  // waits for the stream
+  if (c->pyr_work_bytes > kPyrWorkKept) {
+    CVR_HIP_CHECK(hipFree(c->d_pyr_work));
+    c->d_pyr_work = nullptr;
+    c->pyr_work_bytes = 0;
+  }
   c->pyr_key = key;
   c->pyr_valid = true;
   return 0;

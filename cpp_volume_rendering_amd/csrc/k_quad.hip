@@ -44,17 +44,26 @@ static int make_vol_oct(const T* src, void* dst, int nx, int ny, int nz, hipStre
   return CVR_OK;
 }
 
+int sized_buffer(void** p, size_t* have, size_t bytes) {
+  if (*p && *have == bytes) return CVR_OK;
+  if (*p) CVR_HIP_CHECK(hipFree(*p));
+  *p = nullptr;
+  *have = 0;
+  if (hipMalloc(p, bytes) != hipSuccess) {
+    (void)hipGetLastError();
+    *p = nullptr;
+    return CVR_ERR_NOMEM;
+  }
+  *have = bytes;
+  return CVR_OK;
+}
+
 int build_volume_oct(cvr_ctx* c, hipStream_t st) {
   const size_t cells = brick_cells(c->nx, c->ny, c->nz);
   const size_t bytes = cells * (c->dtype == CVR_U8 ? sizeof(uint2) : sizeof(uint4));
-  if (c->d_vol_oct) CVR_HIP_CHECK(hipFree(c->d_vol_oct));
-  c->d_vol_oct = nullptr;
-  if (hipMalloc(&c->d_vol_oct, bytes) != hipSuccess) {
-    c->d_vol_oct = nullptr;
-    set_error("cvr_set_volume: out of device memory (corner blocks)");
-    return CVR_ERR_NOMEM;
-  }
-  int rc;
+  int rc = sized_buffer(&c->d_vol_oct, &c->vol_oct_bytes, bytes);
+  if (rc == CVR_ERR_NOMEM) set_error("cvr_set_volume: out of device memory (corner blocks)");
+  if (rc != CVR_OK) return rc;
   if (c->dtype == CVR_U8)
     rc = make_vol_oct(static_cast<const uint8_t*>(c->d_vol), c->d_vol_oct, c->nx, c->ny, c->nz, st);
   else
@@ -99,14 +108,18 @@ __global__ __launch_bounds__(256) void k_make_oct(const float* __restrict__ src,
 }
 
 int build_pyramid_oct(cvr_ctx* c, size_t total, int fmt, hipStream_t st) {
-  if (c->d_pyr_oct) CVR_HIP_CHECK(hipFree(c->d_pyr_oct));
-  c->d_pyr_oct = nullptr;
   const size_t rec = fmt == 0 ? 32 : 16;
-  if (hipMalloc(&c->d_pyr_oct, total * rec) != hipSuccess) {
-    c->d_pyr_oct = nullptr;
-    set_error("pyramid: out of device memory (corner blocks)");
-    return CVR_ERR_NOMEM;
+  int rc = sized_buffer(&c->d_pyr_oct, &c->pyr_oct_bytes, total * rec);
+  if (rc == CVR_ERR_NOMEM && c->d_pyr_work) {
+    // the build's workspace is no longer needed once its kernels have run
+    CVR_HIP_CHECK(hipStreamSynchronize(st));
+    CVR_HIP_CHECK(hipFree(c->d_pyr_work));
+    c->d_pyr_work = nullptr;
+    c->pyr_work_bytes = 0;
+    rc = sized_buffer(&c->d_pyr_oct, &c->pyr_oct_bytes, total * rec);
   }
+  if (rc == CVR_ERR_NOMEM) set_error("pyramid: out of device memory (corner blocks)");
+  if (rc != CVR_OK) return rc;
   const PyrGeom& pg = c->pyr;
   for (int l = 0; l < pg.levels; ++l) {
     const int nx = pg.dims[l][0], ny = pg.dims[l][1], nz = pg.dims[l][2];

@@ -428,9 +428,9 @@ int build_sat(cvr_ctx* c, hipStream_t st, bool with_blocks) {
   }
   std::vector<float> lut;
   build_ext_lut(c, lut);
-  if (c->d_ext_lut) CVR_HIP_CHECK(hipFree(c->d_ext_lut));
-  c->d_ext_lut = nullptr;
-  CVR_HIP_CHECK(hipMalloc(&c->d_ext_lut, lut.size() * sizeof(float)));
+  // frames in flight on any stream may still read the table and its blocks
+  CVR_HIP_CHECK(hipDeviceSynchronize());
+  if (!c->d_ext_lut) CVR_HIP_CHECK(hipMalloc(&c->d_ext_lut, 65536 * sizeof(float)));  // the larger type's
   CVR_HIP_CHECK(hipMemcpyAsync(c->d_ext_lut, lut.data(), lut.size() * sizeof(float), hipMemcpyHostToDevice, st));
   const bool timed = c->collect_stats;
   if (timed) {

@@ -155,3 +155,37 @@ def test_light_cache(n, w, h, alpha_max, phong):
     else:
         ref, m = O.render_lc(wl.volume, tf, g, 1, 1, p.ka, p.kd, wl.camera(), w, h, scale=wl.scale)
     check(img, ref, m)
+
+
+def test_buffers_kept_between_volumes_hold_the_new_ones():
+    """Volumes, cones and networks of changing and equal sizes through one handle, against new
+    handles: what a handle keeps is of the call at hand."""
+    def fresh(tech, vol, params):
+        r = N.Renderer(tech)
+        r.set_volume(vol, (1.0, 1.0, 1.0))
+        r.set_transfer_function(*W.seeded_tf(131, 4, alpha_max=0.5))
+        r.set_params(**params)
+        return r
+
+    rng = np.random.default_rng(5)
+    wl = W.cone_blobs(n=24, width=40, height=30, seed=31)
+    kept = {t: fresh(t, rng.integers(0, 256, (8, 8, 8), dtype=np.uint8), {}) for t in (N.DOS, N.EBS)}
+    for shape in ((20, 24, 28), (20, 24, 28), (30, 10, 12), (20, 24, 28)):
+        vol = rng.integers(0, 256, shape, dtype=np.uint8)
+        for tech, many in ((N.DOS, [dict(apply_shadow=1, light_cache=c, sigma0=s) for c in (0, 1) for s in (1.0, 1.5)]),
+                           (N.EBS, [dict(light_cache=c) for c in (0, 1)])):
+            kept[tech].set_volume(vol, (1.0, 1.0, 1.0))
+            kept[tech].set_transfer_function(*W.seeded_tf(131, 4, alpha_max=0.5))
+            for params in many:
+                kept[tech].set_params(**params)
+                a = kept[tech].render(wl.camera(), 40, 30, light=wl.light())
+                b = fresh(tech, vol, params).render(wl.camera(), 40, 30, light=wl.light())
+                assert np.abs(a - b).max() <= 1e-6, (shape, tech, params)  # colours add up in any order
+    net, w = N.Renderer(N.CONE_NN), rng.normal(0, 0.2, N.lib().cvr_nn_param_count()).astype(np.float32)
+    net.nn_set_weights(w)
+    for n in (64, 100, 64, 1):
+        x, t = rng.random((n, 16), np.float32), rng.random((n, 2), np.float32)
+        new = N.Renderer(N.CONE_NN)
+        new.nn_set_weights(w)
+        (la, ga), (lb, gb) = net.nn_gradient(x, t), new.nn_gradient(x, t)
+        assert la == lb and np.array_equal(ga, gb)
