@@ -27,6 +27,9 @@ VolGeom geom_of(const cvr_ctx* c) {
   g.nbx = bricks(c->nx);
   g.nby = bricks(c->ny);
   for (int i = 0; i < 3; ++i) g.vmax[i] = float(n[i] - 1);
+  const size_t rows = size_t(g.nby) * size_t(bricks(c->nz)), lim = size_t(1) << 24;
+  g.narrow = brick_cells(c->nx, c->ny, c->nz) * (c->dtype == CVR_U8 ? 8 : 16) < (size_t(1) << 32) && rows < lim &&
+             size_t(g.nbx) < lim;
   return g;
 }
 

@@ -19,6 +19,8 @@
 // long rays would end last.
 #pragma once
 #include "cvr_common.hpp"
+#include <cmath>
+#include <type_traits>
 
 namespace cvr {
 
@@ -90,26 +92,39 @@ __device__ __forceinline__ float row_last(float v) {
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x15f, 0xf, 0xf, true));
 }
 
+// Sum and (of values >= 0) maximum over each row of 16 lanes, in its last lane.
+template <int kShift> __device__ __forceinline__ float row_shifted(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x110 + kShift, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float row_sum(float v) {
+  v += row_shifted<1>(v);
+  v += row_shifted<2>(v);
+  v += row_shifted<4>(v);
+  return v + row_shifted<8>(v);
+}
+__device__ __forceinline__ float row_max(float v) {  // as whole numbers: the same order, one instruction each
+  int i = __float_as_int(v);
+  i = max(i, __float_as_int(row_shifted<1>(__int_as_float(i))));
+  i = max(i, __float_as_int(row_shifted<2>(__int_as_float(i))));
+  i = max(i, __float_as_int(row_shifted<4>(__int_as_float(i))));
+  return __int_as_float(max(i, __float_as_int(row_shifted<8>(__int_as_float(i)))));
+}
+
 __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Pixel i of the image in square tiles of 1 << tile_log2 pixels (at most 64), row-major, each in
-// Z order; false past the image's edges.
-__device__ __forceinline__ bool tiled_pixel(const RayFrame& rf, int tile_log2, int i, int& px, int& py) {
-  const int tiles_x = (rf.W + (1 << tile_log2) - 1) >> tile_log2, t = i >> (2 * tile_log2), j = i & ((1 << (2 * tile_log2)) - 1);
-  auto even = [](int v) {  // bits 0, 2, 4, ... of v
-    v &= 0x555;
-    v = (v | (v >> 1)) & 0x333;
-    v = (v | (v >> 2)) & 0x70f;
-    return (v | (v >> 4)) & 0x3f;
-  };
-  px = ((t % tiles_x) << tile_log2) + even(j);
-  py = ((t / tiles_x) << tile_log2) + even(j >> 1);
-  return px < rf.W && py < rf.H;
+// Bits 0, 2, 4, ... 10 of v: a Z-order index's x (of v >> 1: y).
+__device__ __forceinline__ int even_bits(int v) {
+  v &= 0x555;
+  v = (v | (v >> 1)) & 0x333;
+  v = (v | (v >> 2)) & 0x70f;
+  return (v | (v >> 4)) & 0x3f;
 }
+// Pixels of the image in square tiles of 1 << tile_log2 pixels (at most 64), row-major, each in
+// Z order.
 inline int tiled_pixels(const RayFrame& rf, int tile_log2) {
   const int m = 1 << tile_log2;
   return ((rf.W + m - 1) / m) * ((rf.H + m - 1) / m) * m * m;
@@ -124,11 +139,11 @@ struct QueueShape {
 // Tiles of 64 x 64 pixels: a unit's rays lie 32 (rays 4) or 16 (rays 16) pixels apart, so long
 // and short ones mix, while the units that run at once stay together (256^3 cone-traced frame
 // at 512^2: 18.7 ms, 23.7 ms in 16 x 16 tiles; EBS 5.0 and 6.6 ms; DOS 4.5 and 6.0 ms).
-// Narrower frames take smaller tiles.  xcd_px: pixels an XCD takes in a row.
+// Narrower frames take smaller tiles, of a unit's rays at least.  xcd_px: pixels an XCD takes in a row.
 inline QueueShape queue_shape(const RayFrame& rf, int rays, int parts, int xcd_px, int waves = 4) {
   const int side = rf.W < rf.H ? rf.W : rf.H;
   QueueShape q{rays, parts, 2, 0, 0};
-  while (q.tile_log2 < 6 && 1 << q.tile_log2 < side) ++q.tile_log2;
+  while (q.tile_log2 < 6 && (1 << q.tile_log2 < side || 1 << (2 * q.tile_log2) < rays)) ++q.tile_log2;
   const int per_wg = rays * waves / parts;  // pixels of a workgroup
   q.blocks = (tiled_pixels(rf, q.tile_log2) + per_wg - 1) / per_wg;
   while (per_wg << q.xcd_log2 < xcd_px) ++q.xcd_log2;
@@ -149,17 +164,24 @@ template <int kSub> __device__ __forceinline__ float group_uniform(float v) {
 }
 
 // The pixels of unit u of a frame: the units of a tile take its pixels in turn, `group`
-// neighbours at a time.
+// neighbours at a time (a power of two, as `rays`).
 struct FramePixels {
   const RayFrame& rf;
-  int tile_log2, first, stride, group;
-  __device__ __forceinline__ FramePixels(const RayFrame& r, const QueueShape& q, int u, int g = 1)
-      : rf(r), tile_log2(q.tile_log2), group(g) {
-    stride = (1 << (2 * q.tile_log2)) / q.rays;  // units of a tile
-    first = u / stride * (1 << (2 * q.tile_log2)) + u % stride * g;
+  int x0, y0, first, stride, group;
+  __device__ __forceinline__ FramePixels(const RayFrame& r, const QueueShape& q, int u, int g = 1) : rf(r), group(g) {
+    const int tiles_x = (rf.W + (1 << q.tile_log2) - 1) >> q.tile_log2;
+    const int log2 = 2 * q.tile_log2 - __builtin_ctz(q.rays);  // of the units of a tile
+    const int t = u >> log2;
+    stride = 1 << log2;
+    first = (u & (stride - 1)) * g;
+    x0 = (t % tiles_x) << q.tile_log2;
+    y0 = (t / tiles_x) << q.tile_log2;
   }
   __device__ __forceinline__ bool operator()(int k, int& px, int& py) const {
-    return tiled_pixel(rf, tile_log2, first + k / group * stride * group + k % group, px, py);
+    const int j = first + (k & ~(group - 1)) * stride + (k & (group - 1));
+    px = x0 + even_bits(j);
+    py = y0 + even_bits(j >> 1);
+    return px < rf.W && py < rf.H;
   }
 };
 
@@ -329,68 +351,79 @@ __device__ __forceinline__ void stage_tf_padded(float4* s_tf, const float4* __re
 
 // The march whose lighting costs less than the queue: lit(p) gives the factor of the colour of
 // the sample at p where it is met.  A lane adds up its own samples' colours and a group of 16 lanes
-// adds up its lanes' when its ray ends.  Takes rays as queue_march does.
+// adds up its lanes' when its ray ends.  The first wavefront sets up the workgroup's rays, one per lane;
+// then all of them take rays from the list.
+constexpr int kListRays = 32;  // of a workgroup (64: 128^3 at 512^2 60 us, 50 with 32)
 template <int kRays> struct RayList {
   float4 tp[kRays];   // entry point (texture space), length
   float4 dir[kRays];  // direction, pixel (bits)
+  int count, next;    // rays listed, taken
 };
-template <typename T, bool kPadded, int kRays, class Pix, class Lit1>
+template <typename T, bool kPadded, bool kSpec, class Pix, class Lit1>
 __device__ __forceinline__ void plain_march(const RayFrame& rf, const VolGeom& g, const float4* tfp, int ntf,
-                                            float step, float et, int rays, Pix&& pix, const float* spec, RayList<kRays>& Q,
+                                            float step, float et, Pix&& pix, const float* spec, RayList<kListRays>& Q,
                                             float4* __restrict__ out, unsigned int& nsamp, unsigned int& nshade,
                                             Lit1&& lit) {
   constexpr int kSub = 16;
   const int lane = threadIdx.x & 63, sub = lane % kSub, base = lane - sub;
-  const uint64_t below = (1ull << lane) - 1ull, below_group = (1ull << base) - 1ull;
-  int px = 0, py = 0;
-  const bool inside = lane < rays && pix(lane, px, py);
-  bool hit = false;
-  f3 t = mk3(0.f, 0.f, 0.f), d = t;
-  float len = 0.f;
-  if (inside) {
-    const f3 eye = ld3(rf.eye);
-    d = camera_ray(rf, px, py);
-    float tn, tf_;
-    hit = ray_box(eye, d, g.G, tn, tf_);
-    t = mk3(__builtin_fmaf(d.x, tn, eye.x), __builtin_fmaf(d.y, tn, eye.y), __builtin_fmaf(d.z, tn, eye.z));
-    t = t + mk3(0.5f * g.G[0], 0.5f * g.G[1], 0.5f * g.G[2]);
-    len = fabsf(tf_ - tn);
-    if (!hit) out[size_t(py) * rf.W + px] = make_float4(0.f, 0.f, 0.f, 0.f);
+  const uint64_t below_group = (1ull << base) - 1ull;
+  if (threadIdx.x < 64) {
+    int px = 0, py = 0;
+    const bool inside = lane < kListRays && pix(lane, px, py);
+    bool hit = false;
+    float4 t = make_float4(0.f, 0.f, 0.f, 0.f), d = t;
+    if (inside) {
+      const f3 eye = ld3(rf.eye), r = camera_ray(rf, px, py);
+      float tn, tf_;
+      hit = ray_box(eye, r, g.G, tn, tf_);
+      f3 e = mk3(__builtin_fmaf(r.x, tn, eye.x), __builtin_fmaf(r.y, tn, eye.y), __builtin_fmaf(r.z, tn, eye.z));
+      e = e + mk3(0.5f * g.G[0], 0.5f * g.G[1], 0.5f * g.G[2]);
+      t = make_float4(e.x, e.y, e.z, fabsf(tf_ - tn));
+      d = make_float4(r.x, r.y, r.z, __int_as_float(py * rf.W + px));
+      if (!hit) out[py * rf.W + px] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    const uint64_t hits = __ballot(hit);
+    if (hit) {
+      const int slot = __popcll(hits & ((1ull << lane) - 1ull));
+      Q.tp[slot] = t;
+      Q.dir[slot] = d;
+    }
+    if (lane == 0) {
+      Q.count = __popcll(hits);
+      Q.next = 0;
+    }
   }
-  const uint64_t hits = __ballot(hit);
-  const int nhit = __popcll(hits), slot = __popcll(hits & below);
-  if (nhit == 0) return;
-  if (hit) {
-    Q.tp[slot] = make_float4(t.x, t.y, t.z, len);
-    Q.dir[slot] = make_float4(d.x, d.y, d.z, __int_as_float(py * rf.W + px));
-  }
-  wave_lds_sync();
+  __syncthreads();
+  const int nhit = __builtin_amdgcn_readfirstlane(Q.count);
   f3 tp, dir;
   float4 acc;  // this lane's share of the colour; opacity of the ray
   float D;
-  int ray, jb, next = 0, pixel;
-  // the next rays for the groups without one (ray -1: none left, and D below every s)
+  int jb, pixel;
+  bool live = false;  // the group has a ray
+  // the next rays for the groups without one (none left: D below every s)
   auto take = [&]() {
-    const uint64_t need = __ballot(ray < 0 && sub == 0);
-    if (ray < 0) {
-      const int mine = next + __popcll(need & below_group), i = min(mine, nhit - 1);
+    const uint64_t need = __ballot(!live && sub == 0);
+    int next = 0;
+    if (lane == 0) next = atomicAdd(&Q.next, __popcll(need));
+    next = __builtin_amdgcn_readfirstlane(next);
+    if (!live) {
+      const int mine = next + __popcll(need & below_group), i = min(mine, kListRays - 1);
       const float4 a = Q.tp[i], b = Q.dir[i];
-      ray = mine < nhit ? mine : -1;
-      tp = mk3(a.x, a.y, a.z);
-      dir = mk3(b.x, b.y, b.z);
-      D = ray < 0 ? -1.f : a.w;
+      live = mine < nhit;
+      tp = live ? mk3(a.x, a.y, a.z) : mk3(0.f, 0.f, 0.f);
+      dir = live ? mk3(b.x, b.y, b.z) : mk3(0.f, 0.f, 0.f);
+      D = live ? a.w : -1.f;
       pixel = __float_as_int(b.w);
       jb = sub;
       acc = make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    next += __popcll(need);
   };
   auto load = [&](RaySample& s, VolTap<T>& v) {
     s = ray_sample(jb, step, D);
     v = volume_tap_load<T>(g, ray_sample_pos(s, tp, dir));
   };
-  ray = -1;
   take();
+  if (!__any(live)) return;
   // One step; the next step's blocks are in flight under it.  False: no rays left.
   auto go = [&](const RaySample& r, const VolTap<T>& tap, RaySample& r1, VolTap<T>& tap1) {
     const bool in_range = jb < kMaxSamples;
@@ -402,7 +435,8 @@ __device__ __forceinline__ void plain_march(const RayFrame& rf, const VolGeom& g
     const bool opaque = valid && src.w > 0.0f;
     const float alpha = opaque ? 1.0f - __expf(-src.w * r.h) : 0.f;
     const uint64_t valids = __ballot(valid);
-    float wa = acc.w;
+    const float w0 = acc.w;
+    float wa = w0;
     uint64_t over = 0;
     bool taken = valid;
     if (__any(opaque)) {
@@ -414,11 +448,13 @@ __device__ __forceinline__ void plain_march(const RayFrame& rf, const VolGeom& g
       float mine = taken ? (1.0f - wb) * alpha : 0.f;
       if (opaque && taken) {
         const Lit l = lit(ray_sample_pos(r, tp, dir));
-        const float ws = mine * l.s;
+        if (kSpec) {
+          const float ws = mine * l.s;
+          acc.x = __builtin_fmaf(spec[0], ws, acc.x);
+          acc.y = __builtin_fmaf(spec[1], ws, acc.y);
+          acc.z = __builtin_fmaf(spec[2], ws, acc.z);
+        }
         mine *= l.m;
-        acc.x = __builtin_fmaf(spec[0], ws, acc.x);
-        acc.y = __builtin_fmaf(spec[1], ws, acc.y);
-        acc.z = __builtin_fmaf(spec[2], ws, acc.z);
       }
       acc.x = __builtin_fmaf(mine, src.x, acc.x);
       acc.y = __builtin_fmaf(mine, src.y, acc.y);
@@ -431,19 +467,13 @@ __device__ __forceinline__ void plain_march(const RayFrame& rf, const VolGeom& g
       // some group's ray has ended (or some group has none)
       const unsigned int mine = (unsigned int)(over >> base) & 0xffffu;
       const bool ended = mine != 0 || !((valids >> (base + kSub - 1)) & 1);
-      if (__any(ended && ray >= 0)) {
-        float4 c = acc;
-        if (mine) c.w = __shfl(wa, base + __builtin_ctz(mine));
-#pragma unroll
-        for (int o = kSub / 2; o > 0; o /= 2) {
-          c.x += __shfl_xor(c.x, o);
-          c.y += __shfl_xor(c.y, o);
-          c.z += __shfl_xor(c.z, o);
-        }
-        if (ended && ray >= 0 && sub == 0) out[pixel] = c;
-        if (ended) ray = -1;
+      if (__any(ended && live)) {
+        // the opacity does not fall along a ray: that of its last sample is the largest
+        const float4 c = make_float4(row_sum(acc.x), row_sum(acc.y), row_sum(acc.z), row_max(taken ? wa : w0));
+        if (ended && live && sub == kSub - 1) out[pixel] = c;
+        if (ended) live = false;
         take();
-        if (!__any(ray >= 0)) return false;
+        if (!__any(live)) return false;
         if (ended) load(r1, tap1);
       }
     }
@@ -454,6 +484,106 @@ __device__ __forceinline__ void plain_march(const RayFrame& rf, const VolGeom& g
   load(ra, ta);
   while (go(ra, ta, rb, tb) && go(rb, tb, ra, ta)) {
   }
+}
+
+// The same march with a lane to a ray, for frames whose rays are alike: no samples are taken past a
+// ray's end, and the opacity recurrence needs no other lane.  Samples in groups of four, the next
+// group's blocks in flight under one (two register sets alternate).
+template <typename T, bool kPadded, class Lit1>
+__device__ __forceinline__ void lane_march(const RayFrame& rf, const VolGeom& g, const float4* tfp, int ntf, float step,
+                                           float et, int px, int py, float4* __restrict__ out, unsigned int& nsamp,
+                                           unsigned int& nshade, Lit1&& lit) {
+  constexpr int kGroup = 4;
+  if (px >= rf.W || py >= rf.H) return;
+  const f3 eye = ld3(rf.eye), dir = camera_ray(rf, px, py);
+  float tn, tf_;
+  float4 dst = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (ray_box(eye, dir, g.G, tn, tf_)) {
+    f3 tp = mk3(__builtin_fmaf(dir.x, tn, eye.x), __builtin_fmaf(dir.y, tn, eye.y), __builtin_fmaf(dir.z, tn, eye.z));
+    tp = tp + mk3(0.5f * g.G[0], 0.5f * g.G[1], 0.5f * g.G[2]);
+    const float D = fabsf(tf_ - tn);
+    auto load = [&](VolTap<T>* t, int j0) {
+#pragma unroll
+      for (int k = 0; k < kGroup; ++k) t[k] = volume_tap_load<T>(g, ray_sample_pos(ray_sample(j0 + k, step, D), tp, dir));
+    };
+    auto group = [&](const VolTap<T>* t, int j0) {  // true: the ray ends in this group
+      float4 src[kGroup];
+      float m[kGroup];
+#pragma unroll
+      for (int k = 0; k < kGroup; ++k) {
+        const float d = volume_tap_lerp<T>(t[k]);
+        src[k] = kPadded ? sample_tf_padded(tfp, ntf, d) : sample_tf(tfp, ntf, d);
+        m[k] = src[k].w > 0.0f ? lit(ray_sample_pos(ray_sample(j0 + k, step, D), tp, dir)).m : 0.f;
+      }
+#pragma unroll
+      for (int k = 0; k < kGroup; ++k) {
+        const RaySample r = ray_sample(j0 + k, step, D);
+        if (!(r.s < D) || j0 + k >= kMaxSamples) return true;
+        ++nsamp;
+        if (src[k].w > 0.0f) {
+          ++nshade;
+          const float alpha = 1.0f - __expf(-src[k].w * r.h), w = (1.0f - dst.w) * alpha * m[k];
+          dst.x = __builtin_fmaf(w, src[k].x, dst.x);
+          dst.y = __builtin_fmaf(w, src[k].y, dst.y);
+          dst.z = __builtin_fmaf(w, src[k].z, dst.z);
+          dst.w = opacity_after(alpha, dst.w);
+          if (dst.w > et) return true;
+        }
+      }
+      return false;
+    };
+    VolTap<T> a[kGroup], b[kGroup];
+    load(a, 0);
+    for (int j0 = 0;; j0 += 2 * kGroup) {
+      load(b, j0 + kGroup);
+      if (group(a, j0)) break;
+      load(a, j0 + 2 * kGroup);
+      if (group(b, j0 + kGroup)) break;
+    }
+  }
+  out[py * rf.W + px] = dst;
+}
+// Pixel of this lane in workgroups of 16 x 16 pixels, a wavefront 8 x 8 of them.
+__device__ __forceinline__ void lane_pixel(const RayFrame& rf, int& px, int& py) {
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  int tx, ty;
+  super_tile(xcd_remap(blockIdx.x, gridDim.x), (rf.W + 15) >> 4, (rf.H + 15) >> 4, 16, 32, tx, ty);
+  px = tx * 16 + (w & 1) * 8 + (lane & 7);
+  py = ty * 16 + (w >> 1) * 8 + (lane >> 3);
+}
+
+// Whether every ray of the frame starts inside the volume's box.
+inline bool eye_inside(const RayFrame& rf, const VolGeom& g) {
+  for (int i = 0; i < 3; ++i)
+    if (!(std::fabs(rf.eye[i]) < 0.5f * g.G[i])) return false;
+  return true;
+}
+// How the plain and the light-cache frames are marched.
+enum { kGroups = 0, kPhong = 1, kLanes = 2 };
+struct MarchShape {
+  int mode, blocks;
+  QueueShape qs;
+};
+// A lane to a ray (kLanes) in frames of kLanePixels and more from inside the volume: all their rays
+// hit it and go about as far (dense
+// volume of 291 x 336 x 306 at 576 x 442 39 us, 53 in groups; 128^3 at 701 x 433 173
+// and 175; but 400 x 327 of 128^3 about 120 and 89, and from outside 128^3 at 512^2 93 and 50).
+constexpr size_t kLanePixels = 1 << 17;
+inline MarchShape march_shape(const RayFrame& rf, const VolGeom& g, bool phong) {
+  MarchShape m;
+  m.qs = queue_shape(rf, kListRays, 4, 512);
+  m.blocks = m.qs.blocks;
+  m.mode = phong ? kPhong : kGroups;
+  if (!phong && size_t(rf.W) * rf.H >= kLanePixels && eye_inside(rf, g)) {
+    m.mode = kLanes;
+    m.blocks = ((rf.W + 15) / 16) * ((rf.H + 15) / 16);
+  }
+  return m;
+}
+template <class F> inline void with_mode(int mode, F&& f) {
+  if (mode == kLanes) f(std::integral_constant<int, kLanes>{});
+  else if (mode == kPhong) f(std::integral_constant<int, kPhong>{});
+  else f(std::integral_constant<int, kGroups>{});
 }
 
 }  // namespace cvr

@@ -50,29 +50,34 @@ struct LcK {
   float ks;          // Phong specular weight, 0 without shadows (Kspecular counts with ApplyShadow)
 };
 
-constexpr int kLcRays = 8;
-
-// PH: the Blinn-Phong branch.
-template <typename T, bool PH>
+// kMode: kGroups, kPhong (with Blinn-Phong) or kLanes.
+template <typename T, int kMode>
 __global__ __launch_bounds__(256) void k_lc_render(RayFrame rf, VolGeom g, LcK L, const float2* __restrict__ lc,
                                                    const float4* __restrict__ tf, int ntf, float step, float et,
                                                    PhongK ph, const float4* __restrict__ grad, QueueShape qs,
                                                    float4* __restrict__ out, unsigned long long* __restrict__ counters) {
-  __shared__ RayList<kLcRays> list[4];
+  __shared__ RayList<kListRays> list;
   extern __shared__ float4 s_tf[];
   stage_tf_padded(s_tf, tf, ntf);
   __syncthreads();
   const float inv_k = 1.0f / (L.ka + L.kd);
-  const FramePixels pix(rf, qs, queue_unit<1>(qs.xcd_log2), 4);
   unsigned int nsamp = 0, nshade = 0;
   const f3 eye = ld3(rf.eye);
-  plain_march<T, true>(rf, g, s_tf, ntf, step, et, qs.rays, pix, ph.spec, list[threadIdx.x >> 6], out, nsamp, nshade, [&](f3 p) {
+  auto lit = [&](f3 p) {
     const float2 I = lc_sample(lc, L.rx, L.ry, L.rz, L.tex_mul, p);
-    if (!PH) return Lit{inv_k * (I.x * L.ka + I.y * L.kd), 0.f};
+    if (kMode != kPhong) return Lit{inv_k * (I.x * L.ka + I.y * L.kd), 0.f};
     float dd, sp;
     if (!phong_terms(grad, g, ph, p, eye, dd, sp)) return Lit{1.f, 0.f};
     return Lit{inv_k * (I.x * L.ka + I.y * (L.kd * dd)), I.y * (L.ks * sp)};
-  });
+  };
+  if constexpr (kMode == kLanes) {
+    int px, py;
+    lane_pixel(rf, px, py);
+    lane_march<T, true>(rf, g, s_tf, ntf, step, et, px, py, out, nsamp, nshade, lit);
+  } else {
+    plain_march<T, true, kMode == kPhong>(rf, g, s_tf, ntf, step, et, FramePixels(rf, qs, queue_unit<4>(qs.xcd_log2), 4),
+                                          ph.spec, list, out, nsamp, nshade, lit);
+  }
   if (counters) {
     atomicAdd(&counters[0], (unsigned long long)nsamp);
     atomicAdd(&counters[1], (unsigned long long)nshade);
@@ -110,25 +115,22 @@ int launch_lc_render(cvr_ctx* c, const RayFrame& rf, int apply_occ, int apply_sd
   L.ka = apply_occ ? ka : 0.f;
   L.kd = apply_sdw ? kd : 0.f;
   L.ks = apply_sdw ? ph.ks : 0.f;
-  const QueueShape qs = queue_shape(rf, kLcRays, 1, 64);
+  const MarchShape ms = march_shape(rf, g, ph.on);
   const size_t shm = size_t(c->tf_size + 2) * sizeof(float4);
   if (c->tf_size > 4096) {
     set_error("cvr_render: light-cache march: transfer function larger than 4096 entries (staged in LDS)");
     return -4;
   }
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
-  auto launch = [&](auto t, auto p) {
+  auto by_mode = [&](auto t) {
     using T = typename decltype(t)::type;
-    constexpr bool PHv = decltype(p)::value;
-    hipLaunchKernelGGL((k_lc_render<T, PHv>), dim3(qs.blocks), dim3(256), shm, st, rf, g, L, c->d_lc, c->d_tf_rgbt,
-                       c->tf_size, step, et, ph, c->d_grad, qs, reinterpret_cast<float4*>(out), cnt);
+    with_mode(ms.mode, [&](auto m) {
+      hipLaunchKernelGGL((k_lc_render<T, decltype(m)::value>), dim3(ms.blocks), dim3(256), shm, st, rf, g, L, c->d_lc,
+                         c->d_tf_rgbt, c->tf_size, step, et, ph, c->d_grad, ms.qs, reinterpret_cast<float4*>(out), cnt);
+    });
   };
-  auto by_phong = [&](auto t) {
-    if (ph.on) launch(t, std::true_type{});
-    else launch(t, std::false_type{});
-  };
-  if (c->dtype == CVR_U8) by_phong(LcVox<uint8_t>{});
-  else by_phong(LcVox<uint16_t>{});
+  if (c->dtype == CVR_U8) by_mode(LcVox<uint8_t>{});
+  else by_mode(LcVox<uint16_t>{});
   CVR_HIP_CHECK(hipGetLastError());
   c->lc_valid = true;
   return CVR_OK;

@@ -14,10 +14,11 @@
 // (plain_march).  A frame's rays have from none to hundreds of samples: with a ray per lane
 // a wavefront ran as long as its longest one, and a 512^2 frame gave the chip about one
 // wavefront with work per SIMD, which waited for its own loads.  What bounds it now is the vector
-// arithmetic of a step (about 150 instructions for 64 samples).  64^3 at 128^2 51 -> 16 us,
-// 128^3 at 512^2 95 -> 55, 400 x 380 x 390 at 1000 x 900 420 -> 206, from inside a volume at 701 x 433
-// 195 -> 190; with Blinn-Phong 161 x 193 x 97 at 1002 x 746 307 -> 172 (shaded where it is met:
-// through the queue of the costlier renderers 243).  The 1D transfer function is staged in LDS.
+// arithmetic of a step (about 140 instructions for 64 samples).  64^3 at 128^2 51 -> 16 us,
+// 128^3 at 512^2 95 -> 50, 400 x 380 x 390 at 1000 x 900 415 -> 203; with Blinn-Phong 161 x 193 x 97
+// at 1002 x 746 307 -> 168 (shaded where it is met: through the queue of the costlier renderers
+// 243).  Large frames from inside the volume keep a lane per ray (march_shape).  The 1D transfer
+// function is staged in LDS.
 #include "cvr_ctx.hpp"
 #include "cvr_queue.hpp"
 #include <type_traits>
@@ -26,30 +27,34 @@ namespace cvr {
 
 template <class T> struct VoxTag { typedef T type; };
 
-constexpr int kPlainRays = 8;
-
-// PH: the Blinn-Phong branch.
-template <typename T, bool TF_LDS, bool PH>
+// kMode: kGroups, kPhong (with Blinn-Phong) or kLanes.
+template <typename T, bool TF_LDS, int kMode>
 __global__ __launch_bounds__(256) void k_rc1p(RayFrame rf, VolGeom g, const float4* __restrict__ tf, int ntf,
                                                float step, float et, PhongK ph, const float4* __restrict__ grad,
                                                float ka, float kd, QueueShape qs, float4* __restrict__ out,
                                                unsigned long long* __restrict__ counters) {
-  __shared__ RayList<kPlainRays> list[4];
+  __shared__ RayList<kListRays> list;
   extern __shared__ float4 s_tf[];
   if (TF_LDS) {
     stage_tf_padded(s_tf, tf, ntf);
     __syncthreads();
   }
   const float4* tfp = TF_LDS ? s_tf : tf;
-  const int u = queue_unit<1>(qs.xcd_log2);
   unsigned int nsamp = 0, nshade = 0;
   const f3 eye = ld3(rf.eye);
-  plain_march<T, TF_LDS>(rf, g, tfp, ntf, step, et, qs.rays, FramePixels(rf, qs, u, 4), ph.spec, list[threadIdx.x >> 6],
-                         out, nsamp, nshade, [&](f3 p) {
-                           float dd, sp;
-                           if (!PH || !phong_terms(grad, g, ph, p, eye, dd, sp)) return Lit{1.f, 0.f};
-                           return Lit{ka + kd * dd, ph.ks * sp};
-                         });
+  auto lit = [&](f3 p) {
+    float dd, sp;
+    if (kMode != kPhong || !phong_terms(grad, g, ph, p, eye, dd, sp)) return Lit{1.f, 0.f};
+    return Lit{ka + kd * dd, ph.ks * sp};
+  };
+  if constexpr (kMode == kLanes) {
+    int px, py;
+    lane_pixel(rf, px, py);
+    lane_march<T, TF_LDS>(rf, g, tfp, ntf, step, et, px, py, out, nsamp, nshade, lit);
+  } else {
+    plain_march<T, TF_LDS, kMode == kPhong>(rf, g, tfp, ntf, step, et, FramePixels(rf, qs, queue_unit<4>(qs.xcd_log2), 4),
+                                            ph.spec, list, out, nsamp, nshade, lit);
+  }
   if (counters) {
     atomicAdd(&counters[0], (unsigned long long)nsamp);
     atomicAdd(&counters[1], (unsigned long long)nshade);
@@ -88,24 +93,21 @@ int launch_rc1p(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* o
   const float4* gr = ph.on ? c->d_grad : nullptr;
   bool lds = c->tf_size <= 4096;
   size_t shm = lds ? size_t(c->tf_size + 2) * sizeof(float4) : 0;
-  const QueueShape qs = queue_shape(rf, kPlainRays, 1, 64);
+  const MarchShape ms = march_shape(rf, g, ph.on);
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   float4* o4 = reinterpret_cast<float4*>(out);
-  // the Blinn-Phong branch is a compile-time variant: without it the unrolled groups of
-  // the pipelined march stay small enough for twice the waves per SIMD
-  auto launch = [&](auto t, auto l, auto p) {
+  auto launch = [&](auto t, auto l, auto m) {
     using T = typename decltype(t)::type;
-    constexpr bool L = decltype(l)::value, PHv = decltype(p)::value;
-    hipLaunchKernelGGL((k_rc1p<T, L, PHv>), dim3(qs.blocks), dim3(256), L ? shm : 0, st, rf, g, c->d_tf_rgbt,
-                       c->tf_size, step, et, ph, gr, P.ka, P.kd, qs, o4, cnt);
+    constexpr bool L = decltype(l)::value;
+    hipLaunchKernelGGL((k_rc1p<T, L, decltype(m)::value>), dim3(ms.blocks), dim3(256), L ? shm : 0, st, rf, g,
+                       c->d_tf_rgbt, c->tf_size, step, et, ph, gr, P.ka, P.kd, ms.qs, o4, cnt);
   };
-  auto by_phong = [&](auto t, auto l) {
-    if (ph.on) launch(t, l, std::true_type{});
-    else launch(t, l, std::false_type{});
+  auto by_mode = [&](auto t, auto l) {
+    with_mode(ms.mode, [&](auto m) { launch(t, l, m); });
   };
   auto by_lds = [&](auto t) {
-    if (lds) by_phong(t, std::true_type{});
-    else by_phong(t, std::false_type{});
+    if (lds) by_mode(t, std::true_type{});
+    else by_mode(t, std::false_type{});
   };
   if (c->dtype == CVR_U8) by_lds(VoxTag<uint8_t>{});
   else by_lds(VoxTag<uint16_t>{});

@@ -157,6 +157,40 @@ def test_light_cache(n, w, h, alpha_max, phong):
     check(img, ref, m)
 
 
+@pytest.mark.parametrize("entries,bits", [(256, 8), (5000, 16)])
+@pytest.mark.parametrize("w,h", [(363, 362), (1024, 128), (400, 327)])
+def test_plain_from_inside(w, h, entries, bits):
+    """A lane to a ray from 2^17 pixels on: one more, just as many, and fewer."""
+    wl = W.cone_blobs(n=24, width=w, height=h, seed=31)
+    vol = wl.volume if bits == 8 else (wl.volume.astype(np.uint16) * 257)
+    rgb, a = W.seeded_tf(131, 4, alpha_max=0.5)
+    rgb[:, 3] = np.round(rgb[:, 3] * (entries - 1) / 255)
+    a[:, 1] = rgb[:, 3]
+    r = N.Renderer(N.RC1P)
+    r.set_volume(vol, wl.scale)
+    r.set_transfer_function(rgb, a, max_density=entries - 1)
+    r.collect_stats()
+    cam = N.Camera((2.0, -1.0, 3.0), (0.0, 0.0, -40.0), (0.0, 1.0, 0.0), 60.0, w / h)
+    img = r.render(cam, w, h)
+    ref, m = O.render_rc1p(vol, O.OTF(rgb, a, max_density=entries - 1), cam, w, h)
+    check(img, ref, m)
+
+
+def test_light_cache_from_inside():
+    w, h = 363, 362
+    wl = W.cone_blobs(n=24, width=w, height=h, seed=31)
+    rgb, a = W.seeded_tf(131, 4, alpha_max=0.5)
+    r = N.Renderer(N.EBS)
+    r.set_volume(wl.volume, wl.scale)
+    r.set_transfer_function(rgb, a)
+    r.set_params(light_cache=1)
+    p = r.params()
+    cam = N.Camera((2.0, -1.0, 3.0), (0.0, 0.0, -40.0), (0.0, 1.0, 0.0), 60.0, w / h)
+    img = r.render(cam, w, h, light=wl.light())
+    ref, m = O.render_lc(wl.volume, O.OTF(rgb, a), r.light_cache(), 1, 1, p.ka, p.kd, cam, w, h, scale=wl.scale)
+    check(img, ref, m)
+
+
 def test_buffers_kept_between_volumes_hold_the_new_ones():
     """Volumes, cones and networks of changing and equal sizes through one handle, against new
     handles: what a handle keeps is of the call at hand."""
