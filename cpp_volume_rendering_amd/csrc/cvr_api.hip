@@ -216,6 +216,7 @@ static void free_all(cvr_ctx* c) {
   if (c->d_sat) (void)hipFree(c->d_sat);
   if (c->d_sat_oct) (void)hipFree(c->d_sat_oct);
   if (c->d_ext_lut) (void)hipFree(c->d_ext_lut);
+  if (c->d_tf_alpha) (void)hipFree(c->d_tf_alpha);
   if (c->d_counters) (void)hipFree(c->d_counters);
   if (c->d_out) (void)hipFree(c->d_out);
   if (c->d_ms_frame) (void)hipFree(c->d_ms_frame);
@@ -540,7 +541,7 @@ int cvr_prepare(cvr_handle h, void* hip_stream) {
   if (rc) return rc;
   DeviceGuard dg(h->device);
   hipStream_t st = static_cast<hipStream_t>(hip_stream);
-  if (h->technique == CVR_EBS) return build_sat(h, st, h->ebs.sat_layout == 0);
+  if (h->technique == CVR_EBS) return build_sat(h, st, ebs_reads_blocks(h->ebs));
   if (h->technique == CVR_CONE_GT) return prepare_gt(h, h->gt);
   if (h->technique == CVR_DOS) return prepare_dos(h, h->dos, st);
   if (h->technique == CVR_CONE_TRACE) return prepare_cone(h, h->cone, st);

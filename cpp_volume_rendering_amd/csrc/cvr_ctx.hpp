@@ -82,6 +82,8 @@ struct cvr_ctx {
   float2* d_sat = nullptr;
   void* d_sat_oct = nullptr;  // corner blocks of the SAT, 64 B per cell (k_sat.hip)
   float* d_ext_lut = nullptr;  // per raw value extinction (GetExtN), 256 or 65536 entries
+  void* d_tf_alpha = nullptr;  // the transfer function's alpha column (FP64) of d_ext_lut
+  size_t tf_alpha_bytes = 0;
   uint64_t sat_built_for = ~0ull;
   uint64_t sat_oct_built_for = ~0ull;  // d_sat_oct holds the blocks of this SAT
 
@@ -167,6 +169,10 @@ int launch_rc1p(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* o
 // Blinn-Phong constants of a render (builds the gradient when shading is on)
 int phong_setup(cvr_ctx* c, int on, int gradient_type, float ks, float shininess, const float spec[3],
                 const RayFrame& rf, const cvr_light* light, PhongK& ph, hipStream_t st);
+// whether a frame reads the SAT's corner blocks: not with the light cache, whose 32^3 cells are
+// done from the linear table in the time that writing the blocks takes (256^3: blocks 245 us and
+// cache 300 us from them, 250 us from the linear table)
+inline bool ebs_reads_blocks(const cvr_ebs_params& P) { return P.sat_layout == 0 && !P.light_cache; }
 // the SAT of the current volume and TF; with_blocks: also its corner blocks
 int build_sat(cvr_ctx* c, hipStream_t st, bool with_blocks = false);
 // volume gradient of `type` for Blinn-Phong shading
