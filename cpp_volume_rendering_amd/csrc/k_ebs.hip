@@ -437,30 +437,121 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   }
 }
 
+// Corner v (as corner_issue numbers them) of a box, in texel coordinates.
+struct Corner {
+  double x, y, z;
+};
+__device__ __forceinline__ Corner box_corner(const EbsK& k, int v, f3 p1, f3 p2) {
+  const float x = (v & 1) ? p1.x : p2.x, y = (v & 4) ? p1.y : p2.y, z = (v & 2) ? p1.z : p2.z;
+  return Corner{double(fminf(fmaxf(x + k.scale[0], k.minSAT[0]), k.maxSAT[0])) * k.sat_tex_mul[0] - 0.5,
+                double(fminf(fmaxf(y + k.scale[1], k.minSAT[1]), k.maxSAT[1])) * k.sat_tex_mul[1] - 0.5,
+                double(fminf(fmaxf(z + k.scale[2], k.minSAT[2]), k.maxSAT[2])) * k.sat_tex_mul[2] - 0.5};
+}
+// The weighted sum of a stream of box sums over the eight lanes of a group, a lane to each of the
+// boxes' corners: next(corner, weight) gives this lane's corner of the next box.  Both exponents
+// are linear in the box sums, so the lanes' shares are added up once, at the end.
+template <class Next>
+__device__ __forceinline__ double corner_sum(const void* __restrict__ sat, const EbsK& k, Next&& next) {
+  const int v = threadIdx.x & 7;
+  const double sign = (v == 0 || v == 3 || v == 5 || v == 6) ? 1.0 : -1.0;
+  double acc = 0.0;
+  Corner c;
+  double wa, wb;
+  TapSlot<1> a, b;
+  if (next(c, wa)) {
+    tap_issue<1>(sat, k, c.x, c.y, c.z, a);
+    for (;;) {
+      const bool more_b = next(c, wb);
+      if (more_b) tap_issue<1>(sat, k, c.x, c.y, c.z, b);
+      acc += wa * tap_eval<1>(a);
+      if (!more_b) break;
+      const bool more_a = next(c, wa);
+      if (more_a) tap_issue<1>(sat, k, c.x, c.y, c.z, a);
+      acc += wb * tap_eval<1>(b);
+      if (!more_a) break;
+    }
+  }
+  acc *= sign;
+  for (int o = 1; o < 8; o *= 2) acc += __shfl_xor(acc, o);
+  return acc;
+}
+
 // Object-space light cache (rc1pextbsd/lightcachecomputation.comp:440-468): cell i holds
 // (AO, shadow) at texture-space position (i + 1/2) * cell, 1 for a term that is off,
-// from the renderer's own AO and shadow evaluations.  One lane per cell.
-template <int L>
-// 64-lane workgroups, at most one wave per SIMD (a 32^3 cache is 512 waves): the box
-// streams' registers beyond the 256 architectural VGPRs live in AGPRs.
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_lc_ebs(EbsK k, const void* __restrict__ sat, const ShadowRow* __restrict__ rows,
+// from the renderer's own AO and shadow boxes (ebs_ao, ebs_shadow_table, ebs_shadow_point).
+// A 32^3 cache is 512 wavefronts with a lane to a cell, half of one per SIMD, each a chain
+// of box sums; with eight lanes to a cell, one to each corner of its boxes, it is 4096 and
+// each lane holds two taps (256^3 with shadows, from the linear table: 267 -> 250 us, and
+// bound by the
+// lines it reads, of which a tap uses 64 bytes in four, and the FP64 lerps; 240 with the cells of an
+// XCD side by side).
+__global__ __launch_bounds__(256) void k_lc_ebs(EbsK k, const void* __restrict__ sat, const ShadowRow* __restrict__ rows,
                                                 int rx, int ry, int rz, f3 cell, float2* __restrict__ lc) {
   extern __shared__ float4 smem[];
   ShadowRow* s_rows = reinterpret_cast<ShadowRow*>(smem);
   ebs_load_rows(rows, k.nrows, s_rows);
-  const int nrows = k.nrows;
   const size_t n = size_t(rx) * ry * rz;
-  const size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+  const size_t i = (size_t(xcd_remap(blockIdx.x, gridDim.x, 7)) * blockDim.x + threadIdx.x) >> 3;
+  if (i >= n) return;  // whole groups of eight lanes
+  const int v = threadIdx.x & 7;
   const int x = int(i % size_t(rx)), y = int((i / size_t(rx)) % size_t(ry)), z = int(i / (size_t(rx) * ry));
   const f3 tp = mk3((float(x) + 0.5f) * cell.x, (float(y) + 0.5f) * cell.y, (float(z) + 0.5f) * cell.z);
-  unsigned int nbox = 0;
   float Io = 1.f, Is = 1.f;
-  if (k.apply_occ) Io = ebs_ao<L>(sat, k, tp);
-  if (k.apply_sdw)
-    Is = k.shadow_type == 1 ? ebs_shadow_table<L>(sat, k, s_rows, nrows, tp, nbox)
-                            : ebs_shadow_point<L>(sat, k, tp, nbox);
-  lc[i] = make_float2(Io, Is);
+  if (k.apply_occ) {
+    const f3 sc = ld3(k.scale);
+    const double rad = k.ao_radius;
+    int gi = 0;
+    const double t = corner_sum(sat, k, [&](Corner& c, double& w) {
+      if (gi >= k.shells) return false;
+      const float r1f = k.ao_radius * float(gi + 1);
+      c = box_corner(k, v, tp - sc * r1f, tp + sc * r1f);
+      // shell i counts (S_i - S_(i-1)) / r_i^2
+      const double r1 = rad * double(gi + 1), r2 = rad * double(gi + 2);
+      w = 1.0 / (r1 * r1) - (gi + 1 < k.shells ? 1.0 / (r2 * r2) : 0.0);
+      ++gi;
+      return true;
+    });
+    const double rn = rad * double(k.shells);
+    Io = __expf(-float((1.0 / (rn * rn)) * t));
+  }
+  if (k.apply_sdw && k.shadow_type == 1) {
+    const float pa = comp(tp, k.axis), lo = k.axis_lo, hi = k.axis_hi;
+    int r = 0;
+    Is = __expf(-float(corner_sum(sat, k, [&](Corner& c, double& w) {
+      if (r >= k.nrows) return false;
+      const ShadowRow& R = s_rows[r];
+      const float nxt = pa + R.next;
+      if (!(nxt > lo && nxt < hi)) return false;
+      c = box_corner(k, v, tp + ld3(R.o1), tp + ld3(R.o2));
+      w = double(R.inv_vq) * double(k.sdw_weight);
+      ++r;
+      return true;
+    })));
+  } else if (k.apply_sdw) {
+    const f3 real = tp - mk3(0.5f * k.g.G[0], 0.5f * k.g.G[1], 0.5f * k.g.G[2]);
+    const f3 cvv = norm3(ld3(k.light_pos) - real);
+    float cv[3] = {cvv.x, cvv.y, cvv.z};
+    ConeGeom<float> cg;
+    cone_setup<float>(cv, k.sdw_angle, k.sdw_interval, k.sdw_initial, k.scale, cg);
+    const int a = cg.axis;
+    const float pa = comp(tp, a), lo = sel3(k.minVol, a), hi = sel3(k.maxVol, a), cva = sel3(cv, a);
+    float apos = cg.apos0;
+    Is = __expf(-float(corner_sum(sat, k, [&](Corner& c, double& w) {
+      if (!((apos / cva) < k.sdw_max_dist)) return false;
+      const float nxt = pa + (apos + cg.interval);
+      if (!(nxt > lo && nxt < hi)) return false;
+      float o1[3], o2[3];
+      cone_box<float>(cg, apos, o1, o2);
+      const f3 p1 = tp + ld3(o1), p2 = tp + ld3(o2);
+      const float vq =
+          (fabsf(p1.x - p2.x) / k.scale[0]) * (fabsf(p1.y - p2.y) / k.scale[1]) * (fabsf(p1.z - p2.z) / k.scale[2]);
+      c = box_corner(k, v, p1, p2);
+      w = double(k.sdw_weight) / double(vq);
+      apos = apos + cg.interval;
+      return true;
+    })));
+  }
+  if (v == 0) lc[i] = make_float2(Io, Is);
 }
 
 int launch_ebs(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out, hipStream_t st) {
@@ -473,7 +564,7 @@ int launch_ebs(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* ou
     set_error("cvr_render: EBS ao_shells >= 1, ao_radius > 0 and sdw_interval > 0 required");
     return -1;
   }
-  int rc = build_sat(c, st, P.sat_layout == 0);
+  int rc = build_sat(c, st, ebs_reads_blocks(P));
   if (rc) return rc;
   EbsK k{};
   k.g = geom_of(c);
@@ -574,12 +665,8 @@ int launch_ebs(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* ou
       return -4;
     }
     const ShadowRow* lrows = static_cast<const ShadowRow*>(c->d_ebs_rows);
-    if (P.sat_layout == 1)
-      hipLaunchKernelGGL(k_lc_ebs<1>, dim3(unsigned((n + 63) / 64)), dim3(64), size_t(k.nrows) * sizeof(ShadowRow), st,
-                         k, static_cast<const void*>(c->d_sat), lrows, rx, ry, rz, cell, c->d_lc);
-    else
-      hipLaunchKernelGGL(k_lc_ebs<0>, dim3(unsigned((n + 63) / 64)), dim3(64), size_t(k.nrows) * sizeof(ShadowRow), st,
-                         k, static_cast<const void*>(c->d_sat_oct), lrows, rx, ry, rz, cell, c->d_lc);
+    hipLaunchKernelGGL(k_lc_ebs, dim3(unsigned((n + 31) / 32)), dim3(256), size_t(k.nrows) * sizeof(ShadowRow), st, k,
+                       static_cast<const void*>(c->d_sat), lrows, rx, ry, rz, cell, c->d_lc);
     CVR_HIP_CHECK(hipGetLastError());
     return launch_lc_render(c, rf, P.apply_occlusion, P.apply_shadow, P.ka, P.kd, step, P.et_threshold, ph, out, st);
   }

@@ -223,3 +223,47 @@ def test_buffers_kept_between_volumes_hold_the_new_ones():
         new.nn_set_weights(w)
         (la, ga), (lb, gb) = net.nn_gradient(x, t), new.nn_gradient(x, t)
         assert la == lb and np.array_equal(ga, gb)
+
+
+@pytest.mark.parametrize("res", [(1, 1, 1), (5, 3, 2), (7, 11, 3), (33, 2, 4)])
+@pytest.mark.parametrize("shadow_type,occ,sdw", [(0, 1, 1), (1, 1, 1), (1, 0, 1), (0, 1, 0)])
+def test_light_cache_cells(res, shadow_type, occ, sdw):
+    """Eight lanes to a cell: fewer cells than a workgroup's, part of the last one's, and each of
+    the terms alone.  The tolerance is that of the cache's own tests."""
+    wl = W.banded_noise(n=20, width=16, height=16, seed=12)
+    vol = np.ascontiguousarray(wl.volume[:, :13, :9])
+    r = N.Renderer(N.EBS)
+    r.set_volume(vol, wl.scale)
+    r.set_transfer_function(wl.rgb_iso, wl.alpha_iso)
+    p = r.params()
+    p.shadow_type, p.apply_occlusion, p.apply_shadow, p.light_cache = shadow_type, occ, sdw, 1
+    p.light_cache_res[:] = list(res)
+    r.set_params(p)
+    p = r.params()
+    light = wl.light()
+    r.render(wl.camera(), 16, 16, light=light)
+    prm = O.ebs_params(p, light)
+    grid = np.array(vol.shape[::-1]) * np.array(wl.scale)
+    prm.sdw_max_dist = np.float32(0.75) * np.float32(float(np.linalg.norm(grid)))
+    ref = O.lc_ebs(vol.shape[::-1], wl.scale, O.sat(vol, O.OTF(wl.rgb_iso, wl.alpha_iso)), prm, res)
+    d = np.abs(r.light_cache().astype(np.float64) - ref)
+    assert d.max() <= 5e-4, d.max()
+
+
+@pytest.mark.parametrize("bits,entries,ext", [(8, 256, 0), (8, 2, 0), (16, 256, 0), (16, 4096, 0), (16, 70000, 0), (16, 256, 1)])
+def test_summed_area_table_of_each_extinction_table(bits, entries, ext):
+    """The table's last cell is the sum of every voxel's extinction, each a 32-bit value of the
+    table: a step of 2^-23 in one of them stands out less than 1e-6 of the sum."""
+    rng = np.random.default_rng(entries)
+    vol = rng.integers(0, 1 << bits, (6, 7, 8)).astype(np.uint8 if bits == 8 else np.uint16)
+    rgb, a = W.seeded_tf(131, 4, alpha_max=0.9)
+    if entries == 2:
+        rgb, a = rgb[[0, -1]], a[[0, -1]]
+    rgb[:, 3] = np.round(rgb[:, 3] * (entries - 1) / 255)
+    a[:, 1] = rgb[:, 3]
+    r = N.Renderer(N.EBS)
+    r.set_volume(vol, (1.0, 1.0, 1.0))
+    r.set_transfer_function(rgb, a, max_density=entries - 1, extinction_input=bool(ext))
+    got = r.get_sat(vol.shape[::-1])
+    ref = O.sat(vol, O.OTF(rgb, a, max_density=entries - 1, extinction_input=bool(ext)))
+    assert np.abs(got - ref).max() <= 1e-6 * ref.max()
