@@ -7,10 +7,6 @@
 
 namespace cvr {
 
-// One step of a cone march: midpoint distance, segment length, pyramid level.
-struct ConeStepF {
-  float tm, dt, lod, pad;
-};
 // One stencil point of the surrogate's features: distance along the axis, segment
 // length, pyramid level.
 struct StencilF {
@@ -56,11 +52,11 @@ template <class Fn> void with_types(int dtype, int fmt, Fn&& fn) {
 
 // Per-frame cone-tracer constants.
 struct ConeK {
-  int n_steps, n_occ, apply_occ, apply_sdw;
+  int n_occ, apply_occ, apply_sdw;
   float ring_cos, ring_sin, ka, kd;
   float L[3];               // shadow cone axis (towards the light)
-  const ConeStepF* so;      // occlusion schedule [n_steps]
-  const ConeStepF* ss;      // shadow schedule [n_steps]
+  ConeSched so, ss;         // occlusion and shadow schedules
+  const ConeLevel* lev;     // [levels]
   const FeatTap* ft;        // surrogate inputs: axial/ring pairs [2*kNOcc], shadow [kNSdw], local [1]
 };
 
@@ -139,35 +135,91 @@ __device__ __forceinline__ float border_falloff(const PyrGeom& pg, f3 tp, float 
   return __expf(-(cx * cx + cy * cy + cz * cz) * inv2sg2);
 }
 
-// textureLod with LINEAR_MIPMAP_LINEAR (lerp of levels floor(lod) and floor(lod)+1,
-// the second clamped to the chain), then the border falloff.
-template <int F>
-__device__ __forceinline__ float gauss_ext(const void* __restrict__ pyr, const PyrGeom& pg, f3 tp, float lod) {
-  const float q = float(pg.levels - 1);
-  lod = fminf(fmaxf(lod, 0.f), q);
-  const int d1 = int(floorf(lod));
-  const int d2 = min(d1 + 1, pg.levels - 1);
-  const float fr = lod - float(d1);
-  const float a = pyr_tri<F>(pyr, pg, d1, tp);
-  const float b = pyr_tri<F>(pyr, pg, d2, tp);
-  return (a * (1.f - fr) + b * fr) * border_falloff(pg, tp, 0.5f * exp2f(-2.f * lod));
+// Byte offset of corner block (x0, y0, z0) in a level of `nbx` x `nby` bricks, records of
+// 2^kShift bytes: brick number, then the 6 bits of in-brick position (brick_index).  The
+// 32-bit form needs the level's records to span less than 4 GiB (PyrGeom::wide = 0); its
+// products are 24-bit (v_mad_u32_u24).
+template <int kShift>
+__device__ __forceinline__ uint32_t oct_offset32(int x0, int y0, int z0, int nbx, int nby) {
+  const uint32_t b = mad24(mad24(uint32_t(z0) >> 2, uint32_t(nby), uint32_t(y0) >> 2), uint32_t(nbx), uint32_t(x0) >> 2);
+  const uint32_t local = ((uint32_t(z0) & 3u) << 4) | ((uint32_t(y0) & 3u) << 2) | (uint32_t(x0) & 3u);
+  return ((b << 6) | local) << kShift;
 }
 
-// The same lookup at a whole level `l` (one trilinear read).
-template <int F>
-__device__ __forceinline__ float gauss_ext_level(const void* __restrict__ pyr, const PyrGeom& pg, f3 tp, int l) {
-  return pyr_tri<F>(pyr, pg, l, tp) * border_falloff(pg, tp, __uint_as_float((126u - 2u * unsigned(l)) << 23));
+// The smallest of the active lanes' values, in a scalar register.
+__device__ __forceinline__ float wave_min(float v) {
+  float m = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+  for (uint64_t b = __ballot(v < m); b; b = __ballot(v < m))
+    m = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), __builtin_ctzll(b)));
+  return m;
 }
 
-template <int F>
-__device__ __forceinline__ float cone_T(const void* __restrict__ pyr, const PyrGeom& pg, const ConeStepF* __restrict__ s,
-                                        int n, f3 p, f3 axis) {
+// Transmittance of a cone of 64 steps and one or two trilinear reads each, the bulk of a
+// cone-traced frame.  Bound by vector instructions and the L1's tag rate (four 16-byte loads of a
+// step's two 32-byte blocks), so whatever is the same for all lanes is in the tables (scalar loads),
+// steps whose level is a whole one read it alone (23 of the 64 of an occlusion cone: the first, within
+// two sigma of level 0, and those past the last level), and steps before the first lane leaves the
+// box do without the border falloff, which is 1 there.  256^3 at 1024^2 68.6 -> 54.5 ms, at 512^2 18.7 -> 14.4 (vector
+// instructions issued in 82 % of the cycles, 0.85 L1 tags a cycle and CU).
+template <int F, bool kWide>
+__device__ __forceinline__ float cone_T(const void* __restrict__ pyr, const PyrGeom& pg,
+                                        const ConeLevel* __restrict__ levels, const ConeSched& S, f3 p, f3 axis) {
+  typedef typename PyrOct<F>::type B;
+  typedef const __attribute__((address_space(4))) ConeStepF* ConstSteps;
+  typedef const __attribute__((address_space(4))) ConeLevel* ConstLevels;
+  const ConstSteps s = (ConstSteps)(uintptr_t)S.s;
+  const ConstLevels lev = (ConstLevels)(uintptr_t)levels;
+  constexpr int kShift = sizeof(B) == 32 ? 5 : 4;
+  // the steps up to which every lane's cone axis is inside the box
+  auto leave = [&](float a, float q, float G) { return ((a > 0.f ? G : 0.f) - q) / a; };
+  const float te = wave_min(fminf(leave(axis.x, p.x, pg.G[0]), fminf(leave(axis.y, p.y, pg.G[1]), leave(axis.z, p.z, pg.G[2]))));
+  int jin = min(max(int(floorf((__log2f(te) - S.log2_t0) * S.inv_log2_q)) + 1, 0), S.n);
+  jin = __builtin_amdgcn_readfirstlane(jin);
+  while (jin > 0 && !(s[jin - 1].tm <= te)) --jin;
   float od = 0.f;
-#pragma unroll 4
-  for (int j = 0; j < n; ++j) {
-    const ConeStepF c = s[j];
-    od += gauss_ext<F>(pyr, pg, p + axis * c.tm, c.lod) * c.dt;
-  }
+  auto read = [&](int l, f3 tp) {
+    const ConstLevels g = lev + l;
+    int x0, y0, z0;
+    float fx, fy, fz;
+    quad_axis_f(fmaf(tp.x, g->ts[0], -0.5f), g->dmax[0], x0, fx);
+    quad_axis_f(fmaf(tp.y, g->ts[1], -0.5f), g->dmax[1], y0, fy);
+    quad_axis_f(fmaf(tp.z, g->ts[2], -0.5f), g->dmax[2], z0, fz);
+    const char* lv = static_cast<const char*>(pyr) + ((size_t(g->boff_hi) << 32) | g->boff_lo);
+    if constexpr (kWide)
+      return pyr_lerp<F>(*reinterpret_cast<const B*>(lv + (brick_index(x0, y0, z0, g->nb[0], g->nb[1]) << kShift)), fx, fy, fz, pg.one);
+    else
+      return pyr_lerp<F>(*reinterpret_cast<const B*>(lv + oct_offset32<kShift>(x0, y0, z0, g->nb[0], g->nb[1])), fx, fy, fz, pg.one);
+  };
+  auto step = [&](auto two, auto border, int j) {
+    const float tm = s[j].tm;
+    const f3 tp = p + axis * tm;
+    float v = read(s[j].level, tp);
+    if constexpr (decltype(two)::value) v = v * s[j].omf + read(s[j].level + 1, tp) * s[j].fr;
+    if constexpr (decltype(border)::value) {
+      const float cx = __builtin_amdgcn_fmed3f(tp.x, 0.f, pg.G[0]) - tp.x;
+      const float cy = __builtin_amdgcn_fmed3f(tp.y, 0.f, pg.G[1]) - tp.y;
+      const float cz = __builtin_amdgcn_fmed3f(tp.z, 0.f, pg.G[2]) - tp.z;
+      v *= __builtin_amdgcn_exp2f((cx * cx + cy * cy + cz * cz) * s[j].fall);
+    }
+    od += v * s[j].dt;
+  };
+  // kAhead steps' loads are in flight together (256^3 at 512^2: 14.6 ms with 2, 14.4 with 3, 17.6 with 4)
+  constexpr int kAhead = 3;
+  auto part = [&](auto two, int b, int e) {
+    const int m = min(max(jin, b), e);
+    int j = b;
+    auto run = [&](auto border, int end) {
+      for (; j + kAhead <= end; j += kAhead)
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) step(two, border, j + u);
+      for (; j < end; ++j) step(two, border, j);
+    };
+    run(std::false_type{}, m);
+    run(std::true_type{}, e);
+  };
+  part(std::false_type{}, 0, S.n0);
+  part(std::true_type{}, S.n0, S.n1);
+  part(std::false_type{}, S.n1, S.n);
   return __expf(-od);
 }
 
@@ -178,21 +230,52 @@ __device__ __forceinline__ void occ_frame(f3 dir, f3& k, f3& up, f3& right) {
   k = mk3(-dir.x, -dir.y, -dir.z);
 }
 
-// 1 axial cone + (n_occ-1) cones whose axes sit on a ring at ring angle from the axis,
-// cosine-weighted like gt_ray_marching.comp:161-168.
-template <int F>
-__device__ __forceinline__ float ct_occlusion(const void* __restrict__ pyr, const PyrGeom& pg, const ConeK& K, f3 p,
-                                              f3 k, f3 up, f3 right) {
-  float num = cone_T<F>(pyr, pg, K.so, K.n_steps, p, k), den = 1.f;
+// Occlusion and shadow of a sample.  Occlusion: 1 axial cone + (n_occ-1) cones whose axes
+// sit on a ring at ring angle from the axis, cosine-weighted like gt_ray_marching.comp:161-168;
+// 0 and not computed for a term that is off.  One loop over all the cones: the march is inlined
+// once.
+template <int F, bool kWide>
+__device__ __forceinline__ void ct_light_at(const void* __restrict__ pyr, const PyrGeom& pg, const ConeK& K, f3 p, f3 dir,
+                                            f3 L, bool occ, bool sdw, float& Io, float& Is) {
+  f3 k, up, right;
+  occ_frame(dir, k, up, right);
+  float num = 0.f, den = 0.f;
   const int nr = K.n_occ - 1;
-  for (int j = 0; j < nr; ++j) {
-    float sphi, cphi;
-    __sincosf(6.283185307179586f * float(j) / float(nr), &sphi, &cphi);
-    const f3 ax = k * K.ring_cos + (up * cphi + right * sphi) * K.ring_sin;
-    num += K.ring_cos * cone_T<F>(pyr, pg, K.so, K.n_steps, p, ax);
-    den += K.ring_cos;
+  Is = 0.f;
+  for (int j = occ ? 0 : K.n_occ; j < K.n_occ + (sdw ? 1 : 0); ++j) {
+    f3 ax = k;
+    float w = 1.f;
+    if (j == K.n_occ) {
+      ax = L;
+    } else if (j > 0) {
+      float sphi, cphi;
+      __sincosf(6.283185307179586f * float(j - 1) / float(nr), &sphi, &cphi);
+      ax = k * K.ring_cos + (up * cphi + right * sphi) * K.ring_sin;
+      w = K.ring_cos;
+    }
+    const bool sd = j == K.n_occ;
+    ConeSched S;
+    S.s = sd ? K.ss.s : K.so.s;
+    S.n = sd ? K.ss.n : K.so.n;
+    S.n0 = sd ? K.ss.n0 : K.so.n0;
+    S.n1 = sd ? K.ss.n1 : K.so.n1;
+    S.log2_t0 = sd ? K.ss.log2_t0 : K.so.log2_t0;
+    S.inv_log2_q = sd ? K.ss.inv_log2_q : K.so.inv_log2_q;
+    const float t = cone_T<F, kWide>(pyr, pg, K.lev, S, p, ax);
+    if (sd) {
+      Is = t;
+    } else {
+      num += w * t;
+      den += w;
+    }
   }
-  return num / den;
+  Io = occ ? num / den : 0.f;
+}
+template <int F>
+__device__ __forceinline__ void ct_light(const void* __restrict__ pyr, const PyrGeom& pg, const ConeK& K, f3 p, f3 dir,
+                                         f3 L, bool occ, bool sdw, float& Io, float& Is) {
+  if (pg.wide) ct_light_at<F, true>(pyr, pg, K, p, dir, L, occ, sdw, Io, Is);
+  else ct_light_at<F, false>(pyr, pg, K, p, dir, L, occ, sdw, Io, Is);
 }
 
 // The surrogate's 16 inputs (see the CPU oracle's nn_features): for occlusion segment i
@@ -202,7 +285,7 @@ __device__ __forceinline__ float ct_occlusion(const void* __restrict__ pyr, cons
 // length kept in registers), so one memory round trip serves the group, and the groups
 // are software-pipelined: the next group's loads are in flight while the current group
 // is interpolated (512^3 surrogate frame at 1024^2, fp16: 5.80 -> 5.57 ms).  Each read is
-// gauss_ext_level's, with the segment length folded into the falloff factor.  Groups of 4
+// one trilinear value times the border falloff, with the segment length folded into the factor.  Groups of 4
 // keep two groups of 32-byte fp32 records within the registers of two waves per SIMD.
 // The groups only order the loads: every input is computed the same way whatever their
 // size.
@@ -213,18 +296,6 @@ typedef const __attribute__((address_space(4))) FeatTap* ConstTaps;
 #endif
 template <int F>
 __host__ __device__ constexpr int feat_group() { return CVR_FEAT_GROUP ? CVR_FEAT_GROUP : 4; }
-
-// Byte offset of corner block (x0, y0, z0) in a level of `nbx` x `nby` bricks, records of
-// 2^kShift bytes: brick number, then the 6 bits of in-brick position (brick_index).  The
-// 32-bit form needs the level's records to span less than 4 GiB (PyrGeom::wide = 0); its
-// products are 24-bit (v_mad_u32_u24).
-template <int kShift>
-__device__ __forceinline__ uint32_t oct_offset32(int x0, int y0, int z0, int nbx, int nby) {
-  const uint32_t b = __umul24(__umul24(uint32_t(z0) >> 2, uint32_t(nby)) + (uint32_t(y0) >> 2), uint32_t(nbx)) +
-                     (uint32_t(x0) >> 2);
-  const uint32_t local = ((uint32_t(z0) & 3u) << 4) | ((uint32_t(y0) & 3u) << 2) | (uint32_t(x0) & 3u);
-  return ((b << 6) | local) << kShift;
-}
 
 template <int F, bool kWide>
 __device__ __forceinline__ void nn_feats_at(const void* __restrict__ pyr, const PyrGeom& pg,

@@ -42,6 +42,28 @@ struct PyrKey {
 };
 // Section table of one directional-occlusion cone: rows (interval, level, d_integral,
 // amplitude), section counts with 1/3/7 Gaussians, sub-cone axes.
+// One step of a cone march: midpoint distance, segment length, and of its pyramid level lod: the
+// weights 1 - fr and fr of the levels `level` and level + 1 (fr 0: the first alone), and the border
+// falloff's -log2(e) / (2 (2^lod)^2).
+struct ConeStepF {
+  float tm, dt, omf, fr, fall;
+  int level, pad[2];
+};
+// A pyramid level as the cone march reads it, 48 bytes of a 64-byte row: texel coordinate per
+// world unit, last texel index per axis, bricks, byte offset of its corner blocks.
+struct ConeLevel {
+  float ts[3], dmax[3];
+  int nb[2];
+  unsigned int boff_lo, boff_hi;
+  int pad[6];
+};
+// A cone's steps.  Steps [0, n0) and [n1, n) read one level, those between two.  Midpoint j lies at
+// exp2(log2_t0 + j / inv_log2_q).
+struct ConeSched {
+  const ConeStepF* s;
+  int n, n0, n1;
+  float log2_t0, inv_log2_q;
+};
 struct DosTable {
   std::vector<float4> rows;
   int n[3] = {0, 0, 0};
@@ -112,7 +134,7 @@ struct cvr_ctx {
   std::vector<float> gt_occ, gt_sdw;
   float* d_gt_rays = nullptr;
   cvr_gt_params gt_rays_for{};
-  int cone_n_steps = 0;
+  cvr::ConeSched cone_sched[2] = {};  // occlusion, shadow: pointers into d_cone_tab
 
   // surrogate network: fp32 master weights, gradient, Adam moments, packed bf16 copy
   float *d_nn_w = nullptr, *d_nn_g = nullptr, *d_nn_m = nullptr, *d_nn_v = nullptr, *d_nn_scalar = nullptr;

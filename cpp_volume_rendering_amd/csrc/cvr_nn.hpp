@@ -201,10 +201,8 @@ __device__ __forceinline__ bool nn_march(const RayFrame& rf, const VolGeom& g, c
           ood_seen |= ood;
         } else if (on && (ood || nk.exact_all)) {
           ++cnt[2];
-          f3 k, up, right;
-          occ_frame(dir, k, up, right);
-          Io = K.apply_occ ? ct_occlusion<F>(pyr, pg, K, p, k, up, right) : 0.f;
-          Is = K.apply_sdw ? cone_T<F>(pyr, pg, K.ss, K.n_steps, p, L) : 0.f;
+          // (the few samples that come here take 64-bit offsets whatever the level's size)
+          ct_light_at<F, true>(pyr, pg, K, p, dir, L, K.apply_occ != 0, K.apply_sdw != 0, Io, Is);
         }
         Io = fminf(fmaxf(Io, 0.f), 1.f);
         Is = fminf(fmaxf(Is, 0.f), 1.f);

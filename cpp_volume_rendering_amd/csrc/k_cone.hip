@@ -11,8 +11,9 @@
 // the border falloff of GetGaussianExtinction, :92-112).
 //
 // The march is queue_march's (cvr_queue.hpp): 256^3 at 1024^2 177 -> 69 ms, at
-// 512^2 162 -> 18.7 ms, at 128^2 146 -> 1.9 ms.  Per step the level index is wave-uniform, so the level geometry stays in SGPRs;
-// the step schedule is read with scalar loads from a small device table.
+// 512^2 162 -> 18.7 ms, at 128^2 146 -> 1.9 ms; with the steps of cone_T (cvr_cone.hpp) 54.5, 14.4 and
+// 1.3 ms.  A step's level is the same in all lanes, so its constants and the level's geometry come
+// through scalar loads from a small device table.
 #include "cvr_cone.hpp"
 #include "cvr_queue.hpp"
 #include <cmath>
@@ -39,10 +40,8 @@ __global__ __launch_bounds__(256) void k_cone_render(RayFrame rf, VolGeom g, Pyr
   const float spec[3] = {0.f, 0.f, 0.f};
   queue_march<T, 64, false, kParts>(rf, g, s_tf, ntf, step, et, qs.rays, FramePixels(rf, qs, u), spec, kParts > 1 ? queue : queue + (threadIdx.x >> 6), out, nsamp, nshade,
                  [&](bool, f3 p, f3 dir) {
-                   f3 k, up, right;
-                   occ_frame(dir, k, up, right);
-                   const float Io = K.apply_occ ? ct_occlusion<F>(pyr, pg, K, p, k, up, right) : 0.f;
-                   const float Is = K.apply_sdw ? cone_T<F>(pyr, pg, K.ss, K.n_steps, p, L) : 0.f;
+                   float Io, Is;
+                   ct_light<F>(pyr, pg, K, p, dir, L, K.apply_occ != 0, K.apply_sdw != 0, Io, Is);
                    return Lit{inv_k * (Io * ka + Is * kd), 0.f};
                  });
   if (counters) {
@@ -65,8 +64,10 @@ __global__ __launch_bounds__(256) void k_cone_points(PyrGeom pg, const void* __r
   const f3 L = norm3(ld3(lights + 3 * i));
   f3 k, up, right;
   occ_frame(d, k, up, right);
-  if (occ) occ[i] = ct_occlusion<F>(pyr, pg, K, p, k, up, right);
-  if (sdw) sdw[i] = cone_T<F>(pyr, pg, K.ss, K.n_steps, p, L);
+  float Io, Is;
+  ct_light<F>(pyr, pg, K, p, d, L, occ != nullptr, sdw != nullptr, Io, Is);
+  if (occ) occ[i] = Io;
+  if (sdw) sdw[i] = Is;
   if (feat) {
     float f[kNFeat];
     nn_feats<F>(pyr, pg, K.ft, p, k, L, f);
@@ -75,18 +76,29 @@ __global__ __launch_bounds__(256) void k_cone_points(PyrGeom pg, const void* __r
 }
 
 // Host side: schedules in double (geometric distances t0 q^j, q = (tmax/t0)^(1/n);
-// level log2(r / (r_sigma sigma0)) for the cone radius r at the step midpoint).
+// level log2(r / (r_sigma sigma0)) for the cone radius r at the step midpoint).  Fills
+// all of S but its device pointer.
 static void schedule(int n, double t0, double tmax, double half_deg, double r_sigma, double sigma0, int levels,
-                     std::vector<ConeStepF>& out) {
+                     std::vector<ConeStepF>& out, ConeSched& S) {
   out.resize(n);
   const double q = std::pow(tmax / t0, 1.0 / n), th = std::tan(half_deg * 3.14159265358979323846 / 180.0);
+  const double log2e = 1.4426950408889634;
   for (int j = 0; j < n; ++j) {
     const double a = t0 * std::pow(q, double(j)), b = t0 * std::pow(q, double(j + 1));
     const double tm = 0.5 * (a + b);
-    double lod = std::log2(tm * th / (r_sigma * sigma0));
-    lod = std::min(std::max(lod, 0.0), double(levels - 1));
-    out[j] = ConeStepF{float(tm), float(b - a), float(lod), 0.f};
+    double l = std::log2(tm * th / (r_sigma * sigma0));
+    l = std::min(std::max(l, 0.0), double(levels - 1));
+    const float lod = float(l), fr = lod - std::floor(lod);
+    out[j] = ConeStepF{float(tm), float(b - a), 1.f - fr, fr, float(-0.5 * log2e * std::exp2(-2.0 * double(lod))),
+                       int(std::floor(lod)), {0, 0}};
   }
+  S.n = n;
+  S.n0 = 0;
+  while (S.n0 < n && out[S.n0].fr == 0.f) ++S.n0;
+  S.n1 = n;
+  while (S.n1 > S.n0 && out[S.n1 - 1].fr == 0.f) --S.n1;
+  S.log2_t0 = float(std::log2(0.5 * t0 * (1.0 + q)));
+  S.inv_log2_q = float(1.0 / std::log2(q));
 }
 
 // The surrogate's stencil: kNOcc geometric segments over [t0, occ_max], each read on
@@ -184,23 +196,41 @@ int prepare_cone(cvr_ctx* c, const cvr_cone_params& P, hipStream_t st) {
     return -1;
   }
   std::vector<ConeStepF> so, ss;
-  schedule(P.n_steps, P.t0, occ_max, P.occ_half_deg, P.r_sigma, P.sigma0, c->pyr.levels, so);
-  schedule(P.n_steps, P.t0, sdw_max, P.sdw_half_deg, P.r_sigma, P.sigma0, c->pyr.levels, ss);
+  ConeSched& So = c->cone_sched[0];
+  ConeSched& Ss = c->cone_sched[1];
+  schedule(P.n_steps, P.t0, occ_max, P.occ_half_deg, P.r_sigma, P.sigma0, c->pyr.levels, so, So);
+  schedule(P.n_steps, P.t0, sdw_max, P.sdw_half_deg, P.r_sigma, P.sigma0, c->pyr.levels, ss, Ss);
+  std::vector<ConeLevel> lev(kMaxLevels);
+  for (int l = 0; l < c->pyr.levels; ++l) {
+    const PyrGeom& pg = c->pyr;
+    for (int a = 0; a < 3; ++a) {
+      lev[l].ts[a] = pg.ts[l][a];
+      lev[l].dmax[a] = pg.dmax[l][a];
+    }
+    lev[l].nb[0] = pg.nb[l][0];
+    lev[l].nb[1] = pg.nb[l][1];
+    const size_t at = pg.boff[l] * (pg.fmt == 0 ? 32u : 16u);  // records of 32 (fp32) or 16 bytes
+    lev[l].boff_lo = unsigned(at & 0xFFFFFFFFu);
+    lev[l].boff_hi = unsigned(at >> 32);
+  }
   std::vector<StencilF> stn;
   stencil(P, occ_max, sdw_max, c->pyr.levels, stn);
   stn.push_back(StencilF{0.f, 1.f, 0.f, 0.f});  // the local opacity: level 0 at the sample
   std::vector<FeatTap> taps(kNFeat);
   for (int i = 0; i < kNFeat; ++i) taps[i] = feat_tap(c->pyr, stn[i]);
-  // [taps (kNFeat x 64 B)] [occlusion schedule] [shadow schedule]
-  const size_t bytes = kNFeat * sizeof(FeatTap) + (so.size() + ss.size()) * sizeof(ConeStepF);
-  if (!c->d_cone_tab) CVR_HIP_CHECK(hipMalloc(&c->d_cone_tab, kNFeat * sizeof(FeatTap) + 2 * kMaxSteps * sizeof(ConeStepF)));
+  // [taps (kNFeat x 64 B)] [levels] [occlusion schedule] [shadow schedule]
+  const size_t tb = kNFeat * sizeof(FeatTap), lb = kMaxLevels * sizeof(ConeLevel), sb = so.size() * sizeof(ConeStepF);
+  if (!c->d_cone_tab) CVR_HIP_CHECK(hipMalloc(&c->d_cone_tab, tb + lb + 2 * kMaxSteps * sizeof(ConeStepF)));
   else CVR_HIP_CHECK(hipDeviceSynchronize());  // earlier renders may still read the old table
-  std::vector<char> buf(bytes);
-  std::memcpy(buf.data(), taps.data(), kNFeat * sizeof(FeatTap));
-  std::memcpy(buf.data() + kNFeat * sizeof(FeatTap), so.data(), so.size() * sizeof(ConeStepF));
-  std::memcpy(buf.data() + kNFeat * sizeof(FeatTap) + so.size() * sizeof(ConeStepF), ss.data(), ss.size() * sizeof(ConeStepF));
-  CVR_HIP_CHECK(hipMemcpy(c->d_cone_tab, buf.data(), bytes, hipMemcpyHostToDevice));
-  c->cone_n_steps = P.n_steps;
+  std::vector<char> buf(tb + lb + 2 * sb);
+  std::memcpy(buf.data(), taps.data(), tb);
+  std::memcpy(buf.data() + tb, lev.data(), lb);
+  std::memcpy(buf.data() + tb + lb, so.data(), sb);
+  std::memcpy(buf.data() + tb + lb + sb, ss.data(), sb);
+  CVR_HIP_CHECK(hipMemcpy(c->d_cone_tab, buf.data(), buf.size(), hipMemcpyHostToDevice));
+  char* dev = static_cast<char*>(c->d_cone_tab);
+  So.s = reinterpret_cast<const ConeStepF*>(dev + tb + lb);
+  Ss.s = reinterpret_cast<const ConeStepF*>(dev + tb + lb + sb);
   c->cone_tab_for = P;
   c->cone_tab_pyr = c->pyr_key;
   c->cone_tab_valid = true;
@@ -209,7 +239,6 @@ int prepare_cone(cvr_ctx* c, const cvr_cone_params& P, hipStream_t st) {
 
 ConeK cone_constants(const cvr_ctx* c, const cvr_cone_params& P, const float L[3]) {
   ConeK K{};
-  K.n_steps = P.n_steps;
   K.n_occ = P.n_occ_cones;
   K.apply_occ = P.apply_occlusion;
   K.apply_sdw = P.apply_shadow;
@@ -221,8 +250,9 @@ ConeK cone_constants(const cvr_ctx* c, const cvr_cone_params& P, const float L[3
   double l = std::sqrt(double(L[0]) * L[0] + double(L[1]) * L[1] + double(L[2]) * L[2]);
   for (int i = 0; i < 3; ++i) K.L[i] = float(L[i] / l);
   K.ft = static_cast<const FeatTap*>(c->d_cone_tab);
-  K.so = reinterpret_cast<const ConeStepF*>(K.ft + kNFeat);
-  K.ss = K.so + P.n_steps;
+  K.lev = reinterpret_cast<const ConeLevel*>(K.ft + kNFeat);
+  K.so = c->cone_sched[0];
+  K.ss = c->cone_sched[1];
   return K;
 }
 

@@ -564,8 +564,10 @@ __global__ __launch_bounds__(256) void k_nn_samples(VolGeom g, PyrGeom pg, const
   float bo, bs;
   nn_base(f, float(K.n_occ - 1) * K.ring_cos, bo, bs);
   // targets are the residuals of the exact tracer to the network-free estimate
-  Tg[size_t(i) * 2] = ct_occlusion<F>(pyr, pg, K, p, k, up, right) - bo;
-  Tg[size_t(i) * 2 + 1] = cone_T<F>(pyr, pg, K.ss, K.n_steps, p, L) - bs;
+  float Io, Is;
+  ct_light<F>(pyr, pg, K, p, dir, L, true, true, Io, Is);
+  Tg[size_t(i) * 2] = Io - bo;
+  Tg[size_t(i) * 2 + 1] = Is - bs;
   if (pos_out) {
     pos_out[size_t(i) * 6 + 0] = p.x; pos_out[size_t(i) * 6 + 1] = p.y; pos_out[size_t(i) * 6 + 2] = p.z;
     pos_out[size_t(i) * 6 + 3] = dir.x; pos_out[size_t(i) * 6 + 4] = dir.y; pos_out[size_t(i) * 6 + 5] = dir.z;

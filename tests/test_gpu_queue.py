@@ -53,6 +53,19 @@ def test_cone(n, w, h, alpha_max):
     check(img, ref, m)
 
 
+# schedules of one step, of steps of one level only, of two levels from the first on, and remainders of
+# the groups in which steps are loaded
+@pytest.mark.parametrize("n_steps,n_levels,half,occ,sdw", [(1, 1, 30, 1, 1), (2, 6, 30, 1, 0), (3, 2, 80, 1, 1),
+                                                           (5, 6, 5, 0, 1), (64, 3, 30, 1, 1), (7, 6, 89, 1, 1)])
+def test_cone_schedules(n_steps, n_levels, half, occ, sdw):
+    wl, tf, r, p, img = scene(N.CONE_TRACE, 24, 17, 13, 0.6, n_steps=n_steps, n_levels=n_levels, occ_half_deg=half,
+                              apply_occlusion=occ, apply_shadow=sdw)
+    pyr = O.OPyr.build(wl.volume, tf, nlev=n_levels)
+    prm = O.cone_params(wl.grid, wl.light(), n_steps=n_steps, occ_half_deg=half, apply_occ=occ, apply_sdw=sdw)
+    ref, m = O.render_cone(wl.volume, tf, pyr, prm, wl.camera(), 17, 13)
+    check(img, ref, m)
+
+
 @pytest.mark.parametrize("n,w,h,alpha_max", SIZES + MANY)
 def test_dos(n, w, h, alpha_max):
     wl, tf, r, p, img = scene(N.DOS, n, w, h, alpha_max, apply_shadow=1, shadow_type=2, base_res=(24, 24, 24))
