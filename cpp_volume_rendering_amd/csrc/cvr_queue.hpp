@@ -489,9 +489,9 @@ __device__ __forceinline__ void plain_march(const RayFrame& rf, const VolGeom& g
 // The same march with a lane to a ray, for frames whose rays are alike: no samples are taken past a
 // ray's end, and the opacity recurrence needs no other lane.  Samples in groups of four, the next
 // group's blocks in flight under one (two register sets alternate).
-template <typename T, bool kPadded, class Lit1>
+template <typename T, bool kPadded, bool kSpec, class Lit1>
 __device__ __forceinline__ void lane_march(const RayFrame& rf, const VolGeom& g, const float4* tfp, int ntf, float step,
-                                           float et, int px, int py, float4* __restrict__ out, unsigned int& nsamp,
+                                           float et, int px, int py, const float* spec, float4* __restrict__ out, unsigned int& nsamp,
                                            unsigned int& nshade, Lit1&& lit) {
   constexpr int kGroup = 4;
   if (px >= rf.W || py >= rf.H) return;
@@ -508,12 +508,13 @@ __device__ __forceinline__ void lane_march(const RayFrame& rf, const VolGeom& g,
     };
     auto group = [&](const VolTap<T>* t, int j0) {  // true: the ray ends in this group
       float4 src[kGroup];
-      float m[kGroup];
+      Lit l[kGroup];
 #pragma unroll
       for (int k = 0; k < kGroup; ++k) {
         const float d = volume_tap_lerp<T>(t[k]);
         src[k] = kPadded ? sample_tf_padded(tfp, ntf, d) : sample_tf(tfp, ntf, d);
-        m[k] = src[k].w > 0.0f ? lit(ray_sample_pos(ray_sample(j0 + k, step, D), tp, dir)).m : 0.f;
+        l[k] = Lit{1.f, 0.f};
+        if (!kSpec && src[k].w > 0.0f) l[k] = lit(ray_sample_pos(ray_sample(j0 + k, step, D), tp, dir));
       }
 #pragma unroll
       for (int k = 0; k < kGroup; ++k) {
@@ -522,7 +523,14 @@ __device__ __forceinline__ void lane_march(const RayFrame& rf, const VolGeom& g,
         ++nsamp;
         if (src[k].w > 0.0f) {
           ++nshade;
-          const float alpha = 1.0f - __expf(-src[k].w * r.h), w = (1.0f - dst.w) * alpha * m[k];
+          if (kSpec) l[k] = lit(ray_sample_pos(r, tp, dir));
+          const float alpha = 1.0f - __expf(-src[k].w * r.h), w0 = (1.0f - dst.w) * alpha, w = w0 * l[k].m;
+          if (kSpec) {
+            const float ws = w0 * l[k].s;
+            dst.x = __builtin_fmaf(spec[0], ws, dst.x);
+            dst.y = __builtin_fmaf(spec[1], ws, dst.y);
+            dst.z = __builtin_fmaf(spec[2], ws, dst.z);
+          }
           dst.x = __builtin_fmaf(w, src[k].x, dst.x);
           dst.y = __builtin_fmaf(w, src[k].y, dst.y);
           dst.z = __builtin_fmaf(w, src[k].z, dst.z);
@@ -552,36 +560,52 @@ __device__ __forceinline__ void lane_pixel(const RayFrame& rf, int& px, int& py)
   py = ty * 16 + (w >> 1) * 8 + (lane >> 3);
 }
 
-// Whether every ray of the frame starts inside the volume's box.
-inline bool eye_inside(const RayFrame& rf, const VolGeom& g) {
-  for (int i = 0; i < 3; ++i)
-    if (!(std::fabs(rf.eye[i]) < 0.5f * g.G[i])) return false;
+// Whether the whole frame looks at the volume's box: 8 x 8 of its rays, the corners' included, hit it.
+inline bool frame_full(const RayFrame& rf, const VolGeom& g) {
+  for (int i = 0; i < 64; ++i) {
+    const float a = (float(i & 7) / 3.5f - 1.0f) * rf.tanfov * rf.aspect, b = (float(i >> 3) / 3.5f - 1.0f) * rf.tanfov;
+    float lo = 0.f, hi = INFINITY;
+    for (int k = 0; k < 3; ++k) {
+      const float d = rf.s[k] * a + rf.u[k] * b + rf.f[k], h = 0.5f * g.G[k];
+      const float x = (-h - rf.eye[k]) / d, y = (h - rf.eye[k]) / d;
+      lo = std::fmax(lo, std::fmin(x, y));
+      hi = std::fmin(hi, std::fmax(x, y));
+    }
+    if (!(lo < hi)) return false;
+  }
   return true;
 }
 // How the plain and the light-cache frames are marched.
-enum { kGroups = 0, kPhong = 1, kLanes = 2 };
+enum { kGroups = 0, kPhong = 1, kLanes = 2 };  // kLanes + kPhong: both
 struct MarchShape {
   int mode, blocks;
   QueueShape qs;
 };
-// A lane to a ray (kLanes) in frames of kLanePixels and more from inside the volume: all their rays
-// hit it and go about as far (dense
-// volume of 291 x 336 x 306 at 576 x 442 39 us, 53 in groups; 128^3 at 701 x 433 173
-// and 175; but 400 x 327 of 128^3 about 120 and 89, and from outside 128^3 at 512^2 93 and 50).
+// A lane to a ray (kLanes) in frames of kLanePixels and more that look at nothing but the volume, where
+// rays go about as far: no lane is without one, and none takes samples past its end.
+//                                                       in groups   a lane each
+//   dense 291 x 336 x 306 from inside at 576 x 442            53 us        39
+//   128^3 from inside at 701 x 433                           175          173
+//   dense 150 x 100 x 120 from its face at 800 x 700         100           72
+//   51 x 31 x 47, Blinn-Phong, at 2000 x 1198               1250          960
+//   128^3 from inside at 400 x 327 (fewer pixels)             89          120
+//   dense 200^3 at 800 x 700, a third of it empty            113          123
+//   128^3 at 512^2, a fifth of it covered                     50           93
 constexpr size_t kLanePixels = 1 << 17;
 inline MarchShape march_shape(const RayFrame& rf, const VolGeom& g, bool phong) {
   MarchShape m;
   m.qs = queue_shape(rf, kListRays, 4, 512);
   m.blocks = m.qs.blocks;
   m.mode = phong ? kPhong : kGroups;
-  if (!phong && size_t(rf.W) * rf.H >= kLanePixels && eye_inside(rf, g)) {
-    m.mode = kLanes;
+  if (size_t(rf.W) * rf.H >= kLanePixels && frame_full(rf, g)) {
+    m.mode += kLanes;
     m.blocks = ((rf.W + 15) / 16) * ((rf.H + 15) / 16);
   }
   return m;
 }
 template <class F> inline void with_mode(int mode, F&& f) {
   if (mode == kLanes) f(std::integral_constant<int, kLanes>{});
+  else if (mode == kLanes + kPhong) f(std::integral_constant<int, kLanes + kPhong>{});
   else if (mode == kPhong) f(std::integral_constant<int, kPhong>{});
   else f(std::integral_constant<int, kGroups>{});
 }

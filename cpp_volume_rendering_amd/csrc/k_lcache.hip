@@ -50,7 +50,7 @@ struct LcK {
   float ks;          // Phong specular weight, 0 without shadows (Kspecular counts with ApplyShadow)
 };
 
-// kMode: kGroups, kPhong (with Blinn-Phong) or kLanes.
+// kMode: kGroups or kLanes, + kPhong (with Blinn-Phong).
 template <typename T, int kMode>
 __global__ __launch_bounds__(256) void k_lc_render(RayFrame rf, VolGeom g, LcK L, const float2* __restrict__ lc,
                                                    const float4* __restrict__ tf, int ntf, float step, float et,
@@ -65,17 +65,17 @@ __global__ __launch_bounds__(256) void k_lc_render(RayFrame rf, VolGeom g, LcK L
   const f3 eye = ld3(rf.eye);
   auto lit = [&](f3 p) {
     const float2 I = lc_sample(lc, L.rx, L.ry, L.rz, L.tex_mul, p);
-    if (kMode != kPhong) return Lit{inv_k * (I.x * L.ka + I.y * L.kd), 0.f};
+    if (!(kMode & kPhong)) return Lit{inv_k * (I.x * L.ka + I.y * L.kd), 0.f};
     float dd, sp;
     if (!phong_terms(grad, g, ph, p, eye, dd, sp)) return Lit{1.f, 0.f};
     return Lit{inv_k * (I.x * L.ka + I.y * (L.kd * dd)), I.y * (L.ks * sp)};
   };
-  if constexpr (kMode == kLanes) {
+  if constexpr ((kMode & kLanes) != 0) {
     int px, py;
     lane_pixel(rf, px, py);
-    lane_march<T, true>(rf, g, s_tf, ntf, step, et, px, py, out, nsamp, nshade, lit);
+    lane_march<T, true, (kMode & kPhong) != 0>(rf, g, s_tf, ntf, step, et, px, py, ph.spec, out, nsamp, nshade, lit);
   } else {
-    plain_march<T, true, kMode == kPhong>(rf, g, s_tf, ntf, step, et, FramePixels(rf, qs, queue_unit<4>(qs.xcd_log2), 4),
+    plain_march<T, true, (kMode & kPhong) != 0>(rf, g, s_tf, ntf, step, et, FramePixels(rf, qs, queue_unit<4>(qs.xcd_log2), 4),
                                           ph.spec, list, out, nsamp, nshade, lit);
   }
   if (counters) {

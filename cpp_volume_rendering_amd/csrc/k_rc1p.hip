@@ -17,7 +17,8 @@
 // arithmetic of a step (about 140 instructions for 64 samples).  64^3 at 128^2 51 -> 16 us,
 // 128^3 at 512^2 95 -> 50, 400 x 380 x 390 at 1000 x 900 415 -> 203; with Blinn-Phong 161 x 193 x 97
 // at 1002 x 746 307 -> 168 (shaded where it is met: through the queue of the costlier renderers
-// 243).  Large frames from inside the volume keep a lane per ray (march_shape).  The 1D transfer
+// 243).  Large frames that look at nothing but the volume keep a lane per ray
+// (march_shape).  The 1D transfer
 // function is staged in LDS.
 #include "cvr_ctx.hpp"
 #include "cvr_queue.hpp"
@@ -27,7 +28,7 @@ namespace cvr {
 
 template <class T> struct VoxTag { typedef T type; };
 
-// kMode: kGroups, kPhong (with Blinn-Phong) or kLanes.
+// kMode: kGroups or kLanes, + kPhong (with Blinn-Phong).
 template <typename T, bool TF_LDS, int kMode>
 __global__ __launch_bounds__(256) void k_rc1p(RayFrame rf, VolGeom g, const float4* __restrict__ tf, int ntf,
                                                float step, float et, PhongK ph, const float4* __restrict__ grad,
@@ -44,15 +45,15 @@ __global__ __launch_bounds__(256) void k_rc1p(RayFrame rf, VolGeom g, const floa
   const f3 eye = ld3(rf.eye);
   auto lit = [&](f3 p) {
     float dd, sp;
-    if (kMode != kPhong || !phong_terms(grad, g, ph, p, eye, dd, sp)) return Lit{1.f, 0.f};
+    if (!(kMode & kPhong) || !phong_terms(grad, g, ph, p, eye, dd, sp)) return Lit{1.f, 0.f};
     return Lit{ka + kd * dd, ph.ks * sp};
   };
-  if constexpr (kMode == kLanes) {
+  if constexpr ((kMode & kLanes) != 0) {
     int px, py;
     lane_pixel(rf, px, py);
-    lane_march<T, TF_LDS>(rf, g, tfp, ntf, step, et, px, py, out, nsamp, nshade, lit);
+    lane_march<T, TF_LDS, (kMode & kPhong) != 0>(rf, g, tfp, ntf, step, et, px, py, ph.spec, out, nsamp, nshade, lit);
   } else {
-    plain_march<T, TF_LDS, kMode == kPhong>(rf, g, tfp, ntf, step, et, FramePixels(rf, qs, queue_unit<4>(qs.xcd_log2), 4),
+    plain_march<T, TF_LDS, (kMode & kPhong) != 0>(rf, g, tfp, ntf, step, et, FramePixels(rf, qs, queue_unit<4>(qs.xcd_log2), 4),
                                             ph.spec, list, out, nsamp, nshade, lit);
   }
   if (counters) {

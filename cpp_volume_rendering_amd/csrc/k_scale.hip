@@ -102,8 +102,9 @@ __global__ __launch_bounds__(256) void k_downscale(const float4* __restrict__ sr
   const int ir_r = int(floorf((x_r + kr / float(dh)) * float(sh) - 0.5f));
   const int il_c = int(ceilf((x_c - kr / float(dw)) * float(sw) - 0.5f));
   const int ir_c = int(floorf((x_c + kr / float(dw)) * float(sw) - 0.5f));
-  for (int t = ty; t < kTaps; t += 16) wts[1][t][tx] = down_weight(kern, x_c, il_c + t, sw, dw);
-  for (int t = tx; t < kTaps; t += 16) wts[0][t][ty] = down_weight(kern, x_r, il_r + t, sh, dh);
+  const int taps = min(kTaps, int(2.f * kr * fmaxf(float(sw) / float(dw), float(sh) / float(dh))) + 2);  // of a set, at most
+  for (int t = ty; t < taps; t += 16) wts[1][t][tx] = down_weight(kern, x_c, il_c + t, sw, dw);
+  for (int t = tx; t < taps; t += 16) wts[0][t][ty] = down_weight(kern, x_r, il_r + t, sh, dh);
   __syncthreads();
   if (jc >= dw || jr >= dh) return;
   float4 f = make_float4(0.f, 0.f, 0.f, 0.f);

@@ -170,10 +170,17 @@ def test_light_cache(n, w, h, alpha_max, phong):
     check(img, ref, m)
 
 
+INSIDE = ((2.0, -1.0, 3.0), (0.0, 0.0, -40.0))
+
+
+@pytest.mark.parametrize("phong", [0, 1])
 @pytest.mark.parametrize("entries,bits", [(256, 8), (5000, 16)])
-@pytest.mark.parametrize("w,h", [(363, 362), (1024, 128), (400, 327)])
-def test_plain_from_inside(w, h, entries, bits):
-    """A lane to a ray from 2^17 pixels on: one more, just as many, and fewer."""
+@pytest.mark.parametrize("w,h,eye,to", [(363, 362, *INSIDE), (1024, 128, *INSIDE), (400, 327, *INSIDE),
+                                        (400, 330, (0.0, 0.0, 16.0), (0.0, 0.0, 0.0)),
+                                        (400, 330, (0.0, 0.0, 26.0), (0.0, 0.0, 0.0))])
+def test_plain_of_full_frames(w, h, eye, to, entries, bits, phong):
+    """A lane to a ray from 2^17 pixels on in frames that the volume fills: one pixel more, just as
+    many, and fewer; from inside, from before a face, and from where the corners miss it."""
     wl = W.cone_blobs(n=24, width=w, height=h, seed=31)
     vol = wl.volume if bits == 8 else (wl.volume.astype(np.uint16) * 257)
     rgb, a = W.seeded_tf(131, 4, alpha_max=0.5)
@@ -182,25 +189,39 @@ def test_plain_from_inside(w, h, entries, bits):
     r = N.Renderer(N.RC1P)
     r.set_volume(vol, wl.scale)
     r.set_transfer_function(rgb, a, max_density=entries - 1)
+    p = r.params()
+    p.apply_gradient_shading, p.shininess = phong, 20.0
+    r.set_params(p)
     r.collect_stats()
-    cam = N.Camera((2.0, -1.0, 3.0), (0.0, 0.0, -40.0), (0.0, 1.0, 0.0), 60.0, w / h)
-    img = r.render(cam, w, h)
-    ref, m = O.render_rc1p(vol, O.OTF(rgb, a, max_density=entries - 1), cam, w, h)
+    cam, light = N.Camera(eye, to, (0.0, 1.0, 0.0), 60.0, w / h), wl.light()
+    img = r.render(cam, w, h, light=light)
+    tf = O.OTF(rgb, a, max_density=entries - 1)
+    if phong:
+        ph = O.phong(p.gradient_type, light, ka=p.ka, kd=p.kd, ks=p.ks, shininess=p.shininess)
+        ref, m = O.render_rc1p_phong(vol, tf, ph, cam, w, h)
+    else:
+        ref, m = O.render_rc1p(vol, tf, cam, w, h)
     check(img, ref, m)
 
 
-def test_light_cache_from_inside():
+@pytest.mark.parametrize("phong", [0, 1])
+def test_light_cache_of_a_full_frame(phong):
     w, h = 363, 362
     wl = W.cone_blobs(n=24, width=w, height=h, seed=31)
     rgb, a = W.seeded_tf(131, 4, alpha_max=0.5)
     r = N.Renderer(N.EBS)
     r.set_volume(wl.volume, wl.scale)
     r.set_transfer_function(rgb, a)
-    r.set_params(light_cache=1)
+    r.set_params(light_cache=1, apply_phong=phong)
     p = r.params()
-    cam = N.Camera((2.0, -1.0, 3.0), (0.0, 0.0, -40.0), (0.0, 1.0, 0.0), 60.0, w / h)
-    img = r.render(cam, w, h, light=wl.light())
-    ref, m = O.render_lc(wl.volume, O.OTF(rgb, a), r.light_cache(), 1, 1, p.ka, p.kd, cam, w, h, scale=wl.scale)
+    cam, light = N.Camera(*INSIDE, (0.0, 1.0, 0.0), 60.0, w / h), wl.light()
+    img = r.render(cam, w, h, light=light)
+    tf, g = O.OTF(rgb, a), r.light_cache()
+    if phong:
+        ph = O.phong(p.gradient_type, light, ka=p.ka, kd=p.kd, ks=p.ks, shininess=p.shininess)
+        ref, m = O.render_lc_phong(wl.volume, tf, g, 1, 1, p.ka, p.kd, ph, cam, w, h, scale=wl.scale)
+    else:
+        ref, m = O.render_lc(wl.volume, tf, g, 1, 1, p.ka, p.kd, cam, w, h, scale=wl.scale)
     check(img, ref, m)
 
 
