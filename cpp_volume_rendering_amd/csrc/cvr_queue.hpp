@@ -560,8 +560,9 @@ __device__ __forceinline__ void lane_pixel(const RayFrame& rf, int& px, int& py)
   py = ty * 16 + (w >> 1) * 8 + (lane >> 3);
 }
 
-// Whether the whole frame looks at the volume's box: 8 x 8 of its rays, the corners' included, hit it.
-inline bool frame_full(const RayFrame& rf, const VolGeom& g) {
+// How many of 8 x 8 rays of the frame, the corners' included, hit the volume's box.
+inline int frame_hits(const RayFrame& rf, const VolGeom& g) {
+  int n = 0;
   for (int i = 0; i < 64; ++i) {
     const float a = (float(i & 7) / 3.5f - 1.0f) * rf.tanfov * rf.aspect, b = (float(i >> 3) / 3.5f - 1.0f) * rf.tanfov;
     float lo = 0.f, hi = INFINITY;
@@ -571,9 +572,9 @@ inline bool frame_full(const RayFrame& rf, const VolGeom& g) {
       lo = std::fmax(lo, std::fmin(x, y));
       hi = std::fmin(hi, std::fmax(x, y));
     }
-    if (!(lo < hi)) return false;
+    n += lo < hi;
   }
-  return true;
+  return n;
 }
 // How the plain and the light-cache frames are marched.
 enum { kGroups = 0, kPhong = 1, kLanes = 2 };  // kLanes + kPhong: both
@@ -581,23 +582,42 @@ struct MarchShape {
   int mode, blocks;
   QueueShape qs;
 };
-// A lane to a ray (kLanes) in frames of kLanePixels and more that look at nothing but the volume, where
-// rays go about as far: no lane is without one, and none takes samples past its end.
-//                                                       in groups   a lane each
-//   dense 291 x 336 x 306 from inside at 576 x 442            53 us        39
-//   128^3 from inside at 701 x 433                           175          173
-//   dense 150 x 100 x 120 from its face at 800 x 700         100           72
-//   51 x 31 x 47, Blinn-Phong, at 2000 x 1198               1250          960
-//   128^3 from inside at 400 x 327 (fewer pixels)             89          120
-//   dense 200^3 at 800 x 700, a third of it empty            113          123
-//   128^3 at 512^2, a fifth of it covered                     50           93
+// A lane to a ray (kLanes) takes no sample past a ray's end and needs no sum over lanes, but a frame
+// takes as long as its longest rays and the lanes beside them wait: it is for frames with many rays for
+// the samples of the longest, and for large ones that look at nothing but the volume.  Pixels that hit
+// the box over samples along its diagonal, plain march:     in groups   a lane each
+//   30^3 at 1100 x 1000                           1320           63 us        48
+//   64^3 at 1100 x 1000                            620           83           84
+//   100^3 at 1600 x 1300                           560          167          133
+//   40^3 at 800 x 700                              500           42           38
+//   100^3 at 1100 x 1000                           400          103          118
+//   64^3 at 700 x 600                              210           44           53
+//   400 x 380 x 390 at 1000 x 900                   80          203          415
+//   64^3 at 700 x 600, from near                  1390          129          120
+//   40^3 at 400 x 330, from near                   700           41           44
+//   dense 200^3 at 800 x 700, from near            590          113          123
+//   dense 291 x 336 x 306 from inside, 576 x 442   240           53           39
+//   128^3 from inside at 701 x 433                 690          175          173
+//   128^3 from inside at 400 x 327                 300           89          120
+// light cache (cache and march):
+//   100^3 at 1100 x 1000, from near               2430          948          913
+//   64^3 at 1100 x 1000                            620          238          277
+// Blinn-Phong, from near:
+//   43 x 27 x 35 at 2241 x 1296                  10800         1012          730
+//   64^3 at 1100 x 1000                           3800          645          613
+//   100^3 at 1100 x 1000                          2430          882          913
+//   64^3 at 700 x 600                             1390          260          358
+constexpr float kLaneRays = 500.f, kLaneCacheRays = 2000.f, kLanePhongRays = 3500.f;
 constexpr size_t kLanePixels = 1 << 17;
-inline MarchShape march_shape(const RayFrame& rf, const VolGeom& g, bool phong) {
+inline MarchShape march_shape(const RayFrame& rf, const VolGeom& g, float step, bool phong, float lane_rays) {
   MarchShape m;
   m.qs = queue_shape(rf, kListRays, 4, 512);
   m.blocks = m.qs.blocks;
   m.mode = phong ? kPhong : kGroups;
-  if (size_t(rf.W) * rf.H >= kLanePixels && frame_full(rf, g)) {
+  const size_t px = size_t(rf.W) * rf.H;
+  const int hits = frame_hits(rf, g);
+  const float steps = std::sqrt(g.G[0] * g.G[0] + g.G[1] * g.G[1] + g.G[2] * g.G[2]) / step;
+  if ((hits == 64 && px >= kLanePixels) || float(px) * float(hits) / 64.f >= steps * (phong ? kLanePhongRays : lane_rays)) {
     m.mode += kLanes;
     m.blocks = ((rf.W + 15) / 16) * ((rf.H + 15) / 16);
   }

@@ -17,8 +17,7 @@
 // arithmetic of a step (about 140 instructions for 64 samples).  64^3 at 128^2 51 -> 16 us,
 // 128^3 at 512^2 95 -> 50, 400 x 380 x 390 at 1000 x 900 415 -> 203; with Blinn-Phong 161 x 193 x 97
 // at 1002 x 746 307 -> 168 (shaded where it is met: through the queue of the costlier renderers
-// 243).  Large frames that look at nothing but the volume keep a lane per ray
-// (march_shape).  The 1D transfer
+// 243).  Frames of many short rays keep a lane per ray (march_shape).  The 1D transfer
 // function is staged in LDS.
 #include "cvr_ctx.hpp"
 #include "cvr_queue.hpp"
@@ -94,7 +93,7 @@ int launch_rc1p(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* o
   const float4* gr = ph.on ? c->d_grad : nullptr;
   bool lds = c->tf_size <= 4096;
   size_t shm = lds ? size_t(c->tf_size + 2) * sizeof(float4) : 0;
-  const MarchShape ms = march_shape(rf, g, ph.on);
+  const MarchShape ms = march_shape(rf, g, step, ph.on, kLaneRays);
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   float4* o4 = reinterpret_cast<float4*>(out);
   auto launch = [&](auto t, auto l, auto m) {

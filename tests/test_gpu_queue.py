@@ -177,10 +177,11 @@ INSIDE = ((2.0, -1.0, 3.0), (0.0, 0.0, -40.0))
 @pytest.mark.parametrize("entries,bits", [(256, 8), (5000, 16)])
 @pytest.mark.parametrize("w,h,eye,to", [(363, 362, *INSIDE), (1024, 128, *INSIDE), (400, 327, *INSIDE),
                                         (400, 330, (0.0, 0.0, 16.0), (0.0, 0.0, 0.0)),
-                                        (400, 330, (0.0, 0.0, 26.0), (0.0, 0.0, 0.0))])
+                                        (400, 330, (0.0, 0.0, 26.0), (0.0, 0.0, 0.0)), (900, 601, (20.0, 9.0, 60.0), (0.0, 0.0, 0.0))])
 def test_plain_of_full_frames(w, h, eye, to, entries, bits, phong):
     """A lane to a ray from 2^17 pixels on in frames that the volume fills: one pixel more, just as
-    many, and fewer; from inside, from before a face, and from where the corners miss it."""
+    many, and fewer; from inside, from before a face, and from where the corners miss it; and in
+    frames of many pixels for the volume's size."""
     wl = W.cone_blobs(n=24, width=w, height=h, seed=31)
     vol = wl.volume if bits == 8 else (wl.volume.astype(np.uint16) * 257)
     rgb, a = W.seeded_tf(131, 4, alpha_max=0.5)
