@@ -81,29 +81,39 @@ __device__ __forceinline__ unsigned int to16(float x, int fmt) {
   return u >> 16;
 }
 
-// Corner blocks of one pyramid level: cell (x, y, z) holds the 2 x 2 x 2 values at
+// Corner blocks of every pyramid level: cell (x, y, z) holds the 2 x 2 x 2 values at
 // (x..x+1, y..y+1, z..z+1), the +1 neighbours clamped to the edge, plane z first, each
-// plane (x, y), (x+1, y), (x, y+1), (x+1, y+1); fp32 as 32 bytes, fp16 / bf16 as 16.
+// plane (x, y), (x+1, y), (x, y+1), (x+1, y+1); fp32 as 32 bytes, fp16 / bf16 as 16.  One launch:
+// workgroup blockIdx.x takes 256 cells, in order, of the first level whose `end` lies past it.
+struct OctEnds {
+  unsigned int end[kMaxLevels];
+};
 template <int FMT>
-__global__ __launch_bounds__(256) void k_make_oct(const float* __restrict__ src, void* __restrict__ dst, int nx, int ny,
-                                                  int nz) {
-  const int x = blockIdx.x * 64 + (threadIdx.x & 63);
-  const int y = blockIdx.y * 4 + (threadIdx.x >> 6);
-  const int z = blockIdx.z;
+__global__ __launch_bounds__(256) void k_make_oct(PyrGeom pg, OctEnds e, const float* __restrict__ pyr,
+                                                  void* __restrict__ blocks) {
+  int l = 0;
+  while (l + 1 < pg.levels && blockIdx.x >= e.end[l]) ++l;
+  const int nx = pg.dims[l][0], ny = pg.dims[l][1], nz = pg.dims[l][2];
+  const unsigned int rows = (unsigned(nx) + 63u) / 64u, per = (unsigned(ny) + 3u) / 4u;
+  unsigned int b = blockIdx.x - (l ? e.end[l - 1] : 0u);
+  const int x = int(b % rows) * 64 + (threadIdx.x & 63);
+  b /= rows;
+  const int y = int(b % per) * 4 + (threadIdx.x >> 6), z = int(b / per);
   if (x >= nx || y >= ny || z >= nz) return;
+  const float* src = pyr + pg.off[l];
   const int x1 = min(x + 1, nx - 1), y1 = min(y + 1, ny - 1), z1 = min(z + 1, nz - 1);
   const size_t sy = size_t(nx), sz = size_t(nx) * ny;
   const size_t r00 = z * sz + y * sy, r01 = z * sz + y1 * sy, r10 = z1 * sz + y * sy, r11 = z1 * sz + y1 * sy;
   const float v[8] = {src[r00 + x], src[r00 + x1], src[r01 + x], src[r01 + x1],
                       src[r10 + x], src[r10 + x1], src[r11 + x], src[r11 + x1]};
-  const size_t i = brick_index(x, y, z, bricks(nx), bricks(ny));
+  const size_t i = pg.boff[l] + brick_index(x, y, z, bricks(nx), bricks(ny));
   if (FMT == 0) {
-    float4* d = static_cast<float4*>(dst) + 2 * i;
+    float4* d = static_cast<float4*>(blocks) + 2 * i;
     d[0] = make_float4(v[0], v[1], v[2], v[3]);
     d[1] = make_float4(v[4], v[5], v[6], v[7]);
   } else {
-    static_cast<uint4*>(dst)[i] = make_uint4(to16(v[0], FMT) | (to16(v[1], FMT) << 16), to16(v[2], FMT) | (to16(v[3], FMT) << 16),
-                                             to16(v[4], FMT) | (to16(v[5], FMT) << 16), to16(v[6], FMT) | (to16(v[7], FMT) << 16));
+    static_cast<uint4*>(blocks)[i] = make_uint4(to16(v[0], FMT) | (to16(v[1], FMT) << 16), to16(v[2], FMT) | (to16(v[3], FMT) << 16),
+                                                to16(v[4], FMT) | (to16(v[5], FMT) << 16), to16(v[6], FMT) | (to16(v[7], FMT) << 16));
   }
 }
 
@@ -121,17 +131,19 @@ int build_pyramid_oct(cvr_ctx* c, size_t total, int fmt, hipStream_t st) {
   if (rc == CVR_ERR_NOMEM) set_error("pyramid: out of device memory (corner blocks)");
   if (rc != CVR_OK) return rc;
   const PyrGeom& pg = c->pyr;
+  OctEnds e{};
+  size_t blocks = 0;
   for (int l = 0; l < pg.levels; ++l) {
-    const int nx = pg.dims[l][0], ny = pg.dims[l][1], nz = pg.dims[l][2];
-    if (nz > 65535) { set_error("corner blocks: depth above 65535"); return CVR_ERR_INVALID; }
-    const dim3 grid(unsigned((nx + 63) / 64), unsigned((ny + 3) / 4), unsigned(nz));
-    void* d = static_cast<char*>(c->d_pyr_oct) + pg.boff[l] * rec;
-    const float* s = c->d_pyr + pg.off[l];
-    if (fmt == 0) hipLaunchKernelGGL(k_make_oct<0>, grid, dim3(256), 0, st, s, d, nx, ny, nz);
-    else if (fmt == 1) hipLaunchKernelGGL(k_make_oct<1>, grid, dim3(256), 0, st, s, d, nx, ny, nz);
-    else hipLaunchKernelGGL(k_make_oct<2>, grid, dim3(256), 0, st, s, d, nx, ny, nz);
-    CVR_HIP_CHECK(hipGetLastError());
+    if (pg.dims[l][2] > 65535) { set_error("corner blocks: depth above 65535"); return CVR_ERR_INVALID; }
+    blocks += size_t((pg.dims[l][0] + 63) / 64) * size_t((pg.dims[l][1] + 3) / 4) * size_t(pg.dims[l][2]);
+    if (blocks >> 31) { set_error("corner blocks: pyramid too large"); return CVR_ERR_INVALID; }
+    e.end[l] = unsigned(blocks);
   }
+  const dim3 grid{unsigned(blocks)};
+  if (fmt == 0) hipLaunchKernelGGL(k_make_oct<0>, grid, dim3(256), 0, st, pg, e, c->d_pyr, c->d_pyr_oct);
+  else if (fmt == 1) hipLaunchKernelGGL(k_make_oct<1>, grid, dim3(256), 0, st, pg, e, c->d_pyr, c->d_pyr_oct);
+  else hipLaunchKernelGGL(k_make_oct<2>, grid, dim3(256), 0, st, pg, e, c->d_pyr, c->d_pyr_oct);
+  CVR_HIP_CHECK(hipGetLastError());
   CVR_HIP_CHECK(hipStreamSynchronize(st));
   return CVR_OK;
 }

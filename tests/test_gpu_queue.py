@@ -302,3 +302,31 @@ def test_summed_area_table_of_each_extinction_table(bits, entries, ext):
     got = r.get_sat(vol.shape[::-1])
     ref = O.sat(vol, O.OTF(rgb, a, max_density=entries - 1, extinction_input=bool(ext)))
     assert np.abs(got - ref).max() <= 1e-6 * ref.max()
+
+
+# levels of at most 4096 voxels go to one workgroup: all but the first, from a level just under and just
+# over that size, none; flat and long grids; the direct and the separable build of level 0; a
+# transfer function too large for LDS.  The tolerance is that of the pyramid's own tests.
+@pytest.mark.parametrize("base,sigma0,entries,bits", [((17, 16, 15), 1.0, 256, 8), ((17, 16, 16), 1.0, 256, 16),
+                                                      ((32, 32, 32), 1.0, 256, 8), ((1, 1, 1), 1.0, 256, 8),
+                                                      ((70, 5, 1), 0.7, 256, 16), ((40, 33, 9), 1.3, 9000, 16),
+                                                      ((64, 64, 64), 1.0, 9000, 16), ((48, 40, 36), 0.7, 9000, 8)])
+def test_pyramid_shapes(base, sigma0, entries, bits):
+    wl = W.plain_blobs(n=32, width=8, height=8, seed=14)
+    vol = wl.volume if bits == 8 else (wl.volume.astype(np.uint16) * 257)
+    rgb, a = wl.rgb_iso.copy(), wl.alpha_iso.copy()
+    rgb[:, 3] = np.round(rgb[:, 3] * (entries - 1) / 255)
+    a[:, 1] = np.round(a[:, 1] * (entries - 1) / 255)
+    r = N.Renderer(N.CONE_TRACE)
+    r.set_volume(vol)
+    r.set_transfer_function(rgb, a, max_density=entries - 1)
+    p = r.params()
+    p.base_res[:] = list(base)
+    p.sigma0, p.n_levels = sigma0, 0
+    r.set_params(p)
+    g = r.pyramid()
+    ref = O.OPyr.build(vol, O.OTF(rgb, a, max_density=entries - 1), base=base, sigma0=sigma0)
+    assert len(g) == ref.levels
+    for l in range(ref.levels):
+        t = ref.level(l)
+        assert g[l].shape == t.shape and (np.abs(g[l] - t) / np.maximum(1.0, np.abs(t))).max() <= 1e-4, l
