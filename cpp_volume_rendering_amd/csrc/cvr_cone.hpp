@@ -4,6 +4,7 @@
 #include "cvr_ctx.hpp"
 #include <hip/hip_fp16.h>
 #include <type_traits>
+#include <vector>
 
 namespace cvr {
 
@@ -109,32 +110,6 @@ __device__ __forceinline__ float pyr_lerp(typename PyrOct<F>::type r, float fx, 
   }
 }
 
-// GL_LINEAR lookup of pyramid level `l` at texture-space point tp: the texel coordinate
-// tp * dims / G - 1/2 is one fma per axis, the read one corner block.
-template <int F>
-__device__ __forceinline__ float pyr_tri(const void* __restrict__ pyr, const PyrGeom& pg, int l, f3 tp) {
-  int x0, y0, z0;
-  float fx, fy, fz;
-  quad_axis_f(fmaf(tp.x, pg.ts[l][0], -0.5f), pg.dmax[l][0], x0, fx);
-  quad_axis_f(fmaf(tp.y, pg.ts[l][1], -0.5f), pg.dmax[l][1], y0, fy);
-  quad_axis_f(fmaf(tp.z, pg.ts[l][2], -0.5f), pg.dmax[l][2], z0, fz);
-  typedef typename PyrOct<F>::type B;
-  return pyr_lerp<F>(static_cast<const B*>(pyr)[pg.boff[l] + brick_index(x0, y0, z0, pg.nb[l][0], pg.nb[l][1])], fx, fy,
-                     fz, pg.one);
-}
-
-// Border falloff of GetGaussianExtinction (rc1pdosct/ray_bbox_marching.comp:96-109):
-// exp(-|clamp(p, 0, G) - p|^2 / (2 (2^lod)^2)); the distance is 0 inside the box, so the
-// factor is exactly 1 there and no branch is needed (the loads of many lookups can then
-// be issued back to back).  inv2sg2 = 1 / (2 (2^lod)^2).
-__device__ __forceinline__ float border_falloff(const PyrGeom& pg, f3 tp, float inv2sg2) {
-  // clamp(p, 0, G) as one median-of-three (p is finite, G > 0)
-  const float cx = __builtin_amdgcn_fmed3f(tp.x, 0.f, pg.G[0]) - tp.x;
-  const float cy = __builtin_amdgcn_fmed3f(tp.y, 0.f, pg.G[1]) - tp.y;
-  const float cz = __builtin_amdgcn_fmed3f(tp.z, 0.f, pg.G[2]) - tp.z;
-  return __expf(-(cx * cx + cy * cy + cz * cz) * inv2sg2);
-}
-
 // Byte offset of corner block (x0, y0, z0) in a level of `nbx` x `nby` bricks, records of
 // 2^kShift bytes: brick number, then the 6 bits of in-brick position (brick_index).  The
 // 32-bit form needs the level's records to span less than 4 GiB (PyrGeom::wide = 0); its
@@ -154,6 +129,42 @@ __device__ __forceinline__ float wave_min(float v) {
   return m;
 }
 
+typedef const __attribute__((address_space(4))) ConeLevel* ConstLevels;
+// GL_LINEAR lookup of level g (the same for all lanes: its geometry comes through scalar loads) at
+// texture-space point tp: the texel coordinate is one fma per axis, the read one corner block.
+template <int F, bool kWide>
+__device__ __forceinline__ float level_read(const void* __restrict__ pyr, ConstLevels g, f3 tp, float one) {
+  typedef typename PyrOct<F>::type B;
+  constexpr int kShift = sizeof(B) == 32 ? 5 : 4;
+  int x0, y0, z0;
+  float fx, fy, fz;
+  quad_axis_f(fmaf(tp.x, g->ts[0], -0.5f), g->dmax[0], x0, fx);
+  quad_axis_f(fmaf(tp.y, g->ts[1], -0.5f), g->dmax[1], y0, fy);
+  quad_axis_f(fmaf(tp.z, g->ts[2], -0.5f), g->dmax[2], z0, fz);
+  const char* lv = static_cast<const char*>(pyr) + ((size_t(g->boff_hi) << 32) | g->boff_lo);
+  if constexpr (kWide)
+    return pyr_lerp<F>(*reinterpret_cast<const B*>(lv + (brick_index(x0, y0, z0, g->nb[0], g->nb[1]) << kShift)), fx, fy, fz, one);
+  else
+    return pyr_lerp<F>(*reinterpret_cast<const B*>(lv + oct_offset32<kShift>(x0, y0, z0, g->nb[0], g->nb[1])), fx, fy, fz, one);
+}
+// Border falloff of GetGaussianExtinction (rc1pdosct/ray_bbox_marching.comp:96-109):
+// exp(-|clamp(p, 0, G) - p|^2 / (2 (2^lod)^2)), `fall` = -log2(e) / (2 (2^lod)^2); the distance is 0
+// inside the box, so the factor is exactly 1 there.
+__device__ __forceinline__ float border_falloff(const PyrGeom& pg, f3 tp, float fall) {
+  // clamp(p, 0, G) as one median-of-three (p is finite, G > 0)
+  const float cx = __builtin_amdgcn_fmed3f(tp.x, 0.f, pg.G[0]) - tp.x;
+  const float cy = __builtin_amdgcn_fmed3f(tp.y, 0.f, pg.G[1]) - tp.y;
+  const float cz = __builtin_amdgcn_fmed3f(tp.z, 0.f, pg.G[2]) - tp.z;
+  return __builtin_amdgcn_exp2f((cx * cx + cy * cy + cz * cz) * fall);
+}
+// The distance along `axis` up to which p + axis t of every active lane is inside the box.
+__device__ __forceinline__ float wave_exit(const PyrGeom& pg, f3 p, f3 axis) {
+  auto leave = [&](float a, float q, float G) { return ((a > 0.f ? G : 0.f) - q) / a; };
+  return wave_min(fminf(leave(axis.x, p.x, pg.G[0]), fminf(leave(axis.y, p.y, pg.G[1]), leave(axis.z, p.z, pg.G[2]))));
+}
+// The levels of a pyramid as the marches read them (kMaxLevels rows).
+std::vector<ConeLevel> cone_levels(const PyrGeom& pg);
+
 // Transmittance of a cone of 64 steps and one or two trilinear reads each, the bulk of a
 // cone-traced frame.  Bound by vector instructions and the L1's tag rate (four 16-byte loads of a
 // step's two 32-byte blocks), so whatever is the same for all lanes is in the tables (scalar loads),
@@ -164,43 +175,22 @@ __device__ __forceinline__ float wave_min(float v) {
 template <int F, bool kWide>
 __device__ __forceinline__ float cone_T(const void* __restrict__ pyr, const PyrGeom& pg,
                                         const ConeLevel* __restrict__ levels, const ConeSched& S, f3 p, f3 axis) {
-  typedef typename PyrOct<F>::type B;
   typedef const __attribute__((address_space(4))) ConeStepF* ConstSteps;
-  typedef const __attribute__((address_space(4))) ConeLevel* ConstLevels;
   const ConstSteps s = (ConstSteps)(uintptr_t)S.s;
   const ConstLevels lev = (ConstLevels)(uintptr_t)levels;
-  constexpr int kShift = sizeof(B) == 32 ? 5 : 4;
   // the steps up to which every lane's cone axis is inside the box
-  auto leave = [&](float a, float q, float G) { return ((a > 0.f ? G : 0.f) - q) / a; };
-  const float te = wave_min(fminf(leave(axis.x, p.x, pg.G[0]), fminf(leave(axis.y, p.y, pg.G[1]), leave(axis.z, p.z, pg.G[2]))));
+  const float te = wave_exit(pg, p, axis);
   int jin = min(max(int(floorf((__log2f(te) - S.log2_t0) * S.inv_log2_q)) + 1, 0), S.n);
   jin = __builtin_amdgcn_readfirstlane(jin);
   while (jin > 0 && !(s[jin - 1].tm <= te)) --jin;
   float od = 0.f;
-  auto read = [&](int l, f3 tp) {
-    const ConstLevels g = lev + l;
-    int x0, y0, z0;
-    float fx, fy, fz;
-    quad_axis_f(fmaf(tp.x, g->ts[0], -0.5f), g->dmax[0], x0, fx);
-    quad_axis_f(fmaf(tp.y, g->ts[1], -0.5f), g->dmax[1], y0, fy);
-    quad_axis_f(fmaf(tp.z, g->ts[2], -0.5f), g->dmax[2], z0, fz);
-    const char* lv = static_cast<const char*>(pyr) + ((size_t(g->boff_hi) << 32) | g->boff_lo);
-    if constexpr (kWide)
-      return pyr_lerp<F>(*reinterpret_cast<const B*>(lv + (brick_index(x0, y0, z0, g->nb[0], g->nb[1]) << kShift)), fx, fy, fz, pg.one);
-    else
-      return pyr_lerp<F>(*reinterpret_cast<const B*>(lv + oct_offset32<kShift>(x0, y0, z0, g->nb[0], g->nb[1])), fx, fy, fz, pg.one);
-  };
   auto step = [&](auto two, auto border, int j) {
     const float tm = s[j].tm;
     const f3 tp = p + axis * tm;
-    float v = read(s[j].level, tp);
-    if constexpr (decltype(two)::value) v = v * s[j].omf + read(s[j].level + 1, tp) * s[j].fr;
-    if constexpr (decltype(border)::value) {
-      const float cx = __builtin_amdgcn_fmed3f(tp.x, 0.f, pg.G[0]) - tp.x;
-      const float cy = __builtin_amdgcn_fmed3f(tp.y, 0.f, pg.G[1]) - tp.y;
-      const float cz = __builtin_amdgcn_fmed3f(tp.z, 0.f, pg.G[2]) - tp.z;
-      v *= __builtin_amdgcn_exp2f((cx * cx + cy * cy + cz * cz) * s[j].fall);
-    }
+    float v = level_read<F, kWide>(pyr, lev + s[j].level, tp, pg.one);
+    if constexpr (decltype(two)::value)
+      v = v * s[j].omf + level_read<F, kWide>(pyr, lev + s[j].level + 1, tp, pg.one) * s[j].fr;
+    if constexpr (decltype(border)::value) v *= border_falloff(pg, tp, s[j].fall);
     od += v * s[j].dt;
   };
   // kAhead steps' loads are in flight together (256^3 at 512^2: 14.6 ms with 2, 14.4 with 3, 17.6 with 4)

@@ -64,6 +64,13 @@ struct ConeSched {
   int n, n0, n1;
   float log2_t0, inv_log2_q;
 };
+// One section of a DOS cone as the device reads it: distance, integration weight, amplitude, the
+// border falloff's -log2(e) / (2 (2^level)^2) and the pyramid level (sections double their sigma, so
+// it is a whole one), clamped to the chain.
+struct DosRow {
+  float track, dint, amp, fall;
+  int level, pad[3];
+};
 struct DosTable {
   std::vector<float4> rows;
   int n[3] = {0, 0, 0};
@@ -127,8 +134,9 @@ struct cvr_ctx {
   cvr::DosTable dos_occ, dos_sdw;
   cvr_dos_cone dos_cones_for[2] = {};  // the cones and sigma of the tables in d_dos_rows
   double dos_sigma_for = 0.0;          // 0: none
-  float4* d_dos_rows = nullptr;
-  size_t dos_rows_cap = 0;
+  void* d_dos_rows = nullptr;  // pyramid levels, occlusion rows, shadow rows
+  size_t dos_rows_bytes = 0;
+  std::vector<cvr::ConeLevel> dos_lev_for;  // the levels in d_dos_rows
 
   // cone ground truth: sampled ray directions (occlusion, then shadow)
   std::vector<float> gt_occ, gt_sdw;

@@ -101,6 +101,22 @@ static void schedule(int n, double t0, double tmax, double half_deg, double r_si
   S.inv_log2_q = float(1.0 / std::log2(q));
 }
 
+std::vector<ConeLevel> cone_levels(const PyrGeom& pg) {
+  std::vector<ConeLevel> lev(kMaxLevels);
+  for (int l = 0; l < pg.levels; ++l) {
+    for (int a = 0; a < 3; ++a) {
+      lev[l].ts[a] = pg.ts[l][a];
+      lev[l].dmax[a] = pg.dmax[l][a];
+    }
+    lev[l].nb[0] = pg.nb[l][0];
+    lev[l].nb[1] = pg.nb[l][1];
+    const size_t at = pg.boff[l] * (pg.fmt == 0 ? 32u : 16u);  // records of 32 (fp32) or 16 bytes
+    lev[l].boff_lo = unsigned(at & 0xFFFFFFFFu);
+    lev[l].boff_hi = unsigned(at >> 32);
+  }
+  return lev;
+}
+
 // The surrogate's stencil: kNOcc geometric segments over [t0, occ_max], each read on
 // the axis at distance D = sqrt(ab) (level of the axial cone's radius) and at D cos(ring)
 // (level of the ring's radius D sin(ring)); kNSdw segments over [t0, sdw_max] along the
@@ -200,19 +216,7 @@ int prepare_cone(cvr_ctx* c, const cvr_cone_params& P, hipStream_t st) {
   ConeSched& Ss = c->cone_sched[1];
   schedule(P.n_steps, P.t0, occ_max, P.occ_half_deg, P.r_sigma, P.sigma0, c->pyr.levels, so, So);
   schedule(P.n_steps, P.t0, sdw_max, P.sdw_half_deg, P.r_sigma, P.sigma0, c->pyr.levels, ss, Ss);
-  std::vector<ConeLevel> lev(kMaxLevels);
-  for (int l = 0; l < c->pyr.levels; ++l) {
-    const PyrGeom& pg = c->pyr;
-    for (int a = 0; a < 3; ++a) {
-      lev[l].ts[a] = pg.ts[l][a];
-      lev[l].dmax[a] = pg.dmax[l][a];
-    }
-    lev[l].nb[0] = pg.nb[l][0];
-    lev[l].nb[1] = pg.nb[l][1];
-    const size_t at = pg.boff[l] * (pg.fmt == 0 ? 32u : 16u);  // records of 32 (fp32) or 16 bytes
-    lev[l].boff_lo = unsigned(at & 0xFFFFFFFFu);
-    lev[l].boff_hi = unsigned(at >> 32);
-  }
+  const std::vector<ConeLevel> lev = cone_levels(c->pyr);
   std::vector<StencilF> stn;
   stencil(P, occ_max, sdw_max, c->pyr.levels, stn);
   stn.push_back(StencilF{0.f, 1.f, 0.f, 0.f});  // the local opacity: level 0 at the sample

@@ -17,11 +17,11 @@
 // depth, trapezoid sums of amplitude * extinction, I = exp(-depth) averaged over the
 // sub-cones (the 7-packing weights its ring by the adjacent weight).  The march is
 // queue_march's (cvr_queue.hpp; 256^3 at 1024^2 with shadows 41.5 -> 15.6 ms, at 200 x 150
-// 7.2 -> 0.26 ms).  The table row
-// index is wave-uniform, so rows arrive through scalar loads and the level geometry
-// stays in SGPRs.
+// 7.2 -> 0.26 ms; with the rows of dos_cone 12.6 and 0.18 ms).  A section is the same for all lanes:
+// its row and its level's geometry come through scalar loads.
 #include "cvr_cone.hpp"
 #include "cvr_queue.hpp"
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -30,68 +30,88 @@ namespace cvr {
 
 // Per-cone constants of the device integration.
 struct DosConeK {
-  int n1, n3, n7, pad;
-  float init, w, adj7, pad2;
+  int n1, n3, n7;
+  float w, adj7;
   float ax[10][3];  // 3-packing axes, then 7-packing axes, (x, y, z) in the cone frame
 };
 
 struct DosK {
   DosConeK occ, sdw;
-  const float4* occ_rows;
-  const float4* sdw_rows;
+  const ConeLevel* lev;
+  const DosRow* occ_rows;
+  const DosRow* sdw_rows;
   int apply_occ, apply_sdw, shadow_type;
   float spot_cos, ka, kd;
   float eye[3], lpos[3], lfwd[3], lup[3], lright[3];
 };
 
-// GetGaussianExtinction (ray_bbox_marching.comp:92-112) at a section's level: textureLod
-// clamps the level to the chain, the border falloff uses the level as given.
-template <int F>
-__device__ __forceinline__ float dos_ext(const void* __restrict__ pyr, const PyrGeom& pg, f3 tp, float level) {
-  const float lc = fminf(fmaxf(level, 0.f), float(pg.levels - 1));
-  const int d1 = int(floorf(lc));
-  const float fr = lc - float(d1);
-  float a = pyr_tri<F>(pyr, pg, d1, tp);
-  if (fr > 0.f) a = a * (1.f - fr) + pyr_tri<F>(pyr, pg, min(d1 + 1, pg.levels - 1), tp) * fr;
-  return a * border_falloff(pg, tp, 0.5f * exp2f(-2.f * level));
-}
-
-// One cone through its section table; sub-cone axes are k*z + uy*y + vx*x.
-template <int F>
+// One cone through its section table; sub-cone axes are k*z + uy*y + vx*x.  A section's row is the same
+// for all lanes (scalar loads); sections before the first lane leaves the box do without the border
+// falloff, which is 1 there.
+template <int F, bool kWide>
 __device__ __forceinline__ float dos_cone(const void* __restrict__ pyr, const PyrGeom& pg, const DosConeK& C,
-                                          const float4* __restrict__ rows, f3 p, f3 k, f3 uy, f3 vx) {
+                                          const ConeLevel* __restrict__ levels, const DosRow* __restrict__ table, f3 p,
+                                          f3 k, f3 uy, f3 vx) {
+  typedef const __attribute__((address_space(4))) DosRow* ConstRows;
+  const ConstRows rows = (ConstRows)(uintptr_t)table;
+  const ConstLevels lev = (ConstLevels)(uintptr_t)levels;
   float od[7], lt[7];
-  float track = C.init;
   od[0] = 0.f;
   lt[0] = 0.f;
   int i = 0;
-  // the single-cone sections read one level each and their positions do not depend on
-  // the reads: unrolled by 4, four reads are in flight at once and the sums keep their
-  // order (256^3 @ 1024^2 with shadows: 37.7 -> 35.9 ms, the same frame bit for bit)
-#pragma unroll 4
-  for (; i < C.n1; ++i) {
-    const float4 s = rows[i];
-    const float at = dos_ext<F>(pyr, pg, p + k * track, s.y) * s.w;
-    od[0] += (lt[0] + at) * s.z * C.w;
-    lt[0] = at;
-    track += s.x;
+  // GetGaussianExtinction (ray_bbox_marching.comp:92-112) of row i at axis d
+  auto ext = [&](auto border, int i, f3 d) {
+    const f3 tp = p + d * rows[i].track;
+    float v = level_read<F, kWide>(pyr, lev + rows[i].level, tp, pg.one);
+    if constexpr (decltype(border)::value) v *= border_falloff(pg, tp, rows[i].fall);
+    return v * rows[i].amp;
+  };
+  auto add = [&](int j, int i, float at) {
+    od[j] += (lt[j] + at) * rows[i].dint * C.w;
+    lt[j] = at;
+  };
+  // the single-cone sections in groups whose reads are in flight together (256^3 at 1024^2: 15.0 ms
+  // with 2, 13.5 with 4, 12.6 with 8, 12.4 with 10, whose remainders cost small volumes more; the
+  // 7-packing's registers are more than any of them need)
+  constexpr int kAhead = 8;
+  const float te = wave_exit(pg, p, k);
+  auto group = [&](auto border) {
+    float at[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) at[u] = ext(border, i + u, k);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) add(0, i + u, at[u]);
+  };
+  for (; i + kAhead <= C.n1; i += kAhead) {
+    if (rows[i + kAhead - 1].track <= te) group(std::false_type{});
+    else group(std::true_type{});
   }
+  for (; i < C.n1; ++i) add(0, i, ext(std::true_type{}, i, k));
   if (C.n3 + C.n7 == 0) return __expf(-od[0]);
   od[1] = od[2] = od[0];
   lt[1] = lt[2] = lt[0];
   f3 d3[3];
 #pragma unroll
   for (int j = 0; j < 3; ++j) d3[j] = k * C.ax[j][2] + uy * C.ax[j][1] + vx * C.ax[j][0];
-  for (const int e = i + C.n3; i < e; ++i) {
-    const float4 s = rows[i];
+  auto sections = [&](auto count, const f3* d, int e) {
+    constexpr int kN = decltype(count)::value;
+    float t = wave_exit(pg, p, d[0]);
 #pragma unroll
-    for (int j = 0; j < 3; ++j) {
-      const float at = dos_ext<F>(pyr, pg, p + d3[j] * track, s.y) * s.w;
-      od[j] += (lt[j] + at) * s.z * C.w;
-      lt[j] = at;
+    for (int j = 1; j < kN; ++j) t = fminf(t, wave_exit(pg, p, d[j]));
+    for (; i < e; ++i) {
+      float at[kN];
+      if (rows[i].track <= t) {
+#pragma unroll
+        for (int j = 0; j < kN; ++j) at[j] = ext(std::false_type{}, i, d[j]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < kN; ++j) at[j] = ext(std::true_type{}, i, d[j]);
+      }
+#pragma unroll
+      for (int j = 0; j < kN; ++j) add(j, i, at[j]);
     }
-    track += s.x;
-  }
+  };
+  sections(std::integral_constant<int, 3>{}, d3, i + C.n3);
   if (C.n7 == 0) return (__expf(-od[0]) + __expf(-od[1]) + __expf(-od[2])) / 3.0f;
   // 3 -> 7: each outer cone inherits the depth of the 3-cone it came from, the centre
   // cone their mean (Cone7RayOcclusion, :127-137)
@@ -107,30 +127,36 @@ __device__ __forceinline__ float dos_cone(const void* __restrict__ pyr, const Py
   f3 d7[7];
 #pragma unroll
   for (int j = 0; j < 7; ++j) d7[j] = k * C.ax[3 + j][2] + uy * C.ax[3 + j][1] + vx * C.ax[3 + j][0];
-  for (const int e = i + C.n7; i < e; ++i) {
-    const float4 s = rows[i];
-#pragma unroll
-    for (int j = 0; j < 7; ++j) {
-      const float at = dos_ext<F>(pyr, pg, p + d7[j] * track, s.y) * s.w;
-      od[j] += (lt[j] + at) * s.z * C.w;
-      lt[j] = at;
-    }
-    track += s.x;
-  }
+  sections(std::integral_constant<int, 7>{}, d7, i + C.n7);
   const float ring = __expf(-od[1]) + __expf(-od[2]) + __expf(-od[3]) + __expf(-od[4]) + __expf(-od[5]) + __expf(-od[6]);
   return (__expf(-od[0]) + ring * C.adj7) / (1.0f + C.adj7 * 6.0f);
 }
 
 // Shadow cone of ShadowEvaluationKernel (:533-562).  `wp` is the world position.
-template <int F>
+template <int F, bool kWide>
 __device__ __forceinline__ float dos_shadow(const void* __restrict__ pyr, const PyrGeom& pg, const DosK& K, f3 p,
                                             f3 wp) {
-  if (K.shadow_type == 2) return dos_cone<F>(pyr, pg, K.sdw, K.sdw_rows, p, ld3(K.lfwd), ld3(K.lup), ld3(K.lright));
-  const f3 k = norm3(ld3(K.lpos) - wp);
-  if (K.shadow_type == 1 && dot3(k, ld3(K.lfwd)) < K.spot_cos) return 0.f;
-  const f3 u1 = norm3(cross3(k, ld3(K.lright)));
-  const f3 v1 = norm3(cross3(k, u1));
-  return dos_cone<F>(pyr, pg, K.sdw, K.sdw_rows, p, k, v1, u1);
+  f3 k = ld3(K.lfwd), up = ld3(K.lup), right = ld3(K.lright);
+  if (K.shadow_type != 2) {
+    k = norm3(ld3(K.lpos) - wp);
+    if (K.shadow_type == 1 && dot3(k, ld3(K.lfwd)) < K.spot_cos) return 0.f;
+    const f3 u1 = norm3(cross3(k, right));
+    up = norm3(cross3(k, u1));
+    right = u1;
+  }
+  return dos_cone<F, kWide>(pyr, pg, K.sdw, K.lev, K.sdw_rows, p, k, up, right);
+}
+// Both terms at p: the occlusion cone along k in the frame (up, right); 0 for one that is off.
+template <int F>
+__device__ __forceinline__ void dos_light(const void* __restrict__ pyr, const PyrGeom& pg, const DosK& K, f3 p, f3 wp, f3 k,
+                                          f3 up, f3 right, float& Io, float& Is) {
+  auto both = [&](auto wide) {
+    constexpr bool kWide = decltype(wide)::value;
+    Io = K.apply_occ ? dos_cone<F, kWide>(pyr, pg, K.occ, K.lev, K.occ_rows, p, k, up, right) : 0.f;
+    Is = K.apply_sdw ? dos_shadow<F, kWide>(pyr, pg, K, p, wp) : 0.f;
+  };
+  if (pg.wide) both(std::true_type{});
+  else both(std::false_type{});
 }
 
 constexpr int kRays = 4;
@@ -153,13 +179,10 @@ __global__ __launch_bounds__(256) void k_dos_render(RayFrame rf, VolGeom g, PyrG
   queue_march<T, 64, false, kParts>(rf, g, s_tf, ntf, step, et, qs.rays, FramePixels(rf, qs, u), ph.spec, kParts > 1 ? queue : queue + (threadIdx.x >> 6), out, nsamp, nshade,
                  [&](bool, f3 p, f3 dir) {
                    const f3 wp = p - half;
-                   float Io = 0.f, Is = 0.f;
-                   if (K.apply_occ) {
-                     f3 axis, up, right;
-                     occ_frame(dir, axis, up, right);
-                     Io = dos_cone<F>(pyr, pg, K.occ, K.occ_rows, p, norm3(eye - wp), up, right);
-                   }
-                   if (K.apply_sdw) Is = dos_shadow<F>(pyr, pg, K, p, wp);
+                   float Io, Is;
+                   f3 axis, up, right;
+                   occ_frame(dir, axis, up, right);
+                   dos_light<F>(pyr, pg, K, p, wp, norm3(eye - wp), up, right, Io, Is);
                    if (!ph.on) return Lit{inv_k * (Io * ka + Is * kd), 0.f};
                    // Phong branch (:627-643): a sample whose gradient vanishes keeps its colour
                    float dd, sp;
@@ -186,15 +209,11 @@ __global__ __launch_bounds__(256) void k_lc_dos(PyrGeom pg, const void* __restri
   const int x = int(i % size_t(rx)), y = int((i / size_t(rx)) % size_t(ry)), z = int(i / (size_t(rx) * ry));
   const f3 tp = mk3((float(x) + 0.5f) * cell.x, (float(y) + 0.5f) * cell.y, (float(z) + 0.5f) * cell.z);
   const f3 wp = tp - half;
-  float Io = 1.f, Is = 1.f;
-  if (K.apply_occ) {
-    const f3 k = norm3(ld3(K.eye) - wp);
-    const f3 vr = norm3(cross3(mk3(-k.x, -k.y, -k.z), cam_up));
-    const f3 vu = norm3(cross3(k, vr));
-    Io = dos_cone<F>(pyr, pg, K.occ, K.occ_rows, tp, k, vu, vr);
-  }
-  if (K.apply_sdw) Is = dos_shadow<F>(pyr, pg, K, tp, wp);
-  lc[i] = make_float2(Io, Is);
+  const f3 k = norm3(ld3(K.eye) - wp);
+  const f3 vr = norm3(cross3(mk3(-k.x, -k.y, -k.z), cam_up));
+  float Io, Is;
+  dos_light<F>(pyr, pg, K, tp, wp, k, norm3(cross3(k, vr)), vr, Io, Is);
+  lc[i] = make_float2(K.apply_occ ? Io : 1.f, K.apply_sdw ? Is : 1.f);
 }
 
 // ------------------------------------------------------------------ host: section tables
@@ -372,27 +391,37 @@ int prepare_dos(cvr_ctx* c, const cvr_dos_params& P, hipStream_t st) {
   const cvr_dos_cone oc = clamp_cone(P.occ, diag * 0.50f), sc = clamp_cone(P.sdw, diag * 0.75f);
   // the tables of the same cones are kept (building and copying them took 0.05 ms of every frame)
   const double sigma0 = P.sigma0;
-  if (c->dos_sigma_for == sigma0 && std::memcmp(&c->dos_cones_for[0], &oc, sizeof(oc)) == 0 &&
+  const std::vector<ConeLevel> lev = cone_levels(c->pyr);
+  if (c->dos_sigma_for == sigma0 && c->dos_lev_for.size() == lev.size() &&
+      std::memcmp(c->dos_lev_for.data(), lev.data(), lev.size() * sizeof(ConeLevel)) == 0 && std::memcmp(&c->dos_cones_for[0], &oc, sizeof(oc)) == 0 &&
       std::memcmp(&c->dos_cones_for[1], &sc, sizeof(sc)) == 0)
     return CVR_OK;
   c->dos_sigma_for = 0.0;
   CVR_HIP_CHECK(hipDeviceSynchronize());  // frames in flight may still read the rows
   if ((rc = dos_build_table(oc, P.sigma0, c->dos_occ))) return rc;
   if ((rc = dos_build_table(sc, P.sigma0, c->dos_sdw))) return rc;
-  const size_t n = c->dos_occ.rows.size() + c->dos_sdw.rows.size();
-  if (n > c->dos_rows_cap) {
-    if (c->d_dos_rows) CVR_HIP_CHECK(hipFree(c->d_dos_rows));
-    c->d_dos_rows = nullptr;
-    c->dos_rows_cap = 0;
-    if (hipMalloc(&c->d_dos_rows, n * sizeof(float4)) != hipSuccess) {
-      set_error("dos: out of device memory");
-      return CVR_ERR_NOMEM;
+  // [levels] [occlusion rows] [shadow rows]
+  std::vector<DosRow> rows;
+  for (const DosTable* T : {&c->dos_occ, &c->dos_sdw}) {
+    float track = T->init;
+    for (const float4& r : T->rows) {
+      const double level = double(r.y);  // log2(sigma / sigma0), a whole number
+      DosRow d{track, r.z, r.w, float(-0.5 * 1.4426950408889634 * std::exp2(-2.0 * level)), 0, {0, 0, 0}};
+      d.level = std::min(std::max(int(std::lround(level)), 0), c->pyr.levels - 1);
+      rows.push_back(d);
+      track += r.x;
     }
-    c->dos_rows_cap = n;
   }
-  std::vector<float4> all(c->dos_occ.rows);
-  all.insert(all.end(), c->dos_sdw.rows.begin(), c->dos_sdw.rows.end());
-  CVR_HIP_CHECK(hipMemcpy(c->d_dos_rows, all.data(), n * sizeof(float4), hipMemcpyHostToDevice));
+  const size_t lb = lev.size() * sizeof(ConeLevel), rb = rows.size() * sizeof(DosRow);
+  if ((rc = sized_buffer(&c->d_dos_rows, &c->dos_rows_bytes, lb + rb))) {
+    if (rc == CVR_ERR_NOMEM) set_error("dos: out of device memory");
+    return rc;
+  }
+  std::vector<char> buf(lb + rb);
+  std::memcpy(buf.data(), lev.data(), lb);
+  std::memcpy(buf.data() + lb, rows.data(), rb);
+  CVR_HIP_CHECK(hipMemcpy(c->d_dos_rows, buf.data(), buf.size(), hipMemcpyHostToDevice));
+  c->dos_lev_for = lev;
   c->dos_cones_for[0] = oc;
   c->dos_cones_for[1] = sc;
   c->dos_sigma_for = sigma0;
@@ -404,7 +433,6 @@ static DosConeK cone_k(const DosTable& T) {
   k.n1 = T.n[0];
   k.n3 = T.n[1];
   k.n7 = T.n[2];
-  k.init = T.init;
   k.w = T.w;
   k.adj7 = T.adj7;
   std::memcpy(k.ax, T.axes, sizeof(k.ax));
@@ -418,8 +446,9 @@ int launch_dos(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* ou
   DosK K{};
   K.occ = cone_k(c->dos_occ);
   K.sdw = cone_k(c->dos_sdw);
-  K.occ_rows = c->d_dos_rows;
-  K.sdw_rows = c->d_dos_rows + c->dos_occ.rows.size();
+  K.lev = static_cast<const ConeLevel*>(c->d_dos_rows);
+  K.occ_rows = reinterpret_cast<const DosRow*>(K.lev + kMaxLevels);
+  K.sdw_rows = K.occ_rows + c->dos_occ.rows.size();
   K.apply_occ = P.apply_occlusion;
   K.apply_sdw = P.apply_shadow;
   K.shadow_type = P.shadow_type;
@@ -461,8 +490,9 @@ int launch_dos(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* ou
   }
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   float4* o4 = reinterpret_cast<float4*>(out);
-  // small frames: workgroups whose wavefronts share their rays (100 x 100 0.41 ms, 0.82 ms with
-  // rays of their own; 200 x 150 0.26 and 0.48; 400 x 300 2.2 and 1.7; 1024^2 19.4 and 15.6)
+  // small frames: workgroups whose wavefronts share their rays (measured with the first rows of
+  // dos_cone: 100 x 100 0.41 ms, 0.82 ms with rays of their own; 200 x 150 0.26 and 0.48; 400 x 300 2.2
+  // and 1.7; 1024^2 19.4 and 15.6)
   const bool shared = size_t(rf.W) * rf.H < (1 << 16);
   const QueueShape qs = queue_shape(rf, kRays, shared ? 4 : 1, shared ? 64 : 256);
   with_types(c->dtype, c->pyr.fmt, [&](auto t, auto f) {
