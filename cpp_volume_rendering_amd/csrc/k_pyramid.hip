@@ -8,11 +8,10 @@
 // Levels are stored in one fp32 buffer, level 0 first, x fastest.  Opacity levels
 // live in a scratch buffer only while the chain is built.
 //
-// Level 0: the direct build sums 343 samples of the volume per voxel (8x8x4 voxel bricks per
-// 256-lane workgroup, the weights in LDS); the separable one (when the voxel spacing and sigma are
-// commensurate) samples a lattice once, see k_pyr_lattice / k_pyr_sep.  Levels above are products
-// over the axes: three passes of linear reads each (k_pyr_axis), the small ones together in one
-// workgroup (k_pyr_tail).
+// Direct build: one lane per output voxel, 8x8x4 voxel bricks per 256-lane workgroup;
+// the 343 weights are the same for every voxel and sit in LDS.  Separable build (used
+// when the voxel spacing and sigma are commensurate, as in every default configuration):
+// see k_pyr_lattice / k_pyr_sep below.
 #include "cvr_ctx.hpp"
 #include <array>
 #include <algorithm>
@@ -37,6 +36,18 @@ static dim3 cells_grid(int n0, int n1, int n2) {
   return dim3(unsigned((n0 + 63) / 64), unsigned(std::min((n1 + 3) / 4, 65535)), unsigned(std::min(n2, 65535)));
 }
 
+// Tap k of output cell o along an axis: the centre rounded, then one fused addition, spelled out so that
+// every build takes the same samples (the compiler would choose which product to fuse).
+__device__ __forceinline__ float tap_pos(int o, int k, float vs, float sigma) {
+  float c;
+  {
+#pragma clang fp contract(off)
+    c = (float(o) + 0.5f) * vs;
+  }
+  asm("" : "+v"(c));
+  return __builtin_fmaf(sigma, float(k), c);
+}
+
 struct PyrBuild {
   int bx, by, bz;  // output level dims
   int px, py, pz;  // previous level dims (levels >= 1)
@@ -52,7 +63,7 @@ __device__ __forceinline__ bool outside01(float x, float y, float z) {
 // alone, and so does its share of the block's offset (brick_index is a sum of three terms): they are
 // computed once per axis, 7 along x in registers, and the 343 taps are left with an addition, a load,
 // the lerp and the table read from LDS (128^3 level of a 34 x 29 x 28 volume 0.75 ms; the
-// next step of that volume and its DOS frame 3.45 -> 0.86 ms).
+// next step of that volume and its DOS frame 3.45 -> 1.57 ms with k_pyr_next's).
 constexpr int kTfLds = 8192;
 template <typename T, bool TF_LDS>
 __global__ __launch_bounds__(256) void k_pyr_level0(PyrBuild b, VolGeom g, const float4* __restrict__ tf_rgba,
@@ -79,13 +90,12 @@ __global__ __launch_bounds__(256) void k_pyr_level0(PyrBuild b, VolGeom g, const
   const int y = blockIdx.y * 8 + ((threadIdx.x >> 3) & 7);
   const int z = blockIdx.z * 4 + (threadIdx.x >> 6);
   if (x >= b.bx || y >= b.by || z >= b.bz) return;
-  const float gx = (float(x) + 0.5f) * b.vs[0], gy = (float(y) + 0.5f) * b.vs[1], gz = (float(z) + 0.5f) * b.vs[2];
   typedef typename VolOct<T>::type RT;
   const RT* __restrict__ oct = static_cast<const RT*>(g.oct);
   // tap k of an axis: false outside the box; its cell's term of the block number (`rows`: bricks
   // of a step along the axis, `in`: cells of one inside a brick) and weight
-  auto tap = [&](int axis, float centre, int k, size_t rows, int in, size_t& off, float& f) {
-    const float p = centre + float(k) * b.sigma, t = p / b.G[axis];
+  auto tap = [&](int axis, int o, int k, size_t rows, int in, size_t& off, float& f) {
+    const float p = tap_pos(o, k, b.vs[axis], b.sigma), t = p / b.G[axis];
     int c;
     quad_axis_f(p * g.tex_mul[axis] - 0.5f, g.vmax[axis], c, f);
     off = size_t(c >> 2) * rows * 64u + size_t((c & 3) * in);
@@ -95,16 +105,16 @@ __global__ __launch_bounds__(256) void k_pyr_level0(PyrBuild b, VolGeom g, const
   float fx[7];
   bool vx[7];
 #pragma unroll
-  for (int k = 0; k < 7; ++k) vx[k] = tap(0, gx, k - 3, 1, 1, ox[k], fx[k]);
+  for (int k = 0; k < 7; ++k) vx[k] = tap(0, x, k - 3, 1, 1, ox[k], fx[k]);
   float acc = 0.f;
   for (int kz = 0; kz < 7; ++kz) {
     size_t oz;
     float fz;
-    if (!tap(2, gz, kz - 3, size_t(g.nbx) * size_t(g.nby), 16, oz, fz)) continue;
+    if (!tap(2, z, kz - 3, size_t(g.nbx) * size_t(g.nby), 16, oz, fz)) continue;
     for (int ky = 0; ky < 7; ++ky) {
       size_t oy;
       float fy;
-      if (!tap(1, gy, ky - 3, size_t(g.nbx), 4, oy, fy)) continue;
+      if (!tap(1, y, ky - 3, size_t(g.nbx), 4, oy, fy)) continue;
       const RT* row = oct + (oz + oy);
       RT r[7];
 #pragma unroll
@@ -143,82 +153,17 @@ __device__ __forceinline__ float tex3_f(const float* __restrict__ a, int nx, int
   return c0 + fz * (c1 - c0);
 }
 
-// Level i >= 1 along one axis: the trilinear read of the level before and the Gaussian are
-// products over the axes, so any level is three passes of 7 linear reads each, whatever its
-// spacing (the direct sum of 343 trilinear reads is left for when the passes' temporaries find no
-// memory).  in: in0 x in1 x in2, of which `axis` shrinks to b_n; `vs` and G the axis's spacing and size.
-__global__ __launch_bounds__(256) void k_pyr_axis(const float* __restrict__ in, float* __restrict__ out, int in0, int in1,
-                                                  int in2, int axis, int b_n, float vs, float G, float sigma, SepW w,
-                                                  float scale) {
-  const int o0 = axis == 0 ? b_n : in0, o1 = axis == 1 ? b_n : in1, o2 = axis == 2 ? b_n : in2;
-  for_cells(o0, o1, o2, [&](int x, int y, int z) {
-    const size_t s1 = size_t(in0), s2 = size_t(in0) * in1;
-    const int o = axis == 0 ? x : axis == 1 ? y : z, n = axis == 0 ? in0 : axis == 1 ? in1 : in2;
-    const size_t step = axis == 0 ? 1 : axis == 1 ? s1 : s2;
-    const size_t base = (axis == 0 ? 0 : size_t(x)) + (axis == 1 ? 0 : y * s1) + (axis == 2 ? 0 : z * s2);
-    const float c = (float(o) + 0.5f) * vs;
-    float acc = 0.f;
-#pragma unroll
-    for (int t = 0; t < 7; ++t) {
-      const float u = (c + float(t - 3) * sigma) / G;
-      int i0, i1;
-      float f;
-      lin_axis(u * float(n) - 0.5f, n, i0, i1, f);
-      const float a = in[base + i0 * step], b = in[base + i1 * step];
-      if (!(u < 0.f || u > 1.f)) acc += w.g[t] * (a + f * (b - a));
-    }
-    out[x + size_t(o0) * (y + size_t(o1) * z)] = acc * scale;
-  });
-}
-
-// The levels from `first` on, each of the one before, in one workgroup: the level before `first` has
-// at most kTailCells voxels, and the passes of k_pyr_axis run in LDS.  Three launches a level for a
-// few thousand voxels left the GPU waiting for the host.
-constexpr int kTailCells = 4096;
-__global__ __launch_bounds__(1024) void k_pyr_tail(PyrGeom pg, int first, float sigma0, float* __restrict__ op, SepW w,
-                                                   float norm) {
-  __shared__ float buf[3][kTailCells];
-  const int* P = pg.dims[first - 1];
-  for (int i = threadIdx.x; i < P[0] * P[1] * P[2]; i += 1024) buf[0][i] = op[pg.off[first - 1] + i];
-  __syncthreads();
-  for (int l = first; l < pg.levels; ++l) {
-    int n[3] = {pg.dims[l - 1][0], pg.dims[l - 1][1], pg.dims[l - 1][2]};
-    const float sigma = ldexpf(sigma0, l);
-#pragma unroll
-    for (int axis = 0; axis < 3; ++axis) {
-      const float* in = buf[axis];
-      float* out = buf[(axis + 1) % 3];
-      const int s1 = n[0], s2 = n[0] * n[1], len = n[axis];
-      const float G = pg.G[axis], vs = G / float(pg.dims[l][axis]);
-      n[axis] = pg.dims[l][axis];
-      for (int i = threadIdx.x; i < n[0] * n[1] * n[2]; i += 1024) {
-        const int x = i % n[0], y = i / n[0] % n[1], z = i / (n[0] * n[1]);
-        const int o = axis == 0 ? x : axis == 1 ? y : z, step = axis == 0 ? 1 : axis == 1 ? s1 : s2;
-        const int base = (axis == 0 ? 0 : x) + (axis == 1 ? 0 : y * s1) + (axis == 2 ? 0 : z * s2);
-        const float c = (float(o) + 0.5f) * vs;
-        float acc = 0.f;
-#pragma unroll
-        for (int t = 0; t < 7; ++t) {
-          const float u = (c + float(t - 3) * sigma) / G;
-          int i0, i1;
-          float f;
-          lin_axis(u * float(len) - 0.5f, len, i0, i1, f);
-          const float a = in[base + i0 * step], b = in[base + i1 * step];
-          if (!(u < 0.f || u > 1.f)) acc += w.g[t] * (a + f * (b - a));
-        }
-        if (axis == 2) {
-          acc *= norm;
-          op[pg.off[l] + i] = acc;
-        }
-        out[i] = acc;
-      }
-      __syncthreads();
-    }
-  }
-}
-
-__global__ __launch_bounds__(256) void k_pyr_next(PyrBuild b, const float* __restrict__ prev_op,
+// Direct build of a level from the one before, as level 0's: the cells, weights and inside tests of a
+// tap once per axis, 7 along x in registers, each tap's sums in the order of tex3_f.  A small level
+// has a lane or none per SIMD, each a chain of 343 taps: from LDS where the level before fits.
+constexpr int kPrevLds = 36000;  // voxels of the level before that LDS holds
+template <bool kLds>
+__global__ __launch_bounds__(256) void k_pyr_next(PyrBuild b, const float* __restrict__ prev_global,
                                                   float* __restrict__ out_op) {
+  extern __shared__ float s_prev[];
+  if (kLds)
+    for (int i = threadIdx.x; i < b.px * b.py * b.pz; i += 256) s_prev[i] = prev_global[i];
+  const float* prev_op = kLds ? s_prev : prev_global;
   __shared__ float s_w[343];
   __shared__ float s_wsum;
   for (int i = threadIdx.x; i < 343; i += blockDim.x) {
@@ -237,43 +182,75 @@ __global__ __launch_bounds__(256) void k_pyr_next(PyrBuild b, const float* __res
   const int y = blockIdx.y * 8 + ((threadIdx.x >> 3) & 7);
   const int z = blockIdx.z * 4 + (threadIdx.x >> 6);
   if (x >= b.bx || y >= b.by || z >= b.bz) return;
-  const float gx = (float(x) + 0.5f) * b.vs[0], gy = (float(y) + 0.5f) * b.vs[1], gz = (float(z) + 0.5f) * b.vs[2];
+  auto tap = [&](int axis, int o, int k, int n, int& i0, int& i1, float& f) {
+    const float t = tap_pos(o, k, b.vs[axis], b.sigma) / b.G[axis];
+    lin_axis(t * float(n) - 0.5f, n, i0, i1, f);
+    return !(t < 0.f || t > 1.f);
+  };
+  int x0[7], x1[7];
+  float fx[7];
+  bool vx[7];
+#pragma unroll
+  for (int k = 0; k < 7; ++k) vx[k] = tap(0, x, k - 3, b.px, x0[k], x1[k], fx[k]);
+  const size_t sy = size_t(b.px), sz = size_t(b.px) * b.py;
   float acc = 0.f;
-  for (int i = 0; i < 343; ++i) {
-    const int kx = i % 7 - 3, ky = (i / 7) % 7 - 3, kz = i / 49 - 3;
-    const float tx = (gx + float(kx) * b.sigma) / b.G[0];
-    const float ty = (gy + float(ky) * b.sigma) / b.G[1];
-    const float tz = (gz + float(kz) * b.sigma) / b.G[2];
-    if (outside01(tx, ty, tz)) continue;
-    acc += s_w[i] * tex3_f(prev_op, b.px, b.py, b.pz, tx, ty, tz);
+  for (int kz = 0; kz < 7; ++kz) {
+    int z0, z1;
+    float fz;
+    if (!tap(2, z, kz - 3, b.pz, z0, z1, fz)) continue;
+    for (int ky = 0; ky < 7; ++ky) {
+      int y0, y1;
+      float fy;
+      if (!tap(1, y, ky - 3, b.py, y0, y1, fy)) continue;
+      const float *r00 = prev_op + (y0 * sy + z0 * sz), *r10 = prev_op + (y1 * sy + z0 * sz);
+      const float *r01 = prev_op + (y0 * sy + z1 * sz), *r11 = prev_op + (y1 * sy + z1 * sz);
+#pragma unroll
+      for (int k = 0; k < 7; ++k) {
+        const float c00 = r00[x0[k]] + fx[k] * (r00[x1[k]] - r00[x0[k]]);
+        const float c10 = r10[x0[k]] + fx[k] * (r10[x1[k]] - r10[x0[k]]);
+        const float c01 = r01[x0[k]] + fx[k] * (r01[x1[k]] - r01[x0[k]]);
+        const float c11 = r11[x0[k]] + fx[k] * (r11[x1[k]] - r11[x0[k]]);
+        const float c0 = c00 + fy * (c10 - c00), c1 = c01 + fy * (c11 - c01);
+        if (vx[k]) acc += s_w[(kz * 7 + ky) * 7 + k] * (c0 + fz * (c1 - c0));
+      }
+    }
   }
   out_op[size_t(x) + size_t(b.bx) * (y + size_t(b.by) * z)] = acc / s_wsum;
 }
 
 // ---------------------------------------------------------------------------------
-// Separable build of level 0.  The 7^3 taps of output voxel x along axis a sit at (x + 1/2) vs_a +
+// Separable build.  The 7^3 taps of output voxel x along axis a sit at (x + 1/2) vs_a +
 // i sigma (i = -3..3).  When vs_a = m_a delta_a and sigma = q_a delta_a for small
 // integers m_a, q_a, every tap of every output voxel lies on the lattice (1/2) vs_a +
 // (n - 3 q_a) delta_a, n = m_a x + q_a (i + 3), and the weights factor as
 // sigma^3 g_i g_j g_k (g_i = exp(-i^2 / 2)); the zero outside [0, G] is a per-axis test.
-// So the level is: the TF opacity of the trilinear volume sample evaluated once per lattice
-// point, then three 7-tap passes along x, y and z with output stride m_a and tap stride
-// q_a, normalised by (sum g)^3 -- 3 x 7 taps per voxel instead of 343, the same samples and
-// weights (extcoefvolumegenerator.cpp:230-367).
+// So a level is: its function (TF opacity of the trilinear volume sample for level 0,
+// the trilinear previous level above) evaluated once per lattice point, then three 7-tap
+// passes along x, y and z with output stride m_a and tap stride q_a, normalised by
+// (sum g)^3 -- 3 x 7 taps per voxel instead of 343, the same samples and weights
+// (extcoefvolumegenerator.cpp:230-367).  (Levels above 0 could always be three passes of linear
+// reads: 0.7 ms less where they are built directly.  But another order of their sums moves 16-bit
+// records and, behind them, the surrogate's bf16 inputs across roundings: 4e-4 in a pixel.)
 struct SepAxis {
   int m, q, len;  // output stride, tap stride, lattice points (m (b - 1) + 6 q + 1)
   float half_vs, delta;
 };
 
-template <typename T>
+template <typename T, bool kLevel0>
 __global__ __launch_bounds__(256) void k_pyr_lattice(SepAxis ax, SepAxis ay, SepAxis az, float3 G, VolGeom g,
-                                                     const float4* __restrict__ tf_rgba, int ntf, float* __restrict__ lat) {
+                                                     const float4* __restrict__ tf_rgba, int ntf,
+                                                     const float* __restrict__ prev_op, int px, int py, int pz,
+                                                     float* __restrict__ lat) {
   for_cells(ax.len, ay.len, az.len, [&](int nx, int ny, int nz) {
     const float p0 = ax.half_vs + float(nx - 3 * ax.q) * ax.delta;
     const float p1 = ay.half_vs + float(ny - 3 * ay.q) * ay.delta;
     const float p2 = az.half_vs + float(nz - 3 * az.q) * az.delta;
+    const float tx = p0 / G.x, ty = p1 / G.y, tz = p2 / G.z;
     float v = 0.f;
-    if (!outside01(p0 / G.x, p1 / G.y, p2 / G.z)) v = sample_tf(tf_rgba, ntf, sample_volume_oct<T>(g, mk3(p0, p1, p2))).w;
+    if (!outside01(tx, ty, tz)) {
+      if (kLevel0) v = sample_tf(tf_rgba, ntf, sample_volume_oct<T>(g, mk3(p0, p1, p2))).w;
+      else v = tex3_f(prev_op, px, py, pz, tx, ty, tz);
+    }
     lat[nx + size_t(ax.len) * (ny + size_t(ay.len) * nz)] = v;
   });
 }
@@ -383,28 +360,26 @@ int build_pyramid(cvr_ctx* c, int base_x, int base_y, int base_z, float sigma0, 
   pg.one = 1.0f;
   // frames in flight on any stream may still read the pyramid that is built over
   CVR_HIP_CHECK(hipDeviceSynchronize());
-  // level 0 takes the separable path where voxel spacing and sigma are commensurate on every axis
-  // (true of the default configurations), else the direct build
-  std::array<SepAxis, 3> a{};
-  bool sep = true;
+  // separable path per level: voxel spacing and sigma commensurate on every axis (true at
+  // every level of the default configurations; a level whose size was rounded down from
+  // an odd one may not be, and takes the direct build)
+  std::vector<std::array<SepAxis, 3>> sax(L);
+  std::vector<char> sep(L, 0);
   size_t tmp_floats = 0;
-  int tail = L;  // the first level of k_pyr_tail
-  for (int k = 0; k < 3 && sep; ++k) sep = sep_axis(double(g.G[k]) / double(pg.dims[0][k]), double(sigma0), pg.dims[0][k], a[k]);
-  if (sep) tmp_floats = size_t(a[0].len) * a[1].len * a[2].len + size_t(pg.dims[0][0]) * a[1].len * a[2].len;
-  for (int i = 1; i < L; ++i) {
-    const int* P = pg.dims[i - 1];
-    if (size_t(P[0]) * P[1] * P[2] <= size_t(kTailCells)) {
-      tail = i;
-      break;
-    }
-    tmp_floats = std::max(tmp_floats, size_t(pg.dims[i][0]) * (size_t(P[1]) + pg.dims[i][1]) * P[2]);
+  for (int i = 0; i < L; ++i) {
+    bool ok = true;
+    const double sig = double(sigma0) * std::pow(2.0, double(i));
+    for (int k = 0; k < 3 && ok; ++k) ok = sep_axis(double(g.G[k]) / double(pg.dims[i][k]), sig, pg.dims[i][k], sax[i][k]);
+    sep[i] = ok;
+    if (ok)
+      tmp_floats = std::max(tmp_floats, size_t(sax[i][0].len) * sax[i][1].len * sax[i][2].len +
+                                            size_t(pg.dims[i][0]) * sax[i][1].len * sax[i][2].len);
   }
   // opacities of every level, then the temporaries of the largest level's passes
   int rc = sized_buffer(reinterpret_cast<void**>(&c->d_pyr), &c->pyr_bytes, total * sizeof(float));
   if (!rc) rc = sized_buffer(&c->d_pyr_work, &c->pyr_work_bytes, (total + tmp_floats) * sizeof(float));
   if (rc == CVR_ERR_NOMEM && c->d_pyr) {
-    sep = false;  // no room for the temporaries: the direct build needs none
-    tmp_floats = 0;
+    std::fill(sep.begin(), sep.end(), 0);  // no room for the temporaries: the direct build needs none
     rc = sized_buffer(&c->d_pyr_work, &c->pyr_work_bytes, total * sizeof(float));
   }
   if (rc) {
@@ -421,66 +396,65 @@ int build_pyramid(cvr_ctx* c, int base_x, int base_y, int base_z, float sigma0, 
   }
   const float norm = float(1.0 / (gsum * gsum * gsum));
   const float3 G3 = make_float3(g.G[0], g.G[1], g.G[2]);
-  if (sep) {
+  for (int i = 0; i < L; ++i) {
+    if (!sep[i]) {
+      // direct build of this level (343 taps per voxel)
+      PyrBuild b{};
+      b.bx = pg.dims[i][0]; b.by = pg.dims[i][1]; b.bz = pg.dims[i][2];
+      for (int k = 0; k < 3; ++k) {
+        b.G[k] = g.G[k];
+        b.vs[k] = g.G[k] / float(pg.dims[i][k]);
+      }
+      b.sigma = sigma0 * float(std::pow(2.0, double(i)));
+      dim3 grid((b.bx + 7) / 8, (b.by + 7) / 8, (b.bz + 3) / 4);
+      if (i == 0) {
+        auto go = [&](auto t, auto l) {
+          constexpr bool kL = decltype(l)::value;
+          hipLaunchKernelGGL((k_pyr_level0<decltype(t), kL>), grid, dim3(256), kL ? size_t(c->tf_size) * sizeof(float) : 0,
+                             st, b, g, c->d_tf_rgba, c->tf_size, d_op);
+        };
+        auto by_table = [&](auto t) {
+          if (c->tf_size <= kTfLds) go(t, std::true_type{});
+          else go(t, std::false_type{});
+        };
+        if (c->dtype == CVR_U8) by_table(uint8_t{});
+        else by_table(uint16_t{});
+      } else {
+        b.px = pg.dims[i - 1][0]; b.py = pg.dims[i - 1][1]; b.pz = pg.dims[i - 1][2];
+        const size_t prev = size_t(b.px) * b.py * b.pz;
+        if (prev <= size_t(kPrevLds))
+          hipLaunchKernelGGL(k_pyr_next<true>, grid, dim3(256), prev * sizeof(float), st, b, d_op + pg.off[i - 1],
+                             d_op + pg.off[i]);
+        else
+          hipLaunchKernelGGL(k_pyr_next<false>, grid, dim3(256), 0, st, b, d_op + pg.off[i - 1], d_op + pg.off[i]);
+      }
+      CVR_HIP_CHECK(hipGetLastError());
+      continue;
+    }
+    const std::array<SepAxis, 3>& a = sax[i];
     float* lat = d_tmp;
     float* p1 = d_tmp + size_t(a[0].len) * a[1].len * a[2].len;
     const dim3 nb = cells_grid(a[0].len, a[1].len, a[2].len);
-    if (c->dtype == CVR_U8)
-      hipLaunchKernelGGL(k_pyr_lattice<uint8_t>, nb, dim3(256), 0, st, a[0], a[1], a[2], G3, g, c->d_tf_rgba, c->tf_size,
-                         lat);
-    else
-      hipLaunchKernelGGL(k_pyr_lattice<uint16_t>, nb, dim3(256), 0, st, a[0], a[1], a[2], G3, g, c->d_tf_rgba, c->tf_size,
-                         lat);
-    const int bx = pg.dims[0][0], by = pg.dims[0][1], bz = pg.dims[0][2];
+    if (i == 0) {
+      if (c->dtype == CVR_U8)
+        hipLaunchKernelGGL((k_pyr_lattice<uint8_t, true>), nb, dim3(256), 0, st, a[0], a[1], a[2], G3, g, c->d_tf_rgba,
+                           c->tf_size, nullptr, 0, 0, 0, lat);
+      else
+        hipLaunchKernelGGL((k_pyr_lattice<uint16_t, true>), nb, dim3(256), 0, st, a[0], a[1], a[2], G3, g, c->d_tf_rgba,
+                           c->tf_size, nullptr, 0, 0, 0, lat);
+    } else {
+      hipLaunchKernelGGL((k_pyr_lattice<uint8_t, false>), nb, dim3(256), 0, st, a[0], a[1], a[2], G3, g, nullptr, 0,
+                         d_op + pg.off[i - 1], pg.dims[i - 1][0], pg.dims[i - 1][1], pg.dims[i - 1][2], lat);
+    }
+    CVR_HIP_CHECK(hipGetLastError());
+    const int bx = pg.dims[i][0], by = pg.dims[i][1], bz = pg.dims[i][2];
     // x: lattice -> p1; y: p1 -> the lattice's space; z: -> the level, normalised
     hipLaunchKernelGGL(k_pyr_sep, cells_grid(bx, a[1].len, a[2].len), dim3(256), 0, st, lat, p1, a[0].len, a[1].len,
                        a[2].len, 0, a[0].m, a[0].q, bx, gw, 1.0f);
     hipLaunchKernelGGL(k_pyr_sep, cells_grid(bx, by, a[2].len), dim3(256), 0, st, p1, lat, bx, a[1].len, a[2].len, 1,
                        a[1].m, a[1].q, by, gw, 1.0f);
-    hipLaunchKernelGGL(k_pyr_sep, cells_grid(bx, by, bz), dim3(256), 0, st, lat, d_op, bx, by, a[2].len, 2, a[2].m, a[2].q,
-                       bz, gw, norm);
-    CVR_HIP_CHECK(hipGetLastError());
-  }
-  for (int i = sep ? 1 : 0; i < tail; ++i) {
-    PyrBuild b{};
-    b.bx = pg.dims[i][0]; b.by = pg.dims[i][1]; b.bz = pg.dims[i][2];
-    for (int k = 0; k < 3; ++k) {
-      b.G[k] = g.G[k];
-      b.vs[k] = g.G[k] / float(pg.dims[i][k]);
-    }
-    b.sigma = sigma0 * float(std::pow(2.0, double(i)));
-    const dim3 grid((b.bx + 7) / 8, (b.by + 7) / 8, (b.bz + 3) / 4);
-    if (i == 0) {
-      auto go = [&](auto t, auto l) {
-        constexpr bool kL = decltype(l)::value;
-        hipLaunchKernelGGL((k_pyr_level0<decltype(t), kL>), grid, dim3(256), kL ? size_t(c->tf_size) * sizeof(float) : 0, st,
-                           b, g, c->d_tf_rgba, c->tf_size, d_op);
-      };
-      auto by_table = [&](auto t) {
-        if (c->tf_size <= kTfLds) go(t, std::true_type{});
-        else go(t, std::false_type{});
-      };
-      if (c->dtype == CVR_U8) by_table(uint8_t{});
-      else by_table(uint16_t{});
-    } else if (tmp_floats) {
-      const int* P = pg.dims[i - 1];
-      float *p1 = d_tmp, *p2 = d_tmp + size_t(b.bx) * P[1] * P[2];
-      auto pass = [&](const float* in, float* out, int n0, int n1, int n2, int axis, float scale) {
-        const int bn = pg.dims[i][axis];
-        hipLaunchKernelGGL(k_pyr_axis, cells_grid(axis == 0 ? bn : n0, axis == 1 ? bn : n1, axis == 2 ? bn : n2), dim3(256),
-                           0, st, in, out, n0, n1, n2, axis, bn, b.vs[axis], b.G[axis], b.sigma, gw, scale);
-      };
-      pass(d_op + pg.off[i - 1], p1, P[0], P[1], P[2], 0, 1.0f);
-      pass(p1, p2, b.bx, P[1], P[2], 1, 1.0f);
-      pass(p2, d_op + pg.off[i], b.bx, b.by, P[2], 2, norm);
-    } else {
-      b.px = pg.dims[i - 1][0]; b.py = pg.dims[i - 1][1]; b.pz = pg.dims[i - 1][2];
-      hipLaunchKernelGGL(k_pyr_next, grid, dim3(256), 0, st, b, d_op + pg.off[i - 1], d_op + pg.off[i]);
-    }
-    CVR_HIP_CHECK(hipGetLastError());
-  }
-  if (tail < L) {
-    hipLaunchKernelGGL(k_pyr_tail, dim3(1), dim3(1024), 0, st, pg, tail, sigma0, d_op, gw, norm);
+    hipLaunchKernelGGL(k_pyr_sep, cells_grid(bx, by, bz), dim3(256), 0, st, lat, d_op + pg.off[i], bx, by, a[2].len, 2,
+                       a[2].m, a[2].q, bz, gw, norm);
     CVR_HIP_CHECK(hipGetLastError());
   }
   hipLaunchKernelGGL(k_pyr_tau, dim3(unsigned((total + 255) / 256)), dim3(256), 0, st, d_op, c->d_pyr, total);

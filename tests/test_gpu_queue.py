@@ -304,9 +304,8 @@ def test_summed_area_table_of_each_extinction_table(bits, entries, ext):
     assert np.abs(got - ref).max() <= 1e-6 * ref.max()
 
 
-# levels of at most 4096 voxels go to one workgroup: all but the first, from a level just under and just
-# over that size, none; flat and long grids; the direct and the separable build of level 0; a
-# transfer function too large for LDS.  The tolerance is that of the pyramid's own tests.
+# the direct and the separable build of each level, flat and long grids, and a transfer function too
+# large for LDS.  The tolerance is that of the pyramid's own tests.
 @pytest.mark.parametrize("base,sigma0,entries,bits", [((17, 16, 15), 1.0, 256, 8), ((17, 16, 16), 1.0, 256, 16),
                                                       ((32, 32, 32), 1.0, 256, 8), ((1, 1, 1), 1.0, 256, 8),
                                                       ((70, 5, 1), 0.7, 256, 16), ((40, 33, 9), 1.3, 9000, 16),
