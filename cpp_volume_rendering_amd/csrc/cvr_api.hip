@@ -142,7 +142,7 @@ static void defaults(int technique, void* p) {
     e->ks = 0.8f;  // renderingparameters.cpp:25-26
     e->shininess = 30.0f;
     e->specular[0] = e->specular[1] = e->specular[2] = 1.0f;  // lightsourcelist.cpp:24
-    e->sat_layout = 0;  // corner blocks: 53.2 ms against 61.0 ms at 256^3 @1024^2
+    e->sat_layout = 0;  // corner blocks: 15.7 ms against 20 ms at 256^3 @1024^2
   } else if (technique == CVR_CONE_GT) {
     // crtgtrenderer.cpp:32-51 (both lighting terms on here: with both off the shading
     // divides by zero)
@@ -293,7 +293,7 @@ int cvr_create(int technique, int device, cvr_handle* out) {
   defaults(CVR_DOS, &c->dos);
   defaults(CVR_CONE_TRACE, &c->cone);
   defaults(CVR_CONE_NN, &c->nn);
-  if (hipMalloc(&c->d_counters, 4 * sizeof(unsigned long long)) != hipSuccess ||
+  if (hipMalloc(&c->d_counters, kCountBytes) != hipSuccess ||
       hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {
     free_all(c);
     delete c;
@@ -588,7 +588,7 @@ static int grow_buffer(float** p, size_t* cap, size_t bytes, const char* who) {
 // with the stats and the event timing of the handle.
 static int render_device(cvr_ctx* h, const cvr_camera* cam, const cvr_light* light, int width, int height, float* dst,
                          hipStream_t st) {
-  if (h->collect_stats) CVR_HIP_CHECK(hipMemsetAsync(h->d_counters, 0, 4 * sizeof(unsigned long long), st));
+  if (h->collect_stats) CVR_HIP_CHECK(hipMemsetAsync(h->d_counters, 0, kCountBytes, st));
   RayFrame rf = frame_of(cam, width, height);
   CVR_HIP_CHECK(hipEventRecord(h->ev0, st));
   int rc;
@@ -609,9 +609,12 @@ static int render_device(cvr_ctx* h, const cvr_camera* cam, const cvr_light* lig
 // Reads the counters and the event time of the last render (waits for the stream).
 static int finish_stats(cvr_ctx* h, hipStream_t st) {
   if (!h->collect_stats) return CVR_OK;
-  unsigned long long cnt[4];
-  CVR_HIP_CHECK(hipMemcpyAsync(cnt, h->d_counters, sizeof(cnt), hipMemcpyDeviceToHost, st));
+  unsigned long long lines[kCountLines][kCountStride], cnt[4] = {0, 0, 0, 0};
+  static_assert(sizeof(lines) == kCountBytes, "one copy of the counters");
+  CVR_HIP_CHECK(hipMemcpyAsync(lines, h->d_counters, sizeof(lines), hipMemcpyDeviceToHost, st));
   CVR_HIP_CHECK(hipStreamSynchronize(st));
+  for (const auto& l : lines)
+    for (int i = 0; i < 4; ++i) cnt[i] += l[i];
   h->stats.samples = cnt[0];
   h->stats.shaded_samples = cnt[1];
   h->stats.fallback_samples = cnt[2];

@@ -22,6 +22,17 @@ void set_error(const std::string& msg);
 // caller passes a vanishing step size.
 constexpr int kMaxSamples = 1 << 21;
 
+// Sample counters of a frame (samples, shaded, exact fallbacks, box sums), kept kCountLines times,
+// each on a 128-byte line of its own, and summed on the host.  An addition to one line takes about
+// 12 ns and the next one waits for it: with one line for all wavefronts (an addition per wavefront
+// and counter) counting made the light-cache march of 1024^2 take 3.15 instead of 0.09 ms, with 64
+// lines 0.26; plain frame of 128^3 at 512^2 0.80 -> 0.07 ms, without counting 0.04.
+constexpr int kCountLines = 64, kCountStride = 16;
+constexpr size_t kCountBytes = size_t(kCountLines) * kCountStride * sizeof(unsigned long long);
+__device__ __forceinline__ void count_add(unsigned long long* counters, int which, unsigned int n) {
+  atomicAdd(&counters[(blockIdx.x % kCountLines) * kCountStride + which], (unsigned long long)n);
+}
+
 // --------------------------------------------------------------------------- camera
 // Per-frame ray set-up, computed on the host in double and rounded once.
 // dir(px,py) = normalize(a*s + b*u + f) is the expansion of

@@ -45,8 +45,8 @@ __global__ __launch_bounds__(256) void k_cone_render(RayFrame rf, VolGeom g, Pyr
                    return Lit{inv_k * (Io * ka + Is * kd), 0.f};
                  });
   if (counters) {
-    atomicAdd(&counters[0], (unsigned long long)nsamp);
-    atomicAdd(&counters[1], (unsigned long long)nshade);
+    count_add(counters, 0, nsamp);
+    count_add(counters, 1, nshade);
   }
 }
 

@@ -190,8 +190,8 @@ __global__ __launch_bounds__(256) void k_dos_render(RayFrame rf, VolGeom g, PyrG
                    return Lit{inv_k * (Io * ka + Is * kd * dd), Is * (K.apply_sdw ? ph.ks : 0.f) * sp};
                  });
   if (counters) {
-    atomicAdd(&counters[0], (unsigned long long)nsamp);
-    atomicAdd(&counters[1], (unsigned long long)nshade);
+    count_add(counters, 0, nsamp);
+    count_add(counters, 1, nshade);
   }
 }
 

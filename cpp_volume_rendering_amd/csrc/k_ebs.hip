@@ -431,9 +431,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
                    return Lit{inv_k * (Io * ka + Is * kd * dd), Is * ((k.apply_sdw ? ph.ks : 0.f) * sp)};
                  });
   if (counters) {
-    atomicAdd(&counters[0], (unsigned long long)nsamp);
-    atomicAdd(&counters[1], (unsigned long long)nshade);
-    atomicAdd(&counters[3], (unsigned long long)nbox);
+    count_add(counters, 0, nsamp);
+    count_add(counters, 1, nshade);
+    count_add(counters, 3, nbox);
   }
 }
 

@@ -79,8 +79,8 @@ __global__ __launch_bounds__(256) void k_lc_render(RayFrame rf, VolGeom g, LcK L
                                           ph.spec, list, out, nsamp, nshade, lit);
   }
   if (counters) {
-    atomicAdd(&counters[0], (unsigned long long)nsamp);
-    atomicAdd(&counters[1], (unsigned long long)nshade);
+    count_add(counters, 0, nsamp);
+    count_add(counters, 1, nshade);
   }
 }
 

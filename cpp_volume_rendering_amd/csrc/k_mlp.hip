@@ -630,10 +630,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   if (!kExact && marked && (threadIdx.x & 63) == 0) redo[bid] = 1u;
   if (counters) {
     if (!kExact) {
-      atomicAdd(&counters[0], (unsigned long long)cnt[0]);
-      atomicAdd(&counters[1], (unsigned long long)cnt[1]);
+      count_add(counters, 0, cnt[0]);
+      count_add(counters, 1, cnt[1]);
     } else {
-      atomicAdd(&counters[2], (unsigned long long)cnt[2]);
+      count_add(counters, 2, cnt[2]);
     }
   }
 }

@@ -56,8 +56,8 @@ __global__ __launch_bounds__(256) void k_rc1p(RayFrame rf, VolGeom g, const floa
                                             ph.spec, list, out, nsamp, nshade, lit);
   }
   if (counters) {
-    atomicAdd(&counters[0], (unsigned long long)nsamp);
-    atomicAdd(&counters[1], (unsigned long long)nshade);
+    count_add(counters, 0, nsamp);
+    count_add(counters, 1, nshade);
   }
 }
 

@@ -329,3 +329,20 @@ def test_pyramid_shapes(base, sigma0, entries, bits):
     for l in range(ref.levels):
         t = ref.level(l)
         assert g[l].shape == t.shape and (np.abs(g[l] - t) / np.maximum(1.0, np.abs(t))).max() <= 1e-4, l
+
+
+# The samples counted in a frame do not depend on how its rays are spread over workgroups: the shading
+# queue and the light-cache march count the same frame alike, again after another frame
+@pytest.mark.parametrize("w,h", [(1, 1), (97, 71), (640, 400)])
+@pytest.mark.parametrize("tech", [N.EBS, N.DOS])
+def test_counted_samples(tech, w, h):
+    counts = []
+    for cached in (0, 1):
+        wl, tf, r, p, img = scene(tech, 24, w, h, 0.3, light_cache=cached)
+        s = r.stats()
+        counts.append((s.samples, s.shaded_samples))
+        r.render(wl.camera(), 2 * w, h, light=wl.light())
+        r.render(wl.camera(), w, h, light=wl.light())
+        s = r.stats()
+        counts.append((s.samples, s.shaded_samples))
+    assert counts[0][0] > 0 and len(set(counts)) == 1, counts
