@@ -157,9 +157,14 @@ __device__ __forceinline__ float border_falloff(const PyrGeom& pg, f3 tp, float 
   const float cz = __builtin_amdgcn_fmed3f(tp.z, 0.f, pg.G[2]) - tp.z;
   return __builtin_amdgcn_exp2f((cx * cx + cy * cy + cz * cz) * fall);
 }
-// The distance along `axis` up to which p + axis t of every active lane is inside the box.
+// The distance along `axis` up to which p + axis t of every active lane is inside the box; below 0 where
+// some lane begins outside it (cvr_cone_eval takes any point; a march's samples may lie outside
+// by the rounding of their ray, which kEdge allows for: the falloff there is 1 to two ulps).
+constexpr float kEdge = 1.0f / 4096.0f;
 __device__ __forceinline__ float wave_exit(const PyrGeom& pg, f3 p, f3 axis) {
-  auto leave = [&](float a, float q, float G) { return ((a > 0.f ? G : 0.f) - q) / a; };
+  auto leave = [&](float a, float q, float G) {
+    return q >= -kEdge && q <= G + kEdge ? ((a > 0.f ? G : 0.f) - q) / a : -INFINITY;
+  };
   return wave_min(fminf(leave(axis.x, p.x, pg.G[0]), fminf(leave(axis.y, p.y, pg.G[1]), leave(axis.z, p.z, pg.G[2]))));
 }
 // The levels of a pyramid as the marches read them (kMaxLevels rows).

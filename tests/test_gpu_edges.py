@@ -1,0 +1,47 @@
+"""Calls at the edges of what the entry points accept, against the FP64 oracle."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from cpp_volume_rendering_amd import native as N
+from cpp_volume_rendering_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-3
+
+
+def handle(tech, wl, **params):
+    r = N.Renderer(tech)
+    r.set_volume(wl.volume, wl.scale)
+    r.set_transfer_function(wl.rgb_iso, wl.alpha_iso)
+    if params:
+        r.set_params(**params)
+    return r
+
+
+def check(img, ref, m, stride=1):
+    s = O.compare(img, ref, m, TOL, stride)
+    print(s)
+    assert s["max_abs"] <= TOL, s
+    assert s["n_over_tol"] <= 0.005 * s["n_pixels"] + 1, s
+
+
+# a point past each face, past an edge and past a corner, a point on a face and one inside, with cones that
+# lead into the box, along the face and away from it; one point a call and 64 of them, whose lanes all
+# begin outside.  The tolerance is that of the points inside.
+@pytest.mark.parametrize("copies", [1, 64])
+@pytest.mark.parametrize("pos", [(-6, 30, 30), (70, 30, 30), (30, -3, 31), (30, 66, 33), (30, 30, -9), (33, 30, 67.5),
+                                 (-4, -5, 30), (69, 68, 70), (0, 30, 30), (30, 64, 30), (20, 41, 30)])
+def test_cone_points_outside_the_box(pos, copies):
+    wl = W.cone_blobs(n=64, width=8, height=8)
+    r = handle(N.CONE_TRACE, wl)
+    pyr = O.OPyr.wrap(wl.grid, [a.astype(np.float64) for a in r.pyramid()])
+    inwards = np.array([32.0, 31.0, 33.0]) - pos
+    for light in (inwards, -inwards, np.array([0.3, 0.9, -0.2])):
+        light = light / np.linalg.norm(light)
+        at, d, li = (np.tile(v, (copies, 1)).astype(np.float32) for v in (np.array(pos, np.float64), -inwards, light))
+        occ, sdw, feat = r.cone_eval(at, d, li)
+        prm = O.cone_params(wl.grid, light_fwd=light)
+        ro, rs, rf = O.cone_points(pyr, prm, at, d)
+        for a, b in ((occ, ro), (sdw, rs), (feat, rf)):
+            assert np.abs(a - b).max() <= 2e-4
