@@ -273,7 +273,8 @@ __device__ __forceinline__ void queue_march(const RayFrame& rf, const VolGeom& g
           const float alpha = opaque ? 1.0f - __expf(-src.w * r.h) : 0.f;
           const float wb = opacity_before<kSub>(alpha, w), wa = opacity_after(alpha, wb);
           mine = (1.0f - wb) * alpha;
-          const uint64_t over = (__ballot(wa > et) >> base) & kGroupMask;
+          // (a transparent sample ends no ray, also where the threshold is below 0)
+          const uint64_t over = (__ballot(opaque && wa > et) >> base) & kGroupMask;
           const int last = over ? __builtin_ctzll(over) : kSub - 1;  // over: the ray ends with that sample
           w = kSub == 64 ? lane_value(wa, last) : __shfl(wa, base + last);
           taken = valid && sub <= last;
@@ -352,7 +353,7 @@ __device__ __forceinline__ void stage_tf_padded(float4* s_tf, const float4* __re
 // The march whose lighting costs less than the queue: lit(p) gives the factor of the colour of
 // the sample at p where it is met.  A lane adds up its own samples' colours and a group of 16 lanes
 // adds up its lanes' when its ray ends.  The first wavefront sets up the workgroup's rays, one per lane;
-// then all of them take rays from the list.
+// then all of them take rays from the list.  et is not below 0 (march_shape).
 constexpr int kListRays = 32;  // of a workgroup (64: 128^3 at 512^2 60 us, 50 with 32)
 template <int kRays> struct RayList {
   float4 tp[kRays];   // entry point (texture space), length
@@ -609,7 +610,7 @@ struct MarchShape {
 //   64^3 at 700 x 600                             1390          260          358
 constexpr float kLaneRays = 500.f, kLaneCacheRays = 2000.f, kLanePhongRays = 3500.f;
 constexpr size_t kLanePixels = 1 << 17;
-inline MarchShape march_shape(const RayFrame& rf, const VolGeom& g, float step, bool phong, float lane_rays) {
+inline MarchShape march_shape(const RayFrame& rf, const VolGeom& g, float step, float et, bool phong, float lane_rays) {
   MarchShape m;
   m.qs = queue_shape(rf, kListRays, 4, 512);
   m.blocks = m.qs.blocks;
@@ -617,7 +618,10 @@ inline MarchShape march_shape(const RayFrame& rf, const VolGeom& g, float step, 
   const size_t px = size_t(rf.W) * rf.H;
   const int hits = frame_hits(rf, g);
   const float steps = std::sqrt(g.G[0] * g.G[0] + g.G[1] * g.G[1] + g.G[2] * g.G[2]) / step;
-  if ((hits == 64 && px >= kLanePixels) || float(px) * float(hits) / 64.f >= steps * (phong ? kLanePhongRays : lane_rays)) {
+  // plain_march ends a ray by the opacity before a sample, lane_march with an opaque one: the same but
+  // where the threshold is below 0
+  if (et < 0.f || (hits == 64 && px >= kLanePixels) ||
+      float(px) * float(hits) / 64.f >= steps * (phong ? kLanePhongRays : lane_rays)) {
     m.mode += kLanes;
     m.blocks = ((rf.W + 15) / 16) * ((rf.H + 15) / 16);
   }

@@ -115,7 +115,7 @@ int launch_lc_render(cvr_ctx* c, const RayFrame& rf, int apply_occ, int apply_sd
   L.ka = apply_occ ? ka : 0.f;
   L.kd = apply_sdw ? kd : 0.f;
   L.ks = apply_sdw ? ph.ks : 0.f;
-  const MarchShape ms = march_shape(rf, g, step, ph.on, kLaneCacheRays);
+  const MarchShape ms = march_shape(rf, g, step, et, ph.on, kLaneCacheRays);
   const size_t shm = size_t(c->tf_size + 2) * sizeof(float4);
   if (c->tf_size > 4096) {
     set_error("cvr_render: light-cache march: transfer function larger than 4096 entries (staged in LDS)");

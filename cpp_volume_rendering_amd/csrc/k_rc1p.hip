@@ -93,7 +93,7 @@ int launch_rc1p(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* o
   const float4* gr = ph.on ? c->d_grad : nullptr;
   bool lds = c->tf_size <= 4096;
   size_t shm = lds ? size_t(c->tf_size + 2) * sizeof(float4) : 0;
-  const MarchShape ms = march_shape(rf, g, step, ph.on, kLaneRays);
+  const MarchShape ms = march_shape(rf, g, step, et, ph.on, kLaneRays);
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   float4* o4 = reinterpret_cast<float4*>(out);
   auto launch = [&](auto t, auto l, auto m) {

@@ -45,3 +45,43 @@ def test_cone_points_outside_the_box(pos, copies):
         ro, rs, rf = O.cone_points(pyr, prm, at, d)
         for a, b in ((occ, ro), (sdw, rs), (feat, rf)):
             assert np.abs(a - b).max() <= 2e-4
+
+
+# a threshold below 0 ends a ray with its first opaque sample, whatever came before it
+@pytest.mark.parametrize("et", [-1.0, 0.0])
+@pytest.mark.parametrize("tech,cached", [(N.EBS, 0), (N.EBS, 1), (N.CONE_TRACE, 0), (N.CONE_NN, 0)])
+def test_threshold_not_above_zero(tech, cached, et):
+    wl = W.cone_blobs(n=64, width=48, height=37, seed=15)
+    wl.rgb_iso, wl.alpha_iso = W.seeded_tf(131, 4)
+    wl.alpha_iso[1, 0] = 0.0  # rays of more than 64 transparent samples before the first opaque one
+    r, cam, light = handle(tech, wl), wl.camera(), wl.light()
+    p = r.params()
+    if tech == N.CONE_NN:
+        p.cone.et_threshold = et
+        wts = np.random.default_rng(3).normal(0, 0.1, N.lib().cvr_nn_param_count()).astype(np.float32)
+        r.nn_set_weights(wts)
+    else:
+        p.et_threshold = et
+        if tech == N.EBS:
+            p.light_cache = cached
+    r.set_params(p)
+    if tech == N.CONE_NN:
+        r.nn_set_weights(wts)
+    img = r.render(cam, 48, 37, light=light)
+    tf = O.OTF(wl.rgb_iso, wl.alpha_iso)
+    if tech == N.EBS and cached:
+        ref, m = O.render_lc(wl.volume, tf, r.light_cache(), 1, 1, p.ka, p.kd, cam, 48, 37, et=et, scale=wl.scale)
+    elif tech == N.EBS:
+        prm = O.ebs_params(p, light)
+        prm.sdw_max_dist = np.float32(0.75) * np.float32(np.linalg.norm(wl.grid))
+        ref, m = O.render_ebs(wl.volume, tf, O.sat(wl.volume, tf), prm, cam, 48, 37, et=et)
+    else:
+        pyr = O.OPyr.wrap(wl.grid, [a.astype(np.float64) for a in r.pyramid()])
+        prm = O.cone_params(wl.grid, light)
+        if tech == N.CONE_TRACE:
+            ref, m = O.render_cone(wl.volume, tf, pyr, prm, cam, 48, 37, et=et)
+        else:
+            ref, m, _ = O.render_nn(wl.volume, tf, pyr, prm, wts, cam, 48, 37, et=et)
+    assert 0 < ref[..., 3].max() < 0.5
+    # the margin is the oracle's distance of an opacity from the threshold: none is near one below 0
+    check(img, ref, m if et > 0 else None)
