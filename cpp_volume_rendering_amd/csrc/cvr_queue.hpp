@@ -125,33 +125,44 @@ __device__ __forceinline__ int even_bits(int v) {
 }
 // Pixels of the image in square tiles of 1 << tile_log2 pixels (at most 64), row-major, each in
 // Z order.
-inline int tiled_pixels(const RayFrame& rf, int tile_log2) {
-  const int m = 1 << tile_log2;
-  return ((rf.W + m - 1) / m) * ((rf.H + m - 1) / m) * m * m;
+__host__ __device__ inline long long tiled_pixels(int w, int h, int tile_log2) {
+  const long long m = 1 << tile_log2;
+  return ((w + m - 1) / m) * ((h + m - 1) / m) * m * m;
 }
 
 // How a frame's rays are dealt out: `rays` per unit (a wavefront, or a workgroup whose four
 // wavefronts share them: parts 4), the tile whose pixels the units take in turn, workgroups,
-// and runs of 1 << xcd_log2 workgroups per XCD (xcd_remap).
+// and runs of 1 << xcd_log2 workgroups per XCD (xcd_remap).  first: the launch's first workgroup of
+// them (for_launches).
 struct QueueShape {
-  int rays, parts, tile_log2, blocks, xcd_log2;
+  int rays, tile_log2, blocks, xcd_log2, first;
 };
 // Tiles of 64 x 64 pixels: a unit's rays lie 32 (rays 4) or 16 (rays 16) pixels apart, so long
 // and short ones mix, while the units that run at once stay together (256^3 cone-traced frame
 // at 512^2: 18.7 ms, 23.7 ms in 16 x 16 tiles; EBS 5.0 and 6.6 ms; DOS 4.5 and 6.0 ms).
 // Narrower frames take smaller tiles, of a unit's rays at least.  xcd_px: pixels an XCD takes in a row.
-inline QueueShape queue_shape(const RayFrame& rf, int rays, int parts, int xcd_px, int waves = 4) {
-  const int side = rf.W < rf.H ? rf.W : rf.H;
-  QueueShape q{rays, parts, 2, 0, 0};
+inline QueueShape queue_shape(int w, int h, int rays, int parts, int xcd_px, int waves = 4) {
+  const int side = w < h ? w : h;
+  QueueShape q{rays, 2, 0, 0, 0};
   while (q.tile_log2 < 6 && (1 << q.tile_log2 < side || 1 << (2 * q.tile_log2) < rays)) ++q.tile_log2;
   const int per_wg = rays * waves / parts;  // pixels of a workgroup
-  q.blocks = (tiled_pixels(rf, q.tile_log2) + per_wg - 1) / per_wg;
+  q.blocks = int((tiled_pixels(w, h, q.tile_log2) + per_wg - 1) / per_wg);
   while (per_wg << q.xcd_log2 < xcd_px) ++q.xcd_log2;
   return q;
 }
+// A launch may have fewer than 2^32 lanes, and a frame of 2^28 pixels takes up to 2^36 (64 a pixel where
+// four wavefronts share four rays): launch(shape, workgroups) for each run of at most 2^31 lanes.
+template <class F> inline void for_launches(QueueShape q, int total, int threads, F&& launch) {
+  const int most = int((1ll << 31) / threads);
+  for (q.first = 0;; q.first += most) {
+    const int left = total - q.first;
+    launch(q, left < most ? left : most);
+    if (left <= most) break;
+  }
+}
 // The unit of this wavefront.
-template <int kParts> __device__ __forceinline__ int queue_unit(int xcd_log2) {
-  const int waves = int(blockDim.x) >> 6, bid = xcd_remap(blockIdx.x, gridDim.x, xcd_log2);
+template <int kParts> __device__ __forceinline__ int queue_unit(const QueueShape& q) {
+  const int waves = int(blockDim.x) >> 6, bid = q.first + xcd_remap(blockIdx.x, gridDim.x, q.xcd_log2);
   return kParts > 1 ? bid : bid * waves + int(threadIdx.x >> 6);
 }
 
@@ -552,11 +563,12 @@ __device__ __forceinline__ void lane_march(const RayFrame& rf, const VolGeom& g,
   }
   out[py * rf.W + px] = dst;
 }
-// Pixel of this lane in workgroups of 16 x 16 pixels, a wavefront 8 x 8 of them.
-__device__ __forceinline__ void lane_pixel(const RayFrame& rf, int& px, int& py) {
+// Pixel of this lane in workgroups of 16 x 16 pixels (`first`: the launch's first), a wavefront 8 x 8 of
+// them.
+__device__ __forceinline__ void lane_pixel(const RayFrame& rf, int first, int& px, int& py) {
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   int tx, ty;
-  super_tile(xcd_remap(blockIdx.x, gridDim.x), (rf.W + 15) >> 4, (rf.H + 15) >> 4, 16, 32, tx, ty);
+  super_tile(first + xcd_remap(blockIdx.x, gridDim.x), (rf.W + 15) >> 4, (rf.H + 15) >> 4, 16, 32, tx, ty);
   px = tx * 16 + (w & 1) * 8 + (lane & 7);
   py = ty * 16 + (w >> 1) * 8 + (lane >> 3);
 }
@@ -612,7 +624,7 @@ constexpr float kLaneRays = 500.f, kLaneCacheRays = 2000.f, kLanePhongRays = 350
 constexpr size_t kLanePixels = 1 << 17;
 inline MarchShape march_shape(const RayFrame& rf, const VolGeom& g, float step, float et, bool phong, float lane_rays) {
   MarchShape m;
-  m.qs = queue_shape(rf, kListRays, 4, 512);
+  m.qs = queue_shape(rf.W, rf.H, kListRays, 4, 512);
   m.blocks = m.qs.blocks;
   m.mode = phong ? kPhong : kGroups;
   const size_t px = size_t(rf.W) * rf.H;

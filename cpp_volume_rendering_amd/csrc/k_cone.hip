@@ -32,7 +32,7 @@ __global__ __launch_bounds__(256) void k_cone_render(RayFrame rf, VolGeom g, Pyr
   __shared__ WaveQueue<kRays> queue[4];
   for (int i = threadIdx.x; i < ntf; i += blockDim.x) s_tf[i] = tf[i];
   __syncthreads();
-  const int u = queue_unit<kParts>(qs.xcd_log2);
+  const int u = queue_unit<kParts>(qs);
   unsigned int nsamp = 0, nshade = 0;
   const float ka = K.apply_occ ? K.ka : 0.f, kd = K.apply_sdw ? K.kd : 0.f;
   const float inv_k = 1.0f / (ka + kd);
@@ -280,12 +280,14 @@ int launch_cone(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* o
   // small frames: workgroups whose wavefronts share their rays (128^2 1.9 ms, 3.4 ms with rays
   // of their own; 512^2 18.7 and 19.9; 1024^2 70.4 and 68.6)
   const bool shared = size_t(rf.W) * rf.H < (1 << 19);
-  const QueueShape qs = queue_shape(rf, kRays, shared ? 4 : 1, shared ? 64 : 256);
+  const QueueShape shape = queue_shape(rf.W, rf.H, kRays, shared ? 4 : 1, shared ? 64 : 256);
   with_types(c->dtype, c->pyr.fmt, [&](auto t, auto f) {
     using T = typename decltype(t)::type;
     auto launch = [&](auto parts) {
-      hipLaunchKernelGGL((k_cone_render<T, decltype(f)::value, decltype(parts)::value>), dim3(qs.blocks), dim3(256), shm,
-                         st, rf, g, c->pyr, c->d_pyr_oct, K, c->d_tf_rgbt, c->tf_size, step, P.et_threshold, qs, o4, cnt);
+      for_launches(shape, shape.blocks, 256, [&](const QueueShape& qs, int blocks) {
+        hipLaunchKernelGGL((k_cone_render<T, decltype(f)::value, decltype(parts)::value>), dim3(blocks), dim3(256), shm,
+                           st, rf, g, c->pyr, c->d_pyr_oct, K, c->d_tf_rgbt, c->tf_size, step, P.et_threshold, qs, o4, cnt);
+      });
     };
     if (shared) launch(std::integral_constant<int, 4>{});
     else launch(std::integral_constant<int, 1>{});

@@ -170,7 +170,7 @@ __global__ __launch_bounds__(256) void k_dos_render(RayFrame rf, VolGeom g, PyrG
   __shared__ WaveQueue<kRays> queue[4];
   for (int i = threadIdx.x; i < ntf; i += blockDim.x) s_tf[i] = tf[i];
   __syncthreads();
-  const int u = queue_unit<kParts>(qs.xcd_log2);
+  const int u = queue_unit<kParts>(qs);
   const f3 eye = ld3(rf.eye);
   const f3 half = mk3(0.5f * g.G[0], 0.5f * g.G[1], 0.5f * g.G[2]);
   unsigned int nsamp = 0, nshade = 0;
@@ -494,13 +494,15 @@ int launch_dos(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* ou
   // dos_cone: 100 x 100 0.41 ms, 0.82 ms with rays of their own; 200 x 150 0.26 and 0.48; 400 x 300 2.2
   // and 1.7; 1024^2 19.4 and 15.6)
   const bool shared = size_t(rf.W) * rf.H < (1 << 16);
-  const QueueShape qs = queue_shape(rf, kRays, shared ? 4 : 1, shared ? 64 : 256);
+  const QueueShape shape = queue_shape(rf.W, rf.H, kRays, shared ? 4 : 1, shared ? 64 : 256);
   with_types(c->dtype, c->pyr.fmt, [&](auto t, auto f) {
     using T = typename decltype(t)::type;
     auto launch = [&](auto parts) {
-      hipLaunchKernelGGL((k_dos_render<T, decltype(f)::value, decltype(parts)::value>), dim3(qs.blocks), dim3(256), shm, st,
-                         rf, g, c->pyr, c->d_pyr_oct, K, c->d_tf_rgbt, c->tf_size, step, P.et_threshold, ph, c->d_grad, qs,
-                         o4, cnt);
+      for_launches(shape, shape.blocks, 256, [&](const QueueShape& qs, int blocks) {
+        hipLaunchKernelGGL((k_dos_render<T, decltype(f)::value, decltype(parts)::value>), dim3(blocks), dim3(256), shm, st,
+                           rf, g, c->pyr, c->d_pyr_oct, K, c->d_tf_rgbt, c->tf_size, step, P.et_threshold, ph, c->d_grad,
+                           qs, o4, cnt);
+      });
     };
     if (shared) launch(std::integral_constant<int, 4>{});
     else launch(std::integral_constant<int, 1>{});

@@ -408,7 +408,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   for (int i = threadIdx.x; i < ntf; i += blockDim.x) s_tf[i] = tf[i];
   ebs_load_rows(rows, k.nrows, s_rows);
   const int nrows = k.nrows;
-  const int u = queue_unit<kParts>(qs.xcd_log2);
+  const int u = queue_unit<kParts>(qs);
   const f3 eye = ld3(rf.eye);
   unsigned int nsamp = 0, nshade = 0, nbox = 0;
   const float ka = k.apply_occ ? k.ka : 0.f, kd = k.apply_sdw ? k.kd : 0.f;
@@ -682,15 +682,17 @@ int launch_ebs(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* ou
   // small frames: workgroups whose wavefronts share their rays (100 x 100 0.51 ms, 1.0 ms with
   // rays of their own; 400 x 300, point light 3.6 and 4.3; 512^2 5.3 and 5.0; 1024^2 19.4 and 16.0)
   const bool shared = waves == 4 && size_t(rf.W) * rf.H < 200000;
-  const QueueShape qs = queue_shape(rf, kRays, shared ? 4 : 1, shared ? 64 : 256, waves);
+  const QueueShape shape = queue_shape(rf.W, rf.H, kRays, shared ? 4 : 1, shared ? 64 : 256, waves);
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   const void* sat = P.sat_layout == 1 ? static_cast<const void*>(c->d_sat) : c->d_sat_oct;
   const ShadowRow* rows = static_cast<const ShadowRow*>(c->d_ebs_rows);
   float4* o4 = reinterpret_cast<float4*>(out);
   auto launch = [&](auto t, auto l, auto pt, auto parts) {
-    hipLaunchKernelGGL((k_ebs<typename decltype(t)::type, decltype(l)::value, decltype(pt)::value, decltype(parts)::value>), dim3(qs.blocks),
-                       dim3(64 * waves), shm, st, rf, k, c->d_tf_rgbt, c->tf_size, sat, rows, step, P.et_threshold, ph,
-                       c->d_grad, qs, o4, cnt);
+    for_launches(shape, shape.blocks, 64 * waves, [&](const QueueShape& qs, int blocks) {
+      hipLaunchKernelGGL((k_ebs<typename decltype(t)::type, decltype(l)::value, decltype(pt)::value, decltype(parts)::value>),
+                         dim3(blocks), dim3(64 * waves), shm, st, rf, k, c->d_tf_rgbt, c->tf_size, sat, rows, step,
+                         P.et_threshold, ph, c->d_grad, qs, o4, cnt);
+    });
   };
   auto by_light = [&](auto t, auto l) {
     auto by_size = [&](auto pt) {

@@ -103,7 +103,7 @@ __global__ __launch_bounds__(256) void k_gt_render(RayFrame rf, VolGeom g, GtK K
   for (int i = threadIdx.x; i < ntf; i += blockDim.x) s_tf[i] = tf[i];
   for (int i = threadIdx.x; i <= ntf; i += blockDim.x) s_ext[i] = make_float2(tf[max(i - 1, 0)].w, tf[min(i, ntf - 1)].w);
   __syncthreads();
-  const int u = queue_unit<4>(qs.xcd_log2);
+  const int u = queue_unit<4>(qs);
   unsigned int nsamp = 0, nshade = 0;
   const float ka = K.apply_occ ? K.ka : 0.f, kd = K.apply_sdw ? K.kd : 0.f;
   const float inv_k = 1.0f / (ka + kd);
@@ -235,15 +235,17 @@ int launch_gt(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out
   // workgroups whose wavefronts share their rays: a batch is tens to thousands of light-ray
   // steps (128^3 at 256^2 with 16 + 4 rays 5.7 ms, 13.7 ms with rays of their own; 256^3 at 512^2
   // with 4 + 1 11.5 and 12.2)
-  const QueueShape qs = queue_shape(rf, kRays, 4, 64);
+  const QueueShape shape = queue_shape(rf.W, rf.H, kRays, 4, 64);
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   float4* o4 = reinterpret_cast<float4*>(out);
-  if (c->dtype == CVR_U8)
-    hipLaunchKernelGGL(k_gt_render<uint8_t>, dim3(qs.blocks), dim3(256), shm, st, rf, g, K, c->d_tf_rgbt, c->tf_size,
-                       step, P.et_threshold, qs, o4, cnt);
-  else
-    hipLaunchKernelGGL(k_gt_render<uint16_t>, dim3(qs.blocks), dim3(256), shm, st, rf, g, K, c->d_tf_rgbt, c->tf_size,
-                       step, P.et_threshold, qs, o4, cnt);
+  for_launches(shape, shape.blocks, 256, [&](const QueueShape& qs, int blocks) {
+    if (c->dtype == CVR_U8)
+      hipLaunchKernelGGL(k_gt_render<uint8_t>, dim3(blocks), dim3(256), shm, st, rf, g, K, c->d_tf_rgbt, c->tf_size, step,
+                         P.et_threshold, qs, o4, cnt);
+    else
+      hipLaunchKernelGGL(k_gt_render<uint16_t>, dim3(blocks), dim3(256), shm, st, rf, g, K, c->d_tf_rgbt, c->tf_size, step,
+                         P.et_threshold, qs, o4, cnt);
+  });
   CVR_HIP_CHECK(hipGetLastError());
   return CVR_OK;
 }

@@ -72,10 +72,10 @@ __global__ __launch_bounds__(256) void k_lc_render(RayFrame rf, VolGeom g, LcK L
   };
   if constexpr ((kMode & kLanes) != 0) {
     int px, py;
-    lane_pixel(rf, px, py);
+    lane_pixel(rf, qs.first, px, py);
     lane_march<T, true, (kMode & kPhong) != 0>(rf, g, s_tf, ntf, step, et, px, py, ph.spec, out, nsamp, nshade, lit);
   } else {
-    plain_march<T, true, (kMode & kPhong) != 0>(rf, g, s_tf, ntf, step, et, FramePixels(rf, qs, queue_unit<4>(qs.xcd_log2), 4),
+    plain_march<T, true, (kMode & kPhong) != 0>(rf, g, s_tf, ntf, step, et, FramePixels(rf, qs, queue_unit<4>(qs), 4),
                                           ph.spec, list, out, nsamp, nshade, lit);
   }
   if (counters) {
@@ -125,8 +125,10 @@ int launch_lc_render(cvr_ctx* c, const RayFrame& rf, int apply_occ, int apply_sd
   auto by_mode = [&](auto t) {
     using T = typename decltype(t)::type;
     with_mode(ms.mode, [&](auto m) {
-      hipLaunchKernelGGL((k_lc_render<T, decltype(m)::value>), dim3(ms.blocks), dim3(256), shm, st, rf, g, L, c->d_lc,
-                         c->d_tf_rgbt, c->tf_size, step, et, ph, c->d_grad, ms.qs, reinterpret_cast<float4*>(out), cnt);
+      for_launches(ms.qs, ms.blocks, 256, [&](const QueueShape& qs, int blocks) {
+        hipLaunchKernelGGL((k_lc_render<T, decltype(m)::value>), dim3(blocks), dim3(256), shm, st, rf, g, L, c->d_lc,
+                           c->d_tf_rgbt, c->tf_size, step, et, ph, c->d_grad, qs, reinterpret_cast<float4*>(out), cnt);
+      });
     });
   };
   if (c->dtype == CVR_U8) by_mode(LcVox<uint8_t>{});

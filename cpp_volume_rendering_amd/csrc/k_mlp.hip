@@ -909,7 +909,7 @@ NnK nn_consts(cvr_ctx* c) {
 // fit cvr_render_noalloc's array.
 constexpr int kMaxBlocks = 1 << 16;
 static QueueShape nn_shape(const RayFrame& rf, int& sets) {
-  QueueShape q = queue_shape(rf, size_t(rf.W) * rf.H < (1 << 16) ? 4 : 16, 1, 64);
+  QueueShape q = queue_shape(rf.W, rf.H, size_t(rf.W) * rf.H < (1 << 16) ? 4 : 16, 1, 64);
   sets = (q.blocks + kMaxBlocks - 1) / kMaxBlocks;
   q.blocks = (q.blocks + sets - 1) / sets;
   return q;

@@ -49,10 +49,10 @@ __global__ __launch_bounds__(256) void k_rc1p(RayFrame rf, VolGeom g, const floa
   };
   if constexpr ((kMode & kLanes) != 0) {
     int px, py;
-    lane_pixel(rf, px, py);
+    lane_pixel(rf, qs.first, px, py);
     lane_march<T, TF_LDS, (kMode & kPhong) != 0>(rf, g, tfp, ntf, step, et, px, py, ph.spec, out, nsamp, nshade, lit);
   } else {
-    plain_march<T, TF_LDS, (kMode & kPhong) != 0>(rf, g, tfp, ntf, step, et, FramePixels(rf, qs, queue_unit<4>(qs.xcd_log2), 4),
+    plain_march<T, TF_LDS, (kMode & kPhong) != 0>(rf, g, tfp, ntf, step, et, FramePixels(rf, qs, queue_unit<4>(qs), 4),
                                             ph.spec, list, out, nsamp, nshade, lit);
   }
   if (counters) {
@@ -99,8 +99,10 @@ int launch_rc1p(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* o
   auto launch = [&](auto t, auto l, auto m) {
     using T = typename decltype(t)::type;
     constexpr bool L = decltype(l)::value;
-    hipLaunchKernelGGL((k_rc1p<T, L, decltype(m)::value>), dim3(ms.blocks), dim3(256), L ? shm : 0, st, rf, g,
-                       c->d_tf_rgbt, c->tf_size, step, et, ph, gr, P.ka, P.kd, ms.qs, o4, cnt);
+    for_launches(ms.qs, ms.blocks, 256, [&](const QueueShape& qs, int blocks) {
+      hipLaunchKernelGGL((k_rc1p<T, L, decltype(m)::value>), dim3(blocks), dim3(256), L ? shm : 0, st, rf, g,
+                         c->d_tf_rgbt, c->tf_size, step, et, ph, gr, P.ka, P.kd, qs, o4, cnt);
+    });
   };
   auto by_mode = [&](auto t, auto l) {
     with_mode(ms.mode, [&](auto m) { launch(t, l, m); });

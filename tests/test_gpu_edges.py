@@ -85,3 +85,23 @@ def test_threshold_not_above_zero(tech, cached, et):
     assert 0 < ref[..., 3].max() < 0.5
     # the margin is the oracle's distance of an opacity from the threshold: none is near one below 0
     check(img, ref, m if et > 0 else None)
+
+
+def test_frame_of_more_lanes_than_a_launch_may_have():
+    """8192 x 8192 pixels of the ground truth, 64 lanes a pixel, in two launches: rows on both sides of
+    where the second begins, against the oracle."""
+    import torch
+
+    w = h = 8192
+    wl = W.cone_blobs(n=24, width=w, height=h, seed=31)
+    r = handle(N.CONE_GT, wl, occ_rays=2, sdw_rays=1, shadow_type=2)
+    out = torch.full((h, w, 4), -1.0, device="cuda:0")
+    r.render(wl.camera(), w, h, light=wl.light(), out=out)
+    torch.cuda.synchronize()
+    assert float(out.min()) >= 0.0  # every pixel written
+    tf = O.OTF(wl.rgb_iso, wl.alpha_iso)
+    ref, m = O.render_gt(wl.volume, tf, O.gt_params(r.params(), wl.grid, wl.light()), wl.camera(), w, h, stride=64)
+    img = np.zeros((h, w, 4), np.float32)
+    img[::64, ::64] = out[::64, ::64].cpu().numpy()
+    assert ref[:h // 2, ..., 3].max() > 0.2 and ref[h // 2:, ..., 3].max() > 0.2
+    check(img, ref, m, 64)

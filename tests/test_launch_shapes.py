@@ -1,0 +1,51 @@
+"""How frames are dealt out to launches, computed on the host (CPU only: the host half of the kernels'
+header in a small program of its own)."""
+import subprocess
+
+import pytest
+
+from cpp_volume_rendering_amd import build as B
+
+SOURCE = r"""
+#include "cvr_queue.hpp"
+#include <cstdio>
+#include <cstdlib>
+using namespace cvr;
+int main(int, char** v) {
+  const int w = std::atoi(v[1]), h = std::atoi(v[2]), rays = std::atoi(v[3]), parts = std::atoi(v[4]);
+  const QueueShape q = queue_shape(w, h, rays, parts, 64);
+  std::printf("%d %d\n", q.tile_log2, q.blocks);
+  for_launches(q, q.blocks, 256, [&](const QueueShape& s, int blocks) { std::printf("%d %d\n", s.first, blocks); });
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def shapes(tmp_path_factory):
+    d = tmp_path_factory.mktemp("shapes")
+    (d / "shapes.hip").write_text(SOURCE)
+    subprocess.run([B.HIPCC, "-O1", "-std=c++17", f"-I{B.INCLUDE}", f"-I{B.CSRC}", "-x", "hip", "--offload-host-only",
+                    f"--offload-arch={B.ARCH}", str(d / "shapes.hip"), "-o", str(d / "shapes")], check=True,
+                   capture_output=True)
+
+    def run(*args):
+        out = subprocess.run([str(d / "shapes"), *map(str, args)], check=True, capture_output=True, text=True).stdout
+        return [tuple(map(int, line.split())) for line in out.splitlines()]
+
+    return run
+
+
+# ground truth (4 rays, shared), cone tracer and DOS (4, own), EBS (16, own), marches (32, shared)
+@pytest.mark.parametrize("rays,parts", [(4, 4), (4, 1), (16, 1), (32, 4)])
+@pytest.mark.parametrize("w,h", [(1, 1), (333, 64), (1024, 1024), (8191, 8190), (8192, 8192), (16384, 16384), (1 << 28, 1),
+                                 (1, 1 << 28), (65537, 4095)])
+def test_launches_cover_a_frame_within_the_limit_of_lanes(shapes, w, h, rays, parts):
+    (log2, blocks), *launches = shapes(w, h, rays, parts)
+    m, per_wg = 1 << log2, rays * 4 // parts
+    pixels = -(-w // m) * -(-h // m) * m * m
+    assert blocks == -(-pixels // per_wg) and m * m >= rays
+    at = 0
+    for first, n in launches:
+        assert first == at and 0 < n and n * 256 < 1 << 32
+        at += n
+    assert at == blocks
