@@ -405,6 +405,8 @@ int cvr_set_transfer_function(cvr_handle h, int max_density, int extinction_inpu
     rgba[i] = make_float4(r, g, b, opc);
   }
   DeviceGuard dg(h->device);
+  // frames in flight on any stream may still read the tables
+  CVR_HIP_CHECK(hipDeviceSynchronize());
   if (h->tf_size != T) {
     if (h->d_tf_rgbt) CVR_HIP_CHECK(hipFree(h->d_tf_rgbt));
     h->d_tf_rgbt = h->d_tf_rgba = nullptr;
@@ -873,6 +875,7 @@ int cvr_nn_set_weights(cvr_handle h, const float* in, size_t count) {
   DeviceGuard dg(h->device);
   rc = nn_alloc(h);
   if (rc) return rc;
+  CVR_HIP_CHECK(hipDeviceSynchronize());  // frames in flight may still read the packed weights
   CVR_HIP_CHECK(hipMemcpy(h->d_nn_w, in, count * 4, hipMemcpyHostToDevice));
   rc = nn_pack(h, nullptr);
   if (rc) return rc;
@@ -1006,6 +1009,7 @@ int cvr_nn_load(cvr_handle h, const void* in, size_t bytes) {
   DeviceGuard dg(h->device);
   rc = nn_alloc(h);
   if (rc) return rc;
+  CVR_HIP_CHECK(hipDeviceSynchronize());  // as cvr_nn_set_weights
   for (float* d : {h->d_nn_w, h->d_nn_m, h->d_nn_v}) {
     CVR_HIP_CHECK(hipMemcpy(d, p, size_t(np) * 4, hipMemcpyHostToDevice));
     p += size_t(np) * 4;

@@ -58,7 +58,9 @@ __global__ __launch_bounds__(256) void k_gradient(const T* __restrict__ vox, int
 int build_gradient(cvr_ctx* c, int type, hipStream_t st) {
   const uint64_t key = (c->vol_version << 8) | uint64_t(type);
   if (c->d_grad && c->grad_built_for == key) return 0;
-  if (!c->d_grad) {
+  if (c->d_grad) {
+    CVR_HIP_CHECK(hipDeviceSynchronize());  // frames in flight on any stream may still read it
+  } else {
     const size_t cells = brick_cells(c->nx, c->ny, c->nz);
     if (hipMalloc(&c->d_grad, cells * sizeof(float4)) != hipSuccess) {
       c->d_grad = nullptr;

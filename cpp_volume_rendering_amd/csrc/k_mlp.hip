@@ -796,6 +796,12 @@ int nn_train(cvr_ctx* c, hipStream_t st) {
     set_error("surrogate: out of device memory for the training set");
     return -5;
   }
+  // frames in flight on other streams may still read the packed weights that the steps rewrite
+  if (hipDeviceSynchronize() != hipSuccess) {
+    cleanup();
+    set_error("surrogate: waiting for the device before training failed");
+    return CVR_ERR_HIP;
+  }
   rc = nn_generate(c, N.cone, N.seed, n, d_X, d_T, nullptr, st);
   if (!rc) rc = nn_generate(c, N.cone, N.seed ^ 0x5851F42D4C957F2Dull, nv, d_Xv, d_Tv, nullptr, st);
   if (rc) { cleanup(); return rc; }

@@ -7,7 +7,9 @@
  * is success, negative values are errors (cvr_last_error() has the message).
  * The ABI never exits the process.  A handle is not thread-safe: use one
  * handle per host thread.  Inputs are copied; caller buffers stay the
- * caller's.
+ * caller's.  Renders of one handle must not overlap in time on different
+ * streams (they share its buffers); calls that change what a frame reads
+ * (volume, transfer function, network) wait for frames in flight themselves.
  *
  * Coordinates follow the reference: the volume box is [-G/2, G/2] with
  * G = resolution * voxel scale, the image is premultiplied RGBA with row 0 at

@@ -105,3 +105,48 @@ def test_frame_of_more_lanes_than_a_launch_may_have():
     img[::64, ::64] = out[::64, ::64].cpu().numpy()
     assert ref[:h // 2, ..., 3].max() > 0.2 and ref[h // 2:, ..., 3].max() > 0.2
     check(img, ref, m, 64)
+
+
+@pytest.mark.parametrize("edit", ["transfer function", "weights", "checkpoint", "gradient"])
+def test_edits_wait_for_frames_in_flight(edit):
+    """An edit right after a frame of some milliseconds was queued on a non-blocking stream: the frame is the
+    one drawn before the edit, bit for bit (the shared colour sums of a pixel come in any order: to
+    rounding)."""
+    import torch
+
+    w = h = 1024
+    wl = W.cone_blobs(n=96, width=w, height=h, seed=7)
+    cam, light = wl.camera(), wl.light()
+    if edit in ("weights", "checkpoint"):
+        r, rng = handle(N.CONE_NN, wl), np.random.default_rng(5)
+        wa, wb = (rng.normal(0, 0.1, N.lib().cvr_nn_param_count()).astype(np.float32) for _ in range(2))
+        r.nn_set_weights(wb)
+        r.prepare()
+        other = r.nn_save()
+        r.nn_set_weights(wa)
+    elif edit == "gradient":
+        r = handle(N.RC1P, wl, apply_gradient_shading=1, step_size=0.01, et_threshold=1.0)
+    else:
+        r = handle(N.CONE_TRACE, wl)
+    r.prepare()
+    s = torch.cuda.Stream()
+    before, out = (torch.zeros((h, w, 4), device="cuda:0") for _ in range(2))
+    torch.cuda.synchronize()
+    r.render(cam, w, h, light=light, out=before, stream=s.cuda_stream)
+    torch.cuda.synchronize()
+    r.render(cam, w, h, light=light, out=out, stream=s.cuda_stream)
+    if edit == "transfer function":
+        r.set_transfer_function(wl.rgb_iso[:, [1, 2, 0, 3]], wl.alpha_iso * [0.1, 1.0])
+    elif edit == "weights":
+        r.nn_set_weights(wb)
+    elif edit == "checkpoint":
+        r.nn_load(other)
+    else:
+        r.gradient(wl.volume.shape, N.GRADIENT_FINITE_DIFF)
+    torch.cuda.synchronize()
+    # sums of a thousand samples' colours below 1 in another order: 1000 x 2^-24 at most
+    assert float((out - before).abs().max()) <= 6e-5
+    if edit != "gradient":
+        r.render(cam, w, h, light=light, out=out, stream=s.cuda_stream)
+        torch.cuda.synchronize()
+        assert float((out - before).abs().max()) > 1e-3  # the edit is in force
