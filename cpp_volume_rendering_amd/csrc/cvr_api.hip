@@ -344,7 +344,12 @@ int cvr_set_volume(cvr_handle h, int nx, int ny, int nz, int dtype, float sx, fl
   CVR_HIP_CHECK(hipDeviceSynchronize());
   CVR_HIP_CHECK(hipMemcpy(h->d_vol, voxels, bytes, is_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice));
   h->nx = nx; h->ny = ny; h->nz = nz; h->dtype = dtype;
-  if (const int rc = build_volume_oct(h, nullptr)) return rc;
+  if (const int rc = build_volume_oct(h, nullptr)) {
+    (void)hipFree(h->d_vol);  // no volume without its corner blocks, which the marches read
+    h->d_vol = nullptr;
+    h->vol_version++;  // batches that hold the handle look at it again
+    return rc;
+  }
   h->sx = sx; h->sy = sy; h->sz = sz;
   h->vol_version++;
   h->nn_trained = false;
@@ -407,7 +412,7 @@ int cvr_set_transfer_function(cvr_handle h, int max_density, int extinction_inpu
   DeviceGuard dg(h->device);
   // frames in flight on any stream may still read the tables
   CVR_HIP_CHECK(hipDeviceSynchronize());
-  if (h->tf_size != T) {
+  if (h->tf_size != T || !h->d_tf_rgbt) {
     if (h->d_tf_rgbt) CVR_HIP_CHECK(hipFree(h->d_tf_rgbt));
     h->d_tf_rgbt = h->d_tf_rgba = nullptr;
     if (hipMalloc(&h->d_tf_rgbt, both.size() * sizeof(float4)) != hipSuccess) {

@@ -150,3 +150,18 @@ def test_edits_wait_for_frames_in_flight(edit):
         r.render(cam, w, h, light=light, out=out, stream=s.cuda_stream)
         torch.cuda.synchronize()
         assert float((out - before).abs().max()) > 1e-3  # the edit is in force
+
+
+def test_volume_that_is_refused_leaves_none():
+    """A volume too deep for its corner blocks is refused, and so is a frame after it; the next volume is
+    drawn."""
+    wl = W.cone_blobs(n=16, width=8, height=8)
+    r = handle(N.RC1P, wl)
+    deep = np.full((65536, 1, 1), 200, np.uint8)
+    with pytest.raises(N.CvrError):
+        r.set_volume(deep)
+    with pytest.raises(N.CvrError) as e:
+        r.render(wl.camera(), 8, 8)
+    assert e.value.code == N.ERR_STATE
+    r.set_volume(wl.volume, wl.scale)
+    assert r.render(wl.camera(), 8, 8)[..., 3].max() > 0.1
