@@ -33,6 +33,16 @@ __device__ __forceinline__ void count_add(unsigned long long* counters, int whic
   atomicAdd(&counters[(blockIdx.x % kCountLines) * kCountStride + which], (unsigned long long)n);
 }
 
+// A launch may have fewer than 2^32 lanes: launch(first, workgroups) for each run of at most 2^31 lanes.
+template <class F> inline void for_runs(long long total, int threads, F&& launch) {
+  const long long most = (1ll << 31) / threads;
+  for (long long first = 0;; first += most) {
+    const long long left = total - first;
+    launch(first, int(left < most ? left : most));
+    if (left <= most) break;
+  }
+}
+
 // --------------------------------------------------------------------------- camera
 // Per-frame ray set-up, computed on the host in double and rounded once.
 // dir(px,py) = normalize(a*s + b*u + f) is the expansion of

@@ -150,15 +150,13 @@ inline QueueShape queue_shape(int w, int h, int rays, int parts, int xcd_px, int
   while (per_wg << q.xcd_log2 < xcd_px) ++q.xcd_log2;
   return q;
 }
-// A launch may have fewer than 2^32 lanes, and a frame of 2^28 pixels takes up to 2^36 (64 a pixel where
-// four wavefronts share four rays): launch(shape, workgroups) for each run of at most 2^31 lanes.
+// A frame of 2^28 pixels takes up to 2^36 lanes (64 a pixel where four wavefronts share four rays):
+// launch(shape, workgroups) for each launch of it.
 template <class F> inline void for_launches(QueueShape q, int total, int threads, F&& launch) {
-  const int most = int((1ll << 31) / threads);
-  for (q.first = 0;; q.first += most) {
-    const int left = total - q.first;
-    launch(q, left < most ? left : most);
-    if (left <= most) break;
-  }
+  for_runs(total, threads, [&](long long first, int blocks) {
+    q.first = int(first);
+    launch(q, blocks);
+  });
 }
 // The unit of this wavefront.
 template <int kParts> __device__ __forceinline__ int queue_unit(const QueueShape& q) {

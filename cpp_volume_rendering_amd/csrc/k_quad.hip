@@ -83,19 +83,21 @@ __device__ __forceinline__ unsigned int to16(float x, int fmt) {
 
 // Corner blocks of every pyramid level: cell (x, y, z) holds the 2 x 2 x 2 values at
 // (x..x+1, y..y+1, z..z+1), the +1 neighbours clamped to the edge, plane z first, each
-// plane (x, y), (x+1, y), (x, y+1), (x+1, y+1); fp32 as 32 bytes, fp16 / bf16 as 16.  One launch:
-// workgroup blockIdx.x takes 256 cells, in order, of the first level whose `end` lies past it.
+// plane (x, y), (x+1, y), (x, y+1), (x+1, y+1); fp32 as 32 bytes, fp16 / bf16 as 16.  One launch (for
+// pyramids of 2^23 workgroups more, of which the launch's first is `first`): a workgroup takes 256 cells, in
+// order, of the first level whose `end` lies past it.
 struct OctEnds {
   unsigned int end[kMaxLevels];
 };
 template <int FMT>
-__global__ __launch_bounds__(256) void k_make_oct(PyrGeom pg, OctEnds e, const float* __restrict__ pyr,
-                                                  void* __restrict__ blocks) {
+__global__ __launch_bounds__(256) void k_make_oct(PyrGeom pg, OctEnds e, unsigned int first,
+                                                  const float* __restrict__ pyr, void* __restrict__ blocks) {
+  const unsigned int bid = first + blockIdx.x;
   int l = 0;
-  while (l + 1 < pg.levels && blockIdx.x >= e.end[l]) ++l;
+  while (l + 1 < pg.levels && bid >= e.end[l]) ++l;
   const int nx = pg.dims[l][0], ny = pg.dims[l][1], nz = pg.dims[l][2];
   const unsigned int rows = (unsigned(nx) + 63u) / 64u, per = (unsigned(ny) + 3u) / 4u;
-  unsigned int b = blockIdx.x - (l ? e.end[l - 1] : 0u);
+  unsigned int b = bid - (l ? e.end[l - 1] : 0u);
   const int x = int(b % rows) * 64 + (threadIdx.x & 63);
   b /= rows;
   const int y = int(b % per) * 4 + (threadIdx.x >> 6), z = int(b / per);
@@ -139,10 +141,12 @@ int build_pyramid_oct(cvr_ctx* c, size_t total, int fmt, hipStream_t st) {
     if (blocks >> 31) { set_error("corner blocks: pyramid too large"); return CVR_ERR_INVALID; }
     e.end[l] = unsigned(blocks);
   }
-  const dim3 grid{unsigned(blocks)};
-  if (fmt == 0) hipLaunchKernelGGL(k_make_oct<0>, grid, dim3(256), 0, st, pg, e, c->d_pyr, c->d_pyr_oct);
-  else if (fmt == 1) hipLaunchKernelGGL(k_make_oct<1>, grid, dim3(256), 0, st, pg, e, c->d_pyr, c->d_pyr_oct);
-  else hipLaunchKernelGGL(k_make_oct<2>, grid, dim3(256), 0, st, pg, e, c->d_pyr, c->d_pyr_oct);
+  for_runs((long long)blocks, 256, [&](long long at, int n) {
+    const unsigned first = unsigned(at);
+    if (fmt == 0) hipLaunchKernelGGL(k_make_oct<0>, dim3(n), dim3(256), 0, st, pg, e, first, c->d_pyr, c->d_pyr_oct);
+    else if (fmt == 1) hipLaunchKernelGGL(k_make_oct<1>, dim3(n), dim3(256), 0, st, pg, e, first, c->d_pyr, c->d_pyr_oct);
+    else hipLaunchKernelGGL(k_make_oct<2>, dim3(n), dim3(256), 0, st, pg, e, first, c->d_pyr, c->d_pyr_oct);
+  });
   CVR_HIP_CHECK(hipGetLastError());
   CVR_HIP_CHECK(hipStreamSynchronize(st));
   return CVR_OK;

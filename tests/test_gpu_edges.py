@@ -165,3 +165,30 @@ def test_volume_that_is_refused_leaves_none():
     assert e.value.code == N.ERR_STATE
     r.set_volume(wl.volume, wl.scale)
     assert r.render(wl.camera(), 8, 8)[..., 3].max() > 0.1
+
+
+def test_pyramid_of_more_workgroups_than_a_launch_may_have():
+    """A pyramid of 2^24 workgroups of corner blocks, in three launches: cones around where the second and
+    the third begin, and in the first and last slices."""
+    vol = W.cone_blobs(n=64, width=8, height=8).volume[:, 16:32, 30:34].copy()
+    grid = (4.0, 16.0, 64.0)
+    r = N.Renderer(N.CONE_TRACE)
+    r.set_volume(vol)
+    r.set_transfer_function(*W.seeded_tf(103, 4))
+    p = r.params()
+    p.base_res[:], p.n_levels = [1, 1025, 65535], 2
+    r.set_params(p)
+    pyr = O.OPyr.wrap(grid, [a.astype(np.float64) for a in r.pyramid()])
+    per = 257  # workgroups of a slice
+    z = np.array([0.01, (1 << 23) / per / 65535 * 64, (1 << 24) / per / 65535 * 64, 63.99, 40.0])
+    rng = np.random.default_rng(3)
+    pos = np.column_stack([rng.uniform(0.5, 3.5, 40), rng.uniform(1, 15, 40), np.tile(z, 8)])
+    d = rng.normal(0, 1, (40, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    light = np.array([0.3, 0.2, 0.9]) / np.linalg.norm([0.3, 0.2, 0.9])
+    pos, d, li = (np.ascontiguousarray(v, np.float32) for v in (pos, d, np.tile(light, (40, 1))))
+    occ, sdw, feat = r.cone_eval(pos, d, li)
+    ro, rs, rf = O.cone_points(pyr, O.cone_params(grid, light_fwd=light), pos, d)
+    assert ro.min() < 0.9
+    for a, b in ((occ, ro), (sdw, rs), (feat, rf)):
+        assert np.abs(a - b).max() <= 2e-4
