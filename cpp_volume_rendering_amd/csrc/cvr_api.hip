@@ -222,6 +222,7 @@ static void free_all(cvr_ctx* c) {
   if (c->d_ms_frame) (void)hipFree(c->d_ms_frame);
   if (c->d_pyr) (void)hipFree(c->d_pyr);
   if (c->d_pyr_oct) (void)hipFree(c->d_pyr_oct);
+  claim_work(&c->d_pyr_work);
   if (c->d_pyr_work) (void)hipFree(c->d_pyr_work);
   if (c->h_nn_io) (void)hipHostFree(c->h_nn_io);
   if (c->d_nn_redo) (void)hipFree(c->d_nn_redo);
@@ -293,7 +294,7 @@ int cvr_create(int technique, int device, cvr_handle* out) {
   defaults(CVR_DOS, &c->dos);
   defaults(CVR_CONE_TRACE, &c->cone);
   defaults(CVR_CONE_NN, &c->nn);
-  if (hipMalloc(&c->d_counters, kCountBytes) != hipSuccess ||
+  if (device_alloc(&c->d_counters, kCountBytes) != hipSuccess ||
       hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {
     free_all(c);
     delete c;
@@ -334,7 +335,7 @@ int cvr_set_volume(cvr_handle h, int nx, int ny, int nz, int dtype, float sx, fl
     h->d_sat_oct = nullptr;
     if (h->d_grad) CVR_HIP_CHECK(hipFree(h->d_grad));
     h->d_grad = nullptr;
-    if (hipMalloc(&h->d_vol, bytes) != hipSuccess) {
+    if (device_alloc(&h->d_vol, bytes) != hipSuccess) {
       h->d_vol = nullptr;
       set_error("cvr_set_volume: out of device memory");
       return CVR_ERR_NOMEM;
@@ -415,7 +416,7 @@ int cvr_set_transfer_function(cvr_handle h, int max_density, int extinction_inpu
   if (h->tf_size != T || !h->d_tf_rgbt) {
     if (h->d_tf_rgbt) CVR_HIP_CHECK(hipFree(h->d_tf_rgbt));
     h->d_tf_rgbt = h->d_tf_rgba = nullptr;
-    if (hipMalloc(&h->d_tf_rgbt, both.size() * sizeof(float4)) != hipSuccess) {
+    if (device_alloc(&h->d_tf_rgbt, both.size() * sizeof(float4)) != hipSuccess) {
       h->d_tf_rgbt = nullptr;
       set_error("cvr_set_transfer_function: out of device memory");
       return CVR_ERR_NOMEM;
@@ -582,7 +583,7 @@ static int grow_buffer(float** p, size_t* cap, size_t bytes, const char* who) {
   if (*p) CVR_HIP_CHECK(hipFree(*p));
   *p = nullptr;
   *cap = 0;
-  if (hipMalloc(p, bytes) != hipSuccess) {
+  if (device_alloc(p, bytes) != hipSuccess) {
     *p = nullptr;
     set_error(std::string(who) + ": out of device memory");
     return CVR_ERR_NOMEM;
@@ -825,8 +826,8 @@ int cvr_cone_eval(cvr_handle h, int n, const float* pos, const float* dirs, cons
   DeviceGuard dg(h->device);
   DevBuf in, o;
   const size_t n3 = size_t(n) * 3;
-  CVR_HIP_CHECK(hipMalloc(&in.p, 3 * n3 * sizeof(float)));
-  CVR_HIP_CHECK(hipMalloc(&o.p, size_t(n) * 18 * sizeof(float)));
+  CVR_HIP_CHECK(device_alloc(&in.p, 3 * n3 * sizeof(float)));
+  CVR_HIP_CHECK(device_alloc(&o.p, size_t(n) * 18 * sizeof(float)));
   float* dp = static_cast<float*>(in.p);
   float* dout = static_cast<float*>(o.p);
   CVR_HIP_CHECK(hipMemcpy(dp, pos, n3 * 4, hipMemcpyHostToDevice));
@@ -901,8 +902,8 @@ int cvr_nn_eval(cvr_handle h, int n, const float* X, float* Y, int path) {
   if (n == 0) return CVR_OK;
   DeviceGuard dg(h->device);
   DevBuf dx, dy;
-  CVR_HIP_CHECK(hipMalloc(&dx.p, size_t(n) * 16 * 4));
-  CVR_HIP_CHECK(hipMalloc(&dy.p, size_t(n) * 2 * 4));
+  CVR_HIP_CHECK(device_alloc(&dx.p, size_t(n) * 16 * 4));
+  CVR_HIP_CHECK(device_alloc(&dy.p, size_t(n) * 2 * 4));
   CVR_HIP_CHECK(hipMemcpy(dx.p, X, size_t(n) * 16 * 4, hipMemcpyHostToDevice));
   rc = nn_eval(h, static_cast<float*>(dx.p), n, static_cast<float*>(dy.p), path, nullptr);
   if (rc) return rc;
@@ -927,8 +928,8 @@ int cvr_nn_gradient(cvr_handle h, int n, const float* X, const float* T, float* 
   const size_t bytes = (xn + tn + gn) * sizeof(float);
   if (bytes > kNnIoKept) {
     DevBuf dx, dt;
-    CVR_HIP_CHECK(hipMalloc(&dx.p, xn * sizeof(float)));
-    CVR_HIP_CHECK(hipMalloc(&dt.p, tn * sizeof(float)));
+    CVR_HIP_CHECK(device_alloc(&dx.p, xn * sizeof(float)));
+    CVR_HIP_CHECK(device_alloc(&dt.p, tn * sizeof(float)));
     CVR_HIP_CHECK(hipMemcpy(dx.p, X, xn * sizeof(float), hipMemcpyHostToDevice));
     CVR_HIP_CHECK(hipMemcpy(dt.p, T, tn * sizeof(float), hipMemcpyHostToDevice));
     rc = nn_gradient(h, static_cast<float*>(dx.p), static_cast<float*>(dt.p), n, h->d_nn_g, nullptr);

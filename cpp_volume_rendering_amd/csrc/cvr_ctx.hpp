@@ -1,6 +1,7 @@
 // Technique instance state behind a cvr_handle.
 #pragma once
 #include "cvr_common.hpp"
+#include "cvr_memory.hpp"
 #include "cvr_phong.hpp"
 #include "../../include/cvr.h"
 #include <vector>
@@ -119,7 +120,7 @@ struct cvr_ctx {
   // Gaussian extinction pyramid (cone tracers, surrogate)
   float* d_pyr = nullptr;
   size_t pyr_bytes = 0, pyr_oct_bytes = 0;
-  void* d_pyr_work = nullptr;  // opacities and separable passes of a build, kept up to kPyrWorkKept bytes
+  void* d_pyr_work = nullptr;  // opacities and separable passes of a build, idle between builds (claim_work)
   size_t pyr_work_bytes = 0;
   void* d_pyr_oct = nullptr;   // corner blocks of every level (PyrGeom::fmt, k_quad.hip)
   cvr::PyrGeom pyr{};

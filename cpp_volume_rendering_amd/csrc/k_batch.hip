@@ -240,7 +240,7 @@ int grow(void** p, size_t& cap, size_t bytes) {
   if (*p) CVR_HIP_CHECK(hipFree(*p));
   *p = nullptr;
   cap = 0;
-  if (hipMalloc(p, std::max<size_t>(bytes, 256)) != hipSuccess) {
+  if (device_alloc(p, std::max<size_t>(bytes, 256)) != hipSuccess) {
     *p = nullptr;
     set_error("batch: out of device memory");
     return CVR_ERR_NOMEM;
@@ -413,7 +413,7 @@ int tune_step(cvr_batch* b, float* out, hipStream_t st, TimeOf& time_of, cvr_bat
   const size_t px = b->jobs.size() * size_t(b->W) * b->H;
   float4* ref = nullptr;
   double* acc = nullptr;
-  if (hipMalloc(&ref, px * sizeof(float4)) != hipSuccess || hipMalloc(&acc, 2 * sizeof(double)) != hipSuccess) {
+  if (device_alloc(&ref, px * sizeof(float4)) != hipSuccess || device_alloc(&acc, 2 * sizeof(double)) != hipSuccess) {
     if (ref) (void)hipFree(ref);
     set_error("cvr_batch_autotune: out of device memory for the step search");
     return CVR_ERR_NOMEM;
@@ -475,8 +475,8 @@ int cvr_batch_create(int device, int width, int height, cvr_batch_handle* out) {
   b->device = device;
   b->W = width;
   b->H = height;
-  if (hipMalloc(&b->d_heads, kQueues * kMaxVolumes * sizeof(unsigned int)) != hipSuccess ||
-      hipMalloc(&b->d_counters, 4 * sizeof(unsigned long long)) != hipSuccess ||
+  if (device_alloc(&b->d_heads, kQueues * kMaxVolumes * sizeof(unsigned int)) != hipSuccess ||
+      device_alloc(&b->d_counters, 4 * sizeof(unsigned long long)) != hipSuccess ||
       hipStreamCreateWithFlags(&b->cap, hipStreamNonBlocking) != hipSuccess) {
     cvr_batch_destroy(b);
     set_error("cvr_batch_create: HIP allocation failed");

@@ -224,7 +224,7 @@ int prepare_cone(cvr_ctx* c, const cvr_cone_params& P, hipStream_t st) {
   for (int i = 0; i < kNFeat; ++i) taps[i] = feat_tap(c->pyr, stn[i]);
   // [taps (kNFeat x 64 B)] [levels] [occlusion schedule] [shadow schedule]
   const size_t tb = kNFeat * sizeof(FeatTap), lb = kMaxLevels * sizeof(ConeLevel), sb = so.size() * sizeof(ConeStepF);
-  if (!c->d_cone_tab) CVR_HIP_CHECK(hipMalloc(&c->d_cone_tab, tb + lb + 2 * kMaxSteps * sizeof(ConeStepF)));
+  if (!c->d_cone_tab) CVR_HIP_CHECK(device_alloc(&c->d_cone_tab, tb + lb + 2 * kMaxSteps * sizeof(ConeStepF)));
   else CVR_HIP_CHECK(hipDeviceSynchronize());  // earlier renders may still read the old table
   std::vector<char> buf(tb + lb + 2 * sb);
   std::memcpy(buf.data(), taps.data(), tb);

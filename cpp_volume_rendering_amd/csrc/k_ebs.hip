@@ -633,7 +633,7 @@ int launch_ebs(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* ou
       rows.push_back(row);
     }
     k.nrows = int(rows.size());
-    if (!c->d_ebs_rows && hipMalloc(&c->d_ebs_rows, kMaxShadowRows * sizeof(ShadowRow)) != hipSuccess) {
+    if (!c->d_ebs_rows && device_alloc(&c->d_ebs_rows, kMaxShadowRows * sizeof(ShadowRow)) != hipSuccess) {
       c->d_ebs_rows = nullptr;
       set_error("cvr_render: out of device memory (shadow rows)");
       return -5;

@@ -62,7 +62,7 @@ int build_gradient(cvr_ctx* c, int type, hipStream_t st) {
     CVR_HIP_CHECK(hipDeviceSynchronize());  // frames in flight on any stream may still read it
   } else {
     const size_t cells = brick_cells(c->nx, c->ny, c->nz);
-    if (hipMalloc(&c->d_grad, cells * sizeof(float4)) != hipSuccess) {
+    if (device_alloc(&c->d_grad, cells * sizeof(float4)) != hipSuccess) {
       c->d_grad = nullptr;
       set_error("gradient: out of device memory");
       return CVR_ERR_NOMEM;

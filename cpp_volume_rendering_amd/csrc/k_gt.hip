@@ -186,7 +186,7 @@ int prepare_gt(cvr_ctx* c, const cvr_gt_params& P) {
   if (c->d_gt_rays) CVR_HIP_CHECK(hipFree(c->d_gt_rays));
   c->d_gt_rays = nullptr;
   const size_t n = c->gt_occ.size() + c->gt_sdw.size();
-  if (hipMalloc(&c->d_gt_rays, n * sizeof(float)) != hipSuccess) {
+  if (device_alloc(&c->d_gt_rays, n * sizeof(float)) != hipSuccess) {
     c->d_gt_rays = nullptr;
     set_error("gt: out of device memory");
     return CVR_ERR_NOMEM;

@@ -95,7 +95,7 @@ int lc_prepare(cvr_ctx* c, const int res[3]) {
     if (c->d_lc) CVR_HIP_CHECK(hipFree(c->d_lc));
     c->d_lc = nullptr;
     c->lc_cap = 0;
-    CVR_HIP_CHECK(hipMalloc(&c->d_lc, n * sizeof(float2)));
+    CVR_HIP_CHECK(device_alloc(&c->d_lc, n * sizeof(float2)));
     c->lc_cap = n;
   }
   for (int i = 0; i < 3; ++i) c->lc_res[i] = res[i];

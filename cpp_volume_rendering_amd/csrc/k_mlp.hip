@@ -648,7 +648,7 @@ int launch_cone(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* o
 
 static int ensure(void** p, size_t bytes) {
   if (*p) return 0;
-  if (hipMalloc(p, bytes) != hipSuccess) {
+  if (device_alloc(p, bytes) != hipSuccess) {
     *p = nullptr;
     set_error("surrogate: out of device memory");
     return -5;
@@ -696,7 +696,7 @@ static void init_weights(std::vector<float>& w, uint64_t seed) {
 
 // Device buffers of training: the bf16 training packs and the gradient slabs of n samples.
 static int train_buffers(cvr_ctx* c, int n) {
-  if (!c->d_nn_tpack && hipMalloc(&c->d_nn_tpack, kTrainPackBytes) != hipSuccess) {
+  if (!c->d_nn_tpack && device_alloc(&c->d_nn_tpack, kTrainPackBytes) != hipSuccess) {
     c->d_nn_tpack = nullptr;
     set_error("surrogate: out of device memory (training packs)");
     return -5;
@@ -706,7 +706,7 @@ static int train_buffers(cvr_ctx* c, int n) {
     if (c->d_nn_slabs) CVR_HIP_CHECK(hipFree(c->d_nn_slabs));
     c->d_nn_slabs = nullptr;
     c->nn_slabs_cap = 0;
-    if (hipMalloc(&c->d_nn_slabs, need * sizeof(float)) != hipSuccess) {
+    if (device_alloc(&c->d_nn_slabs, need * sizeof(float)) != hipSuccess) {
       c->d_nn_slabs = nullptr;
       set_error("surrogate: out of device memory (gradient slabs)");
       return -5;
@@ -789,9 +789,9 @@ int nn_train(cvr_ctx* c, hipStream_t st) {
     if (d_Yv) (void)hipFree(d_Yv);
     if (d_rng) (void)hipFree(d_rng);
   };
-  if (hipMalloc(&d_X, size_t(n) * kNFeat * 4) != hipSuccess || hipMalloc(&d_T, size_t(n) * 2 * 4) != hipSuccess ||
-      hipMalloc(&d_Xv, size_t(nv) * kNFeat * 4) != hipSuccess || hipMalloc(&d_Tv, size_t(nv) * 2 * 4) != hipSuccess ||
-      hipMalloc(&d_Yv, size_t(nv) * 2 * 4) != hipSuccess || hipMalloc(&d_rng, 2 * kNFeat * 4) != hipSuccess) {
+  if (device_alloc(&d_X, size_t(n) * kNFeat * 4) != hipSuccess || device_alloc(&d_T, size_t(n) * 2 * 4) != hipSuccess ||
+      device_alloc(&d_Xv, size_t(nv) * kNFeat * 4) != hipSuccess || device_alloc(&d_Tv, size_t(nv) * 2 * 4) != hipSuccess ||
+      device_alloc(&d_Yv, size_t(nv) * 2 * 4) != hipSuccess || device_alloc(&d_rng, 2 * kNFeat * 4) != hipSuccess) {
     cleanup();
     set_error("surrogate: out of device memory for the training set");
     return -5;
@@ -982,7 +982,7 @@ int launch_nn(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out
     if (c->d_nn_redo) CVR_HIP_CHECK(hipFree(c->d_nn_redo));
     c->d_nn_redo = nullptr;
     c->nn_redo_cap = 0;
-    if (hipMalloc(&c->d_nn_redo, size_t(tiles) * sizeof(unsigned int)) != hipSuccess) {
+    if (device_alloc(&c->d_nn_redo, size_t(tiles) * sizeof(unsigned int)) != hipSuccess) {
       c->d_nn_redo = nullptr;
       set_error("surrogate: out of device memory");
       return -5;

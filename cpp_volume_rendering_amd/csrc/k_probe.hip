@@ -67,7 +67,7 @@ extern "C" int cvr_probe_gather(int device, size_t working_set_bytes, int reps, 
   while (n * 2 * 32 <= working_set_bytes) n *= 2;
   hipStream_t st = static_cast<hipStream_t>(hip_stream);
   uint4* d = nullptr;
-  if (hipMalloc(&d, n * 32 + 16) != hipSuccess) {
+  if (device_alloc(&d, n * 32 + 16) != hipSuccess) {
     set_error("cvr_probe_gather: out of device memory");
     return CVR_ERR_NOMEM;
   }

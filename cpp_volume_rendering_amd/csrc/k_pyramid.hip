@@ -322,7 +322,7 @@ PyrKey pyr_key_for(const cvr_ctx* c, int base_x, int base_y, int base_z, float s
 
 // A volume that changes every frame rebuilds its pyramid every frame: allocating and freeing
 // its four buffers and the volume's corner blocks took longer than the build (the next 256^3 step and
-// its DOS frame 1.6 to 9 ms with them, 0.54 without).
+// its DOS frame 1.6 to 9 ms with them, 0.54 without).  The workspace lies idle between builds (cvr_memory.hpp).
 constexpr size_t kPyrWorkKept = size_t(1) << 30;
 
 int build_pyramid(cvr_ctx* c, int base_x, int base_y, int base_z, float sigma0, int nlev, int fmt, hipStream_t st) {
@@ -377,6 +377,7 @@ int build_pyramid(cvr_ctx* c, int base_x, int base_y, int base_z, float sigma0, 
   }
   // opacities of every level, then the temporaries of the largest level's passes
   int rc = sized_buffer(reinterpret_cast<void**>(&c->d_pyr), &c->pyr_bytes, total * sizeof(float));
+  claim_work(&c->d_pyr_work);
   if (!rc) rc = sized_buffer(&c->d_pyr_work, &c->pyr_work_bytes, (total + tmp_floats) * sizeof(float));
   if (rc == CVR_ERR_NOMEM && c->d_pyr) {
     std::fill(sep.begin(), sep.end(), 0);  // no room for the temporaries: the direct build needs none
@@ -460,12 +461,16 @@ int build_pyramid(cvr_ctx* c, int base_x, int base_y, int base_z, float sigma0, 
   hipLaunchKernelGGL(k_pyr_tau, dim3(unsigned((total + 255) / 256)), dim3(256), 0, st, d_op, c->d_pyr, total);
   CVR_HIP_CHECK(hipGetLastError());
   c->pyr = pg;
+  // from here on the build's kernels alone need the workspace: the corner blocks may have its room
+  park_work(&c->d_pyr_work, &c->pyr_work_bytes, c->device);
   if (build_pyramid_oct(c, btotal, fmt, st) != CVR_OK) return -5;  // waits for the stream
+  claim_work(&c->d_pyr_work);
   if (c->pyr_work_bytes > kPyrWorkKept) {
     CVR_HIP_CHECK(hipFree(c->d_pyr_work));
     c->d_pyr_work = nullptr;
     c->pyr_work_bytes = 0;
   }
+  park_work(&c->d_pyr_work, &c->pyr_work_bytes, c->device);
   c->pyr_key = key;
   c->pyr_valid = true;
   return 0;

@@ -49,7 +49,7 @@ int sized_buffer(void** p, size_t* have, size_t bytes) {
   if (*p) CVR_HIP_CHECK(hipFree(*p));
   *p = nullptr;
   *have = 0;
-  if (hipMalloc(p, bytes) != hipSuccess) {
+  if (device_alloc(p, bytes) != hipSuccess) {
     (void)hipGetLastError();
     *p = nullptr;
     return CVR_ERR_NOMEM;
@@ -122,14 +122,6 @@ __global__ __launch_bounds__(256) void k_make_oct(PyrGeom pg, OctEnds e, unsigne
 int build_pyramid_oct(cvr_ctx* c, size_t total, int fmt, hipStream_t st) {
   const size_t rec = fmt == 0 ? 32 : 16;
   int rc = sized_buffer(&c->d_pyr_oct, &c->pyr_oct_bytes, total * rec);
-  if (rc == CVR_ERR_NOMEM && c->d_pyr_work) {
-    // the build's workspace is no longer needed once its kernels have run
-    CVR_HIP_CHECK(hipStreamSynchronize(st));
-    CVR_HIP_CHECK(hipFree(c->d_pyr_work));
-    c->d_pyr_work = nullptr;
-    c->pyr_work_bytes = 0;
-    rc = sized_buffer(&c->d_pyr_oct, &c->pyr_oct_bytes, total * rec);
-  }
   if (rc == CVR_ERR_NOMEM) set_error("pyramid: out of device memory (corner blocks)");
   if (rc != CVR_OK) return rc;
   const PyrGeom& pg = c->pyr;

@@ -314,7 +314,7 @@ static int build_ext_lut(cvr_ctx* c, hipStream_t st) {
   const int nvals = c->dtype == CVR_U8 ? 256 : 65536;
   const int md = c->tf_max_density;
   int rc = c->d_ext_lut ? CVR_OK : CVR_ERR_NOMEM;
-  if (rc && hipMalloc(&c->d_ext_lut, 65536 * sizeof(float)) == hipSuccess) rc = CVR_OK;  // the larger type's
+  if (rc && device_alloc(&c->d_ext_lut, 65536 * sizeof(float)) == hipSuccess) rc = CVR_OK;  // the larger type's
   if (!rc) rc = sized_buffer(&c->d_tf_alpha, &c->tf_alpha_bytes, size_t(md + 1) * sizeof(double));
   if (rc) {
     if (rc == CVR_ERR_NOMEM) set_error("cvr_prepare: out of device memory for the extinction table");
@@ -358,7 +358,7 @@ static int build_sat_oct(cvr_ctx* c, hipStream_t st) {
   const int w = c->nx + 2, h = c->ny + 2, d = c->nz + 2;
   const size_t cells = size_t(w) * h * d;
   if (!c->d_sat_oct) {
-    if (hipMalloc(&c->d_sat_oct, cells * 4 * sizeof(float4)) != hipSuccess) {
+    if (device_alloc(&c->d_sat_oct, cells * 4 * sizeof(float4)) != hipSuccess) {
       c->d_sat_oct = nullptr;
       set_error("cvr_prepare: out of device memory for the summed-area table's corner blocks");
       return -5;
@@ -438,7 +438,7 @@ int build_sat(cvr_ctx* c, hipStream_t st, bool with_blocks) {
   const int w = c->nx + 2, h = c->ny + 2, d = c->nz + 2;
   const size_t cells = size_t(w) * h * d;
   if (!c->d_sat) {
-    if (hipMalloc(&c->d_sat, cells * sizeof(float2)) != hipSuccess) {
+    if (device_alloc(&c->d_sat, cells * sizeof(float2)) != hipSuccess) {
       c->d_sat = nullptr;
       set_error("cvr_prepare: out of device memory for the summed-area table");
       return -5;
