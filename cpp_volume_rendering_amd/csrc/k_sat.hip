@@ -444,8 +444,8 @@ int build_sat(cvr_ctx* c, hipStream_t st, bool with_blocks) {
       return -5;
     }
   }
-  // frames in flight on any stream may still read the table and its blocks
-  CVR_HIP_CHECK(hipDeviceSynchronize());
+  // no frame in flight reads the table: the call that made it out of date waited for them, and frames
+  // since then come here first
   if (const int rc = build_ext_lut(c, st)) return rc;
   const bool timed = c->collect_stats;
   if (timed) {
