@@ -913,9 +913,12 @@ int cvr_nn_eval(cvr_handle h, int n, const float* X, float* Y, int path) {
 }
 
 // One step of an optimiser outside the library.  The kernels read the samples from a pinned buffer
-// and write the gradient behind them, so the call waits once; the buffer is kept up to this size
-// (16384 samples: 126 us with device buffers made in the call and a wait for each of four copies, 101
-// with kept buffers and queued copies, 81 now, of which 14 copy the samples and 37 are the kernels').
+// and write the gradient behind them, so the call waits once (16384 samples: 126 us with device buffers made
+// in the call and a wait for each of four copies, 101 with kept buffers and queued copies, 80 now, of which 14
+// copy the samples and 37 are the kernels').  The buffer is kept up to kNnIoKept bytes and grows with n: a size
+// of its own for each n cost two calls of 16384 and 9000 samples in turn 257 us (231 with device buffers, 133
+// now).  Pinning takes 40 us, so a handle's first call (156 us, 170 with a pinned buffer made in it) does
+// without.
 constexpr size_t kNnIoKept = size_t(64) << 20;
 
 int cvr_nn_gradient(cvr_handle h, int n, const float* X, const float* T, float* grad, float* loss) {
@@ -926,7 +929,10 @@ int cvr_nn_gradient(cvr_handle h, int n, const float* X, const float* T, float* 
   DeviceGuard dg(h->device);
   const size_t xn = size_t(n) * 16, tn = size_t(n) * 2, gn = size_t(nn_param_count()) + 1;
   const size_t bytes = (xn + tn + gn) * sizeof(float);
-  if (bytes > kNnIoKept) {
+  const bool first = !h->nn_stepped;
+  h->nn_stepped = true;
+  float* hx = first || bytes > kNnIoKept ? nullptr : pinned_buffer(&h->h_nn_io, &h->nn_io_bytes, bytes);
+  if (!hx) {
     DevBuf dx, dt;
     CVR_HIP_CHECK(device_alloc(&dx.p, xn * sizeof(float)));
     CVR_HIP_CHECK(device_alloc(&dt.p, tn * sizeof(float)));
@@ -939,19 +945,7 @@ int cvr_nn_gradient(cvr_handle h, int n, const float* X, const float* T, float* 
     if (loss) CVR_HIP_CHECK(hipMemcpy(loss, h->d_nn_scalar, sizeof(float), hipMemcpyDeviceToHost));
     return CVR_OK;
   }
-  if (h->nn_io_bytes != bytes) {
-    if (h->h_nn_io) CVR_HIP_CHECK(hipHostFree(h->h_nn_io));
-    h->h_nn_io = nullptr;
-    h->nn_io_bytes = 0;
-    if (hipHostMalloc(reinterpret_cast<void**>(&h->h_nn_io), bytes, hipHostMallocDefault) != hipSuccess) {
-      (void)hipGetLastError();
-      h->h_nn_io = nullptr;
-      set_error("cvr_nn_gradient: out of pinned host memory");
-      return CVR_ERR_NOMEM;
-    }
-    h->nn_io_bytes = bytes;
-  }
-  float *hx = h->h_nn_io, *ht = hx + xn, *hg = ht + tn;
+  float *ht = hx + xn, *hg = ht + tn;
   std::memcpy(hx, X, xn * sizeof(float));
   std::memcpy(ht, T, tn * sizeof(float));
   rc = nn_gradient(h, hx, ht, n, hg, nullptr);

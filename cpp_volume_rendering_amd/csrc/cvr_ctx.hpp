@@ -153,6 +153,7 @@ struct cvr_ctx {
   size_t nn_slabs_cap = 0;
   float* h_nn_io = nullptr;        // cvr_nn_gradient: samples, gradient and loss (pinned, at most kNnIoKept bytes)
   size_t nn_io_bytes = 0;
+  bool nn_stepped = false;         // cvr_nn_gradient has been called
   float nn_lo[16] = {0}, nn_hi[16] = {0};
   bool nn_trained = false;
   uint64_t nn_version = 0;  // bumped whenever the weights or the input range change

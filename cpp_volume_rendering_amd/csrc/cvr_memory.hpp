@@ -1,5 +1,5 @@
-// Device memory: workspaces that a handle keeps between calls are given back where an allocation of any
-// handle finds no room.
+// Memory that a handle keeps between calls: device workspaces, given back where an allocation of any handle
+// finds no room, and pinned buffers.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cstddef>
@@ -64,6 +64,18 @@ template <class T> inline hipError_t device_alloc(T** p, size_t bytes) {
   }
   *p = e == hipSuccess ? static_cast<T*>(q) : nullptr;
   return e;
+}
+
+// A pinned buffer of at least `bytes`, which only grows; null where there is none to be had.
+template <class T> inline T* pinned_buffer(T** p, size_t* have, size_t bytes) {
+  if (*p && *have >= bytes) return *p;
+  if (*p) (void)hipHostFree(*p);
+  void* q = nullptr;
+  const bool ok = hipHostMalloc(&q, bytes, hipHostMallocDefault) == hipSuccess;
+  if (!ok) (void)hipGetLastError();
+  *p = ok ? static_cast<T*>(q) : nullptr;
+  *have = ok ? bytes : 0;
+  return *p;
 }
 
 }  // namespace cvr

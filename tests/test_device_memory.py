@@ -28,6 +28,14 @@ hipError_t hipFree(void* p) {
 }
 hipError_t hipGetDevice(int* d) { *d = 1; return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
+static int pins = 0, frees = 0;
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  ++pins;
+  if (n > 1000) return hipErrorOutOfMemory;
+  *p = std::malloc(n);
+  return hipSuccess;
+}
+hipError_t hipHostFree(void* p) { ++frees; std::free(p); return hipSuccess; }
 }
 using namespace cvr;
 int main() {
@@ -48,7 +56,16 @@ int main() {
   park_work(&b, &bn, 1);
   if (!ok(device_alloc(&r, 30)) || b || bn || !c || used != 95) return 5;
   claim_work(&a);  // it is gone: its owner finds none
-  return a == nullptr ? 0 : 6;
+  if (a) return 6;
+
+  // a pinned buffer grows and is kept for less; where there is none to be had, the next call tries again
+  float* h = nullptr;
+  size_t hn = 0;
+  float* first = pinned_buffer(&h, &hn, 400);
+  if (!first || hn != 400 || pinned_buffer(&h, &hn, 100) != first || pinned_buffer(&h, &hn, 400) != first || pins != 1) return 7;
+  if (!pinned_buffer(&h, &hn, 500) || hn != 500 || pins != 2 || frees != 1) return 8;
+  if (pinned_buffer(&h, &hn, 2000) || h || hn || frees != 2) return 9;
+  return pinned_buffer(&h, &hn, 100) && hn == 100 && frees == 2 ? 0 : 10;
 }
 """
 

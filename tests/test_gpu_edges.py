@@ -192,3 +192,19 @@ def test_pyramid_of_more_workgroups_than_a_launch_may_have():
     assert ro.min() < 0.9
     for a, b in ((occ, ro), (sdw, rs), (feat, rf)):
         assert np.abs(a - b).max() <= 2e-4
+
+
+@pytest.mark.parametrize("sizes", [(100, 700, 100, 3000, 64), (5000, 1, 700)])
+def test_gradient_of_changing_sample_counts(sizes):
+    """Calls of one handle with more and with fewer samples than before: each as a handle's first call,
+    which takes other buffers."""
+    rng = np.random.default_rng(9)
+    w = rng.normal(0, 0.2, N.lib().cvr_nn_param_count()).astype(np.float32)
+    kept = N.Renderer(N.CONE_NN)
+    kept.nn_set_weights(w)
+    for n in sizes:
+        X, T = rng.random((n, 16)).astype(np.float32), rng.normal(0, 0.1, (n, 2)).astype(np.float32)
+        own = N.Renderer(N.CONE_NN)
+        own.nn_set_weights(w)
+        (la, ga), (lb, gb) = kept.nn_gradient(X, T), own.nn_gradient(X, T)
+        assert la == lb and np.array_equal(ga, gb)
