@@ -828,9 +828,8 @@ int nn_train(cvr_ctx* c, hipStream_t st) {
   std::vector<float> w0;
   init_weights(w0, N.seed);
   (void)hipMemcpy(c->d_nn_w, w0.data(), kNParams * 4, hipMemcpyHostToDevice);
-  (void)hipMemset(c->d_nn_m, 0, kNParams * 4);
-  (void)hipMemset(c->d_nn_v, 0, kNParams * 4);
-  (void)hipMemset(c->d_nn_g, 0, kNParams * 4);
+  // on the steps' stream: the null stream's memset need not be done before a non-blocking stream's kernels
+  for (float* p : {c->d_nn_m, c->d_nn_v, c->d_nn_g}) (void)hipMemsetAsync(p, 0, kNParams * 4, st);
   const int B = std::min(N.batch, n);
   const int steps_per_epoch = n / B;
   const int total = steps_per_epoch * N.epochs;
@@ -966,6 +965,11 @@ static int nn_frame(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, floa
   return 0;
 }
 
+__global__ __launch_bounds__(256) void k_clear_marks(unsigned int* __restrict__ p, int n) {
+  const int i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) p[i] = 0u;
+}
+
 int launch_nn(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out, hipStream_t st) {
   const cvr_nn_params& N = c->nn;
   int rc = prepare_cone(c, N.cone, st);
@@ -976,8 +980,8 @@ int launch_nn(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out
   }
   int sets = 1;
   const int tiles = nn_shape(rf, sets).blocks;
-  // workgroup marks for the second pass: zero when allocated, and the second pass clears
-  // what the first sets
+  // workgroup marks for the second pass: cleared when allocated, on the frame's stream, and the second
+  // pass clears what the first sets
   if (size_t(tiles) > c->nn_redo_cap) {
     if (c->d_nn_redo) CVR_HIP_CHECK(hipFree(c->d_nn_redo));
     c->d_nn_redo = nullptr;
@@ -987,7 +991,8 @@ int launch_nn(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out
       set_error("surrogate: out of device memory");
       return -5;
     }
-    CVR_HIP_CHECK(hipMemset(c->d_nn_redo, 0, size_t(tiles) * sizeof(unsigned int)));
+    hipLaunchKernelGGL(k_clear_marks, dim3((tiles + 255) / 256), dim3(256), 0, st, c->d_nn_redo, tiles);
+    CVR_HIP_CHECK(hipGetLastError());
     c->nn_redo_cap = size_t(tiles);
   }
   return nn_frame(c, rf, light, out, c->d_nn_redo, c->collect_stats ? c->d_counters : nullptr, st);
@@ -1021,11 +1026,6 @@ static int scratch_of(int dev, unsigned int** p) {
   }
   *p = g_scratch[dev];
   return CVR_OK;
-}
-
-__global__ __launch_bounds__(256) void k_clear_marks(unsigned int* __restrict__ p, int n) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < n) p[i] = 0u;
 }
 
 int nn_param_count() { return kNParams; }

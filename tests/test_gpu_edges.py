@@ -208,3 +208,29 @@ def test_gradient_of_changing_sample_counts(sizes):
         own.nn_set_weights(w)
         (la, ga), (lb, gb) = kept.nn_gradient(X, T), own.nn_gradient(X, T)
         assert la == lb and np.array_equal(ga, gb)
+
+
+def test_training_and_first_frame_on_a_non_blocking_stream():
+    """Optimiser state and second-pass marks are cleared on the call's stream: the network trained there and
+    its first frame, some of whose samples leave the training range, are the null stream's bit for bit
+    (colours to the rounding of their sums)."""
+    import torch
+
+    wl = W.cone_blobs(n=40, width=96, height=80, seed=21)
+    out, weights, images = torch.zeros((80, 96, 4), device="cuda:0"), [], []
+    for stream in (None, torch.cuda.Stream().cuda_stream):
+        r = handle(N.CONE_NN, wl)
+        p = r.params()
+        p.n_train, p.n_val, p.batch, p.epochs, p.rmse_gate, p.ood_margin = 4096, 1024, 1024, 4, 10.0, -0.02
+        r.set_params(p)
+        torch.cuda.synchronize()
+        r.nn_train(stream=stream)
+        r.render(wl.camera(), 96, 80, light=wl.light(), out=out, stream=stream)
+        torch.cuda.synchronize()
+        weights.append(r.nn_weights())
+        images.append(out.clone())
+        r.collect_stats(True)
+        r.render(wl.camera(), 96, 80, light=wl.light(), out=out, stream=stream)
+        assert r.stats().fallback_samples > 0
+    assert np.array_equal(weights[0], weights[1])
+    assert float((images[0] - images[1]).abs().max()) <= 2e-5  # 300 samples of colours below 1: 300 x 2^-24
