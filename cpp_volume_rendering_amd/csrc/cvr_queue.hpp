@@ -465,10 +465,11 @@ __device__ __forceinline__ void plain_march(const RayFrame& rf, const VolGeom& g
           acc.z = __builtin_fmaf(spec[2], ws, acc.z);
         }
         mine *= l.m;
+        // (here, not for every lane: a transparent entry's colour may be anything, and 0 x NaN is NaN)
+        acc.x = __builtin_fmaf(mine, src.x, acc.x);
+        acc.y = __builtin_fmaf(mine, src.y, acc.y);
+        acc.z = __builtin_fmaf(mine, src.z, acc.z);
       }
-      acc.x = __builtin_fmaf(mine, src.x, acc.x);
-      acc.y = __builtin_fmaf(mine, src.y, acc.y);
-      acc.z = __builtin_fmaf(mine, src.z, acc.z);
       acc.w = row_last(wa);
       nshade += opaque && taken;
     }

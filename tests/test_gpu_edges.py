@@ -234,3 +234,20 @@ def test_training_and_first_frame_on_a_non_blocking_stream():
         assert r.stats().fallback_samples > 0
     assert np.array_equal(weights[0], weights[1])
     assert float((images[0] - images[1]).abs().max()) <= 2e-5  # 300 samples of colours below 1: 300 x 2^-24
+
+
+@pytest.mark.parametrize("tech,params", [(N.RC1P, {}), (N.RC1P, {"apply_gradient_shading": 1}), (N.EBS, {"light_cache": 1}),
+                                         (N.EBS, {}), (N.CONE_TRACE, {})])
+@pytest.mark.parametrize("w,h", [(90, 70), (900, 700)])
+def test_colours_of_transparent_entries_do_not_count(tech, params, w, h):
+    """Entries that are fully transparent, and no opaque sample's neighbours, may hold any colour: NaN gives
+    the frame that 0 gives (bit for bit where a pixel's sum has one order)."""
+    wl = W.cone_blobs(n=32, width=w, height=h, seed=12)
+    frames = []
+    for colour in (0.0, float("inf")):  # the table is NaN between an infinite point and the next
+        wl.rgb_iso = np.array([[colour] * 3 + [0], [0.6, 0.4, 0.7, 20], [0.9, 0.3, 0.5, 255]])
+        wl.alpha_iso = np.array([[0, 0], [0, 40], [0.3, 130], [0.8, 255]])
+        frames.append(handle(tech, wl, **params).render(wl.camera(), w, h, light=wl.light()))
+    assert frames[0][..., 3].max() > 0.3
+    assert np.isfinite(frames[1]).all()
+    assert np.abs(frames[0] - frames[1]).max() <= (1e-5 if tech == N.CONE_TRACE or not params else 0.0)
