@@ -572,6 +572,29 @@ __device__ __forceinline__ void lane_pixel(const RayFrame& rf, int first, int& p
   py = ty * 16 + (w >> 1) * 8 + (lane >> 3);
 }
 
+// The batch's work: tiles of an image in supertiles of 64, dealt to the queues in turn, each cut into kCuts
+// items.
+constexpr int kQueues = 8, kCuts = 4;
+struct BatchShape {
+  int tiles_x, tiles_y, tw_log2, span, nq, nvols;
+};
+// Tiles of one image in queue q.
+__host__ __device__ inline int queue_tiles(const BatchShape& s, int q) {
+  const int t = s.tiles_x * s.tiles_y, st = (t + 63) >> 6;  // tiles, supertiles
+  if (q >= st) return 0;
+  const int mine = (st - 1 - q) / s.nq + 1;
+  return (st - 1) % s.nq == q ? (mine - 1) * 64 + t - (st - 1) * 64 : mine * 64;
+}
+// The shape of a batch of w x h images, at most `jobs` of them of one volume.  A volume's items of a queue are
+// counted in 32 bits, with room for the wavefronts that find none left: where one queue would hold 2^31 items
+// (64 images of 2^26 x 1) there are kQueues.
+inline BatchShape batch_shape(int w, int h, int tw_log2, int span, int queues, int nvols, int jobs) {
+  const int tw = 1 << tw_log2, th = (64 >> tw_log2) * span;
+  BatchShape s{(w + tw - 1) / tw, (h + th - 1) / th, tw_log2, span, queues, nvols};
+  if ((long long)queue_tiles(s, 0) * kCuts * jobs >= (1ll << 31) - (1 << 20)) s.nq = kQueues;
+  return s;
+}
+
 // How many of 8 x 8 rays of the frame, the corners' included, hit the volume's box.
 inline int frame_hits(const RayFrame& rf, const VolGeom& g) {
   int n = 0;

@@ -43,24 +43,12 @@ struct JobDesc {
   int vol;
 };
 
-constexpr int kQueues = 8, kMaxVolumes = 64;
+constexpr int kMaxVolumes = 64;
 
 // The jobs of one volume (a range of the job order), largest volume first.
 struct VolJobs {
   int vol, first, count;
 };
-// Tiles of an image in supertiles of 64, dealt to the queues in turn, each cut into kCuts items.
-constexpr int kCuts = 4;
-struct BatchShape {
-  int tiles_x, tiles_y, tw_log2, span, nq, nvols;
-};
-// Tiles of one image in queue q.
-__host__ __device__ inline int queue_tiles(const BatchShape& s, int q) {
-  const int t = s.tiles_x * s.tiles_y, st = (t + 63) >> 6;  // tiles, supertiles
-  if (q >= st) return 0;
-  const int mine = (st - 1 - q) / s.nq + 1;
-  return (st - 1) % s.nq == q ? (mine - 1) * 64 + t - (st - 1) * 64 : mine * 64;
-}
 
 // The pixels of an item: from pixel `first` of a stack of wave tiles, row by row.
 struct TilePixels {
@@ -212,7 +200,7 @@ struct cvr_batch {
   unsigned int* d_heads = nullptr;
   unsigned long long* d_counters = nullptr;
   size_t cap_vols = 0, cap_jobs = 0, cap_vjobs = 0, cap_order = 0;
-  int n_vjobs = 0;
+  int n_vjobs = 0, most_jobs = 0;  // volumes with jobs, jobs of the one with most
   int max_ntf = 0;
   // graph of (reset, render) for the current jobs / tuning / output
   hipStream_t cap = nullptr;
@@ -352,6 +340,8 @@ int build_tables(cvr_batch* b) {
     ++vj.back().count;
   }
   b->n_vjobs = int(vj.size());
+  b->most_jobs = 0;
+  for (const VolJobs& v : vj) b->most_jobs = std::max(b->most_jobs, v.count);
   int rc;
   if ((rc = grow(reinterpret_cast<void**>(&b->d_vols), b->cap_vols, vd.size() * sizeof(VolDesc)))) return rc;
   if ((rc = grow(reinterpret_cast<void**>(&b->d_jobs), b->cap_jobs, jd.size() * sizeof(JobDesc)))) return rc;
@@ -370,8 +360,8 @@ int build_graph(cvr_batch* b, float* out) {
   int ncu = 0;
   CVR_HIP_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, b->device));
   const int grid = std::max(1, ncu * b->tune.workgroups_per_cu);
-  const int tl = tw_log2_of(b->tune.tile_w), tw = 1 << tl, th = (64 >> tl) * b->tune.span;
-  const BatchShape bs{(b->W + tw - 1) / tw, (b->H + th - 1) / th, tl, b->tune.span, b->tune.queues, b->n_vjobs};
+  const BatchShape bs = batch_shape(b->W, b->H, tw_log2_of(b->tune.tile_w), b->tune.span, b->tune.queues, b->n_vjobs,
+                                    b->most_jobs);
   const size_t shm = size_t(b->max_ntf) * sizeof(float4);
   CVR_HIP_CHECK(hipStreamBeginCapture(b->cap, hipStreamCaptureModeThreadLocal));
   hipLaunchKernelGGL(k_batch_reset, dim3(1), dim3(kQueues * kMaxVolumes), 0, b->cap, b->d_heads, b->d_counters);

@@ -11,7 +11,14 @@ SOURCE = r"""
 #include <cstdio>
 #include <cstdlib>
 using namespace cvr;
-int main(int, char** v) {
+int main(int n, char** v) {
+  if (n == 7) {
+    const BatchShape b = batch_shape(std::atoi(v[1]), std::atoi(v[2]), std::atoi(v[3]), std::atoi(v[4]), std::atoi(v[5]), 1,
+                                     std::atoi(v[6]));
+    std::printf("%d %d %d\n", b.tiles_x, b.tiles_y, b.nq);
+    for (int q = 0; q < b.nq; ++q) std::printf("%d\n", queue_tiles(b, q));
+    return 0;
+  }
   const int w = std::atoi(v[1]), h = std::atoi(v[2]), rays = std::atoi(v[3]), parts = std::atoi(v[4]);
   const QueueShape q = queue_shape(w, h, rays, parts, 64);
   std::printf("%d %d\n", q.tile_log2, q.blocks);
@@ -49,3 +56,18 @@ def test_launches_cover_a_frame_within_the_limit_of_lanes(shapes, w, h, rays, pa
         assert first == at and 0 < n and n * 256 < 1 << 32
         at += n
     assert at == blocks
+
+
+# images a call may have (2^26 pixels, 2^32 in all), flat ones above all: a tile is 4 x 16 span pixels
+@pytest.mark.parametrize("queues", [1, 8])
+@pytest.mark.parametrize("w,h,tw_log2,span,jobs", [(1, 1, 2, 1, 1), (333, 64, 3, 1, 5), (8192, 8192, 2, 1, 64),
+                                                   (1 << 26, 1, 2, 8, 64), (1 << 26, 1, 2, 1, 64), (1, 1 << 26, 5, 1, 64),
+                                                   (1 << 26, 1, 2, 1, 32), (1 << 22, 16, 2, 1, 64)])
+def test_batch_items_are_counted_in_32_bits(shapes, w, h, tw_log2, span, queues, jobs):
+    (tx, ty, nq), *tiles = shapes(w, h, tw_log2, span, queues, jobs)
+    assert tx == -(-w // (1 << tw_log2))
+    assert ty == -(-h // ((64 >> tw_log2) * span))
+    assert sum(t for t, in tiles) == tx * ty and len(tiles) == nq
+    items = [t * 4 * jobs for t, in tiles]
+    assert max(items) < (1 << 31) - (1 << 20)
+    assert nq == (queues if sum(items) < (1 << 31) - (1 << 20) else 8)
