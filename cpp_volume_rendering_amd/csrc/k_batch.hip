@@ -545,13 +545,11 @@ int cvr_batch_render(cvr_batch_handle b, float* out, void* hip_stream) {
   if (b->jobs.empty()) { set_error("cvr_batch_render: no jobs"); return CVR_ERR_STATE; }
   Guard gd(b->device);
   int rc;
-  if (!b->tables_dirty && members_changed(b)) {
-    // a member's buffers or network changed: wait for replays that may still read the
-    // old ones before the tables are rebuilt
-    CVR_HIP_CHECK(hipStreamSynchronize(static_cast<hipStream_t>(hip_stream)));
+  // jobs, the step, a member's buffers or network changed: wait for replays on any stream that may still
+  // read the old tables before they are rebuilt
+  if (b->tables_dirty || members_changed(b)) {
     b->tables_dirty = true;
-  }
-  if (b->tables_dirty) {
+    CVR_HIP_CHECK(hipDeviceSynchronize());
     if ((rc = build_tables(b))) return rc;
     b->dirty = true;
   }

@@ -251,3 +251,33 @@ def test_colours_of_transparent_entries_do_not_count(tech, params, w, h):
     assert frames[0][..., 3].max() > 0.3
     assert np.isfinite(frames[1]).all()
     assert np.abs(frames[0] - frames[1]).max() <= (1e-5 if tech == N.CONE_TRACE or not params else 0.0)
+
+
+def test_new_jobs_wait_for_the_images_in_flight():
+    """New jobs right after a batch was queued on a non-blocking stream, drawn on another into another
+    buffer: the first images are those of the first jobs."""
+    import torch
+
+    wl = W.cone_blobs(n=64, width=256, height=256, seed=8)
+    r = handle(N.CONE_NN, wl)
+    r.nn_set_weights(np.random.default_rng(2).normal(0, 0.1, N.lib().cvr_nn_param_count()).astype(np.float32))
+    r.prepare()
+    b = N.Batch(256, 256)
+    m = b.add_volume(r)
+    jobs = [[(m, wl.camera(az, 10.0), wl.light()) for az in range(a, a + 32)] for a in (0, 180)]
+    s, t = torch.cuda.Stream(), torch.cuda.Stream()
+    out = torch.zeros((4, 32, 256, 256, 4), device="cuda:0")
+    torch.cuda.synchronize()
+    for k in (0, 1):
+        b.set_jobs(jobs[k])
+        b.render(out[k], stream=s.cuda_stream)
+        torch.cuda.synchronize()
+    b.set_jobs(jobs[0])
+    b.render(out[2], stream=s.cuda_stream)
+    torch.cuda.synchronize()
+    b.render(out[2], stream=s.cuda_stream)
+    b.set_jobs(jobs[1])
+    b.render(out[3], stream=t.cuda_stream)
+    torch.cuda.synchronize()
+    assert float((out[0] - out[1]).abs().max()) > 0.1
+    assert float((out[2:] - out[:2]).abs().max()) <= 2e-5  # the order of a pixel's sums: 300 x 2^-24
