@@ -161,11 +161,19 @@ __device__ __forceinline__ float border_falloff(const PyrGeom& pg, f3 tp, float 
 // some lane begins outside it (cvr_cone_eval takes any point; a march's samples may lie outside
 // by the rounding of their ray, which kEdge allows for: the falloff there is 1 to two ulps).
 constexpr float kEdge = 1.0f / 4096.0f;
+// The same of one component: an axis of component 0, of either sign, never leaves (a directional light's cones
+// along an axis have two).
+__host__ __device__ __forceinline__ float axis_exit(float a, float q, float G) {
+  if (!(q >= -kEdge && q <= G + kEdge)) return -INFINITY;
+  return a == 0.f ? INFINITY : ((a > 0.f ? G : 0.f) - q) / a;
+}
 __device__ __forceinline__ float wave_exit(const PyrGeom& pg, f3 p, f3 axis) {
-  auto leave = [&](float a, float q, float G) {
-    return q >= -kEdge && q <= G + kEdge ? ((a > 0.f ? G : 0.f) - q) / a : -INFINITY;
-  };
-  return wave_min(fminf(leave(axis.x, p.x, pg.G[0]), fminf(leave(axis.y, p.y, pg.G[1]), leave(axis.z, p.z, pg.G[2]))));
+  return wave_min(fminf(axis_exit(axis.x, p.x, pg.G[0]),
+                        fminf(axis_exit(axis.y, p.y, pg.G[1]), axis_exit(axis.z, p.z, pg.G[2]))));
+}
+// About how many of a cone's n steps lie up to `te`: clamped before the conversion, as te may be any number.
+__host__ __device__ __forceinline__ int steps_up_to(float log2_te, const ConeSched& S) {
+  return int(fminf(fmaxf(floorf((log2_te - S.log2_t0) * S.inv_log2_q) + 1.0f, 0.0f), float(S.n)));
 }
 // The levels of a pyramid as the marches read them (kMaxLevels rows).
 std::vector<ConeLevel> cone_levels(const PyrGeom& pg);
@@ -185,8 +193,7 @@ __device__ __forceinline__ float cone_T(const void* __restrict__ pyr, const PyrG
   const ConstLevels lev = (ConstLevels)(uintptr_t)levels;
   // the steps up to which every lane's cone axis is inside the box
   const float te = wave_exit(pg, p, axis);
-  int jin = min(max(int(floorf((__log2f(te) - S.log2_t0) * S.inv_log2_q)) + 1, 0), S.n);
-  jin = __builtin_amdgcn_readfirstlane(jin);
+  int jin = __builtin_amdgcn_readfirstlane(steps_up_to(__log2f(te), S));
   while (jin > 0 && !(s[jin - 1].tm <= te)) --jin;
   float od = 0.f;
   auto step = [&](auto two, auto border, int j) {

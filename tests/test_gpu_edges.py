@@ -281,3 +281,23 @@ def test_new_jobs_wait_for_the_images_in_flight():
     torch.cuda.synchronize()
     assert float((out[0] - out[1]).abs().max()) > 0.1
     assert float((out[2:] - out[:2]).abs().max()) <= 2e-5  # the order of a pixel's sums: 300 x 2^-24
+
+
+@pytest.mark.parametrize("tech", [N.CONE_TRACE, N.DOS])
+@pytest.mark.parametrize("fwd", [(0.0, 1.0, 0.0), (-0.0, -1.0, 0.0), (0.0, 0.0, 1.0), (1.0, 0.0, -0.0)])
+def test_lights_along_an_axis(tech, fwd):
+    wl = W.cone_blobs(n=48, width=40, height=33, seed=17)
+    cam, light = wl.camera(), W.light_from_direction(fwd, wl.grid)
+    light.forward[:] = fwd
+    r = handle(tech, wl)
+    if tech == N.DOS:
+        r.set_params(apply_shadow=1, shadow_type=2)
+    img = r.render(cam, 40, 33, light=light)
+    tf = O.OTF(wl.rgb_iso, wl.alpha_iso)
+    pyr = O.OPyr.wrap(wl.grid, [a.astype(np.float64) for a in r.pyramid()])
+    if tech == N.DOS:
+        ref, m = O.render_dos(wl.volume, tf, pyr, O.dos_params(r.params(), wl.grid, light), cam, 40, 33)
+    else:
+        ref, m = O.render_cone(wl.volume, tf, pyr, O.cone_params(wl.grid, light), cam, 40, 33)
+    assert ref[..., 3].max() > 0.3
+    check(img, ref, m)

@@ -71,3 +71,39 @@ def test_batch_items_are_counted_in_32_bits(shapes, w, h, tw_log2, span, queues,
     items = [t * 4 * jobs for t, in tiles]
     assert max(items) < (1 << 31) - (1 << 20)
     assert nq == (queues if sum(items) < (1 << 31) - (1 << 20) else 8)
+
+
+EXITS = r"""
+#include "cvr_cone.hpp"
+#include <cstdio>
+using namespace cvr;
+int main() {
+  const float G = 32.f, inf = INFINITY;
+  for (float zero : {0.f, -0.f})
+    for (float q : {0.f, 5.f, 32.f, -1e-4f, 32.f + 1e-4f})
+      if (axis_exit(zero, q, G) != inf) return 1;
+  if (axis_exit(0.5f, 30.f, G) != 4.f || axis_exit(-0.5f, 3.f, G) != 6.f || axis_exit(1.f, 32.f, G) != 0.f) return 2;
+  for (float a : {0.f, -0.f, 1.f, -1.f, 0.1f})
+    for (float q : {-0.01f, 32.01f, -inf, inf})
+      if (axis_exit(a, q, G) != -inf) return 3;
+  ConeSched S{};
+  S.n = 64;
+  S.log2_t0 = 0.f;
+  for (float r : {8.f, 0.25f, inf}) {
+    S.inv_log2_q = r;
+    for (float t : {-inf, inf, NAN, -1000.f, 1e30f, 0.f, 3.7f})
+      if (steps_up_to(t, S) < 0 || steps_up_to(t, S) > 64) return 4;
+    if (steps_up_to(inf, S) != 64 || steps_up_to(-inf, S) != 0 || steps_up_to(NAN, S) != 0) return 5;
+  }
+  S.inv_log2_q = 8.f;
+  return steps_up_to(2.f, S) == 17 && steps_up_to(1.99f, S) == 16 ? 0 : 6;
+}
+"""
+
+
+def test_cones_along_an_axis_leave_by_the_others(tmp_path):
+    (tmp_path / "e.hip").write_text(EXITS)
+    subprocess.run([B.HIPCC, "-O1", "-std=c++17", f"-I{B.INCLUDE}", f"-I{B.CSRC}", "-x", "hip", "--offload-host-only",
+                    f"--offload-arch={B.ARCH}", str(tmp_path / "e.hip"), "-o", str(tmp_path / "e")], check=True,
+                   capture_output=True)
+    assert subprocess.run([str(tmp_path / "e")]).returncode == 0
