@@ -50,8 +50,8 @@ struct DosK {
 // falloff, which is 1 there.
 template <int F, bool kWide>
 __device__ __forceinline__ float dos_cone(const void* __restrict__ pyr, const PyrGeom& pg, const DosConeK& C,
-                                          const ConeLevel* __restrict__ levels, const DosRow* __restrict__ table, f3 p,
-                                          f3 k, f3 uy, f3 vx) {
+                                          const ConeLevel* __restrict__ levels, const DosRow* __restrict__ table,
+                                          bool inside, f3 p, f3 k, f3 uy, f3 vx) {
   typedef const __attribute__((address_space(4))) DosRow* ConstRows;
   const ConstRows rows = (ConstRows)(uintptr_t)table;
   const ConstLevels lev = (ConstLevels)(uintptr_t)levels;
@@ -74,7 +74,7 @@ __device__ __forceinline__ float dos_cone(const void* __restrict__ pyr, const Py
   // with 2, 13.5 with 4, 12.6 with 8, 12.4 with 10, whose remainders cost small volumes more; the
   // 7-packing's registers are more than any of them need)
   constexpr int kAhead = 8;
-  const float te = wave_exit(pg, p, k);
+  const float te = wave_exit(pg, inside, p, k);
   auto group = [&](auto border) {
     float at[kAhead];
 #pragma unroll
@@ -95,9 +95,9 @@ __device__ __forceinline__ float dos_cone(const void* __restrict__ pyr, const Py
   for (int j = 0; j < 3; ++j) d3[j] = k * C.ax[j][2] + uy * C.ax[j][1] + vx * C.ax[j][0];
   auto sections = [&](auto count, const f3* d, int e) {
     constexpr int kN = decltype(count)::value;
-    float t = wave_exit(pg, p, d[0]);
+    float t = wave_exit(pg, inside, p, d[0]);
 #pragma unroll
-    for (int j = 1; j < kN; ++j) t = fminf(t, wave_exit(pg, p, d[j]));
+    for (int j = 1; j < kN; ++j) t = fminf(t, wave_exit(pg, inside, p, d[j]));
     for (; i < e; ++i) {
       float at[kN];
       if (rows[i].track <= t) {
@@ -134,8 +134,8 @@ __device__ __forceinline__ float dos_cone(const void* __restrict__ pyr, const Py
 
 // Shadow cone of ShadowEvaluationKernel (:533-562).  `wp` is the world position.
 template <int F, bool kWide>
-__device__ __forceinline__ float dos_shadow(const void* __restrict__ pyr, const PyrGeom& pg, const DosK& K, f3 p,
-                                            f3 wp) {
+__device__ __forceinline__ float dos_shadow(const void* __restrict__ pyr, const PyrGeom& pg, const DosK& K, bool inside,
+                                            f3 p, f3 wp) {
   f3 k = ld3(K.lfwd), up = ld3(K.lup), right = ld3(K.lright);
   if (K.shadow_type != 2) {
     k = norm3(ld3(K.lpos) - wp);
@@ -144,16 +144,17 @@ __device__ __forceinline__ float dos_shadow(const void* __restrict__ pyr, const 
     up = norm3(cross3(k, u1));
     right = u1;
   }
-  return dos_cone<F, kWide>(pyr, pg, K.sdw, K.lev, K.sdw_rows, p, k, up, right);
+  return dos_cone<F, kWide>(pyr, pg, K.sdw, K.lev, K.sdw_rows, inside, p, k, up, right);
 }
 // Both terms at p: the occlusion cone along k in the frame (up, right); 0 for one that is off.
 template <int F>
 __device__ __forceinline__ void dos_light(const void* __restrict__ pyr, const PyrGeom& pg, const DosK& K, f3 p, f3 wp, f3 k,
                                           f3 up, f3 right, float& Io, float& Is) {
+  const bool inside = wave_inside(pg, p);
   auto both = [&](auto wide) {
     constexpr bool kWide = decltype(wide)::value;
-    Io = K.apply_occ ? dos_cone<F, kWide>(pyr, pg, K.occ, K.lev, K.occ_rows, p, k, up, right) : 0.f;
-    Is = K.apply_sdw ? dos_shadow<F, kWide>(pyr, pg, K, p, wp) : 0.f;
+    Io = K.apply_occ ? dos_cone<F, kWide>(pyr, pg, K.occ, K.lev, K.occ_rows, inside, p, k, up, right) : 0.f;
+    Is = K.apply_sdw ? dos_shadow<F, kWide>(pyr, pg, K, inside, p, wp) : 0.f;
   };
   if (pg.wide) both(std::true_type{});
   else both(std::false_type{});

@@ -80,12 +80,15 @@ using namespace cvr;
 int main() {
   const float G = 32.f, inf = INFINITY;
   for (float zero : {0.f, -0.f})
-    for (float q : {0.f, 5.f, 32.f, -1e-4f, 32.f + 1e-4f})
+    for (float q : {0.f, 5.f, 32.f})
       if (axis_exit(zero, q, G) != inf) return 1;
   if (axis_exit(0.5f, 30.f, G) != 4.f || axis_exit(-0.5f, 3.f, G) != 6.f || axis_exit(1.f, 32.f, G) != 0.f) return 2;
-  for (float a : {0.f, -0.f, 1.f, -1.f, 0.1f})
-    for (float q : {-0.01f, 32.01f, -inf, inf})
-      if (axis_exit(a, q, G) != -inf) return 3;
+  const float box[3] = {32.f, 16.f, 8.f};
+  for (float e : {0.f, 1e-4f, -1e-4f})
+    if (!in_box(box, f3{e, 4.f, 8.f + e}) || !in_box(box, f3{32.f + e, e, 8.f})) return 3;
+  for (float q : {-0.01f, -inf, inf, NAN})
+    if (in_box(box, f3{q, 4.f, 4.f}) || in_box(box, f3{4.f, q, 4.f}) || in_box(box, f3{4.f, 4.f, q})) return 3;
+  if (in_box(box, f3{32.01f, 4.f, 4.f}) || in_box(box, f3{4.f, 16.01f, 4.f}) || in_box(box, f3{4.f, 4.f, 8.01f})) return 3;
   ConeSched S{};
   S.n = 64;
   S.log2_t0 = 0.f;
