@@ -301,3 +301,116 @@ def test_lights_along_an_axis(tech, fwd):
         ref, m = O.render_cone(wl.volume, tf, pyr, O.cone_params(wl.grid, light), cam, 40, 33)
     assert ref[..., 3].max() > 0.3
     check(img, ref, m)
+
+
+def test_volume_of_more_than_4_gib_of_corner_blocks():
+    """64-bit block offsets, which volumes from 4 GiB of blocks on take: the camera rays of the plain march
+    (lane groups) and of the queue, and light rays, against the oracle."""
+    nx, ny, nz = 840, 830, 784
+    ax = [np.sin(np.linspace(0, k * np.pi, n)) ** 2 for n, k in ((nx, 3), (ny, 2), (nz, 5))]
+    vol = (255.0 * ax[2][:, None, None]).astype(np.float32) * ax[1][:, None].astype(np.float32) * ax[0].astype(np.float32)
+    vol = vol.astype(np.uint8)
+    assert vol.size * 8 > 1 << 32
+    grid, tf = (float(nx), float(ny), float(nz)), W.seeded_tf(107, 4)
+    tf[1][:, 0] *= 0.02  # rays go far into the volume
+    w, h = 24, 18
+    cam, light, otf = W.orbit_camera(grid, w, h, dist_diag=0.9), W.light_from_direction((-0.4, 0.7, 0.6), grid), O.OTF(*tf)
+    for tech in (N.RC1P, N.CONE_GT):
+        r = N.Renderer(tech)
+        r.set_volume(vol)
+        r.set_transfer_function(*tf)
+        if tech == N.CONE_GT:
+            r.set_params(occ_rays=1, sdw_rays=1, shadow_type=2, occ_max_dist=40.0, sdw_max_dist=40.0)
+        img = r.render(cam, w, h, light=light)
+        if tech == N.RC1P:
+            ref, m = O.render_rc1p(vol, otf, cam, w, h)
+        else:
+            ref, m = O.render_gt(vol, otf, O.gt_params(r.params(), grid, light), cam, w, h)
+        assert ref[..., 3].max() > 0.3
+        check(img, ref, m)
+
+
+def test_surrogate_frame_of_two_units_a_wavefront():
+    """2112 x 2112 pixels are more workgroups than there are marks: each takes two sets of rays.  The
+    network's frame against the oracle, the frame of the second pass alone against the cone tracer's, and the
+    first again when no mark is left."""
+    w = h = 2112
+    wl = W.cone_blobs(n=24, width=w, height=h, seed=33)
+    cam, light = wl.camera(), wl.light()
+    r, c = handle(N.CONE_NN, wl), handle(N.CONE_TRACE, wl)
+    p = r.params()
+    p.cone.density_precision = 0
+    r.set_params(p)
+    c.set_params(p.cone)
+    wts = np.random.default_rng(4).normal(0, 0.1, N.lib().cvr_nn_param_count()).astype(np.float32)
+    r.nn_set_weights(wts)
+    first = r.render(cam, w, h, light=light)
+    pyr = O.OPyr.wrap(wl.grid, [a.astype(np.float64) for a in r.pyramid()])
+    tf = O.OTF(wl.rgb_iso, wl.alpha_iso)
+    ref, m, _ = O.render_nn(wl.volume, tf, pyr, O.cone_params(wl.grid, light), wts, cam, w, h, stride=33)
+    img = np.zeros_like(first)
+    img[::33, ::33] = first[::33, ::33]
+    assert ref[: h // 2, ..., 3].max() > 0.2 and ref[h // 2:, ..., 3].max() > 0.2
+    check(img, ref, m, 33)
+    p.ood_margin = -2e30  # no input is in range
+    r.set_params(p)
+    r.collect_stats(True)
+    exact = r.render(cam, w, h, light=light)
+    st = r.stats()
+    assert st.fallback_samples == st.shaded_samples > 0
+    assert np.abs(exact - c.render(cam, w, h, light=light)).max() <= 2e-5
+    p.ood_margin = 0.02
+    r.set_params(p)
+    assert np.array_equal(r.render(cam, w, h, light=light), first) and r.stats().fallback_samples == 0
+
+
+def test_gradient_of_more_samples_than_the_kept_buffer_holds():
+    """940032 samples (64.5 MiB) go through device buffers: the mean of the halves' gradients.  Sums of 14688
+    slabs of one sign in any order: 14688 x 2^-24 of the largest at most."""
+    rng, half = np.random.default_rng(6), 470016
+    r = N.Renderer(N.CONE_NN)
+    r.nn_set_weights(rng.normal(0, 0.2, N.lib().cvr_nn_param_count()).astype(np.float32))
+    X, T = rng.random((2 * half, 16), np.float32), np.full((2 * half, 2), 2.0, np.float32)
+    assert X.nbytes + T.nbytes > 64 << 20
+    (l, g), (la, ga), (lb, gb) = r.nn_gradient(X, T), r.nn_gradient(X[:half], T[:half]), r.nn_gradient(X[half:], T[half:])
+    assert abs(l - 0.5 * (la + lb)) <= 9e-4 * l
+    assert np.abs(g - 0.5 * (ga + gb)).max() <= 9e-4 * np.abs(g).max()
+
+
+@pytest.mark.parametrize("tech,entries", [(N.CONE_TRACE, 4096), (N.DOS, 4096), (N.CONE_GT, 4096), (N.EBS, 4096), (N.CONE_NN, 2048)])
+def test_largest_transfer_functions(tech, entries):
+    """The tables of most entries beside the queues in LDS."""
+    wl = W.cone_blobs(n=32, width=40, height=33, seed=19)
+    cam, light, md = wl.camera(), wl.light(), entries - 1
+    rgb, al = W.seeded_tf(119, 5, max_density=md)
+    r = N.Renderer(tech)
+    r.set_volume(wl.volume)
+    r.set_transfer_function(rgb, al, max_density=md)
+    wts = np.random.default_rng(5).normal(0, 0.1, N.lib().cvr_nn_param_count()).astype(np.float32)
+    if tech == N.CONE_NN:
+        p = r.params()
+        p.cone.density_precision = 0
+        r.set_params(p)
+        r.nn_set_weights(wts)
+    elif tech == N.DOS:
+        r.set_params(apply_shadow=1, shadow_type=2)
+    elif tech == N.CONE_GT:
+        r.set_params(occ_rays=4, sdw_rays=2, shadow_type=2)
+    img = r.render(cam, 40, 33, light=light)
+    tf = O.OTF(rgb, al, max_density=md)
+    if tech == N.EBS:
+        prm = O.ebs_params(r.params(), light)
+        prm.sdw_max_dist = np.float32(0.75) * np.float32(np.linalg.norm(wl.grid))
+        ref, m = O.render_ebs(wl.volume, tf, O.sat(wl.volume, tf), prm, cam, 40, 33)
+    elif tech == N.CONE_GT:
+        ref, m = O.render_gt(wl.volume, tf, O.gt_params(r.params(), wl.grid, light), cam, 40, 33)
+    else:
+        pyr = O.OPyr.wrap(wl.grid, [a.astype(np.float64) for a in r.pyramid()])
+        if tech == N.DOS:
+            ref, m = O.render_dos(wl.volume, tf, pyr, O.dos_params(r.params(), wl.grid, light), cam, 40, 33)
+        elif tech == N.CONE_TRACE:
+            ref, m = O.render_cone(wl.volume, tf, pyr, O.cone_params(wl.grid, light), cam, 40, 33)
+        else:
+            ref, m, _ = O.render_nn(wl.volume, tf, pyr, O.cone_params(wl.grid, light), wts, cam, 40, 33)
+    assert ref[..., 3].max() > 0.3
+    check(img, ref, m)
