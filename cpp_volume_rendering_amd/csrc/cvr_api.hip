@@ -232,6 +232,7 @@ static void free_all(cvr_ctx* c) {
   if (c->d_gt_rays) (void)hipFree(c->d_gt_rays);
   if (c->d_lc) (void)hipFree(c->d_lc);
   if (c->d_grad) (void)hipFree(c->d_grad);
+  if (c->d_short) (void)hipFree(c->d_short);
   if (c->d_ebs_rows) (void)hipFree(c->d_ebs_rows);
   for (void* p : {static_cast<void*>(c->d_nn_w), static_cast<void*>(c->d_nn_g), static_cast<void*>(c->d_nn_m),
                   static_cast<void*>(c->d_nn_v), c->d_nn_pack, c->d_nn_tpack,

@@ -173,6 +173,9 @@ struct cvr_ctx {
   int lc_res[3] = {0, 0, 0};
   bool lc_valid = false;
 
+  int* d_short = nullptr;  // short_tiles of the frame in work
+  size_t short_cap = 0;
+
   // stats
   bool collect_stats = false;
   unsigned long long* d_counters = nullptr;
@@ -214,6 +217,9 @@ int lc_prepare(cvr_ctx* c, const int res[3]);
 int launch_lc_render(cvr_ctx* c, const RayFrame& rf, int apply_occ, int apply_sdw, float ka, float kd, float step,
                      float et, const PhongK& ph, float* out, hipStream_t st);
 int launch_ebs(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out, hipStream_t st);
+// which tiles of a frame have short rays (QueueShape::short_tiles), null if the frame is dealt out in one way
+int short_tiles(cvr_ctx* c, const RayFrame& rf, float step, float et, int px_per_sample, hipStream_t st,
+                const int** tiles);
 // a device buffer of exactly `bytes`: *p if it has that size, else a new one in its place
 int sized_buffer(void** p, size_t* have, size_t bytes);
 int build_volume_oct(cvr_ctx* c, hipStream_t st);

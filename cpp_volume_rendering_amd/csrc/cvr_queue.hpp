@@ -136,6 +136,8 @@ __host__ __device__ inline long long tiled_pixels(int w, int h, int tile_log2) {
 // them (for_launches).
 struct QueueShape {
   int rays, tile_log2, blocks, xcd_log2, first;
+  const int* short_tiles;  // if not null, per tile of 64 x 64 pixels: this launch draws those whose entry is `want`
+  int want;
 };
 // Tiles of 64 x 64 pixels: a unit's rays lie 32 (rays 4) or 16 (rays 16) pixels apart, so long
 // and short ones mix, while the units that run at once stay together (256^3 cone-traced frame
@@ -143,12 +145,19 @@ struct QueueShape {
 // Narrower frames take smaller tiles, of a unit's rays at least.  xcd_px: pixels an XCD takes in a row.
 inline QueueShape queue_shape(int w, int h, int rays, int parts, int xcd_px, int waves = 4) {
   const int side = w < h ? w : h;
-  QueueShape q{rays, 2, 0, 0, 0};
+  QueueShape q{rays, 2, 0, 0, 0, nullptr, 0};
   while (q.tile_log2 < 6 && (1 << q.tile_log2 < side || 1 << (2 * q.tile_log2) < rays)) ++q.tile_log2;
   const int per_wg = rays * waves / parts;  // pixels of a workgroup
   q.blocks = int((tiled_pixels(w, h, q.tile_log2) + per_wg - 1) / per_wg);
   while (per_wg << q.xcd_log2 < xcd_px) ++q.xcd_log2;
   return q;
+}
+// How the tiles of short rays of a frame of shape q are dealt out: `rays` to a wavefront.
+inline QueueShape short_shape(const RayFrame& rf, const QueueShape& q, int rays) {
+  QueueShape s = queue_shape(rf.W, rf.H, rays, 1, 256);
+  s.short_tiles = q.short_tiles;
+  s.want = 1;
+  return s;
 }
 // A frame of 2^28 pixels takes up to 2^36 lanes (64 a pixel where four wavefronts share four rays):
 // launch(shape, workgroups) for each launch of it.
@@ -162,6 +171,13 @@ template <class F> inline void for_launches(QueueShape q, int total, int threads
 template <int kParts> __device__ __forceinline__ int queue_unit(const QueueShape& q) {
   const int waves = int(blockDim.x) >> 6, bid = q.first + xcd_remap(blockIdx.x, gridDim.x, q.xcd_log2);
   return kParts > 1 ? bid : bid * waves + int(threadIdx.x >> 6);
+}
+
+// Whether this launch leaves the workgroup's tile to another (the units of a workgroup are of one tile).
+template <int kParts> __device__ __forceinline__ bool tile_left_out(const QueueShape& q) {
+  if (!q.short_tiles) return false;
+  const int tile = queue_unit<kParts>(q) >> (2 * q.tile_log2 - __builtin_ctz(q.rays));
+  return q.short_tiles[__builtin_amdgcn_readfirstlane(tile)] != q.want;
 }
 
 __device__ __forceinline__ float lane_value(float v, int lane) {

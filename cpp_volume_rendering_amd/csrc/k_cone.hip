@@ -22,14 +22,15 @@
 
 namespace cvr {
 
-constexpr int kRays = 4;
-template <typename T, int F, int kParts>
+constexpr int kRays = 4, kShortRays = 16;
+template <typename T, int F, int kParts, int kRays>
 __global__ __launch_bounds__(256) void k_cone_render(RayFrame rf, VolGeom g, PyrGeom pg, const void* __restrict__ pyr,
                                                      ConeK K, const float4* __restrict__ tf, int ntf, float step,
                                                      float et, QueueShape qs, float4* __restrict__ out,
                                                      unsigned long long* __restrict__ counters) {
   extern __shared__ float4 s_tf[];
   __shared__ WaveQueue<kRays> queue[4];
+  if (tile_left_out<kParts>(qs)) return;
   for (int i = threadIdx.x; i < ntf; i += blockDim.x) s_tf[i] = tf[i];
   __syncthreads();
   const int u = queue_unit<kParts>(qs);
@@ -280,17 +281,22 @@ int launch_cone(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* o
   // small frames: workgroups whose wavefronts share their rays (128^2 1.9 ms, 3.4 ms with rays
   // of their own; 512^2 18.7 and 19.9; 1024^2 70.4 and 68.6)
   const bool shared = size_t(rf.W) * rf.H < (1 << 19);
-  const QueueShape shape = queue_shape(rf.W, rf.H, kRays, shared ? 4 : 1, shared ? 64 : 256);
+  QueueShape shape = queue_shape(rf.W, rf.H, kRays, shared ? 4 : 1, shared ? 64 : 256);
+  if ((rc = short_tiles(c, rf, step, P.et_threshold, 1024, st, &shape.short_tiles))) return rc;
   with_types(c->dtype, c->pyr.fmt, [&](auto t, auto f) {
     using T = typename decltype(t)::type;
-    auto launch = [&](auto parts) {
-      for_launches(shape, shape.blocks, 256, [&](const QueueShape& qs, int blocks) {
-        hipLaunchKernelGGL((k_cone_render<T, decltype(f)::value, decltype(parts)::value>), dim3(blocks), dim3(256), shm,
-                           st, rf, g, c->pyr, c->d_pyr_oct, K, c->d_tf_rgbt, c->tf_size, step, P.et_threshold, qs, o4, cnt);
+    auto launch = [&](const QueueShape& s, auto parts, auto rays) {
+      for_launches(s, s.blocks, 256, [&](const QueueShape& qs, int blocks) {
+        hipLaunchKernelGGL((k_cone_render<T, decltype(f)::value, decltype(parts)::value, decltype(rays)::value>), dim3(blocks),
+                           dim3(256), shm, st, rf, g, c->pyr, c->d_pyr_oct, K, c->d_tf_rgbt, c->tf_size, step,
+                           P.et_threshold, qs, o4, cnt);
       });
     };
-    if (shared) launch(std::integral_constant<int, 4>{});
-    else launch(std::integral_constant<int, 1>{});
+    const std::integral_constant<int, 1> one;
+    const std::integral_constant<int, kRays> few;
+    if (shared) launch(shape, std::integral_constant<int, 4>{}, few);
+    else launch(shape, one, few);
+    if (shape.short_tiles) launch(short_shape(rf, shape, kShortRays), one, std::integral_constant<int, kShortRays>{});
   });
   CVR_HIP_CHECK(hipGetLastError());
   return 0;

@@ -160,8 +160,8 @@ __device__ __forceinline__ void dos_light(const void* __restrict__ pyr, const Py
   else both(std::false_type{});
 }
 
-constexpr int kRays = 4;
-template <typename T, int F, int kParts>
+constexpr int kRays = 4, kShortRays = 16;
+template <typename T, int F, int kParts, int kRays>
 __global__ __launch_bounds__(256) void k_dos_render(RayFrame rf, VolGeom g, PyrGeom pg, const void* __restrict__ pyr,
                                                     DosK K, const float4* __restrict__ tf, int ntf, float step, float et,
                                                     PhongK ph, const float4* __restrict__ grad, QueueShape qs,
@@ -169,6 +169,7 @@ __global__ __launch_bounds__(256) void k_dos_render(RayFrame rf, VolGeom g, PyrG
                                                     unsigned long long* __restrict__ counters) {
   extern __shared__ float4 s_tf[];
   __shared__ WaveQueue<kRays> queue[4];
+  if (tile_left_out<kParts>(qs)) return;
   for (int i = threadIdx.x; i < ntf; i += blockDim.x) s_tf[i] = tf[i];
   __syncthreads();
   const int u = queue_unit<kParts>(qs);
@@ -495,18 +496,22 @@ int launch_dos(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* ou
   // dos_cone: 100 x 100 0.41 ms, 0.82 ms with rays of their own; 200 x 150 0.26 and 0.48; 400 x 300 2.2
   // and 1.7; 1024^2 19.4 and 15.6)
   const bool shared = size_t(rf.W) * rf.H < (1 << 16);
-  const QueueShape shape = queue_shape(rf.W, rf.H, kRays, shared ? 4 : 1, shared ? 64 : 256);
+  QueueShape shape = queue_shape(rf.W, rf.H, kRays, shared ? 4 : 1, shared ? 64 : 256);
+  if ((rc = short_tiles(c, rf, step, P.et_threshold, 1024, st, &shape.short_tiles))) return rc;
   with_types(c->dtype, c->pyr.fmt, [&](auto t, auto f) {
     using T = typename decltype(t)::type;
-    auto launch = [&](auto parts) {
-      for_launches(shape, shape.blocks, 256, [&](const QueueShape& qs, int blocks) {
-        hipLaunchKernelGGL((k_dos_render<T, decltype(f)::value, decltype(parts)::value>), dim3(blocks), dim3(256), shm, st,
-                           rf, g, c->pyr, c->d_pyr_oct, K, c->d_tf_rgbt, c->tf_size, step, P.et_threshold, ph, c->d_grad,
-                           qs, o4, cnt);
+    auto launch = [&](const QueueShape& s, auto parts, auto rays) {
+      for_launches(s, s.blocks, 256, [&](const QueueShape& qs, int blocks) {
+        hipLaunchKernelGGL((k_dos_render<T, decltype(f)::value, decltype(parts)::value, decltype(rays)::value>), dim3(blocks),
+                           dim3(256), shm, st, rf, g, c->pyr, c->d_pyr_oct, K, c->d_tf_rgbt, c->tf_size, step,
+                           P.et_threshold, ph, c->d_grad, qs, o4, cnt);
       });
     };
-    if (shared) launch(std::integral_constant<int, 4>{});
-    else launch(std::integral_constant<int, 1>{});
+    const std::integral_constant<int, 1> one;
+    const std::integral_constant<int, kRays> few;
+    if (shared) launch(shape, std::integral_constant<int, 4>{}, few);
+    else launch(shape, one, few);
+    if (shape.short_tiles) launch(short_shape(rf, shape, kShortRays), one, std::integral_constant<int, kShortRays>{});
   });
   CVR_HIP_CHECK(hipGetLastError());
   return CVR_OK;

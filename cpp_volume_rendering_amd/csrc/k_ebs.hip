@@ -387,7 +387,7 @@ __device__ __forceinline__ void ebs_load_rows(const ShadowRow* __restrict__ rows
   __syncthreads();
 }
 
-constexpr int kRays = 16;
+constexpr int kRays = 16, kShortRays = 32;
 // The march is queue_march's (cvr_queue.hpp).  One wavefront per SIMD: the box streams keep
 // four corner records in flight per lane, which with the FP64 interpolation takes more than
 // the 256 architectural VGPRs; at one wavefront per SIMD the excess lives in AGPRs instead of
@@ -396,11 +396,12 @@ constexpr int kRays = 16;
 // shadows, light table: 66 ms one ray per lane, 23.1 ms queued (30.8 ms with
 // kernel arguments copied to scratch memory for functions called, 28.9 ms at two wavefronts per
 // SIMD), 16.0 ms with the rays dealt out as in queue_shape.
-template <typename T, int L, bool kPoint, int kParts>
+template <typename T, int L, bool kPoint, int kParts, int kRays>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) void k_ebs(RayFrame rf, EbsK k, const float4* __restrict__ tf, int ntf, const void* __restrict__ sat,
            const ShadowRow* __restrict__ rows, float step, float et, PhongK ph, const float4* __restrict__ grad, QueueShape qs,
            float4* __restrict__ out, unsigned long long* __restrict__ counters) {
   extern __shared__ float4 smem[];
+  if (tile_left_out<kParts>(qs)) return;
   const int waves = blockDim.x >> 6;
   WaveQueue<kRays>* queue = reinterpret_cast<WaveQueue<kRays>*>(smem);
   float4* s_tf = reinterpret_cast<float4*>(queue + waves);
@@ -658,8 +659,6 @@ int launch_ebs(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* ou
     for (int i = 0; i < 3; ++i) cs[i] = k.scale[i] * (float(dims[i]) / float(res[i]));  // VolumeScales * (dims / res)
     const f3 cell{cs[0], cs[1], cs[2]};
     const size_t n = size_t(rx) * ry * rz;
-    // one wave per workgroup: a 32^3 cache is 512 waves, which then spread over every CU
-    // instead of half of them (light-cache frame 0.927 -> 0.874 ms, the same cache)
     if (size_t(k.nrows) * sizeof(ShadowRow) > 64 * 1024) {
       set_error("cvr_render: EBS light cache: shadow chain of more than 2048 boxes does not fit LDS");
       return -4;
@@ -682,22 +681,29 @@ int launch_ebs(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* ou
   // small frames: workgroups whose wavefronts share their rays (100 x 100 0.51 ms, 1.0 ms with
   // rays of their own; 400 x 300, point light 3.6 and 4.3; 512^2 5.3 and 5.0; 1024^2 19.4 and 16.0)
   const bool shared = waves == 4 && size_t(rf.W) * rf.H < 200000;
-  const QueueShape shape = queue_shape(rf.W, rf.H, kRays, shared ? 4 : 1, shared ? 64 : 256, waves);
+  QueueShape shape = queue_shape(rf.W, rf.H, kRays, shared ? 4 : 1, shared ? 64 : 256, waves);
+  const size_t short_shm = tables + 4 * sizeof(WaveQueue<kShortRays>);
+  if (short_shm <= 160 * 1024 && (rc = short_tiles(c, rf, step, P.et_threshold, 1024, st, &shape.short_tiles))) return rc;
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   const void* sat = P.sat_layout == 1 ? static_cast<const void*>(c->d_sat) : c->d_sat_oct;
   const ShadowRow* rows = static_cast<const ShadowRow*>(c->d_ebs_rows);
   float4* o4 = reinterpret_cast<float4*>(out);
-  auto launch = [&](auto t, auto l, auto pt, auto parts) {
-    for_launches(shape, shape.blocks, 64 * waves, [&](const QueueShape& qs, int blocks) {
-      hipLaunchKernelGGL((k_ebs<typename decltype(t)::type, decltype(l)::value, decltype(pt)::value, decltype(parts)::value>),
-                         dim3(blocks), dim3(64 * waves), shm, st, rf, k, c->d_tf_rgbt, c->tf_size, sat, rows, step,
+  auto launch = [&](const QueueShape& s, int threads, size_t lds, auto t, auto l, auto pt, auto parts, auto rays) {
+    for_launches(s, s.blocks, threads, [&](const QueueShape& qs, int blocks) {
+      hipLaunchKernelGGL((k_ebs<typename decltype(t)::type, decltype(l)::value, decltype(pt)::value, decltype(parts)::value,
+                                decltype(rays)::value>),
+                         dim3(blocks), dim3(threads), lds, st, rf, k, c->d_tf_rgbt, c->tf_size, sat, rows, step,
                          P.et_threshold, ph, c->d_grad, qs, o4, cnt);
     });
   };
   auto by_light = [&](auto t, auto l) {
     auto by_size = [&](auto pt) {
-      if (shared) launch(t, l, pt, std::integral_constant<int, 4>{});
-      else launch(t, l, pt, std::integral_constant<int, 1>{});
+      const std::integral_constant<int, 1> one;
+      const std::integral_constant<int, kRays> few;
+      if (shared) launch(shape, 256, shm, t, l, pt, std::integral_constant<int, 4>{}, few);
+      else launch(shape, 64 * waves, shm, t, l, pt, one, few);
+      if (shape.short_tiles)
+        launch(short_shape(rf, shape, kShortRays), 256, short_shm, t, l, pt, one, std::integral_constant<int, kShortRays>{});
     };
     if (P.apply_shadow && P.shadow_type != 1) by_size(std::true_type{});
     else by_size(std::false_type{});

@@ -90,26 +90,27 @@ __device__ __forceinline__ float gt_cone(const VolGeom& g, const float2* s_ext, 
   return S / W;
 }
 
-constexpr int kRays = 4;
+constexpr int kRays = 4, kShortRays = 16;
 // The march is queue_march's (cvr_queue.hpp).  128^3 at 256^2 with 16 + 4 rays per sample:
 // 313 -> 5.7 ms (one dependent read per light-ray step at one wavefront per SIMD before).
-template <typename T>
+template <typename T, int kParts, int kRays>
 __global__ __launch_bounds__(256) void k_gt_render(RayFrame rf, VolGeom g, GtK K, const float4* __restrict__ tf,
                                                    int ntf, float step, float et, QueueShape qs, float4* __restrict__ out,
                                                    unsigned long long* __restrict__ counters) {
   extern __shared__ float4 s_tf[];
   __shared__ WaveQueue<kRays> queue[4];
+  if (tile_left_out<kParts>(qs)) return;
   float2* s_ext = reinterpret_cast<float2*>(s_tf + ntf);
   for (int i = threadIdx.x; i < ntf; i += blockDim.x) s_tf[i] = tf[i];
   for (int i = threadIdx.x; i <= ntf; i += blockDim.x) s_ext[i] = make_float2(tf[max(i - 1, 0)].w, tf[min(i, ntf - 1)].w);
   __syncthreads();
-  const int u = queue_unit<4>(qs);
+  const int u = queue_unit<kParts>(qs);
   unsigned int nsamp = 0, nshade = 0;
   const float ka = K.apply_occ ? K.ka : 0.f, kd = K.apply_sdw ? K.kd : 0.f;
   const float inv_k = 1.0f / (ka + kd);
   const f3 half = mk3(0.5f * g.G[0], 0.5f * g.G[1], 0.5f * g.G[2]);
   const float spec[3] = {0.f, 0.f, 0.f};
-  queue_march<T, 64, false, 4>(rf, g, s_tf, ntf, step, et, qs.rays, FramePixels(rf, qs, u), spec, queue, out, nsamp, nshade,
+  queue_march<T, 64, false, kParts>(rf, g, s_tf, ntf, step, et, qs.rays, FramePixels(rf, qs, u), spec, kParts > 1 ? queue : queue + (threadIdx.x >> 6), out, nsamp, nshade,
                  [&](bool, f3 p, f3 dir) {
                    float Io = 0.f, Is = 0.f;
                    if (K.apply_occ) {
@@ -235,17 +236,24 @@ int launch_gt(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out
   // workgroups whose wavefronts share their rays: a batch is tens to thousands of light-ray
   // steps (128^3 at 256^2 with 16 + 4 rays 5.7 ms, 13.7 ms with rays of their own; 256^3 at 512^2
   // with 4 + 1 11.5 and 12.2)
-  const QueueShape shape = queue_shape(rf.W, rf.H, kRays, 4, 64);
+  QueueShape shape = queue_shape(rf.W, rf.H, kRays, 4, 64);
+  if ((rc = short_tiles(c, rf, step, P.et_threshold, 2048, st, &shape.short_tiles))) return rc;
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   float4* o4 = reinterpret_cast<float4*>(out);
-  for_launches(shape, shape.blocks, 256, [&](const QueueShape& qs, int blocks) {
-    if (c->dtype == CVR_U8)
-      hipLaunchKernelGGL(k_gt_render<uint8_t>, dim3(blocks), dim3(256), shm, st, rf, g, K, c->d_tf_rgbt, c->tf_size, step,
-                         P.et_threshold, qs, o4, cnt);
-    else
-      hipLaunchKernelGGL(k_gt_render<uint16_t>, dim3(blocks), dim3(256), shm, st, rf, g, K, c->d_tf_rgbt, c->tf_size, step,
-                         P.et_threshold, qs, o4, cnt);
-  });
+  auto launch = [&](const QueueShape& s, auto parts, auto rays) {
+    constexpr int kP = decltype(parts)::value, kR = decltype(rays)::value;
+    for_launches(s, s.blocks, 256, [&](const QueueShape& qs, int blocks) {
+      if (c->dtype == CVR_U8)
+        hipLaunchKernelGGL((k_gt_render<uint8_t, kP, kR>), dim3(blocks), dim3(256), shm, st, rf, g, K, c->d_tf_rgbt, c->tf_size,
+                           step, P.et_threshold, qs, o4, cnt);
+      else
+        hipLaunchKernelGGL((k_gt_render<uint16_t, kP, kR>), dim3(blocks), dim3(256), shm, st, rf, g, K, c->d_tf_rgbt,
+                           c->tf_size, step, P.et_threshold, qs, o4, cnt);
+    });
+  };
+  launch(shape, std::integral_constant<int, 4>{}, std::integral_constant<int, kRays>{});
+  if (shape.short_tiles)
+    launch(short_shape(rf, shape, kShortRays), std::integral_constant<int, 1>{}, std::integral_constant<int, kShortRays>{});
   CVR_HIP_CHECK(hipGetLastError());
   return CVR_OK;
 }

@@ -346,3 +346,49 @@ def test_counted_samples(tech, w, h):
         s = r.stats()
         counts.append((s.samples, s.shaded_samples))
     assert counts[0][0] > 0 and len(set(counts)) == 1, counts
+
+
+# From inside a volume that is dense on one side and clear on the other: tiles of 64 x 64 pixels whose rays end
+# after a few samples are dealt out apart from the others.  One tile, ragged ones, a frame too small to be
+# looked over, 4 and 16 rays to a wavefront for the other tiles.
+@pytest.mark.parametrize("w,h", [(64, 64), (65, 130), (200, 71), (63, 90), (300, 260)])
+@pytest.mark.parametrize("tech", [N.CONE_TRACE, N.DOS, N.CONE_GT, N.EBS])
+def test_tiles_of_short_rays(tech, w, h):
+    n = 40
+    vol = np.zeros((n, n, n), np.uint8)
+    vol[:, :, : n // 2] = 200
+    vol[:, :, n // 2:] = np.linspace(0, 60, n, dtype=np.uint8)[:, None, None]
+    rgb = np.array([[0.2, 0.5, 0.9, 0], [0.9, 0.6, 0.3, 255]])
+    alpha = np.array([[0.0, 0], [0.0, 50], [0.1, 60], [0.9, 150], [0.95, 255]])
+    grid = (float(n),) * 3
+    r = N.Renderer(tech)
+    r.set_volume(vol)
+    r.set_transfer_function(rgb, alpha)
+    light = W.light_from_direction((0.3, 0.8, -0.4), grid)
+    if tech == N.DOS:
+        r.set_params(apply_shadow=1, shadow_type=2)
+    elif tech == N.CONE_GT:
+        r.set_params(occ_rays=3, sdw_rays=2, shadow_type=2)
+    cam, tf = W.orbit_camera(grid, w, h, az_deg=4.0, el_deg=3.0, dist_diag=0.02, fovy=70.0), O.OTF(rgb, alpha)
+    img = r.render(cam, w, h, light=light)
+    s = 3
+    if tech == N.EBS:
+        prm = O.ebs_params(r.params(), light)
+        prm.sdw_max_dist = np.float32(0.75) * np.float32(np.linalg.norm(grid))
+        ref, m = O.render_ebs(vol, tf, O.sat(vol, tf), prm, cam, w, h, stride=s)
+    elif tech == N.CONE_GT:
+        ref, m = O.render_gt(vol, tf, O.gt_params(r.params(), grid, light), cam, w, h, stride=s)
+    else:
+        pyr = O.OPyr.wrap(grid, [a.astype(np.float64) for a in r.pyramid()])
+        if tech == N.DOS:
+            ref, m = O.render_dos(vol, tf, pyr, O.dos_params(r.params(), grid, light), cam, w, h, stride=s)
+        else:
+            ref, m = O.render_cone(vol, tf, pyr, O.cone_params(grid, light), cam, w, h, stride=s)
+    assert ref[::s, ::s, 3].max() > 0.98 and ref[::s, ::s, 3].min() < 0.5
+    sparse = np.zeros_like(img)
+    sparse[::s, ::s] = img[::s, ::s]
+    st = O.compare(sparse, ref, m, 2e-3, s)
+    assert st["max_abs"] <= 2e-3 and st["n_over_tol"] <= 0.005 * st["n_pixels"] + 1, st
+    r.collect_stats(True)
+    again = r.render(cam, w, h, light=light)
+    assert np.array_equal(again, img) and r.stats().shaded_samples > 0
