@@ -11,7 +11,8 @@
 // four).  Workgroups begin with different volumes, so that all of them are in work at once: when
 // every workgroup began with the largest, each volume had its own tail of waiting wavefronts.
 // 32 images of 256^2 over four volumes of 64^3 to 256^3: 6.6 ms with a barrier at each item, 4.7
-// from the largest on, 4.0 now; 8 of 138 x 147 over four of 43 x 43 x 62: 0.69, 1.10 and 0.41.
+// from the largest on, 3.8 now; 8 of 138 x 147 over four of 43 x 43 x 62: 0.69, 1.10 and 0.41 (before the
+// queues had lines of their own).
 // Which item a queue position is follows from its number, so there is no item list.  Each item
 // is rendered by the same device code as the single-frame surrogate renderer.
 #include "cvr_nn.hpp"
@@ -44,6 +45,10 @@ struct JobDesc {
 };
 
 constexpr int kMaxVolumes = 64;
+// Words between the queues' heads: a line of 128 bytes each.  An addition to a line takes about 12 ns and the
+// next one waits for it; with a volume's heads in one line, 32 images of 261 x 212 of volumes of 34 x 33 x 39
+// and less (110000 items) took 1050 us (605 with an item of 256 pixels a workgroup), 496 now.
+constexpr int kHeadStride = 32;
 
 // The jobs of one volume (a range of the job order), largest volume first.
 struct VolJobs {
@@ -65,7 +70,7 @@ struct TilePixels {
 // Clears the queue heads and the counters (a kernel, so that it can sit in the graph).
 __global__ __launch_bounds__(kQueues * kMaxVolumes) void k_batch_reset(unsigned int* __restrict__ heads,
                                                     unsigned long long* __restrict__ counters) {
-  heads[threadIdx.x] = 0u;
+  heads[threadIdx.x * kHeadStride] = 0u;
   if (threadIdx.x < 4) counters[threadIdx.x] = 0ull;
 }
 
@@ -86,11 +91,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   for (int vi = 0; vi < bs.nvols; ++vi) {
     const int v = (int(blockIdx.x) / bs.nq + vi) % bs.nvols;
     const VolJobs vj = vjobs[v];
-    unsigned int* vheads = heads + v * kQueues;
+    unsigned int* vheads = heads + v * kQueues * kHeadStride;
     if (threadIdx.x == 0) {
       int left = 0;
       for (int q = 0; q < bs.nq; ++q)
-        left |= int(__hip_atomic_load(&vheads[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) <
+        left |= int(__hip_atomic_load(&vheads[q * kHeadStride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) <
                 vj.count * queue_tiles(bs, q) * kCuts;
       s_left = left;
     }
@@ -105,7 +110,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
       const int q = (home + qi) % bs.nq, per_job = queue_tiles(bs, q) * kCuts, n = vj.count * per_job;
       for (;;) {
         int idx = 0;
-        if ((threadIdx.x & 63) == 0) idx = int(atomicAdd(&vheads[q], 1u));
+        if ((threadIdx.x & 63) == 0) idx = int(atomicAdd(&vheads[q * kHeadStride], 1u));
         idx = __builtin_amdgcn_readfirstlane(idx);
         if (idx >= n) break;
         const int job = order[vj.first + idx / per_job], r = idx % per_job, cut = r % kCuts, t = r / kCuts;
@@ -465,7 +470,7 @@ int cvr_batch_create(int device, int width, int height, cvr_batch_handle* out) {
   b->device = device;
   b->W = width;
   b->H = height;
-  if (device_alloc(&b->d_heads, kQueues * kMaxVolumes * sizeof(unsigned int)) != hipSuccess ||
+  if (device_alloc(&b->d_heads, kQueues * kMaxVolumes * kHeadStride * sizeof(unsigned int)) != hipSuccess ||
       device_alloc(&b->d_counters, 4 * sizeof(unsigned long long)) != hipSuccess ||
       hipStreamCreateWithFlags(&b->cap, hipStreamNonBlocking) != hipSuccess) {
     cvr_batch_destroy(b);
