@@ -157,6 +157,8 @@ void light_dir(const RayFrame& rf, const cvr_light* light, float L[3]);
 // step, so that the in-order opacity recurrence takes 16 rounds, not 64 (512^3 at 1024^2 4.74 ms,
 // 4.95 with 64 samples of one ray; from inside a 200 x 190 x 180 volume at 700 x 500 2.64 and 3.0).
 constexpr int kNnRays = 16, kNnSub = 16;
+// Rays of a wavefront with a lane to each (nn_shape).
+constexpr int kLaneNnRays = 64;
 
 // Marches a wavefront's rays (queue_march, pixels from pix) with the surrogate as the
 // lighting: the wave gathers its 64 samples' features and runs the network over them
@@ -167,18 +169,18 @@ constexpr int kNnRays = 16, kNnSub = 16;
 // left the range) for a second pass with kExact, and their pixels are provisional.
 // Which samples a ray takes and their opacities do not depend on the shading, so both
 // passes march it identically.
-template <typename T, int F, bool kExact, class Pix>
+template <typename T, int F, bool kExact, int kSub, int kRays, class Pix>
 __device__ __forceinline__ bool nn_march(const RayFrame& rf, const VolGeom& g, const PyrGeom& pg,
                                          const void* __restrict__ pyr, const ConeK& K, const NnK& nk, const short* sW,
                                          const float* sB, float* sXw, const float4* s_tf, int ntf, float step, float et,
-                                         int rays, Pix&& pix, WaveQueue<kNnRays>& Q, float4* __restrict__ out,
+                                         int rays, Pix&& pix, WaveQueue<kRays>& Q, float4* __restrict__ out,
                                          unsigned int* cnt) {
   const float ka = K.apply_occ ? K.ka : 0.f, kd = K.apply_sdw ? K.kd : 0.f;
   const float inv_k = 1.0f / (ka + kd);
   const f3 L = ld3(K.L);
   const float spec[3] = {0.f, 0.f, 0.f};
   bool ood_seen = false;
-  queue_march<T, kNnSub, true, 1>(
+  queue_march<T, kSub, true, 1>(
       rf, g, s_tf, ntf, step, et, rays, pix, spec, &Q, out, cnt[0], cnt[1], [&](bool on, f3 p, f3 dir) {
         float f[kNFeat];
         bool ood = false;

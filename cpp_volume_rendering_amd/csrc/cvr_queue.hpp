@@ -81,6 +81,7 @@ __device__ __forceinline__ float left_lane(float v, float first) {  // wave_shr:
       __builtin_amdgcn_update_dpp(__float_as_int(first), __float_as_int(v), 0x138, 0xf, 0xf, false));
 }
 template <int kSub> __device__ __forceinline__ float opacity_before(float alpha, float w) {
+  if (kSub == 1) return w;
   if (kSub == 16) return opacity_rounds(alpha, w);
   float b = w;
 #pragma unroll
@@ -224,7 +225,7 @@ __device__ __forceinline__ void queue_march(const RayFrame& rf, const VolGeom& g
                                             WaveQueue<kRays>* queues, float4* __restrict__ out, unsigned int& nsamp, unsigned int& nshade,
                                             Shade&& shade) {
   typedef typename VolOct<T>::type RT;
-  static_assert(kSub == 64 || kSub == 16, "groups are wavefronts or DPP rows");
+  static_assert(kSub == 64 || kSub == 16 || kSub == 1, "groups are wavefronts, DPP rows or lanes");
   constexpr uint64_t kGroupMask = kSub == 64 ? ~0ull : (1ull << (kSub & 63)) - 1ull;
   const int lane = threadIdx.x & 63, sub = lane % kSub, base = lane - sub;
   const int part = kParts > 1 ? int(threadIdx.x >> 6) % kParts : 0;
@@ -301,7 +302,7 @@ __device__ __forceinline__ void queue_march(const RayFrame& rf, const VolGeom& g
           // (a transparent sample ends no ray, also where the threshold is below 0)
           const uint64_t over = (__ballot(opaque && wa > et) >> base) & kGroupMask;
           const int last = over ? __builtin_ctzll(over) : kSub - 1;  // over: the ray ends with that sample
-          w = kSub == 64 ? lane_value(wa, last) : __shfl(wa, base + last);
+          w = kSub == 64 ? lane_value(wa, last) : kSub == 1 ? wa : __shfl(wa, base + last);
           taken = valid && sub <= last;
           ended = ended || over != 0;
         }

@@ -124,7 +124,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         float4* o = out + size_t(job) * img_px;
 #define CVR_BATCH_ITEM(TT, FF)                                                                                      \
   for (int p = 0; p < item_px; p += kNnRays)                                                                        \
-  nn_march<TT, FF, true>(J.rf, V.g, V.pg, V.pyr, K, V.nk, sW, sB, sX[w], s_tf, V.ntf, V.step, V.et,                 \
+  nn_march<TT, FF, true, kNnSub, kNnRays>(J.rf, V.g, V.pg, V.pyr, K, V.nk, sW, sB, sX[w], s_tf, V.ntf, V.step, V.et,                 \
                          kNnRays,          \
                          TilePixels{J.rf, tx * tw, ty * th, bs.tw_log2, cut * item_px + p}, queue[w], o, cnt)
         switch (V.g.dtype * 3 + V.pg.fmt) {

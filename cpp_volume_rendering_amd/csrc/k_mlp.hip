@@ -604,7 +604,7 @@ __global__ void k_feat_range(const float* __restrict__ X, int n, unsigned int* _
 // is marked.  Counters: samples and shaded samples from the first pass, exact fallbacks
 // from the second (which marches a ray exactly as the first did).  A wavefront takes
 // the rays of `sets` units.
-template <typename T, int F, bool kExact>
+template <typename T, int F, bool kExact, bool kLane>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_nn_render(RayFrame rf, VolGeom g, PyrGeom pg, const void* __restrict__ pyr,
                                                    ConeK K, NnK nk, const short* __restrict__ wpack,
                                                    const float* __restrict__ bpack, const float4* __restrict__ tf,
@@ -614,7 +614,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   __shared__ __align__(16) short sW[kPackShorts];
   __shared__ __align__(16) float sB[kNBias];
   __shared__ __align__(16) float sX[4][kWaveScratch];
-  __shared__ WaveQueue<kNnRays> queue[4];
+  constexpr int kRays = kLane ? kLaneNnRays : kNnRays, kSub = kLane ? 1 : kNnSub;
+  __shared__ WaveQueue<kRays> queue[4];
   extern __shared__ float4 s_tf[];
   const int bid = xcd_remap(blockIdx.x, gridDim.x, qs.xcd_log2);
   if (kExact && redo[bid] == 0u) return;  // the same word for every thread of the block
@@ -625,8 +626,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
   unsigned int cnt[3] = {0, 0, 0};
   bool marked = false;
   for (int s = 0; s < sets; ++s)
-    marked |= nn_march<T, F, kExact>(rf, g, pg, pyr, K, nk, sW, sB, sX[w], s_tf, ntf, step, et, qs.rays,
-                                     FramePixels(rf, qs, u * sets + s, 64 / kNnSub), queue[w], out, cnt);
+    marked |= nn_march<T, F, kExact, kSub, kRays>(rf, g, pg, pyr, K, nk, sW, sB, sX[w], s_tf, ntf, step, et, qs.rays,
+                                                  FramePixels(rf, qs, u * sets + s, 4), queue[w], out, cnt);
   if (!kExact && marked && (threadIdx.x & 63) == 0) redo[bid] = 1u;
   if (counters) {
     if (!kExact) {
@@ -912,12 +913,45 @@ NnK nn_consts(cvr_ctx* c) {
 // 4.89 ms; 100 x 90 x 80 at 200 x 150 0.2 and 0.1 ms).  A wavefront takes its rays of `sets`
 // units: more than one for frames of more than kMaxBlocks workgroups, whose marks would not
 // fit cvr_render_noalloc's array.
+//
+// A sample's network costs little beside the march's steps, and where wavefronts are many or rays short a lane to a
+// ray takes fewer of them: frames from inside the box, and large ones of many rays for the samples of the longest.
+// 2 x 2 of a pixel's neighbours lie in a wavefront, as with 16 rays.    a lane per ray and tile   16 rays   64 lanes
+//   256^3 from inside at 1024^2                                                      5676 us         6943       6498
+//   512^3 from inside at 1024^2                                                      9152           10983      10507
+//   64^3 from inside at 1300^2                                                       8094            9654       8828
+//   dense 256^3 from inside at 1024^2                                                 706            1056        818
+//   256^3 from inside at 700^2                                                       3036            3370       3243
+//   128^3 from inside at 600^2                                                       3585            3187       3317
+//   64^3 at 2400^2                                                                   3482            3904       3496
+//   256^3 at 2400^2                                                                 12774           13967      13713
+//   64^3 at 1920 x 1080                                                              1080             975        988
+//   512^3 at 2400 x 2000                                                            17190           17469      18067
+//   256^3 at 1920 x 1080                                                             4374            3170       4651
 constexpr int kMaxBlocks = 1 << 16;
-static QueueShape nn_shape(const RayFrame& rf, int& sets) {
-  QueueShape q = queue_shape(rf.W, rf.H, size_t(rf.W) * rf.H < (1 << 16) ? 4 : 16, 1, 64);
-  sets = (q.blocks + kMaxBlocks - 1) / kMaxBlocks;
-  q.blocks = (q.blocks + sets - 1) / sets;
-  return q;
+constexpr size_t kLanePxInside = 450000, kLanePx = 1 << 21;
+constexpr float kLanePerStep = 6000.f;
+// Two workgroups with 64 rays to a wavefront fit a CU beside tables of this many bytes.
+constexpr size_t kLaneTable = 80 * 1024 - (kPackShorts * 2 + kNBias * 4 + 4 * kWaveScratch * 4 + 4 * sizeof(WaveQueue<kLaneNnRays>));
+struct NnShape {
+  QueueShape q;
+  int sets;
+  bool lane;
+};
+static NnShape nn_shape(const cvr_ctx* c, const RayFrame& rf) {
+  const VolGeom g = geom_of(c);
+  const size_t px = size_t(rf.W) * rf.H;
+  const float step = c->nn.cone.step_size > 0 ? c->nn.cone.step_size : default_step(c);
+  const float steps = std::sqrt(g.G[0] * g.G[0] + g.G[1] * g.G[1] + g.G[2] * g.G[2]) / step;
+  bool inside = true;
+  for (int k = 0; k < 3; ++k) inside = inside && std::fabs(rf.eye[k]) <= 0.5f * g.G[k];
+  NnShape s;
+  s.lane = size_t(c->tf_size) * sizeof(float4) <= kLaneTable &&
+           ((inside && px >= kLanePxInside) || (px >= kLanePx && float(px) >= steps * kLanePerStep));
+  s.q = s.lane ? queue_shape(rf.W, rf.H, kLaneNnRays, 1, 256) : queue_shape(rf.W, rf.H, px < (1 << 16) ? 4 : kNnRays, 1, 64);
+  s.sets = (s.q.blocks + kMaxBlocks - 1) / kMaxBlocks;
+  s.q.blocks = (s.q.blocks + s.sets - 1) / s.sets;
+  return s;
 }
 // The workgroup tiles of the frame as cvr_render_noalloc counts them against its limit:
 // 2 x 2 wave tiles of tile_w x 64 / tile_w pixels, `span` of them stacked.
@@ -946,8 +980,7 @@ static int nn_frame(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, floa
   }
   VolGeom g = geom_of(c);
   const float step = N.cone.step_size > 0 ? N.cone.step_size : default_step(c);
-  int sets = 1;
-  const QueueShape sh = nn_shape(rf, sets);
+  const NnShape sh = nn_shape(c, rf);
   const size_t shm = size_t(c->tf_size) * sizeof(float4);
   if (shm > 32 * 1024) { set_error("surrogate renderer: transfer function larger than 2048 entries"); return -4; }
   short* wp = static_cast<short*>(c->d_nn_pack);
@@ -956,10 +989,17 @@ static int nn_frame(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, floa
   with_types(c->dtype, c->pyr.fmt, [&](auto t, auto f) {
     using T = typename decltype(t)::type;
     constexpr int FF = decltype(f)::value;
-    hipLaunchKernelGGL((k_nn_render<T, FF, false>), dim3(sh.blocks), dim3(256), shm, st, rf, g, c->pyr, c->d_pyr_oct,
-                       K, nk, wp, bp, c->d_tf_rgbt, c->tf_size, step, N.cone.et_threshold, sh, sets, o4, redo, cnt);
-    hipLaunchKernelGGL((k_nn_render<T, FF, true>), dim3(sh.blocks), dim3(256), shm, st, rf, g, c->pyr, c->d_pyr_oct,
-                       K, nk, wp, bp, c->d_tf_rgbt, c->tf_size, step, N.cone.et_threshold, sh, sets, o4, redo, cnt);
+    auto pass = [&](auto exact, auto lane) {
+      hipLaunchKernelGGL((k_nn_render<T, FF, decltype(exact)::value, decltype(lane)::value>), dim3(sh.q.blocks), dim3(256), shm,
+                         st, rf, g, c->pyr, c->d_pyr_oct, K, nk, wp, bp, c->d_tf_rgbt, c->tf_size, step,
+                         N.cone.et_threshold, sh.q, sh.sets, o4, redo, cnt);
+    };
+    auto both = [&](auto lane) {
+      pass(std::false_type{}, lane);
+      pass(std::true_type{}, lane);
+    };
+    if (sh.lane) both(std::true_type{});
+    else both(std::false_type{});
   });
   CVR_HIP_CHECK(hipGetLastError());
   return 0;
@@ -978,8 +1018,7 @@ int launch_nn(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out
     rc = nn_train(c, st);
     if (rc) return rc;
   }
-  int sets = 1;
-  const int tiles = nn_shape(rf, sets).blocks;
+  const int tiles = nn_shape(c, rf).q.blocks;
   // workgroup marks for the second pass: cleared when allocated, on the frame's stream, and the second
   // pass clears what the first sets
   if (size_t(tiles) > c->nn_redo_cap) {
@@ -1073,8 +1112,7 @@ extern "C" int cvr_render_noalloc(cvr_handle h, const cvr_camera* cam, const cvr
   if (rc) return rc;
   hipStream_t st = static_cast<hipStream_t>(hip_stream);
   // the marks must start at zero: a fill kernel (not a memset node) keeps the call capturable
-  int sets = 1;
-  const int blocks = nn_shape(rf, sets).blocks;
+  const int blocks = nn_shape(h, rf).q.blocks;
   hipLaunchKernelGGL(k_clear_marks, dim3((blocks + 255) / 256), dim3(256), 0, st, marks, blocks);
   CVR_HIP_CHECK(hipGetLastError());
   return nn_frame(h, rf, light, out_device, marks, nullptr, st);

@@ -330,14 +330,21 @@ def test_volume_of_more_than_4_gib_of_corner_blocks():
         check(img, ref, m)
 
 
-def test_surrogate_frame_of_two_units_a_wavefront():
-    """2112 x 2112 pixels are more workgroups than there are marks: each takes two sets of rays.  The
-    network's frame against the oracle, the frame of the second pass alone against the cone tracer's, and the
-    first again when no mark is left."""
-    w = h = 2112
+# 2112 x 2112: a lane to a ray, and with a table that leaves no room for that 16 rays to a wavefront, of which
+# more workgroups than there are marks (each takes two sets); from inside with a lane to a ray, a ragged frame
+@pytest.mark.parametrize("w,h,entries,dist", [(2112, 2112, 256, 2.0), (2112, 2112, 1024, 2.0), (701, 645, 256, 0.1)])
+def test_surrogate_frames_of_many_pixels(w, h, entries, dist):
+    """The network's frame against the oracle, the frame of the second pass alone against the cone tracer's,
+    and the first again when no mark is left."""
     wl = W.cone_blobs(n=24, width=w, height=h, seed=33)
-    cam, light = wl.camera(), wl.light()
-    r, c = handle(N.CONE_NN, wl), handle(N.CONE_TRACE, wl)
+    md, light = entries - 1, wl.light()
+    rgb, al = wl.rgb_iso.copy(), wl.alpha_iso.copy()
+    rgb[:, 3], al[:, 1] = np.floor(rgb[:, 3] * md / 255), np.floor(al[:, 1] * md / 255)
+    cam = W.orbit_camera(wl.grid, w, h, dist_diag=dist)
+    r, c = N.Renderer(N.CONE_NN), N.Renderer(N.CONE_TRACE)
+    for x in (r, c):
+        x.set_volume(wl.volume)
+        x.set_transfer_function(rgb, al, max_density=md)
     p = r.params()
     p.cone.density_precision = 0
     r.set_params(p)
@@ -346,12 +353,12 @@ def test_surrogate_frame_of_two_units_a_wavefront():
     r.nn_set_weights(wts)
     first = r.render(cam, w, h, light=light)
     pyr = O.OPyr.wrap(wl.grid, [a.astype(np.float64) for a in r.pyramid()])
-    tf = O.OTF(wl.rgb_iso, wl.alpha_iso)
-    ref, m, _ = O.render_nn(wl.volume, tf, pyr, O.cone_params(wl.grid, light), wts, cam, w, h, stride=33)
+    tf, s = O.OTF(rgb, al, max_density=md), 33 if w > 1000 else 11
+    ref, m, _ = O.render_nn(wl.volume, tf, pyr, O.cone_params(wl.grid, light), wts, cam, w, h, stride=s)
     img = np.zeros_like(first)
-    img[::33, ::33] = first[::33, ::33]
+    img[::s, ::s] = first[::s, ::s]
     assert ref[: h // 2, ..., 3].max() > 0.2 and ref[h // 2:, ..., 3].max() > 0.2
-    check(img, ref, m, 33)
+    check(img, ref, m, s)
     p.ood_margin = -2e30  # no input is in range
     r.set_params(p)
     r.collect_stats(True)
