@@ -175,6 +175,7 @@ struct cvr_ctx {
 
   int* d_short = nullptr;  // short_tiles of the frame in work
   size_t short_cap = 0;
+  bool may_allocate = true;  // false within cvr_render_noalloc
 
   // stats
   bool collect_stats = false;

@@ -1099,8 +1099,13 @@ extern "C" int cvr_render_noalloc(cvr_handle h, const cvr_camera* cam, const cvr
   if (prev != h->device) CVR_HIP_CHECK(hipSetDevice(h->device));
   struct Restore {
     int d;
-    ~Restore() { if (d >= 0) (void)hipSetDevice(d); }
-  } restore{prev != h->device ? prev : -1};
+    cvr_ctx* c;
+    ~Restore() {
+      if (d >= 0) (void)hipSetDevice(d);
+      c->may_allocate = true;
+    }
+  } restore{prev != h->device ? prev : -1, h};
+  h->may_allocate = false;
   hipPointerAttribute_t at{};
   if (hipPointerGetAttributes(&at, out_device) != hipSuccess || at.type != hipMemoryTypeDevice) {
     (void)hipGetLastError();

@@ -69,6 +69,7 @@ int short_tiles(cvr_ctx* c, const RayFrame& rf, float step, float et, int px_per
   if (rf.W < 64 || rf.H < 64 || limit < 4 || frame_hits(rf, g) != 64) return CVR_OK;
   const size_t n = size_t((rf.W + 63) / 64) * size_t((rf.H + 63) / 64);
   if (n > c->short_cap) {
+    if (!c->may_allocate) return CVR_OK;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
     if (hipStreamIsCapturing(st, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
       (void)hipGetLastError();

@@ -421,3 +421,30 @@ def test_largest_transfer_functions(tech, entries):
             ref, m, _ = O.render_nn(wl.volume, tf, pyr, O.cone_params(wl.grid, light), wts, cam, 40, 33)
     assert ref[..., 3].max() > 0.3
     check(img, ref, m)
+
+
+def test_noalloc_of_a_closed_gate_from_inside_allocates_nothing():
+    """The exact tracer's frame from inside looks for tiles of short rays in a buffer that is not there yet:
+    the call goes without, and gives the frame that cvr_render gives with it."""
+    import torch
+
+    w = h = 256
+    wl = W.cone_blobs(n=32, width=w, height=h, seed=3)
+    wl.alpha_iso[:, 0] = 0.9  # dense: every tile is short
+    cam, light = W.orbit_camera(wl.grid, w, h, dist_diag=0.05), wl.light()
+    r = handle(N.CONE_NN, wl)
+    p = r.params()
+    p.force_exact = 1
+    r.set_params(p)
+    r.nn_set_weights(np.zeros(N.lib().cvr_nn_param_count(), np.float32))
+    r.prepare()
+    got, ref = (torch.zeros((h, w, 4), device="cuda:0") for _ in range(2))
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    r.render_noalloc(cam, w, h, got, light=light)
+    torch.cuda.synchronize()
+    assert torch.cuda.mem_get_info()[0] == free
+    r.render(cam, w, h, light=light, out=ref)
+    torch.cuda.synchronize()
+    # a pixel's samples are summed by four wavefronts, or by one: 30 colours of at most 1, 30 x 2^-24
+    assert float(ref[..., 3].max()) > 0.9 and float((got - ref).abs().max()) <= 2e-6
