@@ -482,11 +482,13 @@ __device__ __forceinline__ void plain_march(const RayFrame& rf, const VolGeom& g
           acc.z = __builtin_fmaf(spec[2], ws, acc.z);
         }
         mine *= l.m;
-        // (here, not for every lane: a transparent entry's colour may be anything, and 0 x NaN is NaN)
-        acc.x = __builtin_fmaf(mine, src.x, acc.x);
-        acc.y = __builtin_fmaf(mine, src.y, acc.y);
-        acc.z = __builtin_fmaf(mine, src.z, acc.z);
       }
+      // others' colours may be anything (a transparent entry's NaN): 0 x NaN is NaN.  (Added up above instead, the
+      // 16-bit light-cache march takes 73 registers, 72 here: 64^3 at 300^2 51.5 us, 45.8.)
+      const bool on = opaque && taken;
+      acc.x = on ? __builtin_fmaf(mine, src.x, acc.x) : acc.x;
+      acc.y = on ? __builtin_fmaf(mine, src.y, acc.y) : acc.y;
+      acc.z = on ? __builtin_fmaf(mine, src.z, acc.z) : acc.z;
       acc.w = row_last(wa);
       nshade += opaque && taken;
     }

@@ -237,7 +237,7 @@ int launch_gt(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out
   // steps (128^3 at 256^2 with 16 + 4 rays 5.7 ms, 13.7 ms with rays of their own; 256^3 at 512^2
   // with 4 + 1 11.5 and 12.2)
   QueueShape shape = queue_shape(rf.W, rf.H, kRays, 4, 64);
-  if ((rc = short_tiles(c, rf, step, P.et_threshold, 2048, st, &shape.short_tiles))) return rc;
+  if ((rc = short_tiles(c, rf, step, P.et_threshold, 4096, st, &shape.short_tiles))) return rc;
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   float4* o4 = reinterpret_cast<float4*>(out);
   auto launch = [&](const QueueShape& s, auto parts, auto rays) {

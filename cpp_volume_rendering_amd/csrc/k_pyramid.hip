@@ -358,8 +358,9 @@ int build_pyramid(cvr_ctx* c, int base_x, int base_y, int base_z, float sigma0, 
   VolGeom g = geom_of(c);
   for (int k = 0; k < 3; ++k) pg.G[k] = g.G[k];
   pg.one = 1.0f;
-  // frames in flight on any stream may still read the pyramid that is built over
-  CVR_HIP_CHECK(hipDeviceSynchronize());
+  // frames in flight on any stream may still read the pyramid that is built over, unless a new volume or transfer
+  // function made it out of date: those calls waited for them, and frames since then come here first
+  if (c->pyr_key.vol_v == key.vol_v && c->pyr_key.tf_v == key.tf_v) CVR_HIP_CHECK(hipDeviceSynchronize());
   // separable path per level: voxel spacing and sigma commensurate on every axis (true at
   // every level of the default configurations; a level whose size was rounded down from
   // an odd one may not be, and takes the direct build)
