@@ -614,21 +614,28 @@ inline BatchShape batch_shape(int w, int h, int tw_log2, int span, int queues, i
   return s;
 }
 
-// How many of 8 x 8 rays of the frame, the corners' included, hit the volume's box.
+// Whether ray i of 8 x 8 rays of the frame, the corners' included, hits the volume's box.
+inline bool frame_ray_hits(const RayFrame& rf, const VolGeom& g, int i) {
+  const float a = (float(i & 7) / 3.5f - 1.0f) * rf.tanfov * rf.aspect, b = (float(i >> 3) / 3.5f - 1.0f) * rf.tanfov;
+  float lo = 0.f, hi = INFINITY;
+  for (int k = 0; k < 3; ++k) {
+    const float d = rf.s[k] * a + rf.u[k] * b + rf.f[k], h = 0.5f * g.G[k];
+    const float x = (-h - rf.eye[k]) / d, y = (h - rf.eye[k]) / d;
+    lo = std::fmax(lo, std::fmin(x, y));
+    hi = std::fmin(hi, std::fmax(x, y));
+  }
+  return lo < hi;
+}
+// How many of them do; whether all do (the corners first, which miss from outside).
 inline int frame_hits(const RayFrame& rf, const VolGeom& g) {
   int n = 0;
-  for (int i = 0; i < 64; ++i) {
-    const float a = (float(i & 7) / 3.5f - 1.0f) * rf.tanfov * rf.aspect, b = (float(i >> 3) / 3.5f - 1.0f) * rf.tanfov;
-    float lo = 0.f, hi = INFINITY;
-    for (int k = 0; k < 3; ++k) {
-      const float d = rf.s[k] * a + rf.u[k] * b + rf.f[k], h = 0.5f * g.G[k];
-      const float x = (-h - rf.eye[k]) / d, y = (h - rf.eye[k]) / d;
-      lo = std::fmax(lo, std::fmin(x, y));
-      hi = std::fmin(hi, std::fmax(x, y));
-    }
-    n += lo < hi;
-  }
+  for (int i = 0; i < 64; ++i) n += frame_ray_hits(rf, g, i);
   return n;
+}
+inline bool frame_all_hit(const RayFrame& rf, const VolGeom& g) {
+  for (int i : {0, 7, 56, 63})
+    if (!frame_ray_hits(rf, g, i)) return false;
+  return frame_hits(rf, g) == 64;
 }
 // How the plain and the light-cache frames are marched.
 enum { kGroups = 0, kPhong = 1, kLanes = 2 };  // kLanes + kPhong: both

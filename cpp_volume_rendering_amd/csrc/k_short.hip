@@ -66,7 +66,7 @@ int short_tiles(cvr_ctx* c, const RayFrame& rf, float step, float et, int px_per
   const VolGeom g = geom_of(c);
   const size_t px = size_t(rf.W) * rf.H;
   const int limit = int(std::min(px / px_per_sample, size_t(32)) / 4 * 4);
-  if (rf.W < 64 || rf.H < 64 || limit < 4 || frame_hits(rf, g) != 64) return CVR_OK;
+  if (rf.W < 64 || rf.H < 64 || limit < 4 || !frame_all_hit(rf, g)) return CVR_OK;
   const size_t n = size_t((rf.W + 63) / 64) * size_t((rf.H + 63) / 64);
   if (n > c->short_cap) {
     if (!c->may_allocate) return CVR_OK;
