@@ -77,11 +77,29 @@ def stats_frame(r, wl, cam, light, out, stream):
     return st
 
 
-def gather_bytes(tech, st, r, bpv):
+def cone_reads(p, grid, levels):
+    """Trilinear reads of one sample's cones: a step lies at the level whose Gaussian matches the cone's
+    radius there, clamped to the chain, and reads that level alone where it is a whole one, two otherwise."""
+    diag = math.sqrt(sum(g * g for g in grid))
+
+    def cone(reach, half_deg):
+        q, n = (reach / p.t0) ** (1.0 / p.n_steps), 0
+        for j in range(p.n_steps):
+            tm = 0.5 * p.t0 * (q ** j + q ** (j + 1))
+            lod = math.log2(tm * math.tan(math.radians(half_deg)) / (p.r_sigma * p.sigma0))
+            n += 2 if 0.0 < lod < levels - 1 else 1
+        return n
+
+    occ = cone(p.occ_max_dist if p.occ_max_dist > 0 else 0.5 * diag, p.occ_half_deg)
+    sdw = cone(p.sdw_max_dist if p.sdw_max_dist > 0 else 0.75 * diag, p.sdw_half_deg)
+    return p.n_occ_cones * occ + sdw
+
+
+def gather_bytes(tech, st, r, bpv, grid):
     """Algorithmic bytes one frame gathers: each trilinear read counts its 8 texels (volume
     samples at the voxel size, pyramid reads as fp32 or 16-bit values); the cone tracer
-    reads 2 levels per step, the section-table renderer one level per section and
-    sub-cone, the surrogate 16 whole-level reads per shaded sample."""
+    reads one or two levels per step (cone_reads), the section-table renderer one level per
+    section and sub-cone, the surrogate 16 whole-level reads per shaded sample."""
     from cpp_volume_rendering_amd import native as N
     p = r.params()
     vol = st.samples * 8 * bpv
@@ -98,10 +116,12 @@ def gather_bytes(tech, st, r, bpv):
         return vol + st.shaded_samples * reads * 8 * b
     if tech == N.CONE_TRACE:
         b = 4 if p.density_precision == 0 else 2
-        return vol + st.shaded_samples * (p.n_occ_cones + 1) * p.n_steps * 2 * 8 * b
+        return vol + st.shaded_samples * cone_reads(p, grid, len(r.pyramid())) * 8 * b
     if tech == N.CONE_NN:
         b = 4 if p.cone.density_precision == 0 else 2
-        exact = st.fallback_samples * (p.cone.n_occ_cones + 1) * p.cone.n_steps * 2 * 8 * b
+        exact = 0
+        if st.fallback_samples:
+            exact = st.fallback_samples * cone_reads(p.cone, grid, len(r.pyramid())) * 8 * b
         return vol + st.shaded_samples * 16 * 8 * b + exact
     return vol
 
@@ -516,7 +536,7 @@ def main():
         # the march over the cache: volume taps + 8 float2 cache taps per shaded sample
         gathered = st.samples * 8 * bpv + st.shaded_samples * 8 * 8 + wl.width * wl.height * 16
     else:
-        gathered = gather_bytes(tech, st, r, bpv) + wl.width * wl.height * 16
+        gathered = gather_bytes(tech, st, r, bpv, wl.grid) + wl.width * wl.height * 16
     achieved = gathered / (ms * 1e-3) / 1e9
     config["gathered_bytes_per_frame"] = int(gathered)
     kernel = {N.RC1P: "k_rc1p", N.EBS: "k_ebs", N.DOS: "k_dos_render", N.CONE_TRACE: "k_cone_render",

@@ -75,3 +75,13 @@ def test_more_than_one_gpu_is_refused():
                            timeout=120, env={**os.environ, **env})
         assert r.returncode == 2, (r.returncode, r.stderr[-300:])
         assert "one GPU" in json.loads(r.stdout.strip().splitlines()[-1])["error"]
+
+
+def test_cone_reads_count_one_level_where_a_step_reads_one():
+    p = types.SimpleNamespace(t0=1.0, n_steps=64, occ_half_deg=30.0, sdw_half_deg=10.0, r_sigma=2.0, sigma0=1.0, occ_max_dist=0.0,
+                              sdw_max_dist=0.0, n_occ_cones=8)
+    grid = (256.0,) * 3
+    # 23 of an occlusion cone's 64 steps lie within two sigma of level 0 or past the last of 6 levels; of the
+    # shadow cone, whose radius is 2 at a distance of 11.3 and 64 past its end, the first 27
+    assert bench.cone_reads(p, grid, 6) == 8 * (64 + 41) + 64 + 37
+    assert bench.cone_reads(p, grid, 1) == 9 * 64
