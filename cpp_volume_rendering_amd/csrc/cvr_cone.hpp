@@ -191,8 +191,8 @@ std::vector<ConeLevel> cone_levels(const PyrGeom& pg);
 // step's two 32-byte blocks), so whatever is the same for all lanes is in the tables (scalar loads),
 // steps whose level is a whole one read it alone (23 of the 64 of an occlusion cone: the first, within
 // two sigma of level 0, and those past the last level), and steps before the first lane leaves the
-// box do without the border falloff, which is 1 there.  256^3 at 1024^2 68.6 -> 54.5 ms, at 512^2 18.7 -> 14.4 (vector
-// instructions issued in 82 % of the cycles, 0.85 L1 tags a cycle and CU).
+// box do without the border falloff, which is 1 there.  256^3 at 1024^2 68.6 -> 54.5 ms, at 512^2 18.7 -> 14.4 (0.95
+// vector instructions each four cycles and SIMD, 1.00 L1 tags a cycle and CU, address units 95 % busy).
 template <int F, bool kWide>
 __device__ __forceinline__ float cone_T(const void* __restrict__ pyr, const PyrGeom& pg,
                                         const ConeLevel* __restrict__ levels, const ConeSched& S, bool inside, f3 p, f3 axis) {

@@ -41,8 +41,6 @@ struct PyrKey {
            base[2] == o.base[2] && sigma_bits == o.sigma_bits && nlev == o.nlev && fmt == o.fmt;
   }
 };
-// Section table of one directional-occlusion cone: rows (interval, level, d_integral,
-// amplitude), section counts with 1/3/7 Gaussians, sub-cone axes.
 // One step of a cone march: midpoint distance, segment length, and of its pyramid level lod: the
 // weights 1 - fr and fr of the levels `level` and level + 1 (fr 0: the first alone), and the border
 // falloff's -log2(e) / (2 (2^lod)^2).
@@ -50,7 +48,7 @@ struct ConeStepF {
   float tm, dt, omf, fr, fall;
   int level, pad[2];
 };
-// A pyramid level as the cone march reads it, 48 bytes of a 64-byte row: texel coordinate per
+// A pyramid level as the cone march reads it, 40 bytes of a 64-byte row: texel coordinate per
 // world unit, last texel index per axis, bricks, byte offset of its corner blocks.
 struct ConeLevel {
   float ts[3], dmax[3];
@@ -72,6 +70,8 @@ struct DosRow {
   float track, dint, amp, fall;
   int level, pad[3];
 };
+// Section table of one directional-occlusion cone: rows (interval, level, d_integral,
+// amplitude), section counts with 1/3/7 Gaussians, sub-cone axes.
 struct DosTable {
   std::vector<float4> rows;
   int n[3] = {0, 0, 0};

@@ -1,6 +1,8 @@
 // The shaded march shared by the cone tracer, DOS, EBS, the ground truth and the surrogate:
-// a wavefront marches one ray at a time, 64 consecutive samples per step, and shades the
-// opaque samples it meets 64 at a time.
+// a wavefront marches one ray at a time, 64 consecutive samples per step (the surrogate four
+// rays and 16 samples, or a lane to each of 64 rays), and shades the opaque samples it meets
+// 64 at a time.  The plain and light-cache marches (plain_march, lane_march), whose samples
+// are shaded by one read or none, are below.
 //
 // What bounds a shaded frame is the lighting of its opaque samples (tens to thousands of
 // reads each), and a ray has from none to more than a thousand of them.  With one ray per
@@ -9,7 +11,7 @@
 // tracer), 1.0 (DOS) and 0.3 (EBS) wavefronts per SIMD on average, of 4, 2 and 1 that fit.
 // A sample's position and opacity do not depend on the lighting, so here the march runs
 // ahead of it:
-//  - lane k takes sample 64 n + k of the ray; the opacity recurrence runs in order through
+//  - lane k takes sample 64 n + k of the ray (of 64 samples a step); the opacity recurrence runs in order through
 //    the lanes (each lane from its left neighbour), so the samples taken, their opacities
 //    and the early exit are those of a one-lane march, bit for bit;
 //  - opaque samples go to a queue in LDS; whenever it holds 64, every lane shades one and
@@ -132,7 +134,7 @@ __host__ __device__ inline long long tiled_pixels(int w, int h, int tile_log2) {
 }
 
 // How a frame's rays are dealt out: `rays` per unit (a wavefront, or a workgroup whose four
-// wavefronts share them: parts 4), the tile whose pixels the units take in turn, workgroups,
+// wavefronts share them), the tile whose pixels the units take in turn, workgroups,
 // and runs of 1 << xcd_log2 workgroups per XCD (xcd_remap).  first: the launch's first workgroup of
 // them (for_launches).
 struct QueueShape {
@@ -142,7 +144,8 @@ struct QueueShape {
 };
 // Tiles of 64 x 64 pixels: a unit's rays lie 32 (rays 4) or 16 (rays 16) pixels apart, so long
 // and short ones mix, while the units that run at once stay together (256^3 cone-traced frame
-// at 512^2: 18.7 ms, 23.7 ms in 16 x 16 tiles; EBS 5.0 and 6.6 ms; DOS 4.5 and 6.0 ms).
+// at 512^2: 18.7 ms, 23.7 ms in 16 x 16 tiles; EBS 5.0 and 6.6 ms; DOS 4.5 and 6.0 ms; cone tracer and
+// DOS before cone_T and the rows of dos_cone).
 // Narrower frames take smaller tiles, of a unit's rays at least.  xcd_px: pixels an XCD takes in a row.
 inline QueueShape queue_shape(int w, int h, int rays, int parts, int xcd_px, int waves = 4) {
   const int side = w < h ? w : h;

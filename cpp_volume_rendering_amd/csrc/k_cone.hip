@@ -278,8 +278,8 @@ int launch_cone(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* o
   if (shm > 64 * 1024) { set_error("cone renderer: transfer function larger than 4096 entries"); return -4; }
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   float4* o4 = reinterpret_cast<float4*>(out);
-  // small frames: workgroups whose wavefronts share their rays (128^2 1.9 ms, 3.4 ms with rays
-  // of their own; 512^2 18.7 and 19.9; 1024^2 70.4 and 68.6)
+  // small frames: workgroups whose wavefronts share their rays (256^3 at 128^2 1.3 ms, 2.3 with rays of
+  // their own; 256^2 3.9 and 5.4; 512^2 13.7 and 14.7; 720^2 26.7 and 27.5; 1024^2 53.0 and 52.4)
   const bool shared = size_t(rf.W) * rf.H < (1 << 19);
   QueueShape shape = queue_shape(rf.W, rf.H, kRays, shared ? 4 : 1, shared ? 64 : 256);
   if ((rc = short_tiles(c, rf, step, P.et_threshold, 1024, st, &shape.short_tiles))) return rc;

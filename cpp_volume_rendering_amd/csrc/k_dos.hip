@@ -16,8 +16,8 @@
 // section on the axis, then 3 then 7 sub-cones that inherit their parent's optical
 // depth, trapezoid sums of amplitude * extinction, I = exp(-depth) averaged over the
 // sub-cones (the 7-packing weights its ring by the adjacent weight).  The march is
-// queue_march's (cvr_queue.hpp; 256^3 at 1024^2 with shadows 41.5 -> 15.6 ms, at 200 x 150
-// 7.2 -> 0.26 ms; with the rows of dos_cone 12.6 and 0.18 ms).  A section is the same for all lanes:
+// queue_march's (cvr_queue.hpp; 256^3 at 1024^2 with shadows 41.5 ms a lane per ray, 15.6 queued, 12.6
+// with the rows of dos_cone, 10.7 at three wavefronts per SIMD).  A section is the same for all lanes:
 // its row and its level's geometry come through scalar loads.
 #include "cvr_cone.hpp"
 #include "cvr_queue.hpp"
@@ -497,9 +497,9 @@ int launch_dos(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* ou
   }
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
   float4* o4 = reinterpret_cast<float4*>(out);
-  // small frames: workgroups whose wavefronts share their rays (measured with the first rows of
-  // dos_cone: 100 x 100 0.41 ms, 0.82 ms with rays of their own; 200 x 150 0.26 and 0.48; 400 x 300 2.2
-  // and 1.7; 1024^2 19.4 and 15.6)
+  // small frames: workgroups whose wavefronts share their rays (256^3 at 100^2 0.24 ms, 0.45 with rays of
+  // their own; 200 x 150 0.43 and 0.76; 256^2 0.92 and 1.07, 128^3 0.40 either way; 400 x 300 1.28 and 1.38;
+  // 512^2 3.30 and 3.02; 1024^2 12.7 and 10.7)
   const bool shared = size_t(rf.W) * rf.H < (1 << 16);
   QueueShape shape = queue_shape(rf.W, rf.H, kRays, shared ? 4 : 1, shared ? 64 : 256);
   if ((rc = short_tiles(c, rf, step, P.et_threshold, 1024, st, &shape.short_tiles))) return rc;

@@ -268,23 +268,6 @@ __device__ __forceinline__ void box_stream(const void* __restrict__ sat, const E
   }
 }
 
-// EvaluateSAT3D (:87-100) of one box.
-template <int L>
-__device__ __forceinline__ double box_sum(const void* __restrict__ sat, const EbsK& k, f3 p1, f3 p2) {
-  bool first = true;
-  double S = 0.0;
-  box_stream<L>(
-      sat, k,
-      [&](BoxC& c, float&) {
-        if (!first) return false;
-        c = box_coords(k, p1, p2);
-        first = false;
-        return true;
-      },
-      [&](double v, float) { S = v; });
-  return S;
-}
-
 // ExtinctionAmbientOcclusion (:112-146).
 template <int L>
 __device__ __forceinline__ float ebs_ao(const void* __restrict__ sat, const EbsK& k, f3 tx) {
@@ -678,8 +661,9 @@ int launch_ebs(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* ou
   int waves = 4;
   while (waves > 1 && tables + size_t(waves) * sizeof(WaveQueue<kRays>) > 160 * 1024) waves /= 2;
   const size_t shm = tables + size_t(waves) * sizeof(WaveQueue<kRays>);
-  // small frames: workgroups whose wavefronts share their rays (100 x 100 0.51 ms, 1.0 ms with
-  // rays of their own; 400 x 300, point light 3.6 and 4.3; 512^2 5.3 and 5.0; 1024^2 19.4 and 16.0)
+  // small frames: workgroups whose wavefronts share their rays (256^3 at 100^2 0.58 ms, 1.47 with rays of
+  // their own; 256^2 1.74 and 2.45; 400 x 300 2.62 and 2.46, point light 2.95 and 2.74; 512^2 6.19 and 5.29;
+  // 1024^2 23.6 and 18.9)
   const bool shared = waves == 4 && size_t(rf.W) * rf.H < 200000;
   QueueShape shape = queue_shape(rf.W, rf.H, kRays, shared ? 4 : 1, shared ? 64 : 256, waves);
   const size_t short_shm = tables + 4 * sizeof(WaveQueue<kShortRays>);

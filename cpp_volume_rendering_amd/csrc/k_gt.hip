@@ -38,8 +38,8 @@ __device__ __forceinline__ float ext_of(const float2* s_ext, int ntf, float d) {
 
 // Transmittance of one ray (ConeOcclusionEvaluationRayCasting inner loop, :125-159).  The
 // positions do not depend on the values read, so the next step's block is in flight while
-// a step is composited (with 89 VGPRs, five wavefronts per SIMD cover the rest; two or four
-// steps in flight took 105 and 138 VGPRs and were 1 to 10 % slower).
+// a step is composited (79 VGPRs for 8-bit and 83 for 16-bit volumes: six and five wavefronts
+// per SIMD cover the rest; two or four steps in flight were 1 to 10 % slower).
 template <typename T>
 __device__ __forceinline__ float gt_ray(const VolGeom& g, const float2* s_ext, int ntf, f3 p, f3 w, float dist,
                                         float gap, float rstep) {
@@ -92,7 +92,7 @@ __device__ __forceinline__ float gt_cone(const VolGeom& g, const float2* s_ext, 
 
 constexpr int kRays = 4, kShortRays = 16;
 // The march is queue_march's (cvr_queue.hpp).  128^3 at 256^2 with 16 + 4 rays per sample:
-// 313 -> 5.7 ms (one dependent read per light-ray step at one wavefront per SIMD before).
+// 293 ms a lane per ray with one dependent read per light-ray step at one wavefront per SIMD, 4.3 now.
 template <typename T, int kParts, int kRays>
 __global__ __launch_bounds__(256) void k_gt_render(RayFrame rf, VolGeom g, GtK K, const float4* __restrict__ tf,
                                                    int ntf, float step, float et, QueueShape qs, float4* __restrict__ out,
@@ -234,8 +234,8 @@ int launch_gt(cvr_ctx* c, const RayFrame& rf, const cvr_light* light, float* out
   }
   const size_t shm = size_t(c->tf_size) * sizeof(float4) + size_t(c->tf_size + 1) * sizeof(float2);
   // workgroups whose wavefronts share their rays: a batch is tens to thousands of light-ray
-  // steps (128^3 at 256^2 with 16 + 4 rays 5.7 ms, 13.7 ms with rays of their own; 256^3 at 512^2
-  // with 4 + 1 11.5 and 12.2)
+  // steps (128^3 at 256^2 with 16 + 4 rays 3.2 ms, 3.7 with rays of their own; with 4 + 1 at 100^2 0.54
+  // and 1.40, at 1024^2 24.6 and 24.5; 256^3 at 512^2 19.3 and 24.0)
   QueueShape shape = queue_shape(rf.W, rf.H, kRays, 4, 64);
   if ((rc = short_tiles(c, rf, step, P.et_threshold, 4096, st, &shape.short_tiles))) return rc;
   unsigned long long* cnt = c->collect_stats ? c->d_counters : nullptr;
