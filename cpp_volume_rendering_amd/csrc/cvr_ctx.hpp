@@ -174,7 +174,6 @@ struct cvr_ctx {
   bool lc_valid = false;
 
   int* d_short = nullptr;  // short_tiles of the frame in work
-  size_t short_cap = 0;
   bool may_allocate = true;  // false within cvr_render_noalloc
 
   // stats

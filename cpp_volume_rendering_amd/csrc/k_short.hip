@@ -59,7 +59,10 @@ __global__ __launch_bounds__(64) void k_short_tiles(RayFrame rf, VolGeom g, cons
 
 // Frames whose rays all hit the box (from inside it or close to it) are looked over: others have tiles of
 // many misses and of short and long rays beside each other.  A ray is short up to 32 samples, fewer (pixels /
-// px_per_sample) in frames whose 16 rays to a wavefront would not fill the chip.
+// px_per_sample) in frames whose 16 rays to a wavefront would not fill the chip.  The buffer holds the tiles of
+// the largest frame (2^28 pixels, either side of 64 or more and so at most doubled by its last tile: 1 MiB) from
+// the first on: one that grew would be freed under a captured frame.
+constexpr size_t kMaxTiles = size_t(1) << 18;
 int short_tiles(cvr_ctx* c, const RayFrame& rf, float step, float et, int px_per_sample, hipStream_t st,
                 const int** tiles) {
   *tiles = nullptr;
@@ -68,21 +71,17 @@ int short_tiles(cvr_ctx* c, const RayFrame& rf, float step, float et, int px_per
   const int limit = int(std::min(px / px_per_sample, size_t(32)) / 4 * 4);
   if (rf.W < 64 || rf.H < 64 || limit < 4 || !frame_all_hit(rf, g)) return CVR_OK;
   const size_t n = size_t((rf.W + 63) / 64) * size_t((rf.H + 63) / 64);
-  if (n > c->short_cap) {
+  if (!c->d_short) {
     if (!c->may_allocate) return CVR_OK;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusActive;
     if (hipStreamIsCapturing(st, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) {
       (void)hipGetLastError();
       return CVR_OK;  // nothing may be allocated now
     }
-    if (c->d_short) CVR_HIP_CHECK(hipFree(c->d_short));
-    c->d_short = nullptr;
-    c->short_cap = 0;
-    if (device_alloc(&c->d_short, n * sizeof(int)) != hipSuccess) {
+    if (device_alloc(&c->d_short, kMaxTiles * sizeof(int)) != hipSuccess) {
       (void)hipGetLastError();
       return CVR_OK;
     }
-    c->short_cap = n;
   }
   if (c->dtype == CVR_U8)
     hipLaunchKernelGGL(k_short_tiles<uint8_t>, dim3(unsigned(n)), dim3(64), 0, st, rf, g, c->d_tf_rgbt, c->tf_size, step,

@@ -448,3 +448,34 @@ def test_noalloc_of_a_closed_gate_from_inside_allocates_nothing():
     torch.cuda.synchronize()
     # a pixel's samples are summed by four wavefronts, or by one: 30 colours of at most 1, 30 x 2^-24
     assert float(ref[..., 3].max()) > 0.9 and float((got - ref).abs().max()) <= 2e-6
+
+
+def test_captured_frame_from_inside_outlives_larger_ones():
+    """A captured frame keeps the buffer in which it looks for tiles of short rays: a larger frame, drawn
+    between its replays, takes no new one."""
+    import torch
+
+    w, h = 300, 260
+    wl = W.cone_blobs(n=32, width=w, height=h, seed=3)
+    wl.alpha_iso[:, 0] = 0.9  # dense: every tile is short
+    light, fill = wl.light(), torch.empty(4 << 20, device="cuda:0")
+    r = handle(N.CONE_TRACE, wl)
+    eager, got = (torch.zeros((h, w, 4), device="cuda:0") for _ in range(2))
+    cam = W.orbit_camera(wl.grid, w, h, dist_diag=0.05)
+    r.render(cam, w, h, light=light, out=eager)
+    torch.cuda.synchronize()
+    s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        r.render(cam, w, h, light=light, out=got, stream=s.cuda_stream)
+    large = torch.zeros((4 * h, 4 * w, 4), device="cuda:0")
+    for _ in range(3):
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        r.render(W.orbit_camera(wl.grid, 4 * w, 4 * h, dist_diag=0.05), 4 * w, 4 * h, light=light, out=large)
+        torch.cuda.synchronize()
+        assert torch.cuda.mem_get_info()[0] == free
+        fill.fill_(float("nan"))
+        got.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, eager) and float(eager[..., 3].max()) > 0.9
