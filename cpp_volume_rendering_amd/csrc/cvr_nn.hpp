@@ -154,8 +154,9 @@ ConeK cone_constants(const cvr_ctx* c, const cvr_cone_params& P, const float L[3
 void light_dir(const RayFrame& rf, const cvr_light* light, float L[3]);
 
 // Rays of a wavefront's queue and samples per step of each: four rays at a time share a
-// step, so that the in-order opacity recurrence takes 16 rounds, not 64 (512^3 at 1024^2 4.74 ms,
-// 4.95 with 64 samples of one ray; from inside a 200 x 190 x 180 volume at 700 x 500 2.64 and 3.0).
+// step, so that the in-order opacity recurrence takes 16 rounds, not 64 (in turn on one box, 512^3 at
+// 1024^2 4.74 ms, 4.95 with 64 samples of one ray; from inside a 200 x 190 x 180 volume at 700 x 500 2.64
+// and 3.0; boxes differ, 5.0 to 5.3 ms on others for the first).
 constexpr int kNnRays = 16, kNnSub = 16;
 // Rays of a wavefront with a lane to each (nn_shape).
 constexpr int kLaneNnRays = 64;
